@@ -29,6 +29,9 @@ typedef int i32x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
+// four neighbours on the alignment of one element: one vector memory instruction either way
+typedef f32x4 f32x4_el __attribute__((aligned(4)));
+typedef u16x4 u16x4_el __attribute__((aligned(2)));
 
 __device__ __forceinline__ unsigned short sk_f32_to_bf16(float f) {
   unsigned u = __builtin_bit_cast(unsigned, f);
@@ -37,15 +40,15 @@ __device__ __forceinline__ unsigned short sk_f32_to_bf16(float f) {
   return (unsigned short)(u >> 16);
 }
 
-// C[m][n .. n + ncols) = cast(v): the four neighbours one lane owns; one vector store where the
-// row pitch keeps it aligned and all four columns exist.
+// C[m][n .. n + ncols) = cast(v): the four neighbours one lane owns; one vector store where all
+// four columns exist.
 template <int OUT>
 __device__ __forceinline__ void sk_store_row4(void* C, int64_t ldc, int m, int n, const f32x4& v, int ncols) {
   const int64_t idx = (int64_t)m * ldc + n;
-  const bool vec_ok = (ldc & 3) == 0 && ncols == 4;
+  const bool vec_ok = ncols == 4;
   if constexpr (OUT == ASTERGEMM_F32) {
     float* o = (float*)C + idx;
-    if (vec_ok) *(f32x4*)o = v;
+    if (vec_ok) *(f32x4_el*)o = v;
     else
       for (int r = 0; r < ncols; ++r) o[r] = v[r];
   } else {
@@ -58,7 +61,7 @@ __device__ __forceinline__ void sk_store_row4(void* C, int64_t ldc, int m, int n
       }
     }
     unsigned short* o = (unsigned short*)C + idx;
-    if (vec_ok) *(u16x4*)o = u16x4{h[0], h[1], h[2], h[3]};
+    if (vec_ok) *(u16x4_el*)o = u16x4{h[0], h[1], h[2], h[3]};
     else
       for (int r = 0; r < ncols; ++r) o[r] = h[r];
   }
@@ -697,7 +700,6 @@ __global__ __launch_bounds__(256) void skinny_splitk_reduce_kernel(const float* 
   if (scale_b) scale *= *scale_b;
   const int cg = (N + 3) >> 2;                     // groups of four columns per row
   const int64_t plane = (int64_t)M * N;
-  const bool vec = (N & 3) == 0;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < (int64_t)M * cg;
        i += (int64_t)gridDim.x * blockDim.x) {
     const int m = (int)(i / cg), n = (int)(i - (int64_t)m * cg) * 4;
@@ -710,7 +712,7 @@ __global__ __launch_bounds__(256) void skinny_splitk_reduce_kernel(const float* 
       for (int s = 0; s < 8; ++s) {
         const int sc = (s0 + s) < S ? (s0 + s) : S - 1;
         const float* q = src + sc * plane;
-        if (vec) t[s] = *(const f32x4*)q;
+        if (ncols == 4) t[s] = *(const f32x4_el*)q;
         else
           for (int r = 0; r < 4; ++r) t[s][r] = r < ncols ? q[r] : 0.f;
       }
@@ -973,7 +975,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_fp4m_kernel(const GemmArgs p)
         // sums over this K range only: [range][M][N] fp32, added up by the reduce kernel
         const int ncols = (r1 - n) < 4 ? (r1 - n) : 4;
         float* o = p.workspace + ((int64_t)ks * p.M + m) * p.N + n;
-        if ((p.N & 3) == 0 && ncols == 4) *(f32x4*)o = v;
+        if (ncols == 4) *(f32x4_el*)o = v;
         else
           for (int r = 0; r < ncols; ++r) o[r] = v[r];
       } else if (m < p.M && n < r1) {
@@ -1296,7 +1298,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_regm_kernel(const GemmArgs p)
         // partial sums of this K range: [split][M][N] fp32, finished by the reduce kernel
         const int ncols = (r1 - n) < 4 ? (r1 - n) : 4;
         float* o = p.workspace + ((int64_t)ks * p.M + m) * p.N + n;
-        if ((p.N & 3) == 0 && ncols == 4) *(f32x4*)o = v;
+        if (ncols == 4) *(f32x4_el*)o = v;
         else
           for (int r = 0; r < ncols; ++r) o[r] = v[r];
       } else if (m < p.M && n < r1) {

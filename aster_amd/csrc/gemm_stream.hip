@@ -25,11 +25,13 @@ int launch_stream(const GemmArgs& a, int grid, hipStream_t s) {
   return (int)hipGetLastError();
 }
 
-// Whole 256x256 tiles and whole 128-byte K-steps only; other shapes go to the
-// general tile kernel.
 const char* check_stream(const astergemm_config& c) {
-  // edge tiles are handled in units of 8 operand rows and 16-byte output chunks
-  if (c.M % 8 != 0 || c.N % 8 != 0 || c.M < 8 || c.N < 8) return "M and N must be multiples of 8";
+  // Edge tiles move in units of 8 operand rows and 16-byte output chunks; a unit of A across the
+  // last row is shifted up (edge_row), so M is free from one whole unit on.  The general tile
+  // kernels against these, M not a multiple of 8, back to back: bf16 333x14336x4096 71.0 -> 62.8 us,
+  // 500x4096x14336 158 -> 79, 1537x8192x8192 211 -> 173, 130x4096x4096 47 -> 21; fp8 500x4096x14336
+  // 80.6 -> 53.9, 1537x8192x8192 110 -> 87; MXFP4 333x14336x4096 48.0 -> 25.7, 1537x8192x8192 135 -> 62.
+  if (c.M < 8 || c.N < 8 || c.N % 8 != 0) return "M must be at least 8 and N a multiple of 8";
   // a K tail of 1..7 granules is multiplied after the loop; at least one whole step is needed
   if (row_bytes(c.dtype_ab, c.K) % 16 != 0) return "K must cover a whole number of 16-byte granules";
   if (row_bytes(c.dtype_ab, c.K) < kRowBytes) return "K must cover at least one 128-byte row chunk";
@@ -271,6 +273,8 @@ const char* check_stream_splitk(const astergemm_config& c) {
   if (const char* why = check_stream_whole_k(c)) return why;
   if (c.dtype_ab == ASTERGEMM_MXFP4 && c.K % 512 != 0) return "K must be a multiple of 512";
   const int64_t tiles = ((c.M + 127) / 128) * ((c.N + 127) / 128);
+  // a ragged M with a handful of tiles stays with the 64 x 64 kernels (pinned by the tests)
+  if (c.M % 8 != 0 && tiles < 8) return "split K of a ragged M needs eight output tiles";
   // shorter rows: the unsplit 64 x 64 kernels are ahead (fp8 256x4096x4096: 15.2 against 19.8 us)
   const int64_t min_steps = c.dtype_ab == ASTERGEMM_MXFP4 ? 32 : 64;
   if (row_bytes(c.dtype_ab, c.K) / kRowBytes < min_steps)
@@ -494,6 +498,7 @@ inline TailSplit tail_split_of(int64_t M, int64_t N, int cus) {
     for (int64_t t1 = cut_tiles - 1; t1 >= 1; --t1) {
       if ((t1 * other) % cus != 0) continue;
       const int64_t rest = extent - t1 * 256;
+      if (rest < 8) break;  // the 128 x 128 kernel shifts the edge by up to 8 rows (edge_row)
       const int64_t rest128 = (rest + 127) / 128 * (((along == 1 ? M : N) + 127) / 128);
       const double cost = (double)(t1 * other / cus) +
                           0.55 * (double)((rest128 + 2 * cus - 1) / (2 * cus));

@@ -108,11 +108,17 @@ __device__ __forceinline__ void gemm_stream4_body(const GemmArgs& p, int bid, in
     for (int i = 0; i < NSC; ++i) {
       const int x = wave + i * NW;
       const bool is_a = x < NSR;
-      t.sc[i] = is_a ? p.mx_a + (int64_t)t.row0 * p.mx_ld : p.mx_b + (int64_t)t.col0 * p.mx_ld;
-      // rows past the end of an edge tile re-read the operand's last row
+      // the rows the tile transfers stage (edge_row); rows past the end re-read the operand's last.
+      // A straddling group starts up to 7 rows above the tile, and lane offsets are unsigned: the
+      // base is 8 rows further up
       const int first = is_a ? t.row0 : t.col0, rows = is_a ? p.M : p.N;
+      const int base = WALK ? first : (first < 8 ? 0 : first - 8);
+      t.sc[i] = (is_a ? p.mx_a : p.mx_b) + (int64_t)base * p.mx_ld;
       int r = (x % NSR) * 64 + lane;
-      if constexpr (!WALK) r = first + r < rows ? r : rows - 1 - first;  // the walk has whole tiles
+      if constexpr (!WALK) {                       // the walk has whole tiles
+        r = edge_row(first + r, rows);
+        r = (r < rows ? r : rows - 1) - base;
+      }
       t.sc_off[i] = (unsigned)(r * p.mx_ld);
     }
   };

@@ -44,18 +44,20 @@ __device__ __forceinline__ void static_for(Fn&& f) {
   }
 }
 
-// ---- epilogue shared by the stream kernels -------------------------------------------------
-// Scale, bias and cast in registers, then turn each 16-row slab of the wave tile
-// around in LDS so that every lane stores 16 contiguous bytes and every store
-// instruction covers whole 128-byte lines of C.  (A lane owns 4 consecutive
-// columns of one row per MFMA tile; stored directly that is 8 bytes per lane and
-// 32-byte pieces per row, which costs ~7 % of the kernel.)  The lane id is
-// recomputed here, opaque to the optimiser, so that no lane-derived value has to
-// stay in a VGPR across the K loop.
+// Edge of an operand whose height is not a multiple of 8 (M: a prompt has as many rows as it has
+// tokens): the 8-row group that straddles the end is staged shifted up, as the operand's last 8
+// rows, so that a transfer stays one scalar base and one lane offset.  edge_row says which operand
+// row tile row r (counted from the top of the operand) then holds; rows the shift repeats are
+// multiplied twice, with the same operands in the same order, and stored twice with the same bits.
+// Rows of groups past the end map to >= rows.  Heights of 8 and more; a multiple of 8 maps every
+// row to itself.  What such an M cost before on the general tile kernels: see check_stream.
+__device__ __forceinline__ int edge_row(int r, int rows) {
+  return r >= (rows & ~7) ? r - (-rows & 7) : r;
+}
+
 // Scalar bases of a wave's LH row groups (8 rows each, 8 * NW rows apart) for the global->LDS
-// transfers.  Operand heights are multiples of 8, so a group lies either inside the matrix or
-// wholly past its end; the latter re-read the last 8 rows (their products land in output rows
-// or columns the epilogue does not store).
+// transfers.  A group past the end, or across it (see edge_row), reads the operand's last 8 rows
+// (the products of the former land in output rows or columns the epilogue does not store).
 template <class Plan>
 __device__ __forceinline__ void group_bases(const uint8_t* mat, int64_t ld_bytes, int tile_row0, int wave,
                                             int rows, const uint8_t* (&out)[Plan::LH]) {
@@ -101,7 +103,7 @@ __device__ __forceinline__ void stream_k_tail(const GemmArgs& p,
       }
 #pragma unroll
       for (int m = 0; m < TM; ++m) {
-        int r = row0 + (wm * TM + m) * 16 + li;
+        int r = edge_row(row0 + (wm * TM + m) * 16 + li, p.M);
         r = r < p.M ? r : p.M - 1;
         fat[m][g] = live ? *(const i32x4*)(p.A + (int64_t)r * p.lda_bytes + koff + gran * 16) : zero;
       }
@@ -113,6 +115,14 @@ __device__ __forceinline__ void stream_k_tail(const GemmArgs& p,
   }
 }
 
+// ---- epilogue shared by the stream kernels -------------------------------------------------
+// Scale, bias and cast in registers, then turn each 16-row slab of the wave tile
+// around in LDS so that every lane stores 16 contiguous bytes and every store
+// instruction covers whole 128-byte lines of C.  (A lane owns 4 consecutive
+// columns of one row per MFMA tile; stored directly that is 8 bytes per lane and
+// 32-byte pieces per row, which costs ~7 % of the kernel.)  The lane id is
+// recomputed here, opaque to the optimiser, so that no lane-derived value has to
+// stay in a VGPR across the K loop.
 template <int OUT, int BM, int BN, int WM, int WN>
 __device__ __forceinline__ void stream_epilogue(const GemmArgs& p,
                                                 f32x4 (&acc)[BM / WM / 16][BN / WN / 16],
@@ -174,10 +184,10 @@ __device__ __forceinline__ void stream_epilogue(const GemmArgs& p,
       const int c = t * 64 + lane_e;
       const int r = c / (ROWB / 16), cc = c % (ROWB / 16);
       const i32x4 d = *(const i32x4*)(slab + r * PITCH + cc * 16);
-      uint8_t* out = (uint8_t*)p.C + ((int64_t)(wrow0 + m * 16 + r) * p.ldc + wcol0) * OB + cc * 16;
+      const int row = edge_row(wrow0 + m * 16 + r, p.M);
+      uint8_t* out = (uint8_t*)p.C + ((int64_t)row * p.ldc + wcol0) * OB + cc * 16;
       // edge tiles: N is a multiple of 8, so a 16-byte chunk is inside a row or past its end
-      if (wrow0 + m * 16 + r < p.M && wcol0 + cc * (16 / OB) < p.N)
-        __builtin_nontemporal_store(d, (i32x4*)out);
+      if (row < p.M && wcol0 + cc * (16 / OB) < p.N) __builtin_nontemporal_store(d, (i32x4*)out);
     }
   }
 }

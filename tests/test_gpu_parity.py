@@ -637,6 +637,36 @@ def test_stream_kernels_edge_tiles(gpu, M, N, K, dtype_ab, dtype_c):
     assert np.isnan(pad).all() if dtype_c == "f32" else (pad == 0x7FC1).all()
 
 
+@pytest.mark.parametrize("M", [9, 15, 129, 257, 263, 333])
+@pytest.mark.parametrize("tile", [128, 256])
+@pytest.mark.parametrize("dtype_ab,dtype_c", [("bf16", "bf16"), ("f16", "f32"), ("fp8_e4m3", "bf16"),
+                                              ("mxfp4", "f32")])
+def test_stream_kernels_take_any_row_count(gpu, M, tile, dtype_ab, dtype_c):
+    """M that is no multiple of 8: the last row group is staged shifted up and its rows stored
+    where they belong; nothing behind row M is written.  With and without a K tail."""
+    N = 264
+    for K in ((512,) if dtype_ab == "mxfp4" else (512, 528)):
+        a, b, extra = operands(M, N, K, dtype_ab, seed=57, b_std=0.05)
+        bias = np.random.default_rng(58).standard_normal(N).astype(np.float32)
+        out, name = run_gemm(a, b, M, N, K, dtype_ab, dtype_c, bias=bias, ldc=N + 8,
+                             family=_capi.KERNEL_TILE, wg_tile=(tile, tile), **extra)
+        assert name.startswith("stream_")
+        if dtype_ab == "fp8_e4m3":
+            want = G.gemm_fp8(a, b, extra["scale_a"], extra["scale_b"], out_dtype=_DT[dtype_c], bias=bias)
+        elif dtype_ab == "mxfp4":
+            want = G.gemm(a, b, _DT[dtype_ab], _DT[dtype_c], bias=bias, **extra)
+        else:
+            want = G.gemm(a, b, _DT[dtype_ab], _DT[dtype_c], bias=bias)
+        if M * N >= 4096:
+            check(out, want, dtype_c, N, bar=REL_L2_BAR if dtype_c != "f32" else 1e-5)
+        else:
+            got, ref = G.output_to_f32(out[:, :N], _DT[dtype_c]), G.output_to_f32(want, _DT[dtype_c])
+            # one bf16 rounding step, 2^-8 of the value, and the fp32 sums, far below 1e-4 of the largest
+            assert np.all(np.abs(got - ref) <= 2.0 ** -7 * np.abs(ref) + 1e-4 * np.abs(ref).max())
+        pad = out[:, N:]
+        assert np.isnan(pad).all() if dtype_c == "f32" else (pad == 0x7FC1).all()
+
+
 @pytest.mark.parametrize("M,N,K", [(256, 256, 1024), (264, 520, 1088), (384, 1000, 1152), (256, 384, 1216),
                                    (512, 264, 1408), (256, 256, 1472), (264, 256, 1536), (256, 512, 1600),
                                    (1000, 1024, 1664), (256, 256, 1728), (504, 776, 1800), (256, 128, 2120),
