@@ -61,179 +61,410 @@ __device__ __forceinline__ unsigned e2m1_rne_sat(float x) {
 __global__ void zero_u32_kernel(unsigned* p) { *p = 0u; }
 
 // Source element types: fp32, or the 16-bit types a GEMM of this library writes (both widen
-// to fp32 exactly, so quantising them equals quantising the widened values).
+// to fp32 exactly, so quantising them equals quantising the widened values).  The kernels move the
+// source in 16-byte groups of kPer elements, one group per lane and load.
+typedef int i32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+typedef u32x2 u32x2_a4 __attribute__((aligned(4)));  // fp8 destinations are 4-byte aligned
+typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+
 template <int SRC>
 struct Src {
   static constexpr int kBytes = SRC == ASTERGEMM_F32 ? 4 : 2;
+  static constexpr int kPer = 16 / kBytes;
 };
 template <int SRC>
 __device__ __forceinline__ float widen(unsigned short h) {
   if constexpr (SRC == ASTERGEMM_BF16) return __uint_as_float((unsigned)h << 16);
   else return (float)__builtin_bit_cast(_Float16, h);
 }
-// four consecutive elements (16 or 8 bytes, naturally aligned) as fp32
-template <int SRC>
-__device__ __forceinline__ f32x4 load4(const void* base, int64_t group) {
-  if constexpr (SRC == ASTERGEMM_F32) {
-    return __builtin_nontemporal_load((const f32x4*)base + group);
-  } else {
-    typedef unsigned short u16x4 __attribute__((ext_vector_type(4)));
-    const u16x4 h = __builtin_nontemporal_load((const u16x4*)base + group);
-    return f32x4{widen<SRC>(h[0]), widen<SRC>(h[1]), widen<SRC>(h[2]), widen<SRC>(h[3])};
-  }
-}
 template <int SRC>
 __device__ __forceinline__ float load1(const void* base, int64_t i) {
   if constexpr (SRC == ASTERGEMM_F32) return ((const float*)base)[i];
   else return widen<SRC>(((const unsigned short*)base)[i]);
 }
+// element e of a group as fp32
+template <int SRC>
+__device__ __forceinline__ float element(const i32x4& raw, int e) {
+  if constexpr (SRC == ASTERGEMM_F32) return __builtin_bit_cast(f32x4, raw)[e];
+  else return widen<SRC>(__builtin_bit_cast(u16x8, raw)[e]);
+}
 
 // max over |x| as unsigned bits (non-negative floats order like their bit patterns; NaNs
-// compare above infinity and so survive the maximum, as they do in numpy's max).  Four
-// independent loads per trip; one atomic per workgroup.
+// compare above infinity and so survive the maximum, as they do in numpy's max), in the bits of
+// the source type: two elements per packed 16-bit maximum.
 template <int SRC>
-__global__ __launch_bounds__(256) void absmax_kernel(const void* __restrict__ src, int64_t n,
-                                                     unsigned* __restrict__ out) {
-  __shared__ unsigned wave_max[4];
+struct AbsMax {
+  u16x2 m2 = {0, 0};
   unsigned m = 0;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  const int64_t n4 = n >> 2;
-  int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-  auto fold = [&](const f32x4 v) {
+  __device__ __forceinline__ void fold(const i32x4& raw) {
+    if constexpr (SRC == ASTERGEMM_F32) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const unsigned b = __float_as_uint(v[e]) & 0x7FFFFFFFu;
-      m = b > m ? b : m;
+      for (int e = 0; e < 4; ++e) {
+        const unsigned b = (unsigned)raw[e] & 0x7FFFFFFFu;
+        m = b > m ? b : m;
+      }
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        m2 = __builtin_elementwise_max(m2, __builtin_bit_cast(u16x2, (unsigned)raw[e] & 0x7FFF7FFFu));
     }
-  };
-  for (; i + 3 * stride < n4; i += 4 * stride) {
-    const f32x4 v0 = load4<SRC>(src, i);
-    const f32x4 v1 = load4<SRC>(src, i + stride);
-    const f32x4 v2 = load4<SRC>(src, i + 2 * stride);
-    const f32x4 v3 = load4<SRC>(src, i + 3 * stride);
-    fold(v0), fold(v1), fold(v2), fold(v3);
   }
-  for (; i < n4; i += stride) fold(load4<SRC>(src, i));
-  for (int64_t j = (n4 << 2) + blockIdx.x * (int64_t)blockDim.x + threadIdx.x; j < n; j += stride) {
-    const unsigned b = __float_as_uint(load1<SRC>(src, j)) & 0x7FFFFFFFu;
-    m = b > m ? b : m;
+  // fp32 bits of the maximum (widening keeps the order)
+  __device__ __forceinline__ unsigned bits() const {
+    if constexpr (SRC == ASTERGEMM_F32) return m;
+    else return __float_as_uint(widen<SRC>(m2[0] > m2[1] ? m2[0] : m2[1]));
   }
+};
+
+__device__ __forceinline__ unsigned wave_max64(unsigned m) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     const unsigned o = (unsigned)__shfl_xor((int)m, off, 64);
     m = o > m ? o : m;
   }
+  return m;
+}
+// maximum over a workgroup of NW waves, known to every thread
+template <int NW>
+__device__ __forceinline__ unsigned block_max(unsigned m) {
+  __shared__ unsigned wave_max[NW];
+  m = wave_max64(m);
   if ((threadIdx.x & 63) == 0) wave_max[threadIdx.x >> 6] = m;
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int w = 1; w < 4; ++w) m = wave_max[w] > m ? wave_max[w] : m;
-    if (m != 0) atomicMax(out, m);
-  }
-}
-
-// scale = absmax / 448 in fp32, 1.0 when absmax is zero (or NaN)
-__global__ void fp8_scale_kernel(const unsigned* amax_bits, float* scale) {
-  const float a = __builtin_bit_cast(float, *amax_bits);
-  *scale = (a > 0.0f) ? a / 448.0f : 1.0f;
-}
-
-template <int SRC>
-__global__ __launch_bounds__(256) void quantize_fp8_kernel(const void* __restrict__ src, int64_t n,
-                                                           const float* __restrict__ scale,
-                                                           uint8_t* __restrict__ dst) {
-  const float s = *scale;
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  const int64_t n4 = n >> 2;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n4; i += stride) {
-    const f32x4 v = load4<SRC>(src, i);
-    unsigned w = 0;
+  m = wave_max[0];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) w |= e4m3_rne_sat(v[e] / s) << (8 * e);
-    ((unsigned*)dst)[i] = w;
-  }
-  for (int64_t i = (n4 << 2) + blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n; i += stride)
-    dst[i] = (uint8_t)e4m3_rne_sat(load1<SRC>(src, i) / s);
+  for (int w = 1; w < NW; ++w) m = wave_max[w] > m ? wave_max[w] : m;
+  return m;
 }
 
-// Eight lanes per 32-element block: a lane loads 16 bytes (4 elements), so one wave-wide load
-// covers 1 KB of contiguous source (8 blocks); four such loads are in flight per trip.  The
-// block maximum goes round the 8 lanes with three exchanges; every lane then encodes its 4
-// elements (2 bytes out) and lane 0 of the group writes the scale byte.  CONTIG: ld == K, so
-// block t sits at element 32 t and no (row, column) split is needed.
-// LANES: the scale byte of block c of row r goes where astergemm_shuffle_scales_e8m0_lanes128 puts
-// it (groups of 128 rows, one KiB per group and 8-block step).
-template <int SRC, bool CONTIG, bool LANES = false>
+// This thread's share of max |src[0..n)|: groups first, first + stride, ..., U loads in flight,
+// and the elements behind the last whole group.
+template <int SRC, int U>
+__device__ __forceinline__ unsigned absmax_share(const void* __restrict__ src, int64_t n, int64_t first,
+                                                 int64_t stride) {
+  constexpr int NE = Src<SRC>::kPer;
+  const i32x4* g = (const i32x4*)src;
+  const int64_t ng = n / NE;
+  AbsMax<SRC> am;
+  int64_t i = first;
+  for (; i + (U - 1) * stride < ng; i += U * stride) {
+    i32x4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = g[i + u * stride];
+#pragma unroll
+    for (int u = 0; u < U; ++u) am.fold(v[u]);
+  }
+  for (; i < ng; i += stride) am.fold(g[i]);
+  unsigned m = am.bits();
+  for (int64_t j = ng * NE + first; j < n; j += stride) {
+    const unsigned b = __float_as_uint(load1<SRC>(src, j)) & 0x7FFFFFFFu;
+    m = b > m ? b : m;
+  }
+  return m;
+}
+
+// One atomic per workgroup; the atomics of all workgroups go to one address, which the memory
+// system takes one at a time (2048 workgroups: 20 us of a 30 us call; 256: 3 us).
+template <int SRC>
+__global__ __launch_bounds__(1024) void absmax_kernel(const void* __restrict__ src, int64_t n,
+                                                      unsigned* __restrict__ out) {
+  const unsigned m = block_max<16>(absmax_share<SRC, 4>(
+      src, n, blockIdx.x * (int64_t)1024 + threadIdx.x, (int64_t)gridDim.x * 1024));
+  if (threadIdx.x == 0 && m != 0) atomicMax(out, m);
+}
+
+// ---- e4m3 with one scale per tensor ----------------------------------------------------------
+//
+// scale = absmax / 448 in fp32, 1.0 when absmax is zero (or NaN).  For a finite tensor whose
+// scale is in [2^-60, 2^60] every quotient is at most 448 in magnitude and the converter
+// instruction (nearest even, like the integer form above) needs no saturation; the quotient is the
+// correctly rounded one by two residual corrections with the correctly rounded reciprocal
+// (Markstein's theorem: q' = RN(q + r * RN(1/s)), r = RN(x - q s), is RN(x / s) when q is within
+// one unit in the last place, which the first correction ensures).  x below 2^-11 s encodes to
+// zero whatever its last bits are; anything above keeps r far from the subnormal range.
+struct Fp8Scale {
+  float s, rcp;
+  bool plain;
+  __device__ __forceinline__ explicit Fp8Scale(unsigned amax_bits) {
+    const float a = __uint_as_float(amax_bits);
+    s = (a > 0.0f) ? a / 448.0f : 1.0f;
+    rcp = 1.0f / s;
+    plain = amax_bits < 0x7F800000u && s >= 0x1p-60f && s <= 0x1p60f;
+  }
+  __device__ __forceinline__ float quotient(float x) const {
+    float q = x * rcp;
+    q = fmaf(fmaf(-q, s, x), rcp, q);
+    return copysignf(fmaf(fmaf(-q, s, x), rcp, q), x);  // a correction by +0 turns -0 into +0
+  }
+  __device__ __forceinline__ unsigned code(float x) const { return e4m3_rne_sat(x / s); }
+};
+
+// the codes of four elements, first one in the low byte
+template <int SRC>
+__device__ __forceinline__ unsigned fp8_codes4(const i32x4& raw, int e0, const Fp8Scale& sc) {
+  if (sc.plain) {
+    int w = 0;
+    w = __builtin_amdgcn_cvt_pk_fp8_f32(sc.quotient(element<SRC>(raw, e0)),
+                                        sc.quotient(element<SRC>(raw, e0 + 1)), w, false);
+    w = __builtin_amdgcn_cvt_pk_fp8_f32(sc.quotient(element<SRC>(raw, e0 + 2)),
+                                        sc.quotient(element<SRC>(raw, e0 + 3)), w, true);
+    return (unsigned)w;
+  }
+  unsigned w = 0;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) w |= sc.code(element<SRC>(raw, e0 + e)) << (8 * e);
+  return w;
+}
+// group i of the source to its place in dst
+template <int SRC>
+__device__ __forceinline__ void fp8_store_group(const i32x4& raw, int64_t i, const Fp8Scale& sc,
+                                                uint8_t* __restrict__ dst) {
+  if constexpr (SRC == ASTERGEMM_F32) {
+    ((unsigned*)dst)[i] = fp8_codes4<SRC>(raw, 0, sc);
+  } else {
+    ((u32x2_a4*)dst)[i] = u32x2{fp8_codes4<SRC>(raw, 0, sc), fp8_codes4<SRC>(raw, 4, sc)};
+  }
+}
+
+// Small tensors (the activations of a decode step) in one launch: every workgroup reads the whole
+// source for the maximum -- from L2, all of it in flight at once -- and encodes its own part.
+template <int SRC>
+__global__ __launch_bounds__(1024) void quantize_fp8_small_kernel(const void* __restrict__ src, int n,
+                                                                  uint8_t* __restrict__ dst,
+                                                                  float* __restrict__ scale) {
+  constexpr int NE = Src<SRC>::kPer;
+  const int ng = n / NE;
+  const int i = blockIdx.x * 1024 + threadIdx.x;
+  i32x4 mine = {0, 0, 0, 0};
+  if (i < ng) mine = ((const i32x4*)src)[i];
+  const Fp8Scale sc(block_max<16>(absmax_share<SRC, 8>(src, n, threadIdx.x, 1024)));
+  if (i == 0) *scale = sc.s;
+  if (i < ng) fp8_store_group<SRC>(mine, i, sc, dst);
+  if (blockIdx.x == 0)
+    for (int j = ng * NE + threadIdx.x; j < n; j += 1024) dst[j] = (uint8_t)sc.code(load1<SRC>(src, j));
+}
+
+// Larger ones in two launches instead of the four it takes with the absmax accumulated in *scale
+// (clear, absmax, scale, encode): bf16 500 x 14336 37.4 -> 13.4 us, 4096 x 4096 47.8 -> 19.4, 8192 x
+// 8192 97.4 -> 62.4 (the source is read twice, the second time from the last-level cache; 40 us at
+// the rate of a large copy).  The first leaves one maximum per workgroup in the first 4 * gridDim.x bytes
+// of dst (written over by the codes in the end) and clears *scale, which the second uses as a
+// counter.
+template <int SRC>
+__global__ __launch_bounds__(256) void fp8_absmax_kernel(const void* __restrict__ src, int64_t n,
+                                                         unsigned* __restrict__ partial,
+                                                         unsigned* __restrict__ counter) {
+  const unsigned m = block_max<4>(absmax_share<SRC, 8>(
+      src, n, blockIdx.x * (int64_t)256 + threadIdx.x, (int64_t)gridDim.x * 256));
+  if (threadIdx.x == 0) {
+    partial[blockIdx.x] = m;
+    if (blockIdx.x == 0) *counter = 0u;
+  }
+}
+
+// Every workgroup takes the maximum of the `np` partial ones, counts itself in and encodes its
+// part of the tensor behind the first 4 * np elements; the last one to have counted itself in --
+// everybody has read the partial maxima by then -- encodes those and stores the scale over the
+// counter.  Nobody waits for anybody.  256 workgroups at most: the counter's atomics are taken
+// one at a time (2048 workgroups of 256 threads: 34.7 us instead of 13.4 on 500 x 14336).
+template <int SRC>
+__global__ __launch_bounds__(1024) void quantize_fp8_kernel(const void* __restrict__ src, int64_t n, int np,
+                                                           uint8_t* __restrict__ dst,
+                                                           float* __restrict__ scale) {
+  constexpr int NE = Src<SRC>::kPer, U = 4;
+  __shared__ unsigned arrived;
+  const i32x4* g = (const i32x4*)src;
+  const int64_t ng = n / NE, head = (int64_t)np * 4 / NE;
+  const int64_t stride = (int64_t)gridDim.x * 1024;
+  int64_t i = head + blockIdx.x * (int64_t)1024 + threadIdx.x;
+  i32x4 v[U];
+  auto fetch = [&]() {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (i + u * stride < ng) v[u] = __builtin_nontemporal_load(g + i + u * stride);
+  };
+  fetch();  // in flight while the maximum is found
+  unsigned m = 0;
+  for (int j = threadIdx.x; j < np; j += 1024) {
+    const unsigned o = ((const unsigned*)dst)[j];
+    m = o > m ? o : m;
+  }
+  const Fp8Scale sc(block_max<16>(m));  // its barrier: the workgroup's reads of dst are over
+  if (threadIdx.x == 0) arrived = atomicAdd((unsigned*)scale, 1u);
+  while (i < ng) {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (i + u * stride < ng) fp8_store_group<SRC>(v[u], i + u * stride, sc, dst);
+    i += U * stride;
+    fetch();
+  }
+  for (int64_t j = ng * NE + blockIdx.x * (int64_t)1024 + threadIdx.x; j < n; j += stride)
+    dst[j] = (uint8_t)sc.code(load1<SRC>(src, j));
+  __syncthreads();
+  if (arrived != gridDim.x - 1) return;
+  for (int64_t j = threadIdx.x; j < head; j += 1024) fp8_store_group<SRC>(g[j], j, sc, dst);
+  if (threadIdx.x == 0) *scale = sc.s;
+}
+
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void static_for_pairs(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for_pairs<N, I + 1>(f);
+  }
+}
+
+// ---- MXFP4 -----------------------------------------------------------------------------------
+//
+// A 32-element block is kPB neighbouring lanes with one 16-byte group each: the block maximum goes
+// round them by lane permutes inside the row, every lane encodes its group (the converter
+// instruction divides by the power of two, rounds to nearest even and saturates) and the block's
+// scale byte is known to all of them.
+template <int SRC>
+struct Mx4Group {
+  static constexpr int kPB = 32 / Src<SRC>::kPer;  // lanes per block: 4, or 8 for fp32
+  unsigned w;       // the group's nibbles: 4 bytes, or 2 for fp32
+  uint8_t scale;    // the block's e8m0 byte
+};
+template <int SRC>
+__device__ __forceinline__ Mx4Group<SRC> mx4_encode(const i32x4& raw) {
+  constexpr int NE = Src<SRC>::kPer;
+  AbsMax<SRC> am;
+  am.fold(raw);
+  unsigned mb = am.bits();
+  auto with = [&](unsigned o) { mb = o > mb ? o : mb; };
+  with((unsigned)__builtin_amdgcn_mov_dpp((int)mb, 0xB1, 0xF, 0xF, true));   // lane ^ 1
+  with((unsigned)__builtin_amdgcn_mov_dpp((int)mb, 0x4E, 0xF, 0xF, true));   // lane ^ 2
+  if constexpr (Mx4Group<SRC>::kPB == 8)
+    with((unsigned)__builtin_amdgcn_mov_dpp((int)mb, 0x141, 0xF, 0xF, true));  // 7 - lane of eight
+  // shared exponent = floor(log2(absmax)) - 2; an all-zero block gets exponent 0, a block
+  // holding NaN / inf gets scale byte 0xFF and its elements are scaled by 2^2
+  const bool bad = mb >= 0x7F800000u;
+  int fl;
+  if (mb == 0 || bad) fl = bad ? 0 : 2;                    // -> shared 0 (zero) / -2 (bad)
+  else if (mb >= 0x00800000u) fl = (int)(mb >> 23) - 127;  // normal
+  else fl = -149 + (31 - __builtin_clz(mb));               // fp32 subnormal
+  int sbyte = (fl - 2) + 127;
+  sbyte = sbyte < 0 ? 0 : (sbyte > 254 ? 254 : sbyte);
+  Mx4Group<SRC> r;
+  r.scale = bad ? (uint8_t)0xFF : (uint8_t)sbyte;
+  r.w = 0;
+  if (!bad && sbyte >= 1) {
+    const float s = __uint_as_float((unsigned)sbyte << 23);
+    static_for_pairs<NE / 2>([&](auto P) {
+      constexpr int e = decltype(P)::value;
+      r.w = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(r.w, element<SRC>(raw, 2 * e),
+                                                     element<SRC>(raw, 2 * e + 1), s, e);
+    });
+  } else {
+    const int shift = -(sbyte - 127);
+#pragma unroll
+    for (int e = 0; e < NE; ++e) {
+      // exact scaling by a power of two in two steps (|shift| can exceed the fp32 exponent
+      // range of a single factor)
+      const float q = ldexpf(ldexpf(element<SRC>(raw, e), shift / 2), shift - shift / 2);
+      r.w |= e2m1_rne_sat(q) << (4 * e);
+    }
+  }
+  return r;
+}
+template <int SRC>
+__device__ __forceinline__ void mx4_store(uint8_t* packed, int64_t group, unsigned w) {
+  if constexpr (SRC == ASTERGEMM_F32) *(unsigned short*)(packed + group * 2) = (unsigned short)w;
+  else *(unsigned*)(packed + group * 4) = w;
+}
+
+// Scale bytes row-major: the source as one run of blocks, four 16-byte groups in flight per lane
+// (bf16, 8-byte loads and integer encoding -> this: 4096 x 4096 15.0 -> 9.3 us, 8192 x 8192 50.3 ->
+// 33.0, which is the rate of a large copy).  CONTIG:
+// ld == K, so block t sits at element 32 t and no (row, column) split is needed.
+template <int SRC, bool CONTIG>
 __global__ __launch_bounds__(256) void quantize_mxfp4_kernel(const void* __restrict__ src,
                                                              int64_t nblocks, unsigned bpr,
                                                              int64_t ld,
                                                              uint8_t* __restrict__ packed,
                                                              uint8_t* __restrict__ scales) {
-  constexpr int U = 4;
-  const int lane = threadIdx.x & 63, g = lane >> 3, l8 = lane & 7;
-  const int64_t nwaves = (int64_t)gridDim.x * 4;
-  for (int64_t base = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * (8 * U); base < nblocks;
-       base += nwaves * (8 * U)) {
-    f32x4 v[U];
-    int64_t t[U];
-    bool live[U];
+  constexpr int U = 4, PB = Mx4Group<SRC>::kPB;
+  const int64_t ngroups = nblocks * PB;
+  const int64_t step = (int64_t)gridDim.x * 256;
+  for (int64_t base = blockIdx.x * (int64_t)256 + threadIdx.x; base < ngroups; base += U * step) {
+    i32x4 v[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      t[u] = base + u * 8 + g;
-      live[u] = t[u] < nblocks;
-      if (!live[u]) t[u] = nblocks - 1;  // stay inside the source; nothing is stored
+      // a lane past the end repeats its first group: the lanes of a block stay together (blocks
+      // are whole and both bounds are multiples of kPB), nothing of it is stored
+      const int64_t t = base + u * step < ngroups ? base + u * step : base;
       int64_t off;
       if (CONTIG) {
-        off = t[u] * 32;
+        off = t * Src<SRC>::kPer;
       } else {
-        const unsigned r = (unsigned)t[u] / bpr, c = (unsigned)t[u] - r * bpr;
-        off = (int64_t)r * ld + (int64_t)c * 32;
+        const unsigned blk = (unsigned)(t / PB), r = blk / bpr, c = blk - r * bpr;
+        off = (int64_t)r * ld + (int64_t)c * 32 + (t % PB) * Src<SRC>::kPer;
       }
-      v[u] = load4<SRC>((const uint8_t*)src + off * Src<SRC>::kBytes, l8);
+      v[u] = __builtin_nontemporal_load((const i32x4*)((const uint8_t*)src + off * Src<SRC>::kBytes));
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      unsigned mb = 0;
+      const int64_t t = base + u * step;
+      const Mx4Group<SRC> q = mx4_encode<SRC>(v[u]);
+      if (t < ngroups) {
+        mx4_store<SRC>(packed, t, q.w);
+        if (t % PB == 0) scales[t / PB] = q.scale;
+      }
+    }
+  }
+}
+
+// Scale bytes in lane order (astergemm_shuffle_scales_e8m0_lanes128): a workgroup takes 128 rows x
+// 256 elements, whose scale bytes are one KiB of the plane, collects them in LDS and stores them
+// as whole lines; written where they fall they are single bytes 256 apart (bf16 4096 x 4096 17.6 ->
+// 10.9 us, 8192 x 8192 60.5 -> 32.0).
+template <int SRC>
+__global__ __launch_bounds__(256) void quantize_mxfp4_lanes_kernel(const void* __restrict__ src, int rows,
+                                                                   unsigned bpr, int64_t ld,
+                                                                   uint8_t* __restrict__ packed,
+                                                                   uint8_t* __restrict__ scales) {
+  constexpr int NE = Src<SRC>::kPer, PB = Mx4Group<SRC>::kPB;
+  constexpr int LPR = 256 / NE;                  // lanes per row of the tile
+  constexpr int RPI = 256 / LPR;                 // rows per trip of the workgroup
+  constexpr int U = 8;
+  __shared__ __attribute__((aligned(16))) uint8_t sc[1024];
+  const unsigned steps = bpr >> 3;               // 256-element steps of a row
+  const unsigned grp = blockIdx.x / steps, st = blockIdx.x - grp * steps;
+  const int row0 = (int)grp * 128;
+  const int live = rows - row0 < 128 ? rows - row0 : 128;
+  const int lr = threadIdx.x / LPR, lc = threadIdx.x % LPR;
+  const int c = lc / PB;                         // block 0..7 of the step
+  for (int r0 = 0; r0 < live; r0 += U * RPI) {
+    i32x4 v[U];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const unsigned b = __float_as_uint(v[u][e]) & 0x7FFFFFFFu;
-        mb = b > mb ? b : mb;
-      }
+    for (int u = 0; u < U; ++u) {
+      int r = r0 + u * RPI + lr;
+      r = r < live ? r : live - 1;               // nothing of it is stored
+      const int64_t off = (int64_t)(row0 + r) * ld + (int64_t)st * 256 + lc * NE;
+      v[u] = __builtin_nontemporal_load((const i32x4*)((const uint8_t*)src + off * Src<SRC>::kBytes));
+    }
 #pragma unroll
-      for (int off = 1; off < 8; off <<= 1) {
-        const unsigned o = (unsigned)__shfl_xor((int)mb, off, 64);
-        mb = o > mb ? o : mb;
+    for (int u = 0; u < U; ++u) {
+      const int r = r0 + u * RPI + lr;
+      const Mx4Group<SRC> q = mx4_encode<SRC>(v[u]);
+      if (r < live) {
+        mx4_store<SRC>(packed, ((int64_t)(row0 + r) * bpr + st * 8) * PB + lc, q.w);
+        // (q, i, tile, h): block c = 4 h + q, row 16 tile + i
+        if (lc % PB == 0) sc[((c & 3) * 16 + (r & 15)) * 16 + (r >> 4) * 2 + (c >> 2)] = q.scale;
       }
-      // shared exponent = floor(log2(absmax)) - 2; an all-zero block gets exponent 0, a block
-      // holding NaN / inf gets scale byte 0xFF and its elements are scaled by 2^2
-      const bool bad = mb >= 0x7F800000u;
-      int fl;
-      if (mb == 0 || bad) fl = bad ? 0 : 2;                    // -> shared 0 (zero) / -2 (bad)
-      else if (mb >= 0x00800000u) fl = (int)(mb >> 23) - 127;  // normal
-      else fl = -149 + (31 - __builtin_clz(mb));               // fp32 subnormal
-      int sbyte = (fl - 2) + 127;
-      sbyte = sbyte < 0 ? 0 : (sbyte > 254 ? 254 : sbyte);
-      const int shift = -(sbyte - 127);
-      unsigned w = 0;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        // exact scaling by a power of two in two steps (|shift| can exceed the fp32 exponent
-        // range of a single factor)
-        const float q = ldexpf(ldexpf(v[u][e], shift / 2), shift - shift / 2);
-        w |= e2m1_rne_sat(q) << (4 * e);
-      }
-      if (live[u]) {
-        *(unsigned short*)(packed + t[u] * 16 + l8 * 2) = (unsigned short)w;
-        if (l8 == 0) {
-          int64_t so = t[u];
-          if constexpr (LANES) {
-            const unsigned r = (unsigned)t[u] / bpr, c = (unsigned)t[u] - r * bpr;
-            // (group, step, q, i, tile, h): block c = 8 step + 4 h + q, row r = 128 group + 16 tile + i
-            so = ((int64_t)(r >> 7) * (bpr >> 3) + (c >> 3)) * 1024 +
-                 (((c & 3) * 16 + (r & 15)) * 16 + ((r >> 4) & 7) * 2 + ((c >> 2) & 1));
-          }
-          scales[so] = bad ? (uint8_t)0xFF : (uint8_t)sbyte;
-        }
-      }
+    }
+  }
+  __syncthreads();
+  uint8_t* dst = scales + (int64_t)blockIdx.x * 1024 + threadIdx.x * 16;
+  if (threadIdx.x < 64) {
+    if (live == 128) {
+      *(i32x4*)dst = *(const i32x4*)(sc + threadIdx.x * 16);
+    } else {                                     // bytes of rows past the end stay as they are
+      for (int b = 0; b < 16; ++b)
+        if ((b >> 1) * 16 + (int)(threadIdx.x & 15) < live) dst[b] = sc[threadIdx.x * 16 + b];
     }
   }
 }
@@ -243,6 +474,10 @@ int blocks_for(int64_t work_items) {
   const int64_t b = (work_items + 255) / 256, cap = 256 * 8;
   return (int)(b < 1 ? 1 : (b > cap ? cap : b));
 }
+
+// Up to this many elements the one-launch form quantises to e4m3 (bf16 source, back to back, one
+// launch / two: 65536 elements 4.1 / 6.8 us, 77056 4.1 / 6.8, 229376 7.5 / 6.8, 262144 7.4 / 7.0).
+constexpr int64_t kFp8OneLaunch = 131072;
 
 }  // namespace
 }  // namespace astergemm
@@ -274,8 +509,10 @@ extern "C" int astergemm_absmax(const void* dSrc, int src_dtype, int64_t n, floa
   hipLaunchKernelGGL(zero_u32_kernel, dim3(1), dim3(1), 0, s, (unsigned*)dAbsmax);
   if (n > 0)
     with_src(src_dtype, [&](auto T) {
-      hipLaunchKernelGGL(absmax_kernel<decltype(T)::value>, dim3(blocks_for(n / 4 + 1)), dim3(256),
-                         0, s, dSrc, n, (unsigned*)dAbsmax);
+      constexpr int SRC = decltype(T)::value;
+      const int64_t b = (n / Src<SRC>::kPer + 4 * 1024) / (4 * 1024);
+      hipLaunchKernelGGL(absmax_kernel<SRC>, dim3((unsigned)(b < 256 ? b : 256)), dim3(1024), 0, s, dSrc,
+                         n, (unsigned*)dAbsmax);
     });
   AG_HIP(hipGetLastError());
   return 0;
@@ -290,14 +527,25 @@ extern "C" int astergemm_quantize_fp8_tensor(const void* dSrc, int src_dtype, in
     return ASTERGEMM_EINVAL;
   }
   hipStream_t s = (hipStream_t)stream;
-  // dScale doubles as the absmax accumulator: bits of a non-negative float
-  if (int rc = astergemm_absmax(dSrc, src_dtype, n, dScale, stream)) return rc;
-  hipLaunchKernelGGL(fp8_scale_kernel, dim3(1), dim3(1), 0, s, (const unsigned*)dScale, dScale);
-  if (n > 0)
-    with_src(src_dtype, [&](auto T) {
-      hipLaunchKernelGGL(quantize_fp8_kernel<decltype(T)::value>, dim3(blocks_for(n / 4 + 1)),
-                         dim3(256), 0, s, dSrc, n, dScale, dDst);
-    });
+  (void)hipGetLastError();
+  with_src(src_dtype, [&](auto T) {
+    constexpr int SRC = decltype(T)::value, NE = Src<SRC>::kPer;
+    const int64_t ng = n / NE;
+    if (n <= kFp8OneLaunch) {
+      const unsigned b = (unsigned)((ng + 1023) / 1024);
+      hipLaunchKernelGGL(quantize_fp8_small_kernel<SRC>, dim3(b ? b : 1), dim3(1024), 0, s, dSrc, (int)n,
+                         dDst, dScale);
+      return;
+    }
+    // one partial maximum per workgroup, a multiple of 32 of them (128 bytes of dst), 1024 at most
+    int64_t np = ((ng + 4 * 256 - 1) / (4 * 256) + 31) & ~(int64_t)31;
+    if (np > 1024) np = 1024;
+    hipLaunchKernelGGL(fp8_absmax_kernel<SRC>, dim3((unsigned)np), dim3(256), 0, s, dSrc, n,
+                       (unsigned*)dDst, (unsigned*)dScale);
+    const int64_t b = (ng + 1023) / 1024;
+    hipLaunchKernelGGL(quantize_fp8_kernel<SRC>, dim3((unsigned)(b < 256 ? b : 256)), dim3(1024), 0, s,
+                       dSrc, n, (int)np, dDst, dScale);
+  });
   AG_HIP(hipGetLastError());
   return 0;
 }
@@ -322,21 +570,23 @@ extern "C" int astergemm_quantize_mxfp4_ex(const void* dSrc, int src_dtype, int6
     set_error("astergemm_quantize_mxfp4: more than 2^31 blocks");
     return ASTERGEMM_EINVAL;
   }
-  const dim3 grid(blocks_for(nblocks * 2));  // a workgroup takes 128 blocks per trip
   (void)hipGetLastError();
   with_src(src_dtype, [&](auto T) {
     constexpr int SRC = decltype(T)::value;
-    auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, grid, dim3(256), 0, (hipStream_t)stream, dSrc, nblocks,
-                         (unsigned)(K / 32), ld_src, dPacked, dScales);
-    };
+    const unsigned bpr = (unsigned)(K / 32);
+    hipStream_t st = (hipStream_t)stream;
     if (lanes) {
-      if (ld_src == K) go(quantize_mxfp4_kernel<SRC, true, true>);
-      else go(quantize_mxfp4_kernel<SRC, false, true>);
-    } else {
-      if (ld_src == K) go(quantize_mxfp4_kernel<SRC, true, false>);
-      else go(quantize_mxfp4_kernel<SRC, false, false>);
+      const unsigned grid = (unsigned)((rows + 127) / 128 * (K / 256));
+      hipLaunchKernelGGL(quantize_mxfp4_lanes_kernel<SRC>, dim3(grid), dim3(256), 0, st, dSrc, (int)rows, bpr,
+                         ld_src, dPacked, dScales);
+      return;
     }
+    const dim3 grid(blocks_for((nblocks * Mx4Group<SRC>::kPB + 3) / 4));  // four groups per thread
+    auto go = [&](auto kern) {
+      hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, dSrc, nblocks, bpr, ld_src, dPacked, dScales);
+    };
+    if (ld_src == K) go(quantize_mxfp4_kernel<SRC, true>);
+    else go(quantize_mxfp4_kernel<SRC, false>);
   });
   AG_HIP(hipGetLastError());
   return 0;

@@ -307,3 +307,54 @@ def test_preshuffle_on_the_device_writes_the_bytes_of_the_host_functions(gpu, dt
                             d_mx_src=d_mx.ptr_value, d_mx_dst=d_mo.ptr_value)
     for bf in (d_b, d_o, d_mx, d_mo):
         bf.free()
+
+
+@pytest.mark.parametrize("n", [7, 8, 9, 8191, 131072, 131073, 131080, 300007])
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+def test_fp8_quantiser_one_and_two_launch_forms(n, dtype):
+    """Both sides of the one-launch limit, whole and broken 16-byte groups, every source type, with
+    signed zeros and the maximum in the last element; nothing behind the n codes is written."""
+    rng = np.random.default_rng(n)
+    x = rng.standard_normal(n).astype(np.float32)
+    x[n // 3] = -0.0
+    x[-1] = -9.5
+    src = x if dtype == "f32" else x.astype(np.float16) if dtype == "f16" else (x.view(np.uint32) >> 16).astype(np.uint16)
+    wide = (src.astype(np.uint32) << 16).view(np.float32) if dtype == "bf16" else src.astype(np.float32)
+    a, q, sc = GpuBuffer(src.nbytes + 16), GpuBuffer(n + 64), GpuBuffer(4)
+    a.copy_from_host(src)
+    q.copy_from_host(np.full(n + 64, 0xAB, np.uint8))
+    print(f"quantize_fp8_tensor {dtype} n={n}", flush=True)
+    Q.quantize_fp8_tensor_device(a.ptr_value, n, q.ptr_value, sc.ptr_value, src_dtype=dtype)
+    got, s = np.empty(n + 64, np.uint8), np.empty(1, np.float32)
+    q.copy_to_host(got)
+    sc.copy_to_host(s)
+    qo, so = F.quantize_fp8_tensor(wide)
+    assert s[0].tobytes() == np.float32(so).tobytes()
+    assert np.array_equal(got[:n], qo) and (got[n:] == 0xAB).all()
+
+
+@pytest.mark.parametrize("rows", [1, 15, 127, 128, 129, 300])
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+def test_mxfp4_quantiser_lane_order_edges(rows, dtype):
+    """Row counts round the 128-row groups of the lane order: the plane equals the shuffled
+    row-major one, bytes of rows past the end stay as they are, the nibbles are the same."""
+    from aster_amd.kittens_helpers import shuffle_scales_e8m0_lanes128
+    K = 512
+    x = np.random.default_rng(rows).standard_normal((rows, K)).astype(np.float32)
+    src = x if dtype == "f32" else x.astype(np.float16) if dtype == "f16" else (x.view(np.uint32) >> 16).astype(np.uint16)
+    wide = (src.astype(np.uint32) << 16).view(np.float32) if dtype == "bf16" else src.astype(np.float32)
+    padded = (rows + 127) // 128 * 128
+    a, p, sc = GpuBuffer(src.nbytes), GpuBuffer(rows * K // 2), GpuBuffer(padded * K // 32)
+    a.copy_from_host(src)
+    sc.copy_from_host(np.full(padded * K // 32, 0xAB, np.uint8))
+    print(f"quantize_mxfp4 lanes128 {dtype} rows={rows}", flush=True)
+    Q.quantize_mxfp4_device(a.ptr_value, rows, K, p.ptr_value, sc.ptr_value, src_dtype=dtype,
+                            scales_layout="lanes128")
+    got_p, got_s = np.empty((rows, K // 2), np.uint8), np.empty(padded * K // 32, np.uint8)
+    p.copy_to_host(got_p)
+    sc.copy_to_host(got_s)
+    po, so = F.quantize_mxfp4(wide)
+    plane = np.full((padded, K // 32), 0xAB, np.uint8)
+    plane[:rows] = so
+    assert np.array_equal(got_p, po)
+    assert np.array_equal(got_s, np.asarray(shuffle_scales_e8m0_lanes128(plane)).reshape(-1))
