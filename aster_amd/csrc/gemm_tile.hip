@@ -6,10 +6,14 @@ namespace astergemm {
 namespace {
 
 // ---- host side: variant table ------------------------------------------------
-template <int DT, int OUT, int BM, int BN, int WM, int WN>
+constexpr int tile_lds_bytes(int dt, int bm, int bn, int stages) {
+  return stages * (bm + bn) * (kRowBytes + (dt == ASTERGEMM_MXFP4 ? 8 : 0));
+}
+
+template <int DT, int OUT, int BM, int BN, int WM, int WN, int S>
 int launch_tile(const GemmArgs& a, int grid, hipStream_t s) {
-  constexpr int lds = 2 * (BM + BN) * kRowBytes;
-  auto k = gemm_tile_kernel<DT, OUT, BM, BN, WM, WN>;
+  constexpr int lds = tile_lds_bytes(DT, BM, BN, S);
+  auto k = gemm_tile_kernel<DT, OUT, BM, BN, WM, WN, S>;
   static std::atomic<uint64_t> attr_devs{0};
   if (int e = lds_attr_once(attr_devs, (const void*)k, lds)) return e;
   AG_LAUNCH_KERNEL(k, dim3(grid), dim3(WM * WN * 64), lds, s, a);
@@ -26,27 +30,28 @@ const char* check_tile(const astergemm_config& c) {
   return nullptr;
 }
 
-#define AG_TILE(name, DT, OUT, BM, BN, WM, WN)                                   \
+#define AG_TILE1(name, DT, OUT, BM, BN, WM, WN, S)                               \
   Variant {                                                                      \
-    name, ASTERGEMM_KERNEL_TILE, DT, OUT, BM, BN, kRowBytes, WM, WN, 2, 1,       \
-        2 * (BM + BN) * kRowBytes,                                               \
-        (const void*)gemm_tile_kernel<DT, OUT, BM, BN, WM, WN>,                  \
-        launch_tile<DT, OUT, BM, BN, WM, WN>, check_tile                         \
+    name, ASTERGEMM_KERNEL_TILE, DT, OUT, BM, BN, kRowBytes, WM, WN, S, 1,       \
+        tile_lds_bytes(DT, BM, BN, S),                                           \
+        (const void*)gemm_tile_kernel<DT, OUT, BM, BN, WM, WN, S>,               \
+        launch_tile<DT, OUT, BM, BN, WM, WN, S>, check_tile                      \
   }
+#define AG_TILE(name, DT, BM, BN, WM, WN, S)                                     \
+  AG_TILE1(name "_bf16", DT, ASTERGEMM_BF16, BM, BN, WM, WN, S),                 \
+      AG_TILE1(name "_f32", DT, ASTERGEMM_F32, BM, BN, WM, WN, S),               \
+      AG_TILE1(name "_f16", DT, ASTERGEMM_F16, BM, BN, WM, WN, S)
 
-#define AG_TILE_SET(prefix, DT)                                                        \
-  AG_TILE(prefix "_256x256_w2x4_bf16", DT, ASTERGEMM_BF16, 256, 256, 2, 4),            \
-      AG_TILE(prefix "_256x256_w2x4_f32", DT, ASTERGEMM_F32, 256, 256, 2, 4),          \
-      AG_TILE(prefix "_256x256_w2x4_f16", DT, ASTERGEMM_F16, 256, 256, 2, 4),          \
-      AG_TILE(prefix "_128x128_w2x2_bf16", DT, ASTERGEMM_BF16, 128, 128, 2, 2),        \
-      AG_TILE(prefix "_128x128_w2x2_f32", DT, ASTERGEMM_F32, 128, 128, 2, 2),          \
-      AG_TILE(prefix "_128x128_w2x2_f16", DT, ASTERGEMM_F16, 128, 128, 2, 2),          \
-      AG_TILE(prefix "_128x64_w2x2_bf16", DT, ASTERGEMM_BF16, 128, 64, 2, 2),          \
-      AG_TILE(prefix "_128x64_w2x2_f32", DT, ASTERGEMM_F32, 128, 64, 2, 2),            \
-      AG_TILE(prefix "_128x64_w2x2_f16", DT, ASTERGEMM_F16, 128, 64, 2, 2),            \
-      AG_TILE(prefix "_64x64_w2x2_bf16", DT, ASTERGEMM_BF16, 64, 64, 2, 2),            \
-      AG_TILE(prefix "_64x64_w2x2_f32", DT, ASTERGEMM_F32, 64, 64, 2, 2),              \
-      AG_TILE(prefix "_64x64_w2x2_f16", DT, ASTERGEMM_F16, 64, 64, 2, 2)
+// Stages of LDS (the last number), measured back to back, S = 2 (every K-step waits for its own
+// transfers) / 3 / 4 / 5: 64 x 64 bf16 777x1001x1032 12.4 / 8.1 / 8.1 / 8.3 us, 130x4096x4096 47 / 25.5 /
+// 19.0 / 17.8, MXFP4 300x4096x11008 45 / 32.3 / 32.7 / 41.8 (five stages: one workgroup per CU);
+// 128 x 64 fp8 300x4096x11008 66 / 40.5 / 40.2 / 40.9 (six); 128 x 128 bf16 130x4096x4096 56 / 40.2 / 40.4 / 40.8.
+// 256 x 256 has room for two.
+#define AG_TILE_SET(prefix, DT)                              \
+  AG_TILE(prefix "_256x256_w2x4", DT, 256, 256, 2, 4, 2),    \
+      AG_TILE(prefix "_128x128_w2x2", DT, 128, 128, 2, 2, 4), \
+      AG_TILE(prefix "_128x64_w2x2", DT, 128, 64, 2, 2, 3),  \
+      AG_TILE(prefix "_64x64_w2x2", DT, 64, 64, 2, 2, 4)
 
 const Variant kTileVariants[] = {
     AG_TILE_SET("tile_bf16", ASTERGEMM_BF16),

@@ -21,6 +21,8 @@
 // (srcA = B rows, srcB = A rows) so each lane owns 4 consecutive columns of one
 // C row and the epilogue stores 8/16-byte vectors.
 #pragma once
+#include <type_traits>
+
 #include "astergemm_internal.h"
 
 namespace astergemm {
@@ -131,42 +133,66 @@ __device__ __forceinline__ f32x4 mfma_step(const i32x4* a, const i32x4* b, f32x4
   }
 }
 
+template <int I, int N, class Fn>
+__device__ __forceinline__ void static_for_stages(Fn&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for_stages<I + 1, N>(f);
+  }
+}
+
+// C[row][col .. col + ncols) = cast(v): one vector store where all four columns exist (the vector
+// memory path takes any element alignment, so an odd row pitch costs nothing extra).
 template <int OUT>
-__device__ __forceinline__ void store4(void* C, int64_t idx, f32x4 v, bool vec_ok,
-                                       int ncols) {
+__device__ __forceinline__ void store4(void* C, int64_t idx, f32x4 v, int ncols) {
+  typedef f32x4 f32x4_el __attribute__((aligned(4)));
+  typedef u16x4 u16x4_el __attribute__((aligned(2)));
   if constexpr (OUT == ASTERGEMM_F32) {
     float* p = (float*)C + idx;
-    if (vec_ok && ncols == 4) {
-      *(f32x4*)p = v;
+    if (ncols == 4) {
+      *(f32x4_el*)p = v;
     } else {
       for (int r = 0; r < ncols; ++r) p[r] = v[r];
     }
   } else {
-    const u16x4 hv4 = cast4_16<OUT>(v);
-    const unsigned short h[4] = {hv4.x, hv4.y, hv4.z, hv4.w};
+    const u16x4 h = cast4_16<OUT>(v);
     unsigned short* p = (unsigned short*)C + idx;
-    if (vec_ok && ncols == 4) {
-      u16x4 hv = {h[0], h[1], h[2], h[3]};
-      *(u16x4*)p = hv;
+    if (ncols == 4) {
+      *(u16x4_el*)p = h;
     } else {
       for (int r = 0; r < ncols; ++r) p[r] = h[r];
     }
   }
 }
 
-template <int DT, int OUT, int BM, int BN, int WM, int WN>
+// K loop: LDS is a ring of S stages (A and B rows of one K-step, MXFP4: and their scale bytes).
+// While K-step k is multiplied, the transfers of k + 1 .. k + S - 1 are in flight: with the two
+// stages this kernel had before, every K-step waited for its own transfers, about 0.7 us of memory
+// latency per 128 bytes of row, whatever the tile.  A trip starts with the wait for stage k (the
+// younger ones stay outstanding), one barrier -- stage k is complete for everybody and everybody
+// has stage k - 1 in registers -- and the transfers of k + S - 1 into the slot of k - 1.  Transfers
+// are inline assembly, so that the compiler does not wait for them on its own; nothing else that
+// counts in vmcnt is issued inside the loop.
+template <int DT, int OUT, int BM, int BN, int WM, int WN, int S>
 __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p) {
   constexpr int NW = WM * WN;
   constexpr int TM = BM / WM / 16;  // 16-row MFMA tiles per wave along M
   constexpr int TN = BN / WN / 16;
-  constexpr int STAGE_A = BM * kRowBytes;
-  constexpr int STAGE = (BM + BN) * kRowBytes;
+  constexpr bool FP4 = DT == ASTERGEMM_MXFP4;
+  constexpr int SCALES = (BM + BN) * kRowBytes;  // offset of the scale bytes in a stage (MXFP4)
+  constexpr int STAGE = SCALES + (FP4 ? (BM + BN) * 8 : 0);
   constexpr int LA = BM / 8 / NW;  // 1 KiB (8-row) global->LDS transfers per wave
   constexpr int LB = BN / 8 / NW;
+  // scale transfers: 4 bytes per lane, 32 rows each, round robin over the waves
+  constexpr int NSX = (BM + BN) / 32;
+  constexpr int LS = FP4 ? (NSX + NW - 1) / NW : 0;
+  constexpr int L = LA + LB + LS;
   constexpr int KSUB = Enc<DT>::kSub;
   constexpr int KGRAN = Enc<DT>::kGran;
   static_assert(BM % (8 * NW) == 0 && BN % (8 * NW) == 0, "tile rows per wave");
   static_assert((8 * NW) % 16 == 0, "swizzle phase must not depend on the transfer index");
+  static_assert(S >= 2 && (S - 2) * L <= 63, "the counted wait fits the vmcnt field");
+  static_assert(BM % 32 == 0 && BN % 32 == 0, "scale transfers cover 32 rows");
 
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
 
@@ -194,59 +220,105 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p) {
 #pragma unroll
     for (int j = 0; j < LA; ++j) {
       const int r = j * 8 * NW + wave * 8 + lrow;
-      const int g = slot ^ ((r >> 1) & 7);
       const int rr = (row0 + r < p.M) ? r : (p.M - 1 - row0);
-      a_off[j] = (unsigned)(rr * (int)p.lda_bytes + g * 16);
+      a_off[j] = (unsigned)(rr * (int)p.lda_bytes + g_lane * 16);
     }
 #pragma unroll
     for (int j = 0; j < LB; ++j) {
       const int r = j * 8 * NW + wave * 8 + lrow;
-      const int g = slot ^ ((r >> 1) & 7);
       const int rr = (col0 + r < p.N) ? r : (p.N - 1 - col0);
-      b_off[j] = (unsigned)(rr * (int)p.ldb_bytes + g * 16);
+      b_off[j] = (unsigned)(rr * (int)p.ldb_bytes + g_lane * 16);
     }
   }
+  // MX scales: 8 bytes per row and K-step at [row][8], A rows first
+  const uint8_t* s_base[LS ? LS : 1];
+  unsigned s_off[LS ? LS : 1];
+  unsigned s_dst[LS ? LS : 1];
+  if constexpr (FP4) {
+#pragma unroll
+    for (int j = 0; j < LS; ++j) {
+      int x = wave + j * NW;
+      x = x < NSX ? x : NSX - 1;  // a surplus transfer repeats the last one: the same bytes
+      const bool is_a = x < BM / 32;
+      const int first = is_a ? row0 : col0, rows = is_a ? p.M : p.N;
+      int r = (is_a ? x : x - BM / 32) * 32 + (lane >> 1);
+      r = (first + r < rows) ? r : (rows - 1 - first);
+      s_base[j] = (is_a ? p.mx_a : p.mx_b) + (int64_t)first * p.mx_ld;
+      s_off[j] = (unsigned)(r * p.mx_ld + (lane & 1) * 4);
+      s_dst[j] = (unsigned)(SCALES + x * 256);
+    }
+  }
+  auto m0_of = [&](const uint8_t* dst) { return (unsigned)(size_t)AG_LDS(dst); };
+  // 64 lanes x 16 bytes from (scalar base + lane offset) to LDS at M0 + lane * 16
+  auto g2s = [&](const uint8_t* base, unsigned voff, const uint8_t* dst) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(m0_of(dst)), "v"(voff), "s"(base)
+                 : "memory", "m0");
+  };
+  auto g2s_lane = [&](const uint8_t* src, const uint8_t* dst) {  // the same from an address per lane
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off"
+                 :
+                 : "s"(m0_of(dst)), "v"(src)
+                 : "memory", "m0");
+  };
+  auto g2s_dword = [&](const uint8_t* base, unsigned voff, const uint8_t* dst) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2"
+                 :
+                 : "s"(m0_of(dst)), "v"(voff), "s"(base)
+                 : "memory", "m0");
+  };
+  auto issue = [&](int kt, int slot) {
+    const uint8_t* ga = a_base + (int64_t)kt * kRowBytes;
+    const uint8_t* gb = b_base + (int64_t)kt * kRowBytes;
+    const uint8_t* la = lds + slot * STAGE + wave * 8 * kRowBytes;
+    const uint8_t* lb = la + BM * kRowBytes;
+    if (p.tail_granules != 0 && kt == p.ksteps - 1) {
+      // Last K-step of a row that does not fill 128 bytes: granules past the end of
+      // the row are fetched from a block of zeros instead, so they add nothing.
+      const bool live = g_lane < p.tail_granules;
+#pragma unroll
+      for (int j = 0; j < LA; ++j) g2s_lane(live ? ga + a_off[j] : g_zero16, la + j * 8 * NW * kRowBytes);
+#pragma unroll
+      for (int j = 0; j < LB; ++j) g2s_lane(live ? gb + b_off[j] : g_zero16, lb + j * 8 * NW * kRowBytes);
+    } else {
+#pragma unroll
+      for (int j = 0; j < LA; ++j) g2s(ga, a_off[j], la + j * 8 * NW * kRowBytes);
+#pragma unroll
+      for (int j = 0; j < LB; ++j) g2s(gb, b_off[j], lb + j * 8 * NW * kRowBytes);
+    }
+    if constexpr (FP4) {
+#pragma unroll
+      for (int j = 0; j < LS; ++j) g2s_dword(s_base[j] + kt * 8, s_off[j], lds + slot * STAGE + s_dst[j]);
+    }
+  };
 
-  auto issue_loads = [&](int kt, int stage) {
-    const uint8_t* ga = a_base + (int64_t)kt * kRowBytes;
-    const uint8_t* gb = b_base + (int64_t)kt * kRowBytes;
-    uint8_t* la = lds + stage * STAGE + wave * 8 * kRowBytes;
-    uint8_t* lb = la + STAGE_A;
+  // ---- what the epilogue needs from memory, requested ahead of everything else ---------------
+  const int li = lane & 15, lq = lane >> 4;
+  constexpr bool EARLY = TM * TN <= 16;  // the big tiles have no registers to spare for it
+  float scale = 1.0f;
+  f32x4 bias_v[EARLY ? TN : 1];
+  auto load_bias = [&](int n) {
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (p.bias) {
 #pragma unroll
-    for (int j = 0; j < LA; ++j)
-      __builtin_amdgcn_global_load_lds(AG_GLOBAL(ga + a_off[j]),
-                                       AG_LDS(la + j * 8 * NW * kRowBytes), 16, 0, 0);
-#pragma unroll
-    for (int j = 0; j < LB; ++j)
-      __builtin_amdgcn_global_load_lds(AG_GLOBAL(gb + b_off[j]),
-                                       AG_LDS(lb + j * 8 * NW * kRowBytes), 16, 0, 0);
+      for (int e = 0; e < 4; ++e) {
+        const int col = col0 + (wn * TN + n) * 16 + 4 * lq + e;
+        v[e] = p.bias[col < p.N ? col : p.N - 1];
+      }
+    }
+    return v;
   };
-  // Last K-step of a row that does not fill 128 bytes: granules past the end of
-  // the row are fetched from a block of zeros instead, so they add nothing.
-  auto issue_tail_loads = [&](int kt, int stage) {
-    const uint8_t* ga = a_base + (int64_t)kt * kRowBytes;
-    const uint8_t* gb = b_base + (int64_t)kt * kRowBytes;
-    uint8_t* la = lds + stage * STAGE + wave * 8 * kRowBytes;
-    uint8_t* lb = la + STAGE_A;
-    const bool live = g_lane < p.tail_granules;
+  if constexpr (EARLY) {
 #pragma unroll
-    for (int j = 0; j < LA; ++j)
-      __builtin_amdgcn_global_load_lds(AG_GLOBAL(live ? ga + a_off[j] : g_zero16),
-                                       AG_LDS(la + j * 8 * NW * kRowBytes), 16, 0, 0);
-#pragma unroll
-    for (int j = 0; j < LB; ++j)
-      __builtin_amdgcn_global_load_lds(AG_GLOBAL(live ? gb + b_off[j] : g_zero16),
-                                       AG_LDS(lb + j * 8 * NW * kRowBytes), 16, 0, 0);
-  };
-  auto stage_step = [&](int kt, int stage) {
-    if (p.tail_granules != 0 && kt == p.ksteps - 1) issue_tail_loads(kt, stage);
-    else issue_loads(kt, stage);
-  };
+    for (int n = 0; n < TN; ++n) bias_v[n] = load_bias(n);
+  }
+  if (p.scale_a) scale *= *p.scale_a;
+  if (p.scale_b) scale *= *p.scale_b;
 
   // ---- LDS -> fragment addressing ------------------------------------------
   // Lane (li = lane%16, lq = lane/16) owns row li of a 16-row tile and, for
   // k-substep s, granule s*4+lq (16-bit, fp4) or granules 2*lq, 2*lq+1 (fp8).
-  const int li = lane & 15, lq = lane >> 4;
   unsigned rd_off[KSUB][KGRAN];
 #pragma unroll
   for (int s = 0; s < KSUB; ++s)
@@ -256,26 +328,9 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p) {
       rd_off[s][h] = (unsigned)(li * kRowBytes + ((g ^ (li >> 1)) << 4));
     }
   const unsigned a_rd = (unsigned)(wm * TM * 16 * kRowBytes);
-  const unsigned b_rd = (unsigned)(STAGE_A + wn * TN * 16 * kRowBytes);
-
-  // MX scale rows (fp4 only): lane reads the 8 e8m0 bytes of its row for this
-  // K-step and shifts its own byte down.
-  const uint8_t* mxa_row[DT == ASTERGEMM_MXFP4 ? TM : 1];
-  const uint8_t* mxb_row[DT == ASTERGEMM_MXFP4 ? TN : 1];
-  if constexpr (DT == ASTERGEMM_MXFP4) {
-#pragma unroll
-    for (int m = 0; m < TM; ++m) {
-      int r = row0 + wm * TM * 16 + m * 16 + li;
-      r = r < p.M ? r : p.M - 1;
-      mxa_row[m] = p.mx_a + (int64_t)r * p.mx_ld;
-    }
-#pragma unroll
-    for (int n = 0; n < TN; ++n) {
-      int r = col0 + wn * TN * 16 + n * 16 + li;
-      r = r < p.N ? r : p.N - 1;
-      mxb_row[n] = p.mx_b + (int64_t)r * p.mx_ld;
-    }
-  }
+  const unsigned b_rd = (unsigned)((BM + wn * TN * 16) * kRowBytes);
+  const unsigned sa_rd = (unsigned)(SCALES + (wm * TM * 16 + li) * 8);
+  const unsigned sb_rd = (unsigned)(SCALES + (BM + wn * TN * 16 + li) * 8);
 
   f32x4 acc[TM][TN];
 #pragma unroll
@@ -283,93 +338,93 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p) {
 #pragma unroll
     for (int n = 0; n < TN; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-  // MX scales of a K-step are fetched one step ahead and ahead of that step's tile
-  // transfers in issue order, so that waiting for them (loads return in order) neither
-  // exposes their latency nor drains the transfers of the next stage.
-  i32x2 sa[DT == ASTERGEMM_MXFP4 ? TM : 1], sb[DT == ASTERGEMM_MXFP4 ? TN : 1];
-  i32x2 sa_nx[DT == ASTERGEMM_MXFP4 ? TM : 1], sb_nx[DT == ASTERGEMM_MXFP4 ? TN : 1];
-  auto load_scales = [&](int kt) {
-    if constexpr (DT == ASTERGEMM_MXFP4) {
+  const int nk = p.ksteps;
 #pragma unroll
-      for (int m = 0; m < TM; ++m) sa_nx[m] = *(const i32x2*)(mxa_row[m] + kt * 8);
-#pragma unroll
-      for (int n = 0; n < TN; ++n) sb_nx[n] = *(const i32x2*)(mxb_row[n] + kt * 8);
-    }
-  };
-  load_scales(0);
-  stage_step(0, 0);
+  for (int k = 0; k < S - 1; ++k)
+    if (k < nk) issue(k, k);
 
-  for (int kt = 0; kt < p.ksteps; ++kt) {
-    // All of this wave's transfers for step kt have landed; after the barrier
-    // everybody's have, and everybody is done reading the other stage.
-    __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 15));
-    __syncthreads();
-    if constexpr (DT == ASTERGEMM_MXFP4) {
+  int slot = 0, slot_ld = S - 1;  // stage k is in slot k mod S; the next transfers go to slot_ld
+  auto trip = [&](int kt) {
+    // behind the barrier: stage kt complete, stage kt - 1 in everybody's registers
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (kt + S - 1 < nk) issue(kt + S - 1, slot_ld);
+    const uint8_t* st = lds + slot * STAGE;
+    i32x2 sa[FP4 ? TM : 1], sb[FP4 ? TN : 1];
+    if constexpr (FP4) {
 #pragma unroll
-      for (int m = 0; m < TM; ++m) sa[m] = sa_nx[m];
+      for (int m = 0; m < TM; ++m) sa[m] = *(const i32x2*)(st + sa_rd + m * 128);
 #pragma unroll
-      for (int n = 0; n < TN; ++n) sb[n] = sb_nx[n];
+      for (int n = 0; n < TN; ++n) sb[n] = *(const i32x2*)(st + sb_rd + n * 128);
     }
-    if (kt + 1 < p.ksteps) {
-      load_scales(kt + 1);
-      stage_step(kt + 1, (kt + 1) & 1);
-    }
-
-    const uint8_t* st = lds + (kt & 1) * STAGE;
-#pragma unroll
-    for (int s = 0; s < KSUB; ++s) {
-      i32x4 af[TM][KGRAN], bf[TN][KGRAN];
+    i32x4 af[KSUB][TM][KGRAN], bf[KSUB][TN][KGRAN];
+    auto read_frags = [&](int s) {
 #pragma unroll
       for (int m = 0; m < TM; ++m)
 #pragma unroll
         for (int h = 0; h < KGRAN; ++h)
-          af[m][h] = *(const i32x4*)(st + a_rd + m * 16 * kRowBytes + rd_off[s][h]);
+          af[s][m][h] = *(const i32x4*)(st + a_rd + m * 16 * kRowBytes + rd_off[s][h]);
 #pragma unroll
       for (int n = 0; n < TN; ++n)
 #pragma unroll
         for (int h = 0; h < KGRAN; ++h)
-          bf[n][h] = *(const i32x4*)(st + b_rd + n * 16 * kRowBytes + rd_off[s][h]);
+          bf[s][n][h] = *(const i32x4*)(st + b_rd + n * 16 * kRowBytes + rd_off[s][h]);
+    };
+#pragma unroll
+    for (int s = 0; s < KSUB; ++s) {
+      read_frags(s);
 #pragma unroll
       for (int m = 0; m < TM; ++m)
 #pragma unroll
         for (int n = 0; n < TN; ++n) {
           int xa = 0, xb = 0;
-          if constexpr (DT == ASTERGEMM_MXFP4) {
+          if constexpr (FP4) {
             xa = (int)((unsigned)(s ? sa[m].y : sa[m].x) >> (8 * lq));
             xb = (int)((unsigned)(s ? sb[n].y : sb[n].x) >> (8 * lq));
           }
-          acc[m][n] = mfma_step<DT>(bf[n], af[m], acc[m][n], xb, xa);
+          acc[m][n] = mfma_step<DT>(bf[s][n], af[s][m], acc[m][n], xb, xa);
         }
     }
+    slot = slot == S - 1 ? 0 : slot + 1;
+    slot_ld = slot_ld == S - 1 ? 0 : slot_ld + 1;
+  };
+  int kt = 0;
+  for (; kt + S - 2 < nk; ++kt) {  // S - 2 younger stages have been requested
+    __builtin_amdgcn_s_waitcnt(waitcnt_imm((S - 2) * L, 0));
+    trip(kt);
+  }
+  for (; kt < nk; ++kt) {          // the last S - 2: nothing left to request
+    const int younger = nk - 1 - kt;
+    static_for_stages<0, S - 2>([&](auto G) {
+      constexpr int g = decltype(G)::value;
+      if (younger == g) __builtin_amdgcn_s_waitcnt(waitcnt_imm(g * L, 0));
+    });
+    trip(kt);
   }
 
   // ---- epilogue: scale, bias, cast, vector store ----------------------------
-  float scale = 1.0f;
-  if (p.scale_a) scale *= *p.scale_a;
-  if (p.scale_b) scale *= *p.scale_b;
-  const bool vec_ok = (p.ldc & 3) == 0;
 #pragma unroll
-  for (int m = 0; m < TM; ++m) {
-    const int row = row0 + (wm * TM + m) * 16 + li;
+  for (int n = 0; n < TN; ++n) {
+    const int col = col0 + (wn * TN + n) * 16 + 4 * lq;
+    const f32x4 b = EARLY ? bias_v[EARLY ? n : 0] : load_bias(n);
+    const int ncols = (p.N - col) < 4 ? (p.N - col) : 4;
 #pragma unroll
-    for (int n = 0; n < TN; ++n) {
-      const int col = col0 + (wn * TN + n) * 16 + 4 * lq;
+    for (int m = 0; m < TM; ++m) {
+      const int row = row0 + (wm * TM + m) * 16 + li;
       if (row < p.M && col < p.N) {
         f32x4 v = acc[m][n] * scale;
-        const int ncols = (p.N - col) < 4 ? (p.N - col) : 4;
-        if (p.bias) {
-          for (int r = 0; r < ncols; ++r) v[r] += p.bias[col + r];
-        }
-        store4<OUT>(p.C, (int64_t)row * p.ldc + col, v, vec_ok, ncols);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] += b[e];
+        store4<OUT>(p.C, (int64_t)row * p.ldc + col, v, ncols);
       }
     }
   }
 }
 
 
-template <int DT, int OUT, int BM, int BN, int WM, int WN>
+template <int DT, int OUT, int BM, int BN, int WM, int WN, int S>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_tile_kernel(const GemmArgs p) {
-  gemm_tile_body<DT, OUT, BM, BN, WM, WN>(p);
+  gemm_tile_body<DT, OUT, BM, BN, WM, WN, S>(p);
 }
 
 }  // namespace

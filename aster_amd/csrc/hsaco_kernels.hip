@@ -35,11 +35,11 @@ __device__ __forceinline__ GemmArgs make_args(const void* A, const void* B, void
 // C[M,N] (f32) = A[M,K] (f16) * B[N,K]^T (f16); K % 8 == 0.
 extern "C" __global__ __launch_bounds__(256) void gemm_cdna4(const void* A, const void* B,
                                                              void* C, int M, int N, int K) {
-  gemm_tile_body<ASTERGEMM_F16, ASTERGEMM_F32, 128, 128, 2, 2>(make_args(A, B, C, M, N, K, 2));
+  gemm_tile_body<ASTERGEMM_F16, ASTERGEMM_F32, 128, 128, 2, 2, 2>(make_args(A, B, C, M, N, K, 2));
 }
 
 // Same with bf16 operands and bf16 output.
 extern "C" __global__ __launch_bounds__(256) void gemm_cdna4_bf16(const void* A, const void* B,
                                                                   void* C, int M, int N, int K) {
-  gemm_tile_body<ASTERGEMM_BF16, ASTERGEMM_BF16, 128, 128, 2, 2>(make_args(A, B, C, M, N, K, 2));
+  gemm_tile_body<ASTERGEMM_BF16, ASTERGEMM_BF16, 128, 128, 2, 2, 2>(make_args(A, B, C, M, N, K, 2));
 }

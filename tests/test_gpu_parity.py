@@ -637,6 +637,28 @@ def test_stream_kernels_edge_tiles(gpu, M, N, K, dtype_ab, dtype_c):
     assert np.isnan(pad).all() if dtype_c == "f32" else (pad == 0x7FC1).all()
 
 
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 6, 9])
+@pytest.mark.parametrize("tile", [(64, 64), (128, 64), (128, 128), (256, 256)])
+@pytest.mark.parametrize("dtype_ab", ["bf16", "fp8_e4m3", "mxfp4"])
+def test_tile_kernels_every_stage_count(gpu, steps, tile, dtype_ab):
+    """The LDS ring of the general tile kernels: fewer K-steps than stages, as many, and more; with a
+    K tail (none for MXFP4, whose rows are whole steps); odd M and N, an odd output pitch."""
+    per = {"bf16": 64, "fp8_e4m3": 128, "mxfp4": 256}[dtype_ab]
+    M, N = tile[0] + 5, tile[1] + 3
+    for K in ((per * steps,) if dtype_ab == "mxfp4" else (per * steps, per * (steps - 1) + per // 4)):
+        a, b, extra = operands(M, N, K, dtype_ab, seed=59, b_std=0.05)
+        bias = np.random.default_rng(60).standard_normal(N).astype(np.float32)
+        out, name = run_gemm(a, b, M, N, K, dtype_ab, "f32", bias=bias, family=_capi.KERNEL_TILE,
+                             wg_tile=tile, ldc=N + 2, **extra)
+        assert name.startswith("tile_")
+        if dtype_ab == "fp8_e4m3":
+            want = G.gemm_fp8(a, b, extra["scale_a"], extra["scale_b"], out_dtype=G.F32, bias=bias)
+        else:
+            want = G.gemm(a, b, _DT[dtype_ab], G.F32, bias=bias, **extra)
+        check(out, want, "f32", N, bar=1e-4 if dtype_ab == "fp8_e4m3" else 1e-5)
+        assert np.isnan(out[:, N:]).all()
+
+
 @pytest.mark.parametrize("M", [9, 15, 129, 257, 263, 333])
 @pytest.mark.parametrize("tile", [128, 256])
 @pytest.mark.parametrize("dtype_ab,dtype_c", [("bf16", "bf16"), ("f16", "f32"), ("fp8_e4m3", "bf16"),
