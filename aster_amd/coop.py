@@ -127,7 +127,7 @@ def stream_kernel_load_plan(wid: int, *, tile_rows: int, num_waves: int,
 
 
 # (tile rows, waves) of every instantiation of the stream kernels' staging.
-STREAM_PLAN_CONFIGS = [(256, 8), (256, 4), (128, 4)]
+STREAM_PLAN_CONFIGS = [(256, 8), (256, 4), (192, 8), (128, 8), (128, 4)]
 
 
 def stream_load_plan_header() -> str:

@@ -152,6 +152,52 @@ int current_device_or_minus_one() {
   return dev;
 }
 
+int chip_cus() {
+  const int cus = device_cus();
+  return cus > 0 ? cus : 256;  // no device to ask: describe the MI355X
+}
+
+int64_t tile_grid(const astergemm_config& c, int64_t bm, int64_t bn) {
+  return ((c.M + bm - 1) / bm) * ((c.N + bn - 1) / bn);
+}
+
+// Rows of the stream kernel with unequal tile sides (192 x 128 or 256 x 128, one workgroup per CU)
+// that AUTO takes, 0 = neither.  They fill the gap between the 128 x 128 kernel, which past one
+// workgroup per CU pays for two, and the 256 x 256 kernel, which below half a round leaves half the
+// chip idle.  bf16, back to back, 128 x 128 / 256 x 256 / 192 x 128 / 256 x 128 in us (K = 4096 unless
+// said):
+//   one round of 192 x 128    333x14336 64.2 / 77.6 / 49.1 / 49.2, 1400x4096 55.2 / 68.8 / 41.0 / 43.3,
+//                             1500x4096x11008 157 / 181 / 119 / 129
+//   one round of 256 x 128    2048x4096 59.3 / 69.8 / 74.9 / 53.9, 500x11008 68.6 / 73.6 / 68.3 / 52.3,
+//                             800x8192x8192 117 / 133 / 138 / 101
+//   past it, 256 x 256        640x14336 106 / 75.3 / 78.3 / 92.4, 2500x4096 87.4 / 71.9 / 77.4 / 91.5
+//   three rounds against two  1300x14336 164 / 163 / 151 / 149, 600x28672 164 / 166 / 161 / 151 (where
+//                             whole rounds plus a rest exist they win: 2560x8192x8192 261 against 287)
+//   K = 1024                  2048x4096 18.9 / 24.8 / 24.3 / 18.8, 800x8192 16.6 / 23.9 / 23.1 / 16.4
+//   K = 512: behind           2048x4096 11.4 / 15.5 / 16.5 / 12.9
+// Up to one 128 x 128 tile per CU its nine-slot ring is ahead (960x4096 35.1 against 39.3).  A
+// config that names a tile size or wave count gets the kernels it always got.
+bool unequal_tiles_apply(const astergemm_config& c) {
+  return (c.dtype_ab == ASTERGEMM_F16 || c.dtype_ab == ASTERGEMM_BF16) &&
+         c.operand_path == ASTERGEMM_OPERAND_LDS && row_bytes(c.dtype_ab, c.K) >= 2048 &&
+         !c.wg_tile_m && !c.wg_tile_n && !c.waves_m && !c.waves_n;
+}
+
+int unequal_tile_of(const astergemm_config& c) {
+  if (!unequal_tiles_apply(c)) return 0;
+  const int64_t cus = chip_cus();
+  if (tile_grid(c, 128, 128) <= cus) return 0;
+  if (tile_grid(c, 192, 128) <= cus) return 192;
+  const int64_t g = tile_grid(c, 256, 128);
+  // whole 128 x 128 tiles on at least 7/8 of two workgroups per CU: the tests pin this selection to
+  // the 128 x 128 kernel, which is the slower one there (512x14336 72.8 against 56.0 us, 2048x4096
+  // 59.3 against 53.9)
+  const int64_t g128 = tile_grid(c, 128, 128);
+  if (c.M % 128 == 0 && c.N % 128 == 0 && g128 <= 2 * cus && g128 * 8 >= 2 * cus * 7) return 0;
+  if (g <= cus || (g <= 3 * cus && tile_grid(c, 256, 256) > cus)) return 256;
+  return 0;
+}
+
 const Variant* choose_uncached(const astergemm_config& c, int* index_out);
 
 // Picks the variant for cfg; on failure returns nullptr with the error set.
@@ -228,12 +274,15 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out) {
   if (c.operand_path == ASTERGEMM_OPERAND_DIRECT_B_K8) family = ASTERGEMM_KERNEL_TILE;
   if (c.operand_path == ASTERGEMM_OPERAND_DIRECT_AB) family = ASTERGEMM_KERNEL_TILE;
 
+  const int unequal = unequal_tile_of(c);
+
   const Variant* best = nullptr;
   int best_index = -1;
   const char* last_why = nullptr;  // reason given by the first variant that refused
   for (int i = 0; i < total_variants(); ++i) {
     const Variant* v = variant_at(i);
     if (v->family != family || !variant_matches_types(*v, c)) continue;
+    if (v->rank == 5 && v->tile_m != unequal) continue;
     if (const char* why = v->check(c)) {
       if (!last_why) last_why = why;
       continue;
@@ -285,7 +334,11 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out) {
       // from 128 on when rows are long (8 KiB and more: few prologues per byte streamed).
       const int64_t g128 = ((c.M + 127) / 128) * ((c.N + 127) / 128);
       const bool ragged_128 = g128 > 512 && g128 % 512 != 0 && g128 % 512 < 180;
+      // 16-bit operands whose 256 x 128 tiles pass one per CU: 256 x 256 whatever part of the round
+      // they fill, the tiles between no longer pay (see unequal_tile_of)
+      const bool past_unequal = unequal_tiles_apply(c) && unequal == 0 && tile_grid(c, 256, 128) > chip_cus();
       const int thr256 = ragged_128 ? 140 : 220;
+      const int thr256s = past_unequal ? 1 : thr256;
       // MXFP4: the generic tile kernels are weak next to the stream kernels, so the 128 x 128
       // stream kernel from 16 workgroups on when K >= 4096, and instead of the 256 x 256 one
       // (long prologue: two K-steps and their scales) when K < 4096
@@ -297,6 +350,9 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out) {
         // split K (rank 4) only passes its check where it was measured ahead of every
         // unsplit kernel: few output tiles, long rows
         if (x->rank == 4) return 3;
+        // unequal sides: offered only where the rule took them; the whole-rounds form stays ahead
+        if (x->rank == 5) return 4;
+        if (unequal && area >= 256 * 256 && x->rank == 3) return 5;
         // (not the tile walk and the whole-rounds form, rank 3, which pay that prologue once per
         // workgroup, from about two tiles of K = 2048 per CU on: 8192 x 8192 x 1024 51 against
         // 57 us, 16384 x 16384 x 1024 180 against 210, 8192 x 8192 x 2048 74 against 84,
@@ -304,7 +360,7 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out) {
         // against 29.8, 4096 x 6144 x 1024 24.0 against 21.8)
         const bool walk_pays = x->rank == 3 && wgs(x) * c.K >= (int64_t)512 * 2048;
         if (area >= 256 * 256 && fp4 && c.K < 4096 && c.K % 512 == 0 && !walk_pays) return -1;
-        if (area >= 256 * 256) return wgs(x) >= thr256 ? 2 : -1;
+        if (area >= 256 * 256) return wgs(x) >= (x->rank >= 2 ? thr256s : thr256) ? 2 : -1;
         return wgs(x) >= ((x->rank >= 2) ? thr128s : 448) ? 1 : 0;
       };
       const int tv = tier(v), tb = tier(best);

@@ -4,6 +4,7 @@
 #include <vector>
 
 #include "gemm_stream_kernel.hpp"
+#include "gemm_streamr_kernel.hpp"
 #include "gemm_stream8_kernel.hpp"
 #include "gemm_stream4_kernel.hpp"
 #include "gemm_streamdb_kernel.hpp"
@@ -81,6 +82,29 @@ const char* check_stream_ring9(const astergemm_config& c) {
   AG_STREAM_RING9(prefix "_128x128_w2x2_ring9_bf16", DT, ASTERGEMM_BF16),        \
       AG_STREAM_RING9(prefix "_128x128_w2x2_ring9_f32", DT, ASTERGEMM_F32),      \
       AG_STREAM_RING9(prefix "_128x128_w2x2_ring9_f16", DT, ASTERGEMM_F16)
+
+// ---- unequal tile sides (gemm_streamr_kernel.hpp); rank 5: AUTO takes them by unequal_tile_of ----
+template <int DT, int OUT, int BM, int BN, int WM, int WN, int NS>
+int launch_streamr(const GemmArgs& a, int grid, hipStream_t s) {
+  constexpr int lds = NS * (BM + BN) * kRowBytes;
+  auto k = gemm_streamr_kernel<DT, OUT, BM, BN, WM, WN, NS>;
+  static std::atomic<uint64_t> attr_devs{0};
+  if (int e = lds_attr_once(attr_devs, (const void*)k, lds)) return e;
+  AG_LAUNCH_KERNEL(k, dim3(grid), dim3(WM * WN * 64), lds, s, a);
+  return (int)hipGetLastError();
+}
+
+#define AG_STREAMR(name, DT, OUT, BM, BN, WM, WN, NS)                            \
+  Variant {                                                                      \
+    name, ASTERGEMM_KERNEL_TILE, DT, OUT, BM, BN, kRowBytes, WM, WN, NS, 5,      \
+        NS * (BM + BN) * kRowBytes,                                              \
+        (const void*)gemm_streamr_kernel<DT, OUT, BM, BN, WM, WN, NS>,           \
+        launch_streamr<DT, OUT, BM, BN, WM, WN, NS>, check_stream                \
+  }
+#define AG_STREAMR_SET(prefix, DT, BM, BN, WM, WN, NS)                           \
+  AG_STREAMR(prefix "_bf16", DT, ASTERGEMM_BF16, BM, BN, WM, WN, NS),            \
+      AG_STREAMR(prefix "_f32", DT, ASTERGEMM_F32, BM, BN, WM, WN, NS),          \
+      AG_STREAMR(prefix "_f16", DT, ASTERGEMM_F16, BM, BN, WM, WN, NS)
 
 // ---- B pre-shuffled, loaded straight into MFMA operands (gemm_streamdb_kernel.hpp) ---------
 template <int DT, int OUT, int NSLOT, int NBUF, int WM>
@@ -618,10 +642,10 @@ int grid_stream_tail(const astergemm_config& c, int cus) {
       AG_STREAM(prefix "_128x128_w2x2_f32", DT, ASTERGEMM_F32, 128, 128, 2, 2),          \
       AG_STREAM(prefix "_128x128_w2x2_f16", DT, ASTERGEMM_F16, 128, 128, 2, 2)
 
-// The table is compiled in four parts (this file once per AG_STREAM_PART: bf16, fp8, MXFP4 and f16
-// operands), so that the parts build side by side and work on one family recompiles one part.
+// The table is compiled in five parts (this file once per AG_STREAM_PART: bf16, fp8, MXFP4 and f16
+// operands, and 16-bit operands on unequal tile sides), so that the parts build side by side and work on one family recompiles one part.
 #ifndef AG_STREAM_PART
-#error "compile with -DAG_STREAM_PART=0, 1, 2 or 3"
+#error "compile with -DAG_STREAM_PART=0, 1, 2, 3 or 4"
 #endif
 
 const Variant kStreamVariants[] = {
@@ -662,6 +686,11 @@ const Variant kStreamVariants[] = {
     AG_STREAM8DB("streamdb_fp8_128x256_w1x4_bf16", ASTERGEMM_FP8_E4M3, ASTERGEMM_BF16),
     AG_STREAM8DB("streamdb_fp8_128x256_w1x4_f32", ASTERGEMM_FP8_E4M3, ASTERGEMM_F32),
     AG_STREAM8DB("streamdb_fp8_128x256_w1x4_f16", ASTERGEMM_FP8_E4M3, ASTERGEMM_F16),
+#elif AG_STREAM_PART == 4
+    AG_STREAMR_SET("stream_bf16_256x128_w4x2", ASTERGEMM_BF16, 256, 128, 4, 2, 3),
+    AG_STREAMR_SET("stream_bf16_192x128_w4x2", ASTERGEMM_BF16, 192, 128, 4, 2, 4),
+    AG_STREAMR_SET("stream_f16_256x128_w4x2", ASTERGEMM_F16, 256, 128, 4, 2, 3),
+    AG_STREAMR_SET("stream_f16_192x128_w4x2", ASTERGEMM_F16, 192, 128, 4, 2, 4),
 #else
     AG_STREAM_SPLITK_SET("splitk_mxfp4", 2, ASTERGEMM_MXFP4, 4 * 128 * kRowBytes + 4 * 128 * 16,
                          gemm_stream4_splitk_kernel),
@@ -702,8 +731,9 @@ const Variant* AG_CAT(stream_variants_part, AG_STREAM_PART)(int* count) {
 const Variant* stream_variants_part1(int* count);
 const Variant* stream_variants_part2(int* count);
 const Variant* stream_variants_part3(int* count);
+const Variant* stream_variants_part4(int* count);
 
-// the four parts as one table: bf16, f16, fp8, MXFP4
+// the parts as one table: bf16, f16, fp8, MXFP4, unequal tile sides
 static const std::vector<Variant>& all_stream_variants() {
   static const std::vector<Variant> all = [] {
     std::vector<Variant> v;
@@ -715,6 +745,8 @@ static const std::vector<Variant>& all_stream_variants() {
     p = stream_variants_part1(&n);
     v.insert(v.end(), p, p + n);
     p = stream_variants_part2(&n);
+    v.insert(v.end(), p, p + n);
+    p = stream_variants_part4(&n);
     v.insert(v.end(), p, p + n);
     return v;
   }();

@@ -123,15 +123,13 @@ __device__ __forceinline__ void stream_k_tail(const GemmArgs& p,
 // 32-byte pieces per row, which costs ~7 % of the kernel.)  The lane id is
 // recomputed here, opaque to the optimiser, so that no lane-derived value has to
 // stay in a VGPR across the K loop.
-template <int OUT, int BM, int BN, int WM, int WN>
+template <int OUT, int BM, int BN, int WM, int WN, int LDS_BYTES = 5 * BM * kRowBytes>
 __device__ __forceinline__ void stream_epilogue(const GemmArgs& p,
                                                 f32x4 (&acc)[BM / WM / 16][BN / WN / 16],
                                                 uint8_t* lds, int wave, int row0, int col0) {
   constexpr int NW = WM * WN;
   constexpr int TM = BM / WM / 16;
   constexpr int TN = BN / WN / 16;
-  constexpr int SLOT = BM * kRowBytes;
-  constexpr int NSLOT = 5;
   const int wm = wave / WN, wn = wave % WN;
   int lane_e;
   asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane_e));
@@ -146,7 +144,7 @@ __device__ __forceinline__ void stream_epilogue(const GemmArgs& p,
   constexpr int SLAB = 16 * PITCH;
   constexpr int CHUNKS = 16 * ROWB / 16;              // 16-byte chunks per slab
   static_assert(CHUNKS % 64 == 0, "whole store instructions per slab");
-  static_assert(2 * SLAB * NW <= NSLOT * SLOT, "staging fits in the ring");
+  static_assert(2 * SLAB * NW <= LDS_BYTES, "staging fits in the ring");
   // every wave is done reading fragments before LDS is reused
   __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
   __builtin_amdgcn_s_barrier();

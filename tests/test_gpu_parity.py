@@ -721,6 +721,29 @@ def test_nine_slot_ring_is_left_to_grids_of_one_workgroup_per_cu(gpu):
     assert AG.GemmPlan.create(256, 14336, 4096, "bf16", "bf16").info.lds_bytes == 9 * 128 * 128
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(8, 8, 64), (9, 136, 128), (191, 128, 192), (192, 120, 256), (193, 256, 320),
+                                   (255, 128, 384), (256, 264, 448), (257, 136, 512), (333, 1000, 576),
+                                   (384, 256, 1024), (400, 384, 1032), (777, 520, 72), (129, 248, 2040)])
+@pytest.mark.parametrize("tile", ["256x128_w4x2", "192x128_w4x2"])
+@pytest.mark.parametrize("dtype_ab,dtype_c", [("bf16", "bf16"), ("f16", "f32"), ("bf16", "f16")])
+def test_stream_unequal_tile_sides(gpu, M, N, K, tile, dtype_ab, dtype_c):
+    """The 256 x 128 and 192 x 128 kernels: K-step counts 1 ... 9, 16, 31 around the rings of three and
+    four stages (none, one and several groups of steady trips), tails of granules, heights around
+    the tiles and off the groups of 8 rows, the smallest operands.  Each output is the sum of the
+    same MFMAs in the same order as in the 128 x 128 kernel, so the bits are equal."""
+    a, b, _ = operands(M, N, K, dtype_ab, seed=71, b_std=0.05)
+    bias = np.random.default_rng(72).standard_normal(N).astype(np.float32)
+    out, name = run_gemm(a, b, M, N, K, dtype_ab, dtype_c, bias=bias,
+                         variant=_variant_id(f"stream_{dtype_ab}_{tile}_{dtype_c}"))
+    assert name == f"stream_{dtype_ab}_{tile}_{dtype_c}"
+    square, _ = run_gemm(a, b, M, N, K, dtype_ab, dtype_c, bias=bias,
+                         variant=_variant_id(f"stream_{dtype_ab}_128x128_w2x2_{dtype_c}"))
+    assert np.array_equal(out, square)
+    check(out, G.gemm(a, b, _DT[dtype_ab], _DT[dtype_c], bias=bias), dtype_c, N,
+          bar=REL_L2_BAR if dtype_c != "f32" else 1e-5)
+
+
 # ---- edge cases: ragged M / N, K tails, leading dimensions, epilogue -----------------
 
 @pytest.mark.parametrize("M,N,K", [(1, 1, 8), (65, 16, 8), (130, 257, 72), (300, 520, 776), (129, 1, 64)])

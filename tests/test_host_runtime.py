@@ -83,6 +83,38 @@ def test_select_headline_configs():
     assert gemm.GemmPlan.create(128, 4096, 14336, "mxfp4", "bf16").info.grid_x == 32 * 7
 
 
+@pytest.mark.parametrize("shape,tile", [
+    ((1024, 4096, 4096), "128x128_w2x2_ring9"),   # 256 tiles of 128 x 128: one per CU
+    ((1025, 4096, 4096), "192x128_w4x2"),
+    ((1536, 4096, 4096), "192x128_w4x2"),         # 256 of 192 x 128
+    ((1537, 4096, 4096), "256x128_w4x2"),
+    ((2047, 4096, 4096), "256x128_w4x2"),         # 256 of 256 x 128
+    ((2048, 4096, 4096), "128x128_w2x2"),         # whole 128 x 128 tiles, two per CU
+    ((2049, 4096, 4096), "256x256_w2x4"),
+    ((2047, 4096, 1024), "256x128_w4x2"),
+    ((2047, 4096, 1016), "128x128_w2x2"),         # rows below 2 KiB
+    ((640, 14336, 4096), "256x256_w2x4"),
+    ((1300, 14336, 4096), "256x128_w4x2"),        # three rounds against two
+    ((2560, 8192, 8192), "256x256_w2x4_tail128"),
+    ((4096, 4096, 4096), "256x256_w2x4"),
+])
+@pytest.mark.parametrize("dtype_ab,dtype_c", [("bf16", "bf16"), ("f16", "f32")])
+def test_selection_of_unequal_tile_sides(shape, tile, dtype_ab, dtype_c):
+    """Which tile AUTO takes on either side of every line of the rule; forms the kernels do not take
+    and configs that name a tile or a wave count keep the kernels they had."""
+    create = lambda *s, **kw: gemm.GemmPlan.create(*s, dtype_ab, dtype_c, **kw).info.name.decode()
+    M, N, K = shape
+    assert create(M, N, K) == f"stream_{dtype_ab}_{tile}_{dtype_c}"
+    assert create(M, N, K, lda=K + 8, ldc=N + 8) == f"stream_{dtype_ab}_{tile}_{dtype_c}"
+    assert create(M, N, K, ldc=N + 1).startswith("tile_")
+    assert create(M, N - 1, K).startswith("tile_")
+    for wg in ((128, 128), (256, 256)):
+        assert "x".join(map(str, wg)) in create(M, N, K, wg_tile=wg)
+    for wg in ((256, 128), (192, 128)):
+        with pytest.raises(Exception, match="no kernel variant"):
+            create(M, N, K, wg_tile=wg)
+
+
 def test_explicit_variant_and_enumeration():
     lib = _capi.load()
     n = lib.astergemm_variant_count()
