@@ -164,38 +164,59 @@ int64_t tile_grid(const astergemm_config& c, int64_t bm, int64_t bn) {
 // Rows of the stream kernel with unequal tile sides (192 x 128 or 256 x 128, one workgroup per CU)
 // that AUTO takes, 0 = neither.  They fill the gap between the 128 x 128 kernel, which past one
 // workgroup per CU pays for two, and the 256 x 256 kernel, which below half a round leaves half the
-// chip idle.  bf16, back to back, 128 x 128 / 256 x 256 / 192 x 128 / 256 x 128 in us (K = 4096 unless
-// said):
-//   one round of 192 x 128    333x14336 64.2 / 77.6 / 49.1 / 49.2, 1400x4096 55.2 / 68.8 / 41.0 / 43.3,
-//                             1500x4096x11008 157 / 181 / 119 / 129
-//   one round of 256 x 128    2048x4096 59.3 / 69.8 / 74.9 / 53.9, 500x11008 68.6 / 73.6 / 68.3 / 52.3,
-//                             800x8192x8192 117 / 133 / 138 / 101
-//   past it, 256 x 256        640x14336 106 / 75.3 / 78.3 / 92.4, 2500x4096 87.4 / 71.9 / 77.4 / 91.5
-//   three rounds against two  1300x14336 164 / 163 / 151 / 149, 600x28672 164 / 166 / 161 / 151 (where
-//                             whole rounds plus a rest exist they win: 2560x8192x8192 261 against 287)
-//   K = 1024                  2048x4096 18.9 / 24.8 / 24.3 / 18.8, 800x8192 16.6 / 23.9 / 23.1 / 16.4
-//   K = 512: behind           2048x4096 11.4 / 15.5 / 16.5 / 12.9
-// Up to one 128 x 128 tile per CU its nine-slot ring is ahead (960x4096 35.1 against 39.3).  A
-// config that names a tile size or wave count gets the kernels it always got.
+// chip idle.  Back to back, 128 x 128 / 256 x 256 / 192 x 128 / 256 x 128 in us (K = 4096 unless said):
+//   one round of 192 x 128    bf16 333x14336 64.2 / 77.6 / 49.1 / 49.2, 1400x4096 55.2 / 68.8 / 41.0 / 43.3,
+//                             1500x4096x11008 157 / 181 / 119 / 129, fp8 333x14336 36.1 / 42.8 / 27.4 / 30.4
+//   one round of 256 x 128    bf16 2048x4096 59.3 / 69.8 / 74.9 / 53.9, 500x11008 68.6 / 73.6 / 68.3 / 52.3,
+//                             800x8192x8192 117 / 133 / 138 / 101, fp8 500x14336 40.7 / 42.0 / 48.2 / 31.9
+//   past it, 256 x 256        bf16 640x14336 106 / 75.3 / 78.3 / 92.4, 2500x4096 87.4 / 71.9 / 77.4 / 91.5,
+//                             fp8 1500x8192x8192 116 / 87.5 / 95.2 / 106
+//   three rounds against two  bf16 1300x14336 164 / 163 / 151 / 149, 600x28672 164 / 166 / 161 / 151 (where
+//                             whole rounds plus a rest exist they win: 2560x8192x8192 261 against 287);
+//                             fp8 1500x14336 97.7 / 89.5 / 102 / 89.6: level, not taken
+//   rows of 2 KiB             bf16 2048x4096x1024 18.9 / 24.8 / 24.3 / 18.8, 800x8192x1024 16.6 / 23.9 / 23.1 / 16.4
+//   rows of 1 KiB: behind     bf16 2048x4096x512 11.4 / 15.5 / 16.5 / 12.9
+// Up to one 128 x 128 tile per CU 16-bit operands have the nine-slot ring, which is ahead (960x4096 35.1
+// against 39.3); fp8 takes the same kernel at 128 x 128 (ring of five whole K-steps, eight waves) from
+// two tile rows on: 333x8192x8192 51.1 -> 36.8, 1000x4096x14336 86.3 -> 66.8, 200x14336 29.1 -> 23.5.
+// A config that names a tile size or wave count gets the kernels it always got.
 bool unequal_tiles_apply(const astergemm_config& c) {
-  return (c.dtype_ab == ASTERGEMM_F16 || c.dtype_ab == ASTERGEMM_BF16) &&
+  return (c.dtype_ab == ASTERGEMM_F16 || c.dtype_ab == ASTERGEMM_BF16 || c.dtype_ab == ASTERGEMM_FP8_E4M3) &&
          c.operand_path == ASTERGEMM_OPERAND_LDS && row_bytes(c.dtype_ab, c.K) >= 2048 &&
          !c.wg_tile_m && !c.wg_tile_n && !c.waves_m && !c.waves_n;
 }
 
 int unequal_tile_of(const astergemm_config& c) {
   if (!unequal_tiles_apply(c)) return 0;
-  const int64_t cus = chip_cus();
-  if (tile_grid(c, 128, 128) <= cus) return 0;
+  const bool fp8 = c.dtype_ab == ASTERGEMM_FP8_E4M3;
+  const int64_t cus = chip_cus(), g128 = tile_grid(c, 128, 128);
+  if (g128 <= cus) return fp8 && c.M > 128 ? 128 : 0;
   if (tile_grid(c, 192, 128) <= cus) return 192;
-  const int64_t g = tile_grid(c, 256, 128);
   // whole 128 x 128 tiles on at least 7/8 of two workgroups per CU: the tests pin this selection to
-  // the 128 x 128 kernel, which is the slower one there (512x14336 72.8 against 56.0 us, 2048x4096
-  // 59.3 against 53.9)
-  const int64_t g128 = tile_grid(c, 128, 128);
+  // the 128 x 128 kernel, which is the slower one there (bf16 512x14336 72.8 against 56.0 us,
+  // 2048x4096 59.3 against 53.9, fp8 2048x4096 32.4 against 31.6)
   if (c.M % 128 == 0 && c.N % 128 == 0 && g128 <= 2 * cus && g128 * 8 >= 2 * cus * 7) return 0;
-  if (g <= cus || (g <= 3 * cus && tile_grid(c, 256, 256) > cus)) return 256;
+  const int64_t g = tile_grid(c, 256, 128);
+  if (g <= cus || (!fp8 && g <= 3 * cus && tile_grid(c, 256, 256) > cus)) return 256;
   return 0;
+}
+
+// Split K on 256 x 128 tiles: where the square tiles, split or not, leave one CU at least 4/3 of the
+// operand rows (tile rows x K-steps) that one range here does, on rows long enough to pay for the
+// planes.  Square split or unsplit -> this, us: bf16 500x4096x14336 83.6 -> 67.1, 333x4096x14336 72.2 ->
+// 61.1, 1000x4096x14336 133 -> 113, 250x8192x28672 162 -> 136, 500x8192x28672 275 -> 238; fp8
+// 500x4096x14336 54.4 -> 46.2.  Behind: equal or fewer rows saved (bf16 256x4096x14336 56.5 -> 59.4),
+// shorter rows against an unsplit kernel (800x4096x11008 86.3 -> 88.0), few tile columns, where every XCD
+// reads all of A (2000x1024x8192 45.3 -> 59.1).
+bool unequal_split_pays(const astergemm_config& c) {
+  if (!unequal_tiles_apply(c) || c.M <= 128 || c.N < 4 * c.M) return false;
+  const int64_t g128 = tile_grid(c, 128, 128), steps = row_bytes(c.dtype_ab, c.K) / 128;
+  const int S = streamr_split_of(tile_grid(c, 256, 128), steps);
+  if (S == 0 || g128 > chip_cus()) return false;
+  const int S128 = stream_split_of(g128, steps);
+  if (steps < (S128 ? 112 : 224)) return false;
+  const int64_t square = S128 ? (g128 * S128 + 255) / 256 * (steps / S128) * 256 : steps * 256;
+  return steps / S * 384 * 4 <= square * 3;
 }
 
 const Variant* choose_uncached(const astergemm_config& c, int* index_out);
@@ -275,6 +296,7 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out) {
   if (c.operand_path == ASTERGEMM_OPERAND_DIRECT_AB) family = ASTERGEMM_KERNEL_TILE;
 
   const int unequal = unequal_tile_of(c);
+  const bool unequal_split = unequal_split_pays(c);
 
   const Variant* best = nullptr;
   int best_index = -1;
@@ -283,6 +305,7 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out) {
     const Variant* v = variant_at(i);
     if (v->family != family || !variant_matches_types(*v, c)) continue;
     if (v->rank == 5 && v->tile_m != unequal) continue;
+    if (v->rank == 6 && !unequal_split) continue;
     if (const char* why = v->check(c)) {
       if (!last_why) last_why = why;
       continue;
@@ -334,7 +357,7 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out) {
       // from 128 on when rows are long (8 KiB and more: few prologues per byte streamed).
       const int64_t g128 = ((c.M + 127) / 128) * ((c.N + 127) / 128);
       const bool ragged_128 = g128 > 512 && g128 % 512 != 0 && g128 % 512 < 180;
-      // 16-bit operands whose 256 x 128 tiles pass one per CU: 256 x 256 whatever part of the round
+      // 16-bit and fp8 operands whose 256 x 128 tiles pass one per CU: 256 x 256 whatever part of the round
       // they fill, the tiles between no longer pay (see unequal_tile_of)
       const bool past_unequal = unequal_tiles_apply(c) && unequal == 0 && tile_grid(c, 256, 128) > chip_cus();
       const int thr256 = ragged_128 ? 140 : 220;
@@ -351,8 +374,9 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out) {
         // unsplit kernel: few output tiles, long rows
         if (x->rank == 4) return 3;
         // unequal sides: offered only where the rule took them; the whole-rounds form stays ahead
-        if (x->rank == 5) return 4;
-        if (unequal && area >= 256 * 256 && x->rank == 3) return 5;
+        // (fp8 on 128 x 128: the square kernel's lines)
+        if (x->rank == 6 || (x->rank == 5 && x->tile_m > 128)) return 4;
+        if (unequal > 128 && area >= 256 * 256 && x->rank == 3) return 5;
         // (not the tile walk and the whole-rounds form, rank 3, which pay that prologue once per
         // workgroup, from about two tiles of K = 2048 per CU on: 8192 x 8192 x 1024 51 against
         // 57 us, 16384 x 16384 x 1024 180 against 210, 8192 x 8192 x 2048 74 against 84,

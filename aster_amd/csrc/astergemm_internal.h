@@ -140,6 +140,15 @@ inline int stream_split_of(int64_t tiles, int64_t ksteps, bool even_ranges = fal
   return best;
 }
 
+// K ranges of the split-K kernel on 256 x 128 tiles: the largest divisor up to 4 that leaves at most
+// one workgroup per CU; 0 if there is none.
+inline int streamr_split_of(int64_t tiles, int64_t ksteps) {
+  int best = 0;
+  for (int S = 2; S <= 4; ++S)
+    if (ksteps % S == 0 && ksteps / S >= 8 && tiles * S <= 256) best = S;
+  return best;
+}
+
 // Split-K support shared by the decode and the tile kernels (gemm_skinny.hip): the fp32
 // workspace of a (device, stream), and the kernel that adds `splits` planes [M][N] of
 // a.workspace in index order, applies a's scales and bias and stores a.C in `out_dtype`.

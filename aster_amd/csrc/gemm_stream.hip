@@ -94,16 +94,16 @@ int launch_streamr(const GemmArgs& a, int grid, hipStream_t s) {
   return (int)hipGetLastError();
 }
 
-#define AG_STREAMR(name, DT, OUT, BM, BN, WM, WN, NS)                            \
+#define AG_STREAMR(name, DT, OUT, BM, BN, WM, WN, NS)                      \
   Variant {                                                                      \
     name, ASTERGEMM_KERNEL_TILE, DT, OUT, BM, BN, kRowBytes, WM, WN, NS, 5,      \
         NS * (BM + BN) * kRowBytes,                                              \
         (const void*)gemm_streamr_kernel<DT, OUT, BM, BN, WM, WN, NS>,           \
         launch_streamr<DT, OUT, BM, BN, WM, WN, NS>, check_stream                \
   }
-#define AG_STREAMR_SET(prefix, DT, BM, BN, WM, WN, NS)                           \
-  AG_STREAMR(prefix "_bf16", DT, ASTERGEMM_BF16, BM, BN, WM, WN, NS),            \
-      AG_STREAMR(prefix "_f32", DT, ASTERGEMM_F32, BM, BN, WM, WN, NS),          \
+#define AG_STREAMR_SET(prefix, DT, BM, BN, WM, WN, NS)                     \
+  AG_STREAMR(prefix "_bf16", DT, ASTERGEMM_BF16, BM, BN, WM, WN, NS),      \
+      AG_STREAMR(prefix "_f32", DT, ASTERGEMM_F32, BM, BN, WM, WN, NS),    \
       AG_STREAMR(prefix "_f16", DT, ASTERGEMM_F16, BM, BN, WM, WN, NS)
 
 // ---- B pre-shuffled, loaded straight into MFMA operands (gemm_streamdb_kernel.hpp) ---------
@@ -328,6 +328,58 @@ int splits_stream_splitk(const astergemm_config& c) {
   AG_STREAM_SPLITK(prefix "_128x128_w2x2_bf16", KIND, DT, ASTERGEMM_BF16, LDS, FUNC),   \
       AG_STREAM_SPLITK(prefix "_128x128_w2x2_f32", KIND, DT, ASTERGEMM_F32, LDS, FUNC), \
       AG_STREAM_SPLITK(prefix "_128x128_w2x2_f16", KIND, DT, ASTERGEMM_F16, LDS, FUNC)
+
+// ---- split K on the 256 x 128 tiles; rank 6: AUTO takes them by unequal_split_pays --------------
+template <int DT, int OUT>
+int launch_streamr_splitk(const GemmArgs& a0, int grid, hipStream_t s) {
+  (void)grid;
+  constexpr int lds = 3 * (256 + 128) * kRowBytes;
+  auto k = gemm_streamr_splitk_kernel<DT, 256, 128, 4, 2, 3>;
+  static std::atomic<uint64_t> attr_devs{0};
+  if (int e = lds_attr_once(attr_devs, (const void*)k, lds)) return e;
+  const int tiles = a0.tiles_m * a0.tiles_n;
+  const int S = streamr_split_of(tiles, a0.ksteps);
+  if (S == 0 || a0.tail_granules != 0) return (int)hipErrorInvalidValue;
+  GemmArgs a = a0;
+  if (!a.workspace) {
+    if (int rc = splitk_workspace_for((size_t)S * a.M * a.N * sizeof(float), s, &a.workspace))
+      return rc;
+  }
+  GemmArgs part = a;
+  part.split_k = S;
+  part.ksteps = a.ksteps / S;
+  part.ldc = a.N;
+  part.scale_a = part.scale_b = part.bias = nullptr;
+  AG_LAUNCH_KERNEL(k, dim3(tiles * S), dim3(512), lds, s, part);
+  if (const hipError_t e = hipGetLastError(); e != hipSuccess) return (int)e;
+  return splitk_reduce(OUT, a, S, s);
+}
+
+int splits_streamr_splitk(const astergemm_config& c) {
+  const int64_t tiles = ((c.M + 255) / 256) * ((c.N + 127) / 128);
+  const int S = streamr_split_of(tiles, row_bytes(c.dtype_ab, c.K) / kRowBytes);
+  return S < 1 ? 1 : S;
+}
+
+const char* check_streamr_splitk(const astergemm_config& c) {
+  if (const char* why = check_stream_whole_k(c)) return why;
+  if (row_bytes(c.dtype_ab, c.K) / kRowBytes < 64) return "split K needs rows of at least 8 KiB";
+  if (splits_streamr_splitk(c) < 2) return "split K needs at most 128 output tiles of 256 x 128 and 2..4 K ranges";
+  return nullptr;
+}
+
+#define AG_STREAMR_SPLITK(name, DT, OUT)                                         \
+  Variant {                                                                      \
+    name, ASTERGEMM_KERNEL_TILE, DT, OUT, 256, 128, kRowBytes, 4, 2, 3, 6,       \
+        3 * (256 + 128) * kRowBytes,                                             \
+        (const void*)gemm_streamr_splitk_kernel<DT, 256, 128, 4, 2, 3>,          \
+        launch_streamr_splitk<DT, OUT>, check_streamr_splitk,                    \
+        ASTERGEMM_OPERAND_LDS, splits_streamr_splitk                             \
+  }
+#define AG_STREAMR_SPLITK_SET(prefix, DT)                                        \
+  AG_STREAMR_SPLITK(prefix "_256x128_w4x2_bf16", DT, ASTERGEMM_BF16),            \
+      AG_STREAMR_SPLITK(prefix "_256x128_w4x2_f32", DT, ASTERGEMM_F32),          \
+      AG_STREAMR_SPLITK(prefix "_256x128_w4x2_f16", DT, ASTERGEMM_F16)
 
 template <int DT, int OUT, int BM, int BN, int WM, int WN>
 int launch_stream8(const GemmArgs& a, int grid, hipStream_t s) {
@@ -691,6 +743,12 @@ const Variant kStreamVariants[] = {
     AG_STREAMR_SET("stream_bf16_192x128_w4x2", ASTERGEMM_BF16, 192, 128, 4, 2, 4),
     AG_STREAMR_SET("stream_f16_256x128_w4x2", ASTERGEMM_F16, 256, 128, 4, 2, 3),
     AG_STREAMR_SET("stream_f16_192x128_w4x2", ASTERGEMM_F16, 192, 128, 4, 2, 4),
+    AG_STREAMR_SET("stream_fp8_256x128_w4x2", ASTERGEMM_FP8_E4M3, 256, 128, 4, 2, 3),
+    AG_STREAMR_SET("stream_fp8_192x128_w4x2", ASTERGEMM_FP8_E4M3, 192, 128, 4, 2, 4),
+    AG_STREAMR_SET("stream_fp8_128x128_w4x2", ASTERGEMM_FP8_E4M3, 128, 128, 4, 2, 5),
+    AG_STREAMR_SPLITK_SET("splitk_bf16", ASTERGEMM_BF16),
+    AG_STREAMR_SPLITK_SET("splitk_f16", ASTERGEMM_F16),
+    AG_STREAMR_SPLITK_SET("splitk_fp8", ASTERGEMM_FP8_E4M3),
 #else
     AG_STREAM_SPLITK_SET("splitk_mxfp4", 2, ASTERGEMM_MXFP4, 4 * 128 * kRowBytes + 4 * 128 * 16,
                          gemm_stream4_splitk_kernel),

@@ -1,5 +1,7 @@
-// Stream kernel with unequal tile sides, 16-bit operands: C[M,N] = epi(A[M,K] * B[N,K]^T) on
-// 256 x 128 and 192 x 128 tiles, one eight-wave workgroup per CU.
+// Stream kernel with unequal tile sides, 16-bit and fp8 operands: C[M,N] = epi(A[M,K] * B[N,K]^T)
+// on 256 x 128 and 192 x 128 tiles (fp8 also 128 x 128), one eight-wave workgroup per CU.  What it
+// measured against the square tiles stands at the rules of selection (unequal_tile_of,
+// unequal_split_pays).
 //
 // What bounds it: the operand bytes a CU receives from its XCD's L2 (23-31 B/clk in every kernel
 // of this family), not the matrix cores.  A 256 x 128 tile brings in 384 rows for 32768 outputs,
@@ -7,7 +9,7 @@
 // the chip these are the shapes between.
 //
 // LDS is a ring of NS stages, each one whole K-step (128 bytes of every row of A's and B's tile):
-// three of 48 KiB, or four of 40 KiB.  Unlike the ring of gemm_stream_body, whose halves trade
+// three of 48 KiB, four of 40 KiB or five of 32 KiB.  Unlike the ring of gemm_stream_body, whose halves trade
 // places and must be equal, a stage is refilled as a whole: when K-step k is in registers its stage
 // is requested for K-step k + NS, so NS - 1 K-steps are on their way at any time.  Swizzle, staging
 // plan, fragment order, sums and epilogue are those of gemm_stream_body, so the bits are too.
@@ -18,7 +20,7 @@ namespace astergemm {
 namespace {
 
 template <int DT, int OUT, int BM, int BN, int WM, int WN, int NS>
-__global__ __launch_bounds__(WM* WN * 64) void gemm_streamr_kernel(const GemmArgs p) {
+__device__ __forceinline__ void gemm_streamr_body(const GemmArgs& p, int bid) {
   constexpr int NW = WM * WN;
   constexpr int TM = BM / WM / 16;
   constexpr int TN = BN / WN / 16;
@@ -43,7 +45,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_streamr_kernel(const GemmArg
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave / WN, wn = wave % WN;
   int tile_m, tile_n;
-  map_tile(blockIdx.x, p.tiles_m, p.tiles_n, p.group_m, tile_m, tile_n);
+  map_tile(bid, p.tiles_m, p.tiles_n, p.group_m, tile_m, tile_n);
   const int row0 = tile_m * BM, col0 = tile_n * BN;
 
   // ---- global -> LDS: 128-byte rows, granule index XOR ((row >> 1) & 7) ----------------------
@@ -174,6 +176,186 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_streamr_kernel(const GemmArg
 
   if (p.tail_granules) stream_k_tail<DT, BM, BN, WM, WN>(p, acc, wave, row0, col0, nk);
   stream_epilogue<OUT, BM, BN, WM, WN, NS * STAGE>(p, acc, lds, wave, row0, col0);
+}
+
+// The same for fp8 e4m3.  A K-step is one v_mfma_scale_f32_16x16x128_f8f6f4 per 16 x 16 tile with
+// 32 bytes of each operand per lane (granules lq and 4 + lq, as in gemm_stream8_body, so the bits
+// are the same).  64 accumulators leave room for two whole sets of fragments (2 x 64 registers), so
+// trip k multiplies set k mod 2 and reads K-step k + 1 into the other one.  The stage is a scalar that
+// rotates from trip to trip: unrolled over six trips (both sets, three stages) it spilled 400 dwords.
+template <int DT, int OUT, int BM, int BN, int WM, int WN, int NS>
+__device__ __forceinline__ void gemm_stream8r_body(const GemmArgs& p, int bid) {
+  constexpr int NW = WM * WN;
+  constexpr int TM = BM / WM / 16;
+  constexpr int TN = BN / WN / 16;
+  using PlanA = StreamLoadPlan<BM, NW>;
+  using PlanB = StreamLoadPlan<BN, NW>;
+  constexpr int LA = PlanA::LH, LB = PlanB::LH, L = LA + LB;
+  constexpr int B_AT = BM * kRowBytes;
+  constexpr int STAGE = (BM + BN) * kRowBytes;
+  constexpr int NF = TM + TN;
+  constexpr int NMF = TM * TN;
+  constexpr int RPM = (2 * NF + NMF - 1) / NMF;               // 16-byte LDS reads behind each MFMA
+  static_assert(PlanA::TILE_ROWS == 8 && PlanA::TILE_LDS_BYTES == 8 * kRowBytes, "transfer tile");
+  static_assert(DT == ASTERGEMM_FP8_E4M3, "fp8 operands");
+  static_assert(NS * STAGE <= 160 * 1024, "LDS of a CU");
+  static_assert(LA * 8 * NW == BM && LB * 8 * NW == BN, "whole transfers");
+  static_assert((8 * NW) % 16 == 0, "swizzle phase must not depend on the transfer index");
+  static_assert(L <= NMF, "at most one transfer per MFMA");
+  static_assert((NS - 1) * L <= 63, "vmcnt field");
+
+  extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / WN, wn = wave % WN;
+  int tile_m, tile_n;
+  map_tile(bid, p.tiles_m, p.tiles_n, p.group_m, tile_m, tile_n);
+  const int row0 = tile_m * BM, col0 = tile_n * BN;
+
+  const int lrow = lane >> 3;
+  const int g_lane = (lane & 7) ^ (((wave * 8 + lrow) >> 1) & 7);
+  const unsigned a_off = (unsigned)(lrow * (int)p.lda_bytes + g_lane * 16);
+  const unsigned b_off = (unsigned)(lrow * (int)p.ldb_bytes + g_lane * 16);
+  const uint8_t* a_base[LA];
+  const uint8_t* b_base[LB];
+  group_bases<PlanA>(p.A, p.lda_bytes, row0, wave, p.M, a_base);
+  group_bases<PlanB>(p.B, p.ldb_bytes, col0, wave, p.N, b_base);
+  const int nk = p.ksteps - (p.tail_granules ? 1 : 0);
+
+  auto g2s = [&](const uint8_t* base, unsigned voff, uint8_t* dst) {
+    const unsigned m0v = (unsigned)(size_t)AG_LDS(dst);
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
+                 :
+                 : "s"(m0v), "v"(voff), "s"(base)
+                 : "memory", "m0");
+  };
+  // transfer j (0 ... L - 1) of K-step k: B's rows first, then A's
+  auto issue1 = [&](int k, int stage, auto jc) {
+    constexpr int J = decltype(jc)::value;
+    if constexpr (J < LB)
+      g2s(b_base[J] + (int64_t)k * kRowBytes, b_off,
+          lds + stage * STAGE + B_AT + PlanB::lds_offset(wave, J));
+    else
+      g2s(a_base[J - LB] + (int64_t)k * kRowBytes, a_off,
+          lds + stage * STAGE + PlanA::lds_offset(wave, J - LB));
+  };
+
+  const int li = lane & 15, lq = lane >> 4;
+  unsigned rd_off[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+    rd_off[h] = (unsigned)(li * kRowBytes + (((h * 4 + lq) ^ (li >> 1)) << 4));
+  const unsigned a_rd = (unsigned)(wm * TM * 16 * kRowBytes);
+  const unsigned b_rd = (unsigned)(B_AT + wn * TN * 16 * kRowBytes);
+  i32x8 fa[2][TM], fb[2][TN];
+  // read I: half I & 1 of fragment I / 2 (below TN a B tile, else an A tile) into set S
+  auto read_half = [&](int stage, auto set, auto idx) {
+    constexpr int S = decltype(set)::value;
+    constexpr int F = decltype(idx)::value / 2, H = decltype(idx)::value % 2;
+    const unsigned at = F < TN ? b_rd + F * 16 * kRowBytes : a_rd + (F - TN) * 16 * kRowBytes;
+    const i32x4 v = *(const i32x4*)(lds + stage * STAGE + at + rd_off[H]);
+    i32x8* f;
+    if constexpr (F < TN) f = &fb[S][F];
+    else f = &fa[S][F - TN];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) (*f)[H * 4 + e] = v[e];
+  };
+
+  f32x4 acc[TM][TN];
+#pragma unroll
+  for (int m = 0; m < TM; ++m)
+#pragma unroll
+    for (int n = 0; n < TN; ++n) acc[m][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  static_for<0, NS>([&](auto ic) {
+    constexpr int I = decltype(ic)::value;
+    if (nk > I) static_for<0, L>([&](auto jc) { issue1(I, I, jc); });
+  });
+  {
+    const int behind = (nk < NS ? nk : NS) - 1;  // K-steps requested behind K-step 0
+    static_for<0, NS>([&](auto ic) {
+      constexpr int I = decltype(ic)::value;
+      if (behind == I) __builtin_amdgcn_s_waitcnt(waitcnt_imm(I * L, 15));
+    });
+  }
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  static_for<0, 2 * NF>([&](auto ic) { read_half(0, std::integral_constant<int, 0>{}, ic); });
+  __builtin_amdgcn_sched_barrier(0);
+
+  // Trip k: K-step k + 1 has landed (k + 2 ... k + NS - 1 may be in flight) and K-step k is in
+  // registers for everybody, which frees its stage for k + NS.
+  int stage = 0;  // k mod NS
+  auto trip = [&](int k, auto set, auto steady) {
+    constexpr int S = decltype(set)::value;
+    const int next = stage + 1 == NS ? 0 : stage + 1;
+    constexpr bool STEADY = decltype(steady)::value;
+    const bool do_rd = STEADY || k + 1 < nk;
+    if (do_rd) {
+      if (STEADY || k + NS - 1 < nk) __builtin_amdgcn_s_waitcnt(waitcnt_imm((NS - 2) * L, 0));
+      else __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, 0));
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
+    const bool do_ld = STEADY || k + NS < nk;
+    static_for<0, NMF>([&](auto mc) {
+      constexpr int I = decltype(mc)::value;
+      constexpr int n = I / TM, m = I % TM;
+      // cbsz = blgp = 0: both operands OCP e4m3; zero scale operands select the unscaled form
+      acc[m][n] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fb[S][n], fa[S][m], acc[m][n], 0, 0,
+                                                                   0, 0, 0, 0);
+      if constexpr (I < L) {
+        if (do_ld) issue1(k + NS, stage, mc);
+      }
+      if (do_rd)
+        static_for<I * RPM, (I + 1) * RPM>([&](auto rc) {
+          if constexpr (decltype(rc)::value < 2 * NF)
+            read_half(next, std::integral_constant<int, S ^ 1>{}, rc);
+        });
+      __builtin_amdgcn_sched_barrier(0);
+    });
+    stage = next;
+  };
+  using S0 = std::integral_constant<int, 0>;
+  using S1 = std::integral_constant<int, 1>;
+  int k = 0;
+  // steady: K-step k + 1 + NS exists for the second trip of a pair
+#pragma unroll 1
+  for (; k + 2 + NS <= nk; k += 2) {
+    trip(k, S0{}, std::true_type{});
+    trip(k + 1, S1{}, std::true_type{});
+  }
+#pragma unroll 1
+  for (; k < nk; k += 2) {
+    trip(k, S0{}, std::false_type{});
+    if (k + 1 < nk) trip(k + 1, S1{}, std::false_type{});
+  }
+  __builtin_amdgcn_sched_barrier(0);
+
+  if (p.tail_granules) stream_k_tail<DT, BM, BN, WM, WN>(p, acc, wave, row0, col0, nk);
+  stream_epilogue<OUT, BM, BN, WM, WN, NS * STAGE>(p, acc, lds, wave, row0, col0);
+}
+
+template <int DT, int OUT, int BM, int BN, int WM, int WN, int NS>
+__global__ __launch_bounds__(WM* WN * 64) void gemm_streamr_kernel(const GemmArgs p) {
+  if constexpr (DT == ASTERGEMM_FP8_E4M3) gemm_stream8r_body<DT, OUT, BM, BN, WM, WN, NS>(p, blockIdx.x);
+  else gemm_streamr_body<DT, OUT, BM, BN, WM, WN, NS>(p, blockIdx.x);
+}
+
+// Split K (see gemm_stream_splitk_kernel): copy s of the tile grid multiplies K steps
+// [s * p.ksteps, (s + 1) * p.ksteps) into plane s of the fp32 workspace.
+template <int DT, int BM, int BN, int WM, int WN, int NS>
+__global__ __launch_bounds__(WM* WN * 64) void gemm_streamr_splitk_kernel(const GemmArgs p) {
+  const int tiles = p.tiles_m * p.tiles_n;
+  const int ks = blockIdx.x / tiles;
+  const int bid = blockIdx.x - ks * tiles;
+  GemmArgs q = p;
+  q.A = p.A + (int64_t)ks * p.ksteps * kRowBytes;
+  q.B = p.B + (int64_t)ks * p.ksteps * kRowBytes;
+  q.C = p.workspace + (int64_t)ks * p.M * p.N;
+  if constexpr (DT == ASTERGEMM_FP8_E4M3) gemm_stream8r_body<DT, ASTERGEMM_F32, BM, BN, WM, WN, NS>(q, bid);
+  else gemm_streamr_body<DT, ASTERGEMM_F32, BM, BN, WM, WN, NS>(q, bid);
 }
 
 }  // namespace

@@ -722,26 +722,56 @@ def test_nine_slot_ring_is_left_to_grids_of_one_workgroup_per_cu(gpu):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(8, 8, 64), (9, 136, 128), (191, 128, 192), (192, 120, 256), (193, 256, 320),
-                                   (255, 128, 384), (256, 264, 448), (257, 136, 512), (333, 1000, 576),
-                                   (384, 256, 1024), (400, 384, 1032), (777, 520, 72), (129, 248, 2040)])
-@pytest.mark.parametrize("tile", ["256x128_w4x2", "192x128_w4x2"])
-@pytest.mark.parametrize("dtype_ab,dtype_c", [("bf16", "bf16"), ("f16", "f32"), ("bf16", "f16")])
-def test_stream_unequal_tile_sides(gpu, M, N, K, tile, dtype_ab, dtype_c):
-    """The 256 x 128 and 192 x 128 kernels: K-step counts 1 ... 9, 16, 31 around the rings of three and
-    four stages (none, one and several groups of steady trips), tails of granules, heights around
-    the tiles and off the groups of 8 rows, the smallest operands.  Each output is the sum of the
-    same MFMAs in the same order as in the 128 x 128 kernel, so the bits are equal."""
-    a, b, _ = operands(M, N, K, dtype_ab, seed=71, b_std=0.05)
+@pytest.mark.parametrize("M,N,steps,tail", [(8, 8, 1, 0), (9, 136, 2, 0), (191, 128, 3, 0), (192, 120, 4, 0),
+                                            (193, 256, 5, 0), (255, 128, 6, 0), (256, 264, 7, 0),
+                                            (257, 136, 8, 0), (333, 1000, 9, 0), (384, 256, 16, 0),
+                                            (400, 384, 16, 1), (777, 520, 1, 1), (129, 248, 31, 7)])
+@pytest.mark.parametrize("dtype_ab,dtype_c,tile", [
+    (ab, c, t) for ab, c in (("bf16", "bf16"), ("f16", "f32"), ("bf16", "f16"), ("fp8_e4m3", "bf16"), ("fp8_e4m3", "f32"))
+    for t in ("256x128_w4x2", "192x128_w4x2", "128x128_w4x2") if ab == "fp8_e4m3" or not t.startswith("128")])
+def test_stream_unequal_tile_sides(gpu, M, N, steps, tail, tile, dtype_ab, dtype_c):
+    """The 256 x 128 and 192 x 128 kernels (fp8 also 128 x 128 with eight waves): 128-byte K-steps 1 ... 9,
+    16, 31 around the rings of three, four and five stages (none, one and several groups of steady
+    trips), tails of 16-byte granules, heights around the tiles and off the groups of 8 rows, the
+    smallest operands.  Each output is the sum of the same MFMAs in the same order as in the square
+    128 x 128 kernel, so the bits are equal."""
+    fp8 = dtype_ab == "fp8_e4m3"
+    K = (steps * 128 + tail * 16) // (1 if fp8 else 2)
+    a, b, ex = operands(M, N, K, dtype_ab, seed=71, b_std=0.05)
     bias = np.random.default_rng(72).standard_normal(N).astype(np.float32)
+    pre = "stream_fp8" if fp8 else f"stream_{dtype_ab}"
     out, name = run_gemm(a, b, M, N, K, dtype_ab, dtype_c, bias=bias,
-                         variant=_variant_id(f"stream_{dtype_ab}_{tile}_{dtype_c}"))
-    assert name == f"stream_{dtype_ab}_{tile}_{dtype_c}"
+                         variant=_variant_id(f"{pre}_{tile}_{dtype_c}"), **ex)
+    assert name == f"{pre}_{tile}_{dtype_c}"
     square, _ = run_gemm(a, b, M, N, K, dtype_ab, dtype_c, bias=bias,
-                         variant=_variant_id(f"stream_{dtype_ab}_128x128_w2x2_{dtype_c}"))
+                         variant=_variant_id(f"{pre}_128x128_w2x2_{dtype_c}"), **ex)
     assert np.array_equal(out, square)
-    check(out, G.gemm(a, b, _DT[dtype_ab], _DT[dtype_c], bias=bias), dtype_c, N,
-          bar=REL_L2_BAR if dtype_c != "f32" else 1e-5)
+    want = (G.gemm_fp8(a, b, ex["scale_a"], ex["scale_b"], out_dtype=_DT[dtype_c], bias=bias) if fp8
+            else G.gemm(a, b, _DT[dtype_ab], _DT[dtype_c], bias=bias))
+    # the fp8 MFMA adds its 128 products in a width narrower than fp32 (measured rel-L2 about 1.3e-5)
+    check(out, want, dtype_c, N, bar=REL_L2_BAR if dtype_c != "f32" else 1e-4 if fp8 else 1e-5)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,dtype_ab,dtype_c", [(129, 1032, "bf16", "bf16"), (300, 1288, "bf16", "f32"),
+                                                  (512, 2048, "f16", "f16"), (500, 4096, "fp8_e4m3", "bf16"),
+                                                  (257, 4096, "fp8_e4m3", "f32")])
+def test_split_k_on_unequal_tiles(gpu, M, N, dtype_ab, dtype_c):
+    """Split K on 256 x 128 tiles: edge tiles, a padded output pitch, two and four ranges, the same
+    bits on a second run."""
+    fp8 = dtype_ab == "fp8_e4m3"
+    K = 14336
+    a, b, ex = operands(M, N, K, dtype_ab, seed=95, b_std=0.05)
+    bias = np.random.default_rng(96).standard_normal(N).astype(np.float32)
+    name = f"splitk_{'fp8' if fp8 else dtype_ab}_256x128_w4x2_{dtype_c}"
+    run = lambda: run_gemm(a, b, M, N, K, dtype_ab, dtype_c, bias=bias, ldc=N + 8,
+                           variant=_variant_id(name), **ex)
+    out, ran = run()
+    assert ran == name
+    want = (G.gemm_fp8(a, b, ex["scale_a"], ex["scale_b"], out_dtype=_DT[dtype_c], bias=bias) if fp8
+            else G.gemm(a, b, _DT[dtype_ab], _DT[dtype_c], bias=bias))
+    check(out, want, dtype_c, N, bar=REL_L2_BAR if dtype_c != "f32" else 1e-4 if fp8 else 1e-5)
+    assert np.array_equal(out[:, :N].view(np.uint8), run()[0][:, :N].view(np.uint8))
 
 
 # ---- edge cases: ragged M / N, K tails, leading dimensions, epilogue -----------------

@@ -115,6 +115,28 @@ def test_selection_of_unequal_tile_sides(shape, tile, dtype_ab, dtype_c):
             create(M, N, K, wg_tile=wg)
 
 
+@pytest.mark.parametrize("shape,name", [
+    ((500, 4096, 14336), "splitk_{}_256x128_w4x2"),
+    ((256, 4096, 14336), "splitk_{}_128x128_w2x2"),    # as many operand rows per CU as before
+    ((128, 4096, 14336), "splitk_{}_128x128_w2x2"),
+    ((2000, 1024, 8192), "{}_128x128"),                # few tile columns
+    ((500, 4096, 14352), "{}_128x128"),                # K tail
+    ((333, 14336, 4096), "stream_{}_192x128_w4x2"),
+    ((500, 11008, 4096), "stream_{}_256x128_w4x2"),
+    ((1500, 8192, 8192), "stream_{}_256x256_w2x4"),
+])
+def test_selection_of_unequal_tile_sides_bf16_and_fp8(shape, name):
+    """The lines that both operand widths share, and what stays with the square tiles."""
+    for dtype, tag in (("bf16", "bf16"), ("fp8_e4m3", "fp8")):
+        got = gemm.GemmPlan.create(*shape, dtype, "bf16").info.name.decode()
+        if "_128x128" in name:
+            assert "128x128" in got, (dtype, got)
+        else:
+            assert got == name.format(tag) + "_bf16", (dtype, got)
+    p = gemm.GemmPlan.create(500, 4096, 14336, "bf16", "bf16")
+    assert p.workspace_bytes() == 4 * 500 * 4096 * 4 and p.info.grid_x == 64 * 4
+
+
 def test_explicit_variant_and_enumeration():
     lib = _capi.load()
     n = lib.astergemm_variant_count()
