@@ -25,7 +25,8 @@ LIB_PATH = os.path.join(LIB_DIR, "libastergemm.so")
 OBJ_DIR = os.path.join(ROOT, "build", "obj")
 
 # (object stem, source file, extra flags).  gemm_stream.hip holds the variant table of the stream
-# kernels in five parts (bf16, fp8, MXFP4, f16 operands, 16-bit operands on unequal tile sides) and is compiled once per part.
+# kernels in five parts (bf16, fp8, MXFP4, f16 operands, unequal tile sides) and is compiled once
+# per part.
 UNITS = [("gemm_stream_p0", "gemm_stream.hip", ["-DAG_STREAM_PART=0"]),
          ("gemm_stream_p3", "gemm_stream.hip", ["-DAG_STREAM_PART=3"]),
          ("gemm_stream_p2", "gemm_stream.hip", ["-DAG_STREAM_PART=2"]),

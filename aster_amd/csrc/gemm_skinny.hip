@@ -1066,7 +1066,9 @@ int launch_skinny_fp4m_t(const GemmArgs& a0, int S, hipStream_t s) {
   const KRangeGrid kg = krange_grid(MH, a.N, S, cus);
   a.tiles_n = kg.rows;
   a.split_k = S;
+  std::unique_lock<std::mutex> order;  // see splitk_order
   if (S > 1 && !a.workspace) {
+    order = std::unique_lock<std::mutex>(splitk_order());
     if (int rc = splitk_workspace((size_t)S * a.M * a.N * sizeof(float), s, &a.workspace)) return rc;
   }
   AG_LAUNCH_KERNEL(k, dim3(kg.grid), dim3(512), lds, s, a);
@@ -1408,7 +1410,9 @@ int launch_skinny_regm_t(const GemmArgs& a0, int S, hipStream_t s) {
   const KRangeGrid kg = krange_grid(MH, a.N, S, cus);
   a.tiles_n = kg.rows;
   a.split_k = S;
+  std::unique_lock<std::mutex> order;  // see splitk_order
   if (S > 1 && !a.workspace) {
+    order = std::unique_lock<std::mutex>(splitk_order());
     if (int rc = splitk_workspace((size_t)S * a.M * a.N * sizeof(float), s, &a.workspace)) return rc;
   }
   AG_LAUNCH_KERNEL(k, dim3(kg.grid), dim3(512), lds, s, a);
@@ -2015,6 +2019,11 @@ const Variant* skinny_variants() { return kSkinnyVariants; }
 
 int splitk_workspace_for(size_t bytes, hipStream_t stream, float** out) {
   return splitk_workspace(bytes, stream, out);
+}
+
+std::mutex& splitk_order() {
+  static std::mutex m;
+  return m;
 }
 
 void splitk_workspace_release(hipStream_t stream) { splitk_workspace_drop(stream); }

@@ -1,6 +1,7 @@
 // Stream kernels (whole-ring, hand-scheduled MFMA loops) for f16 / bf16, fp8 and MXFP4:
 // launchers, shape checks and the variant table.  Kept apart from gemm_tile.hip so that the
 // two halves of the kernel set compile side by side.
+#include <mutex>
 #include <vector>
 
 #include "gemm_stream_kernel.hpp"
@@ -278,7 +279,9 @@ int launch_stream_splitk(const GemmArgs& a0, int grid, hipStream_t s) {
   const int S = stream_split_of(tiles, a0.ksteps, KIND == 2);
   if (S == 0) return (int)hipErrorInvalidValue;
   GemmArgs a = a0;
+  std::unique_lock<std::mutex> order;  // see splitk_order
   if (!a.workspace) {
+    order = std::unique_lock<std::mutex>(splitk_order());
     if (int rc = splitk_workspace_for((size_t)S * a.M * a.N * sizeof(float), s, &a.workspace))
       return rc;
   }
@@ -341,7 +344,9 @@ int launch_streamr_splitk(const GemmArgs& a0, int grid, hipStream_t s) {
   const int S = streamr_split_of(tiles, a0.ksteps);
   if (S == 0 || a0.tail_granules != 0) return (int)hipErrorInvalidValue;
   GemmArgs a = a0;
+  std::unique_lock<std::mutex> order;  // see splitk_order
   if (!a.workspace) {
+    order = std::unique_lock<std::mutex>(splitk_order());
     if (int rc = splitk_workspace_for((size_t)S * a.M * a.N * sizeof(float), s, &a.workspace))
       return rc;
   }
@@ -695,7 +700,8 @@ int grid_stream_tail(const astergemm_config& c, int cus) {
       AG_STREAM(prefix "_128x128_w2x2_f16", DT, ASTERGEMM_F16, 128, 128, 2, 2)
 
 // The table is compiled in five parts (this file once per AG_STREAM_PART: bf16, fp8, MXFP4 and f16
-// operands, and 16-bit operands on unequal tile sides), so that the parts build side by side and work on one family recompiles one part.
+// operands, and unequal tile sides), so that the parts build side by side and work on one family
+// recompiles one part.
 #ifndef AG_STREAM_PART
 #error "compile with -DAG_STREAM_PART=0, 1, 2, 3 or 4"
 #endif
