@@ -138,6 +138,7 @@ struct ChoiceCacheEntry {
   astergemm_config cfg;
   int dev;
   int index;
+  bool plain;
 };
 constexpr int kChoiceCache = 16;
 thread_local ChoiceCacheEntry g_choice_cache[kChoiceCache];
@@ -219,24 +220,34 @@ bool unequal_split_pays(const astergemm_config& c) {
   return steps / S * 384 * 4 <= square * 3;
 }
 
-const Variant* choose_uncached(const astergemm_config& c, int* index_out);
+// Split K where a kernel without K ranges (or with fewer) takes the problem too: 256 x 128 tiles, and
+// 128 x 128 tiles of a ragged M.  A call that has no scratch of its own for them -- the built-in scratch
+// or a caller's workspace too small, a stream under capture, whose graph may be replayed beside other work
+// on the library's buffer -- runs the other kernel instead of being refused.
+bool optional_split(const Variant& v, const astergemm_config& c) {
+  return v.family == ASTERGEMM_KERNEL_TILE && (v.rank == 6 || (v.rank == 4 && c.M % 8 != 0));
+}
 
-// Picks the variant for cfg; on failure returns nullptr with the error set.
-const Variant* choose(const astergemm_config& c, int* index_out) {
+const Variant* choose_uncached(const astergemm_config& c, int* index_out, bool plain);
+
+// Picks the variant for cfg (`plain`: leaving the optional splits out); on failure returns nullptr with
+// the error set.
+const Variant* choose(const astergemm_config& c, int* index_out, bool plain = false) {
   const int dev = current_device_or_minus_one();
   for (int i = 0; i < g_choice_cache_used; ++i) {
     const ChoiceCacheEntry& e = g_choice_cache[i];
-    if (e.dev == dev && memcmp(&e.cfg, &c, sizeof(c)) == 0) {
+    if (e.dev == dev && e.plain == plain && memcmp(&e.cfg, &c, sizeof(c)) == 0) {
       if (index_out) *index_out = e.index;
       return variant_at(e.index);
     }
   }
   int index = -1;
-  const Variant* v = choose_uncached(c, &index);
+  const Variant* v = choose_uncached(c, &index, plain);
   if (!v) return nullptr;  // refusals are not remembered: the message is made again
   ChoiceCacheEntry& e = g_choice_cache[g_choice_cache_next];
   memcpy(&e.cfg, &c, sizeof(c));
   e.dev = dev;
+  e.plain = plain;
   e.index = index;
   g_choice_cache_next = (g_choice_cache_next + 1) % kChoiceCache;
   if (g_choice_cache_used < kChoiceCache) ++g_choice_cache_used;
@@ -244,7 +255,7 @@ const Variant* choose(const astergemm_config& c, int* index_out) {
   return v;
 }
 
-const Variant* choose_uncached(const astergemm_config& c, int* index_out) {
+const Variant* choose_uncached(const astergemm_config& c, int* index_out, bool plain) {
   g_choose_rc = ASTERGEMM_ENOTSUP;
   if (const char* why = validate_problem(c)) {
     set_error("astergemm: invalid config: %s", why);
@@ -279,13 +290,14 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out) {
   // partial sums than split K on the 128 x 128 kernel (bf16 64x8192x28672: 107 against 94 us;
   // 64x4096x28672 level at 57.5 against 58.5); up to 32 KiB the decode kernel is ahead
   // (64x8192x16384: 60 against 81 us, 64x14336x8192: 53 against 63, fp8 64x8192x28672: 56
-  // against 60)
+  // against 60).  Not for M off the groups of 8: f16 50x8192x28672 91 against 100 us back to back, but
+  // 127 against 110 on buffers that no kernel has read yet
   if (c.family == ASTERGEMM_KERNEL_AUTO && family == ASTERGEMM_KERNEL_SKINNY && c.M > 32 &&
       (is16 || c.dtype_ab == ASTERGEMM_FP8_E4M3) && row_bytes(c.dtype_ab, c.K) > 32768) {
     for (int i = 0; i < total_variants(); ++i) {
       const Variant* v = variant_at(i);
       if (v->family == ASTERGEMM_KERNEL_TILE && v->rank == 4 && variant_matches_types(*v, c) &&
-          v->check(c) == nullptr) {
+          !optional_split(*v, c) && v->check(c) == nullptr) {
         family = ASTERGEMM_KERNEL_TILE;
         break;
       }
@@ -306,6 +318,7 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out) {
     if (v->family != family || !variant_matches_types(*v, c)) continue;
     if (v->rank == 5 && v->tile_m != unequal) continue;
     if (v->rank == 6 && !unequal_split) continue;
+    if (plain && optional_split(*v, c)) continue;
     if (const char* why = v->check(c)) {
       if (!last_why) last_why = why;
       continue;
@@ -545,6 +558,57 @@ int build_args(const Variant& v, const astergemm_config& c, const astergemm_oper
   return 0;
 }
 
+bool is_capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (!s) return false;  // the null stream is never captured
+  if (hipStreamIsCapturing(s, &st) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return st != hipStreamCaptureStatusNone;
+}
+
+// What a call with these operands on this stream runs: cfg's variant, or for an optional split without
+// scratch of the call's own the kernel it stands in for; *other is then the one of the two that does
+// not run (nullptr for configs with one kernel).
+const Variant* choose_for_call(const astergemm_config& c, const astergemm_operands& ops, void* stream,
+                               const Variant** other = nullptr) {
+  const Variant* v = choose(c, nullptr);
+  if (other) *other = nullptr;
+  if (!v || c.variant != 0 || !optional_split(*v, c)) return v;
+  const Variant* plain = choose(c, nullptr, true);
+  const bool fits = ops.dWorkspace ? ops.workspace_bytes >= workspace_need(*v, c)
+                                   : !is_capturing((hipStream_t)stream);
+  if (other) *other = fits ? plain : v;
+  return fits ? v : plain;
+}
+
+// The one-time steps of v's first launch, without a launch; the operands are never read.
+int prime(const Variant& v, const astergemm_config& c, void* any, size_t any_bytes, void* stream) {
+  GemmArgs a;
+  astergemm_operands o;
+  memset(&o, 0, sizeof(o));
+  o.dA = o.dB = o.dC = any;
+  o.dScaleA = o.dScaleB = o.dBias = (const float*)any;
+  o.dMxA = o.dMxB = (const uint8_t*)any;
+  if (any_bytes) {
+    o.dWorkspace = any;
+    o.workspace_bytes = any_bytes;
+  }
+  if (int rc = build_args(v, c, o, &a)) return rc;
+  (void)hipGetLastError();
+  LaunchScope scope(stream, /*prepare_only=*/true);
+  const int e = v.launch(a, grid_of(v, c), (hipStream_t)stream);
+  return e != 0 ? launch_fail(e, v.name, __FILE__, __LINE__) : 0;
+}
+
+// A config with an optional split has two kernels: an eager launch of one readies the other, so that a
+// later capture finds either of them ready; with `library_ws` also the stream's workspace.
+void prime_other(const Variant* other, const astergemm_config& c, void* stream, bool library_ws) {
+  if (other && !is_capturing((hipStream_t)stream))
+    (void)prime(*other, c, (void*)(uintptr_t)4096, library_ws ? 0 : (size_t)-1, stream);
+}
+
 // ---- the entry point that allocates nothing ------------------------------------------------
 // Partial sums of rows cut into K ranges go to this array instead of an allocation.  Its name is
 // a host-side handle only: the device address is looked up once per device.
@@ -644,16 +708,19 @@ int astergemm_run(const astergemm_config* cfg, const astergemm_operands* ops, vo
     set_error("astergemm_run: null argument");
     return ASTERGEMM_EINVAL;
   }
-  int index = -1;
-  const Variant* v = choose(*cfg, &index);
+  const Variant* other = nullptr;
+  const Variant* v = choose_for_call(*cfg, *ops, stream, &other);
   if (!v) return g_choose_rc;
   if (cfg->M == 0 || cfg->N == 0) return 0;
   GemmArgs a;
   if (int rc = build_args(*v, *cfg, *ops, &a)) return rc;
   (void)hipGetLastError();  // the launchers report hipGetLastError(): drop what an earlier call left
-  LaunchScope scope(stream);
-  const int e = v->launch(a, grid_of(*v, *cfg), (hipStream_t)stream);
-  if (e != 0) return launch_fail(e, v->name, __FILE__, __LINE__);
+  {
+    LaunchScope scope(stream);
+    const int e = v->launch(a, grid_of(*v, *cfg), (hipStream_t)stream);
+    if (e != 0) return launch_fail(e, v->name, __FILE__, __LINE__);
+  }
+  prime_other(other, *cfg, stream, /*library_ws=*/!ops->dWorkspace);
   return 0;
 }
 
@@ -675,22 +742,13 @@ int astergemm_prepare(const astergemm_config* cfg) {
   // The launcher runs with every one-time step (function attributes, cached device facts) and
   // without the kernel launches; the operands are never read.  Partial sums, where the config
   // has any, point at the built-in scratch when they fit, so that nothing is allocated either.
-  GemmArgs a;
-  astergemm_operands o;
-  memset(&o, 0, sizeof(o));
-  o.dA = o.dB = o.dC = scratch_ptr;
-  o.dScaleA = o.dScaleB = o.dBias = (const float*)scratch_ptr;
-  o.dMxA = o.dMxB = (const uint8_t*)scratch_ptr;
-  if (workspace_need(*v, *cfg) <= (size_t)ASTERGEMM_NOALLOC_SCRATCH_BYTES) {
-    o.dWorkspace = scratch_ptr;
-    o.workspace_bytes = (size_t)ASTERGEMM_NOALLOC_SCRATCH_BYTES;
-  }
-  if (int rc = build_args(*v, *cfg, o, &a)) return rc;
-  (void)hipGetLastError();
-  LaunchScope scope(nullptr, /*prepare_only=*/true);
-  const int e = v->launch(a, grid_of(*v, *cfg), nullptr);
-  if (e != 0) return launch_fail(e, v->name, __FILE__, __LINE__);
-  return 0;
+  const bool optional = cfg->variant == 0 && optional_split(*v, *cfg);
+  const size_t need = workspace_need(*v, *cfg), scratch = ASTERGEMM_NOALLOC_SCRATCH_BYTES;
+  if (int rc = prime(*v, *cfg, scratch_ptr, need <= scratch ? scratch : optional ? need : 0, nullptr))
+    return rc;
+  if (!optional) return 0;
+  v = choose(*cfg, &index, true);
+  return v ? prime(*v, *cfg, scratch_ptr, (size_t)-1, nullptr) : g_choose_rc;
 }
 
 int astergemm_workspace_bytes(const astergemm_config* cfg, size_t* bytes) {
@@ -711,8 +769,13 @@ int astergemm_run_noalloc(const astergemm_config* cfg, const astergemm_operands*
     set_error("astergemm_run_noalloc: null argument");
     return ASTERGEMM_EINVAL;
   }
-  int index = -1;
-  const Variant* v = choose(*cfg, &index);
+  // calls on one device share the built-in scratch: an optional split does not bring a config to it
+  const Variant* v = choose(*cfg, nullptr);
+  const Variant* other = nullptr;
+  if (v && cfg->variant == 0 && optional_split(*v, *cfg)) {
+    other = v;
+    v = choose(*cfg, nullptr, /*plain=*/true);
+  }
   if (!v) return g_choose_rc;
   if (cfg->M == 0 || cfg->N == 0) return 0;
   const size_t need = workspace_need(*v, *cfg);
@@ -734,9 +797,12 @@ int astergemm_run_noalloc(const astergemm_config* cfg, const astergemm_operands*
   GemmArgs a;
   if (int rc = build_args(*v, *cfg, o, &a)) return rc;
   (void)hipGetLastError();
-  LaunchScope scope(stream);
-  const int e = v->launch(a, grid_of(*v, *cfg), (hipStream_t)stream);
-  if (e != 0) return launch_fail(e, v->name, __FILE__, __LINE__);
+  {
+    LaunchScope scope(stream);
+    const int e = v->launch(a, grid_of(*v, *cfg), (hipStream_t)stream);
+    if (e != 0) return launch_fail(e, v->name, __FILE__, __LINE__);
+  }
+  prime_other(other, *cfg, stream, /*library_ws=*/false);
   return 0;
 }
 
@@ -746,8 +812,7 @@ int astergemm_bench_rotate(const astergemm_config* cfg, const astergemm_operands
     set_error("astergemm_bench_rotate: bad argument");
     return ASTERGEMM_EINVAL;
   }
-  int index = -1;
-  const Variant* v = choose(*cfg, &index);
+  const Variant* v = choose_for_call(*cfg, ops[0], stream);
   if (!v) return g_choose_rc;
   *total_ns = 0;
   if (cfg->M == 0 || cfg->N == 0) return 0;
@@ -777,8 +842,7 @@ int astergemm_bench_graph(const astergemm_config* cfg, const astergemm_operands*
     set_error("astergemm_bench_graph: bad argument");
     return ASTERGEMM_EINVAL;
   }
-  int index = -1;
-  const Variant* v = choose(*cfg, &index);
+  const Variant* v = choose_for_call(*cfg, ops[0], nullptr);
   if (!v) return g_choose_rc;
   *total_ns = 0;
   if (cfg->M == 0 || cfg->N == 0) return 0;
@@ -898,8 +962,7 @@ int astergemm_bench(const astergemm_config* cfg, const astergemm_operands* ops, 
     set_error("astergemm_bench: bad argument");
     return ASTERGEMM_EINVAL;
   }
-  int index = -1;
-  const Variant* v = choose(*cfg, &index);
+  const Variant* v = choose_for_call(*cfg, *ops, stream);
   if (!v) return g_choose_rc;
   if (cfg->M == 0 || cfg->N == 0) {
     for (int i = 0; i < iters; ++i) times_ns[i] = 0;

@@ -239,7 +239,8 @@ int astergemm_workspace_bytes(const astergemm_config* cfg, size_t* bytes);
  * the reference.  ops->dWorkspace is ignored: the partial sums of K ranges go
  * to a scratch array built into the library, ASTERGEMM_NOALLOC_SCRATCH_BYTES
  * per device, held until the process ends; a config that needs more is refused
- * with ASTERGEMM_EINVAL.  Every call on a device shares that array, whatever
+ * with ASTERGEMM_EINVAL, unless a kernel without K ranges (or with fewer) takes
+ * it, which then runs.  Every call on a device shares that array, whatever
  * its stream: calls that overlap on one device race (calls on one stream are
  * ordered and safe).  Nothing in the array has to start at zero: every launch
  * writes all the planes it later adds.  The array's address is looked up on

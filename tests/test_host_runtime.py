@@ -379,6 +379,21 @@ def test_workspace_query_and_caller_workspace_checks():
         gemm.GemmPlan.create(256, 256, 256).run_noalloc(None, None, None)
 
 
+@pytest.mark.parametrize("M,N,K", [(500, 4096, 14336), (333, 4096, 14336), (250, 8192, 28672)])
+def test_split_k_does_not_refuse_a_call_without_scratch(M, N, K):
+    """Problems that a kernel without K ranges takes too: AUTO cuts them, and a call whose scratch does not
+    hold the partial sums gets that kernel (here: as far as the checks of its pointers)."""
+    p = gemm.GemmPlan.create(M, N, K)
+    assert p.workspace_bytes() > _capi.NOALLOC_SCRATCH_BYTES
+    with pytest.raises(_capi.AsterGemmError, match="non-null"):
+        p.run_noalloc(None, None, None)
+    with pytest.raises(_capi.AsterGemmError, match="dWorkspace must be 16-byte aligned"):
+        p.run(4096, 4096, 4096, workspace=4096 + 4, workspace_bytes=16)
+    with pytest.raises(_capi.AsterGemmError, match="workspace of"):  # a kernel asked for by number is that one
+        gemm.GemmPlan.create(M, N, K, variant=p.info.variant).run(4096, 4096, 4096, workspace=4096,
+                                                                  workspace_bytes=16)
+
+
 def test_reported_grid_is_the_launched_grid_of_the_k_range_kernels():
     # S K ranges x R row ranges, one workgroup per CU: the description comes from the same
     # function the launcher uses (the number of CUs is 0 without a device: one row range)

@@ -70,6 +70,42 @@ def test_noalloc_refuses_what_the_scratch_cannot_hold(gpu):
     assert err.value.code == -22 and "scratch" in str(err.value)
 
 
+@pytest.mark.parametrize("M,N,K", [(333, 4096, 14336), (130, 1032, 8192)])
+def test_split_configs_without_scratch_of_their_own(gpu, M, N, K):
+    """AUTO cuts these into K ranges where the library's buffer may be used; the entry point without
+    allocations and a capture (several replays, eager work between them) run the other kernel."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    b = (torch.randn(N, K, generator=g, device="cuda") * 0.02).to(torch.bfloat16)
+    ref = a.float() @ b.float().T
+    plan = AG.GemmPlan.create(M, N, K, "bf16", "bf16")
+    assert plan.workspace_bytes() > 0
+    c = torch.zeros(M, N, device="cuda", dtype=torch.bfloat16)
+
+    def check():
+        torch.cuda.synchronize()
+        rel = float((c.float() - ref).norm() / ref.norm())
+        c.zero_()
+        assert rel <= 4e-3, rel      # bf16 rounding of the output, 1.7e-3, and the order of fp32 sums
+
+    ptrs = (a.data_ptr(), b.data_ptr(), c.data_ptr())
+    print(f"{plan.info.name.decode()} M={M} N={N} K={K}", flush=True)
+    torch.cuda.synchronize()
+    plan.run(*ptrs)
+    check()
+    plan.run_noalloc(*ptrs)
+    check()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        plan.run(*ptrs, stream=torch.cuda.current_stream().cuda_stream)
+    for _ in range(3):
+        graph.replay()
+        check()
+        plan.run(*ptrs)
+        check()
+
+
 def test_caller_workspace_matches_the_library_workspace(gpu):
     M, N, K = 96, 1000, 16384
     rng = np.random.default_rng(11)
