@@ -137,6 +137,11 @@ def test_selection_of_unequal_tile_sides_bf16_and_fp8(shape, name):
     assert p.workspace_bytes() == 4 * 500 * 4096 * 4 and p.info.grid_x == 64 * 4
 
 
+def test_long_decode_rows_off_the_groups_of_8_stay_with_the_decode_kernel():
+    for M, start in ((33, "skinnyx_"), (50, "skinnyx_"), (56, "splitk_"), (63, "skinnyx_"), (64, "splitk_")):
+        assert gemm.GemmPlan.create(M, 8192, 28672, "f16", "f16").info.name.decode().startswith(start), M
+
+
 def test_explicit_variant_and_enumeration():
     lib = _capi.load()
     n = lib.astergemm_variant_count()
