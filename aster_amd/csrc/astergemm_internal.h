@@ -154,8 +154,9 @@ inline int streamr_split_of(int64_t tiles, int64_t ksteps) {
 // workspace of a (device, stream), and the kernel that adds `splits` planes [M][N] of
 // a.workspace in index order, applies a's scales and bias and stores a.C in `out_dtype`.
 int splitk_workspace_for(size_t bytes, hipStream_t stream, float** out);
-// Held by a launcher from the lookup of the library's workspace to the launch of the kernel that adds it
-// up: two host threads on one stream would otherwise enqueue product, product, sum, sum.
+// Held by a launcher from the lookup of the workspace to the launch of the kernel that adds it up, whoever
+// owns that memory (the library's buffer of the stream, the built-in scratch, the caller): two host threads
+// on one stream that share it would otherwise enqueue product, product, sum, sum.
 std::mutex& splitk_order();
 // Frees the workspace of a (synchronised) stream that is about to be destroyed.
 void splitk_workspace_release(hipStream_t stream);

@@ -1067,8 +1067,8 @@ int launch_skinny_fp4m_t(const GemmArgs& a0, int S, hipStream_t s) {
   a.tiles_n = kg.rows;
   a.split_k = S;
   std::unique_lock<std::mutex> order;  // see splitk_order
+  if (S > 1) order = std::unique_lock<std::mutex>(splitk_order());
   if (S > 1 && !a.workspace) {
-    order = std::unique_lock<std::mutex>(splitk_order());
     if (int rc = splitk_workspace((size_t)S * a.M * a.N * sizeof(float), s, &a.workspace)) return rc;
   }
   AG_LAUNCH_KERNEL(k, dim3(kg.grid), dim3(512), lds, s, a);
@@ -1411,8 +1411,8 @@ int launch_skinny_regm_t(const GemmArgs& a0, int S, hipStream_t s) {
   a.tiles_n = kg.rows;
   a.split_k = S;
   std::unique_lock<std::mutex> order;  // see splitk_order
+  if (S > 1) order = std::unique_lock<std::mutex>(splitk_order());
   if (S > 1 && !a.workspace) {
-    order = std::unique_lock<std::mutex>(splitk_order());
     if (int rc = splitk_workspace((size_t)S * a.M * a.N * sizeof(float), s, &a.workspace)) return rc;
   }
   AG_LAUNCH_KERNEL(k, dim3(kg.grid), dim3(512), lds, s, a);

@@ -279,9 +279,8 @@ int launch_stream_splitk(const GemmArgs& a0, int grid, hipStream_t s) {
   const int S = stream_split_of(tiles, a0.ksteps, KIND == 2);
   if (S == 0) return (int)hipErrorInvalidValue;
   GemmArgs a = a0;
-  std::unique_lock<std::mutex> order;  // see splitk_order
+  std::lock_guard<std::mutex> order(splitk_order());
   if (!a.workspace) {
-    order = std::unique_lock<std::mutex>(splitk_order());
     if (int rc = splitk_workspace_for((size_t)S * a.M * a.N * sizeof(float), s, &a.workspace))
       return rc;
   }
@@ -344,9 +343,8 @@ int launch_streamr_splitk(const GemmArgs& a0, int grid, hipStream_t s) {
   const int S = streamr_split_of(tiles, a0.ksteps);
   if (S == 0 || a0.tail_granules != 0) return (int)hipErrorInvalidValue;
   GemmArgs a = a0;
-  std::unique_lock<std::mutex> order;  // see splitk_order
+  std::lock_guard<std::mutex> order(splitk_order());
   if (!a.workspace) {
-    order = std::unique_lock<std::mutex>(splitk_order());
     if (int rc = splitk_workspace_for((size_t)S * a.M * a.N * sizeof(float), s, &a.workspace))
       return rc;
   }

@@ -130,6 +130,70 @@ def test_caller_workspace_matches_the_library_workspace(gpu):
         bf.free()
 
 
+@pytest.mark.parametrize("M,N,K,dtype,kernel", [
+    (128, 1024, 8192, "bf16", "splitk_bf16_128x128_w2x2_bf16"),
+    (129, 1032, 8192, "bf16", "splitk_bf16_256x128_w4x2_bf16"),
+    (50, 1032, 28672, "bf16", "skinnyx_bf16_m64_bf16"), (16, 520, 14336, "mxfp4", "skinnyx_mxfp4_m64_bf16")])
+def test_two_host_threads_on_one_stream_keep_products_and_sums_in_pairs(gpu, M, N, K, dtype, kernel):
+    """Split K and the K ranges of the decode kernels: two threads enqueue different activations on one
+    stream and share the partial sums' memory (the library's buffer, the built-in scratch, a caller's
+    buffer); each call's product and sum stay together, so every output has the bits of the call alone."""
+    import threading
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M)
+    if dtype == "mxfp4":
+        draw = lambda rows: torch.randint(0, 256, (rows, K // 2), generator=g, device="cuda", dtype=torch.uint8)
+        mx = lambda rows: torch.randint(118, 123, (rows, K // 32), generator=g, device="cuda", dtype=torch.uint8)
+        mb, mas = mx(N), [mx(M) for _ in range(2)]
+        scales = [dict(mx_a=m.data_ptr(), mx_b=mb.data_ptr()) for m in mas]
+    else:
+        draw = lambda rows: torch.randn(rows, K, generator=g, device="cuda").to(torch.bfloat16)
+        scales = [{}, {}]
+    w, xs = draw(N), [draw(M) for _ in range(2)]
+    lib, info = _capi.load(), _capi.KernelInfo()
+    plan = AG.GemmPlan.create(M, N, K, dtype, "bf16")
+    for i in range(lib.astergemm_variant_count()):
+        _capi.check(lib.astergemm_variant_info(i, ctypes.byref(plan.config), ctypes.byref(info)))
+        if info.name.decode() == kernel:
+            plan = AG.GemmPlan.create(M, N, K, dtype, "bf16", variant=info.variant)
+    assert plan.info.name.decode() == kernel
+    need = plan.workspace_bytes()
+    assert 0 < need <= _capi.NOALLOC_SCRATCH_BYTES
+    own = torch.zeros(need, device="cuda", dtype=torch.uint8)
+    want = torch.zeros(2, M, N, device="cuda", dtype=torch.bfloat16)
+    n = 100
+    outs = torch.zeros(2, n, M, N, device="cuda", dtype=torch.bfloat16)
+    torch.cuda.synchronize()
+    for i in range(2):
+        plan.run(xs[i].data_ptr(), w.data_ptr(), want[i].data_ptr(), **scales[i])
+    assert not torch.equal(want[0], want[1])
+    for way in ("run", "run_noalloc", "caller"):
+        print(f"{way} {plan.info.name.decode()} M={M} N={N} K={K}", flush=True)
+        outs.zero_()
+        torch.cuda.synchronize()
+        call = plan.run_noalloc if way == "run_noalloc" else plan.run
+        extra = dict(workspace=own.data_ptr(), workspace_bytes=need) if way == "caller" else {}
+        start, failed = threading.Barrier(2), []
+
+        def work(i):
+            try:
+                start.wait(30)
+                for r in range(n):
+                    call(xs[i].data_ptr(), w.data_ptr(), outs[i, r].data_ptr(), **scales[i], **extra)
+            except Exception as exc:
+                failed.append(exc)
+
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        torch.cuda.synchronize()
+        assert not failed, failed
+        for i in range(2):
+            assert torch.equal(outs[i], want[i].expand(n, M, N)), way
+
+
 def _hip():
     # the HIP runtime the library itself is linked against, found through the library's own handle
     # (another copy of libamdhip64 may be loaded in this process, e.g. the one torch ships, and a
