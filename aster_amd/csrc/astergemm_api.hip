@@ -43,6 +43,13 @@ struct LaunchScope {
   ~LaunchScope() { launch_context() = LaunchContext{}; }
 };
 
+// Leaves the thread's error text as it was: for work whose failure is none of the call's.
+struct KeepError {
+  char text[sizeof(g_err)];
+  KeepError() { memcpy(text, g_err, sizeof(text)); }
+  ~KeepError() { memcpy(g_err, text, sizeof(text)); }
+};
+
 // The error text of a launcher's status; a first launch refused inside a capture says what to do.
 int launch_fail(int e, const char* name, const char* file, int line) {
   if ((hipError_t)e == hipErrorStreamCaptureUnsupported) {
@@ -138,7 +145,7 @@ struct ChoiceCacheEntry {
   astergemm_config cfg;
   int dev;
   int index;
-  bool plain;
+  int avoid;
 };
 constexpr int kChoiceCache = 16;
 thread_local ChoiceCacheEntry g_choice_cache[kChoiceCache];
@@ -228,26 +235,39 @@ bool optional_split(const Variant& v, const astergemm_config& c) {
   return v.family == ASTERGEMM_KERNEL_TILE && (v.rank == 6 || (v.rank == 4 && c.M % 8 != 0));
 }
 
-const Variant* choose_uncached(const astergemm_config& c, int* index_out, bool plain);
+// The kernels that fetch MXFP4 scale rows in 16-byte granules; row-major planes may lie on any 8-byte
+// boundary, and the general tile kernels take those.
+bool needs_mx16(const Variant& v) {
+  return v.dtype_ab == ASTERGEMM_MXFP4 && v.family == ASTERGEMM_KERNEL_TILE &&
+         v.operand_path == ASTERGEMM_OPERAND_LDS &&
+         !(&v >= tile_variants() && &v < tile_variants() + num_tile_variants());
+}
+bool planes_off_16(const astergemm_config& c, const astergemm_operands& ops) {
+  return c.dtype_ab == ASTERGEMM_MXFP4 && ((((uintptr_t)ops.dMxA) | ((uintptr_t)ops.dMxB)) & 15) != 0;
+}
 
-// Picks the variant for cfg (`plain`: leaving the optional splits out); on failure returns nullptr with
-// the error set.
-const Variant* choose(const astergemm_config& c, int* index_out, bool plain = false) {
+// What a selection leaves out because of the call's pointers.
+enum Avoid { kAvoidOptionalSplits = 1, kAvoidMx16 = 2 };
+
+const Variant* choose_uncached(const astergemm_config& c, int* index_out, int avoid);
+
+// Picks the variant for cfg, leaving out what `avoid` says; on failure returns nullptr with the error set.
+const Variant* choose(const astergemm_config& c, int* index_out, int avoid = 0) {
   const int dev = current_device_or_minus_one();
   for (int i = 0; i < g_choice_cache_used; ++i) {
     const ChoiceCacheEntry& e = g_choice_cache[i];
-    if (e.dev == dev && e.plain == plain && memcmp(&e.cfg, &c, sizeof(c)) == 0) {
+    if (e.dev == dev && e.avoid == avoid && memcmp(&e.cfg, &c, sizeof(c)) == 0) {
       if (index_out) *index_out = e.index;
       return variant_at(e.index);
     }
   }
   int index = -1;
-  const Variant* v = choose_uncached(c, &index, plain);
+  const Variant* v = choose_uncached(c, &index, avoid);
   if (!v) return nullptr;  // refusals are not remembered: the message is made again
   ChoiceCacheEntry& e = g_choice_cache[g_choice_cache_next];
   memcpy(&e.cfg, &c, sizeof(c));
   e.dev = dev;
-  e.plain = plain;
+  e.avoid = avoid;
   e.index = index;
   g_choice_cache_next = (g_choice_cache_next + 1) % kChoiceCache;
   if (g_choice_cache_used < kChoiceCache) ++g_choice_cache_used;
@@ -255,7 +275,7 @@ const Variant* choose(const astergemm_config& c, int* index_out, bool plain = fa
   return v;
 }
 
-const Variant* choose_uncached(const astergemm_config& c, int* index_out, bool plain) {
+const Variant* choose_uncached(const astergemm_config& c, int* index_out, int avoid) {
   g_choose_rc = ASTERGEMM_ENOTSUP;
   if (const char* why = validate_problem(c)) {
     set_error("astergemm: invalid config: %s", why);
@@ -318,7 +338,8 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out, bool p
     if (v->family != family || !variant_matches_types(*v, c)) continue;
     if (v->rank == 5 && v->tile_m != unequal) continue;
     if (v->rank == 6 && !unequal_split) continue;
-    if (plain && optional_split(*v, c)) continue;
+    if ((avoid & kAvoidOptionalSplits) && optional_split(*v, c)) continue;
+    if ((avoid & kAvoidMx16) && needs_mx16(*v)) continue;
     if (const char* why = v->check(c)) {
       if (!last_why) last_why = why;
       continue;
@@ -568,15 +589,16 @@ bool is_capturing(hipStream_t s) {
   return st != hipStreamCaptureStatusNone;
 }
 
-// What a call with these operands on this stream runs: cfg's variant, or for an optional split without
-// scratch of the call's own the kernel it stands in for; *other is then the one of the two that does
-// not run (nullptr for configs with one kernel).
+// What a call with these operands on this stream runs: cfg's variant among those that read its scale
+// planes, or for an optional split without scratch of the call's own the kernel it stands in for; *other
+// is then the one of the two that does not run (nullptr for configs with one kernel).
 const Variant* choose_for_call(const astergemm_config& c, const astergemm_operands& ops, void* stream,
                                const Variant** other = nullptr) {
-  const Variant* v = choose(c, nullptr);
+  const int planes = planes_off_16(c, ops) ? kAvoidMx16 : 0;
+  const Variant* v = choose(c, nullptr, planes);
   if (other) *other = nullptr;
   if (!v || c.variant != 0 || !optional_split(*v, c)) return v;
-  const Variant* plain = choose(c, nullptr, true);
+  const Variant* plain = choose(c, nullptr, planes | kAvoidOptionalSplits);
   const bool fits = ops.dWorkspace ? ops.workspace_bytes >= workspace_need(*v, c)
                                    : !is_capturing((hipStream_t)stream);
   if (other) *other = fits ? plain : v;
@@ -746,9 +768,18 @@ int astergemm_prepare(const astergemm_config* cfg) {
   const size_t need = workspace_need(*v, *cfg), scratch = ASTERGEMM_NOALLOC_SCRATCH_BYTES;
   if (int rc = prime(*v, *cfg, scratch_ptr, need <= scratch ? scratch : optional ? need : 0, nullptr))
     return rc;
-  if (!optional) return 0;
-  v = choose(*cfg, &index, true);
-  return v ? prime(*v, *cfg, scratch_ptr, (size_t)-1, nullptr) : g_choose_rc;
+  if (cfg->variant != 0) return 0;
+  // the kernels that other pointers than the usual ones lead to (choose_for_call)
+  for (int avoid = 1; avoid <= (kAvoidOptionalSplits | kAvoidMx16); ++avoid) {
+    const Variant* o;
+    {
+      KeepError keep;  // a named tile may exist for 16-byte planes only
+      o = choose(*cfg, &index, avoid);
+    }
+    if (!o || o == v) continue;
+    if (int rc = prime(*o, *cfg, scratch_ptr, (size_t)-1, nullptr)) return rc;
+  }
+  return 0;
 }
 
 int astergemm_workspace_bytes(const astergemm_config* cfg, size_t* bytes) {
@@ -770,11 +801,12 @@ int astergemm_run_noalloc(const astergemm_config* cfg, const astergemm_operands*
     return ASTERGEMM_EINVAL;
   }
   // calls on one device share the built-in scratch: an optional split does not bring a config to it
-  const Variant* v = choose(*cfg, nullptr);
+  const int planes = planes_off_16(*cfg, *ops) ? kAvoidMx16 : 0;
+  const Variant* v = choose(*cfg, nullptr, planes);
   const Variant* other = nullptr;
   if (v && cfg->variant == 0 && optional_split(*v, *cfg)) {
     other = v;
-    v = choose(*cfg, nullptr, /*plain=*/true);
+    v = choose(*cfg, nullptr, planes | kAvoidOptionalSplits);
   }
   if (!v) return g_choose_rc;
   if (cfg->M == 0 || cfg->N == 0) return 0;
@@ -926,6 +958,7 @@ int astergemm_tune(const astergemm_config* cfg, const astergemm_operands* ops, i
     // a caller's workspace too small for this variant's K ranges: the variant is skipped, the
     // tune goes on with the others
     if (ops->dWorkspace && ops->workspace_bytes < workspace_need(*v, *cfg)) continue;
+    if (needs_mx16(*v) && planes_off_16(*cfg, *ops)) continue;
     GemmArgs a;
     if ((rc = build_args(*v, *cfg, *ops, &a)) != 0) break;
     const int grid = grid_of(*v, *cfg);

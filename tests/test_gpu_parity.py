@@ -774,6 +774,47 @@ def test_split_k_on_unequal_tiles(gpu, M, N, dtype_ab, dtype_c):
     assert np.array_equal(out[:, :N].view(np.uint8), run()[0][:, :N].view(np.uint8))
 
 
+@pytest.mark.parametrize("M,N,K", [(333, 1032, 1024), (336, 1032, 4096), (300, 520, 14336), (304, 520, 14336),
+                                   (16, 520, 4096)])
+def test_mxfp4_scale_planes_on_8_byte_boundaries(gpu, M, N, K):
+    """Planes 8 bytes off a 16-byte boundary, for ragged and whole M, a split-K shape and a decode one:
+    the bits of the general tile kernel (decode: of the same kernel) on aligned planes."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(K + M)
+    draw = lambda rows: torch.randint(0, 256, (rows, K // 2), generator=g, device="cuda", dtype=torch.uint8)
+    mx = lambda rows: torch.randint(118, 123, (rows, K // 32), generator=g, device="cuda", dtype=torch.uint8)
+    a, b, ma, mb = draw(M), draw(N), mx(M), mx(N)
+
+    def off8(plane):
+        buf = torch.zeros(plane.numel() + 16, device="cuda", dtype=torch.uint8)
+        at = 8 if buf.data_ptr() % 16 == 0 else 0
+        buf[at:at + plane.numel()] = plane.reshape(-1)
+        return buf, buf.data_ptr() + at
+
+    (keep_a, off_a), (keep_b, off_b) = off8(ma), off8(mb)
+    plan = AG.GemmPlan.create(M, N, K, "mxfp4", "bf16")
+    decode = M <= 64
+    ref_plan = plan if decode else next(
+        AG.GemmPlan.create(M, N, K, "mxfp4", "bf16", variant=v) for v, name, ab, out in _tile_variants()
+        if ab == "mxfp4" and out == "bf16" and name.startswith("tile_mxfp4_64x64_w2x2"))
+    want, aligned, got = (torch.zeros(M, N, device="cuda", dtype=torch.bfloat16) for _ in range(3))
+    torch.cuda.synchronize()
+    print(f"{plan.info.name.decode()} M={M} N={N} K={K}", flush=True)
+    ref_plan.run(a.data_ptr(), b.data_ptr(), want.data_ptr(), mx_a=ma.data_ptr(), mx_b=mb.data_ptr())
+    plan.run(a.data_ptr(), b.data_ptr(), aligned.data_ptr(), mx_a=ma.data_ptr(), mx_b=mb.data_ptr())
+    for run in (plan.run, plan.run_noalloc):
+        for pa, pb in ((off_a, off_b), (off_a, mb.data_ptr()), (ma.data_ptr(), off_b)):
+            got.zero_()
+            torch.cuda.synchronize()
+            run(a.data_ptr(), b.data_ptr(), got.data_ptr(), mx_a=pa, mx_b=pb)
+            torch.cuda.synchronize()
+            assert torch.equal(got, want)
+    # bf16 rounding of the output on both sides (1.7e-3 each) and the order of fp32 sums
+    assert float((aligned.float() - want.float()).norm() / want.float().norm()) <= 4e-3
+    best = plan.tune(a.data_ptr(), b.data_ptr(), got.data_ptr(), iters=1, mx_a=off_a, mx_b=off_b)
+    assert decode or best.info.name.decode().startswith("tile_mxfp4_")
+
+
 # ---- edge cases: ragged M / N, K tails, leading dimensions, epilogue -----------------
 
 @pytest.mark.parametrize("M,N,K", [(1, 1, 8), (65, 16, 8), (130, 257, 72), (300, 520, 776), (129, 1, 64)])

@@ -399,6 +399,34 @@ def test_split_k_does_not_refuse_a_call_without_scratch(M, N, K):
                                                                   workspace_bytes=16)
 
 
+def _no_device():
+    n = ctypes.c_int()
+    return _capi.load().aster_rt_get_device_count(ctypes.byref(n)) != 0 or n.value == 0
+
+
+@pytest.mark.parametrize("M,N,K,kernel", [(333, 14336, 4096, "stream_mxfp4_"), (336, 14336, 4096, "stream_mxfp4_"),
+                                          (500, 4096, 14336, "splitk_mxfp4_"), (512, 4096, 14336, "splitk_mxfp4_"),
+                                          (2561, 8192, 8192, "stream_mxfp4_"), (2048, 8192, 8192, "stream_mxfp4_"),
+                                          (333, 4096, 11008, "tile_mxfp4_")])
+def test_mxfp4_scale_planes_on_8_byte_boundaries_are_taken(M, N, K, kernel):
+    """The stream kernels fetch scale rows in 16-byte granules; a call whose row-major planes lie on another
+    8-byte boundary gets the general tile kernel instead of their refusal.  Without a device every call
+    ends in the launcher of the kernel it was given to, whose name the error holds."""
+    if not _no_device():
+        pytest.skip("the pointers are made up")
+    p = gemm.GemmPlan.create(M, N, K, "mxfp4", "bf16")
+    assert p.info.name.decode().startswith(kernel)
+    for run in (p.run, p.run_noalloc):
+        for a, b in ((8, 0), (0, 8), (8, 8)):
+            with pytest.raises(_capi.AsterGemmError, match=r"\(tile_mxfp4_") as err:
+                run(4096, 4096, 4096, mx_a=4096 + a, mx_b=4096 + b)
+            assert "invalid argument" not in str(err.value)
+        with pytest.raises(_capi.AsterGemmError, match="8-byte aligned"):
+            run(4096, 4096, 4096, mx_a=4096 + 4, mx_b=4096)
+    with pytest.raises(_capi.AsterGemmError, match=r"\(" + kernel):
+        p.run(4096, 4096, 4096, mx_a=4096, mx_b=4096, workspace=4096, workspace_bytes=1 << 40)
+
+
 def test_reported_grid_is_the_launched_grid_of_the_k_range_kernels():
     # S K ranges x R row ranges, one workgroup per CU: the description comes from the same
     # function the launcher uses (the number of CUs is 0 without a device: one row range)
