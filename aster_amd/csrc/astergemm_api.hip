@@ -624,11 +624,29 @@ int prime(const Variant& v, const astergemm_config& c, void* any, size_t any_byt
   return e != 0 ? launch_fail(e, v.name, __FILE__, __LINE__) : 0;
 }
 
+int index_of(const Variant& v) {
+  if (&v >= tile_variants() && &v < tile_variants() + num_tile_variants()) return (int)(&v - tile_variants());
+  if (&v >= stream_variants() && &v < stream_variants() + num_stream_variants())
+    return num_tile_variants() + (int)(&v - stream_variants());
+  return num_tile_variants() + num_stream_variants() + (int)(&v - skinny_variants());
+}
+
 // A config with an optional split has two kernels: an eager launch of one readies the other, so that a
-// later capture finds either of them ready; with `library_ws` also the stream's workspace.
-void prime_other(const Variant* other, const astergemm_config& c, void* stream, bool library_ws) {
-  if (other && !is_capturing((hipStream_t)stream))
-    (void)prime(*other, c, (void*)(uintptr_t)4096, library_ws ? 0 : (size_t)-1, stream);
+// later capture finds either of them ready.  (The stream's workspace is: the kernel a capture runs has no
+// more K ranges than the split it stands in for, by the lines of unequal_split_pays.)  Once per kernel and device (these launchers have one kernel
+// each whatever the config); done on every call it cost such a call 0.5-0.7 of 8.3 us of host time.
+// A failure is that later launch's to report, not the call's that has just succeeded.
+void ready_other(const Variant* other, const astergemm_config& c, void* stream) {
+  if (!other) return;
+  static std::vector<std::atomic<uint64_t>> ready((size_t)total_variants());
+  const int dev = current_device_or_minus_one();
+  if (dev < 0) return;
+  std::atomic<uint64_t>& devs = ready[(size_t)index_of(*other)];
+  const uint64_t bit = (uint64_t)1 << (dev & 63);
+  if ((devs.load(std::memory_order_acquire) & bit) || is_capturing((hipStream_t)stream)) return;
+  KeepError keep;
+  if (prime(*other, c, (void*)(uintptr_t)4096, (size_t)-1, stream) == 0)
+    devs.fetch_or(bit, std::memory_order_release);
 }
 
 // ---- the entry point that allocates nothing ------------------------------------------------
@@ -742,7 +760,7 @@ int astergemm_run(const astergemm_config* cfg, const astergemm_operands* ops, vo
     const int e = v->launch(a, grid_of(*v, *cfg), (hipStream_t)stream);
     if (e != 0) return launch_fail(e, v->name, __FILE__, __LINE__);
   }
-  prime_other(other, *cfg, stream, /*library_ws=*/!ops->dWorkspace);
+  ready_other(other, *cfg, stream);
   return 0;
 }
 
@@ -834,7 +852,7 @@ int astergemm_run_noalloc(const astergemm_config* cfg, const astergemm_operands*
     const int e = v->launch(a, grid_of(*v, *cfg), (hipStream_t)stream);
     if (e != 0) return launch_fail(e, v->name, __FILE__, __LINE__);
   }
-  prime_other(other, *cfg, stream, /*library_ws=*/false);
+  ready_other(other, *cfg, stream);
   return 0;
 }
 

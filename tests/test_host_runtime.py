@@ -137,6 +137,30 @@ def test_selection_of_unequal_tile_sides_bf16_and_fp8(shape, name):
     assert p.workspace_bytes() == 4 * 500 * 4096 * 4 and p.info.grid_x == 64 * 4
 
 
+def test_no_split_on_unequal_tiles_has_fewer_planes_than_the_square_split_it_replaces():
+    """An eager call leaves its stream a workspace of the size it needed, and a captured call of the same
+    config, which runs the square kernel, cannot make it larger."""
+    lib, info, found = _capi.load(), _capi.KernelInfo(), 0
+    for dtype, tag in (("bf16", "bf16"), ("fp8_e4m3", "fp8")):
+        for N in range(1024, 9000, 1024):
+            for K in (4096, 8192, 11008, 14336, 16384, 28672, 57344):
+                for M in range(136, 1025, 56):
+                    p = gemm.GemmPlan.create(M, N, K, dtype, "bf16")
+                    if p.info.name.decode() != f"splitk_{tag}_256x128_w4x2_bf16":
+                        continue
+                    for i in range(lib.astergemm_variant_count()):
+                        _capi.check(lib.astergemm_variant_info(i, ctypes.byref(p.config), ctypes.byref(info)))
+                        if info.name.decode() == f"splitk_{tag}_128x128_w2x2_bf16":
+                            break
+                    try:
+                        square = gemm.GemmPlan.create(M, N, K, dtype, "bf16", variant=info.variant)
+                    except _capi.AsterGemmError:
+                        continue                 # not cut into K ranges on square tiles
+                    found += 1
+                    assert square.workspace_bytes() <= p.workspace_bytes(), (M, N, K, dtype)
+    assert found > 20
+
+
 def test_long_decode_rows_off_the_groups_of_8_stay_with_the_decode_kernel():
     for M, start in ((33, "skinnyx_"), (50, "skinnyx_"), (56, "splitk_"), (63, "skinnyx_"), (64, "splitk_")):
         assert gemm.GemmPlan.create(M, 8192, 28672, "f16", "f16").info.name.decode().startswith(start), M

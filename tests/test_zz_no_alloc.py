@@ -130,6 +130,50 @@ def test_caller_workspace_matches_the_library_workspace(gpu):
         bf.free()
 
 
+def test_an_eager_split_call_readies_its_stream_for_a_capture_of_the_same_config(gpu):
+    """512 x 4096 x 14336: an eager call runs split K on 256 x 128 tiles , a captured one on 128 x 128,
+    whose planes go to the library's buffer of the stream, which cannot grow inside a capture.  Every replay
+    has the bits of that kernel, with eager calls between the replays; a call that succeeds leaves the
+    thread's last error as it was."""
+    import torch
+    M, N, K = 512, 4096, 14336
+    g = torch.Generator(device="cuda").manual_seed(5)
+    a = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    b = (torch.randn(N, K, generator=g, device="cuda") * 0.02).to(torch.bfloat16)
+    eager, got, want = (torch.zeros(M, N, device="cuda", dtype=torch.bfloat16) for _ in range(3))
+    plan = AG.GemmPlan.create(M, N, K, "bf16", "bf16")
+    assert plan.info.name.decode() == "splitk_bf16_256x128_w4x2_bf16"
+    lib, info = _capi.load(), _capi.KernelInfo()
+    for i in range(lib.astergemm_variant_count()):
+        _capi.check(lib.astergemm_variant_info(i, ctypes.byref(plan.config), ctypes.byref(info)))
+        if info.name.decode() == "splitk_bf16_128x128_w2x2_bf16":
+            square = AG.GemmPlan.create(M, N, K, "bf16", "bf16", variant=info.variant)
+    assert 0 < square.workspace_bytes() <= plan.workspace_bytes()
+    stream = torch.cuda.Stream()
+    with pytest.raises(_capi.AsterGemmError, match="non-null"):
+        plan.run(None, None, None)
+    torch.cuda.synchronize()
+    print("eager, capture, replays", flush=True)
+    plan.run(a.data_ptr(), b.data_ptr(), eager.data_ptr(), stream=stream.cuda_stream)
+    assert "non-null" in _capi.last_error()
+    stream.synchronize()
+    first = eager.clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        plan.run(a.data_ptr(), b.data_ptr(), got.data_ptr(), stream=stream.cuda_stream)
+    square.run(a.data_ptr(), b.data_ptr(), want.data_ptr())
+    torch.cuda.synchronize()
+    for _ in range(3):
+        got.zero_()
+        eager.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            graph.replay()
+        plan.run(a.data_ptr(), b.data_ptr(), eager.data_ptr(), stream=stream.cuda_stream)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want) and torch.equal(eager, first)
+
+
 @pytest.mark.parametrize("M,N,K,dtype,kernel", [
     (128, 1024, 8192, "bf16", "splitk_bf16_128x128_w2x2_bf16"),
     (129, 1032, 8192, "bf16", "splitk_bf16_256x128_w4x2_bf16"),
