@@ -591,16 +591,17 @@ bool is_capturing(hipStream_t s) {
 
 // What a call with these operands on this stream runs: cfg's variant among those that read its scale
 // planes, or for an optional split without scratch of the call's own the kernel it stands in for; *other
-// is then the one of the two that does not run (nullptr for configs with one kernel).
+// is then the one of the two that does not run (nullptr for configs with one kernel).  `captured`: the call
+// is going to be captured, whatever the stream does now.
 const Variant* choose_for_call(const astergemm_config& c, const astergemm_operands& ops, void* stream,
-                               const Variant** other = nullptr) {
+                               const Variant** other = nullptr, bool captured = false) {
   const int planes = planes_off_16(c, ops) ? kAvoidMx16 : 0;
   const Variant* v = choose(c, nullptr, planes);
   if (other) *other = nullptr;
   if (!v || c.variant != 0 || !optional_split(*v, c)) return v;
   const Variant* plain = choose(c, nullptr, planes | kAvoidOptionalSplits);
   const bool fits = ops.dWorkspace ? ops.workspace_bytes >= workspace_need(*v, c)
-                                   : !is_capturing((hipStream_t)stream);
+                                   : !captured && !is_capturing((hipStream_t)stream);
   if (other) *other = fits ? plain : v;
   return fits ? v : plain;
 }
@@ -633,9 +634,9 @@ int index_of(const Variant& v) {
 
 // A config with an optional split has two kernels: an eager launch of one readies the other, so that a
 // later capture finds either of them ready.  (The stream's workspace is: the kernel a capture runs has no
-// more K ranges than the split it stands in for, by the lines of unequal_split_pays.)  Once per kernel and device (these launchers have one kernel
-// each whatever the config); done on every call it cost such a call 0.5-0.7 of 8.3 us of host time.
-// A failure is that later launch's to report, not the call's that has just succeeded.
+// more K ranges than the split it stands in for, by the lines of unequal_split_pays.)  Once per kernel and
+// device (these launchers have one kernel each whatever the config); done on every call it cost such a
+// call 0.5-0.7 of 8.3 us of host time.  A failure is that later launch's to report, not the call's that has just succeeded.
 void ready_other(const Variant* other, const astergemm_config& c, void* stream) {
   if (!other) return;
   static std::vector<std::atomic<uint64_t>> ready((size_t)total_variants());
@@ -647,6 +648,27 @@ void ready_other(const Variant* other, const astergemm_config& c, void* stream) 
   KeepError keep;
   if (prime(*other, c, (void*)(uintptr_t)4096, (size_t)-1, stream) == 0)
     devs.fetch_or(bit, std::memory_order_release);
+}
+
+// One operand set of a timed rotation: what astergemm_run would launch for it.
+struct TimedSet {
+  const Variant* v;
+  int grid;
+  GemmArgs args;
+  int launch(hipStream_t s) const { return v->launch(args, grid, s); }
+};
+int timed_sets(const astergemm_config& c, const astergemm_operands* ops, int n, void* stream, bool captured,
+               std::vector<TimedSet>* out) {
+  out->resize((size_t)n);
+  for (int i = 0; i < n; ++i) {
+    TimedSet& t = (*out)[(size_t)i];
+    t.v = choose_for_call(c, ops[i], stream, nullptr, captured);
+    if (!t.v) return g_choose_rc;
+    if (c.M == 0 || c.N == 0) continue;
+    t.grid = grid_of(*t.v, c);
+    if (int rc = build_args(*t.v, c, ops[i], &t.args)) return rc;
+  }
+  return 0;
 }
 
 // ---- the entry point that allocates nothing ------------------------------------------------
@@ -862,26 +884,22 @@ int astergemm_bench_rotate(const astergemm_config* cfg, const astergemm_operands
     set_error("astergemm_bench_rotate: bad argument");
     return ASTERGEMM_EINVAL;
   }
-  const Variant* v = choose_for_call(*cfg, ops[0], stream);
-  if (!v) return g_choose_rc;
+  std::vector<TimedSet> sets;
+  if (int rc = timed_sets(*cfg, ops, n_ops, stream, /*captured=*/false, &sets)) return rc;
   *total_ns = 0;
   if (cfg->M == 0 || cfg->N == 0) return 0;
-  std::vector<GemmArgs> args((size_t)n_ops);
-  for (int i = 0; i < n_ops; ++i)
-    if (int rc = build_args(*v, *cfg, ops[i], &args[(size_t)i])) return rc;
   hipStream_t s = (hipStream_t)stream;
   LaunchScope scope(stream);
-  const int grid = grid_of(*v, *cfg);
   EventPair ev;
   AG_HIP(ev.create());
   int le = (int)hipEventRecord(ev.e0, s);
   (void)hipGetLastError();
-  for (int i = 0; i < iters && le == 0; ++i) le = v->launch(args[(size_t)(i % n_ops)], grid, s);
+  for (int i = 0; i < iters && le == 0; ++i) le = sets[(size_t)(i % n_ops)].launch(s);
   if (le == 0) le = (int)hipEventRecord(ev.e1, s);
   if (le == 0) le = (int)hipEventSynchronize(ev.e1);
   float ms = 0.f;
   if (le == 0) le = (int)hipEventElapsedTime(&ms, ev.e0, ev.e1);
-  if (le != 0) return hip_fail((hipError_t)le, v->name, __FILE__, __LINE__);
+  if (le != 0) return hip_fail((hipError_t)le, sets[0].v->name, __FILE__, __LINE__);
   *total_ns = (int64_t)((double)ms * 1e6);
   return 0;
 }
@@ -892,14 +910,10 @@ int astergemm_bench_graph(const astergemm_config* cfg, const astergemm_operands*
     set_error("astergemm_bench_graph: bad argument");
     return ASTERGEMM_EINVAL;
   }
-  const Variant* v = choose_for_call(*cfg, ops[0], nullptr);
-  if (!v) return g_choose_rc;
+  std::vector<TimedSet> sets;  // what captured calls launch
+  if (int rc = timed_sets(*cfg, ops, n_ops, nullptr, /*captured=*/true, &sets)) return rc;
   *total_ns = 0;
   if (cfg->M == 0 || cfg->N == 0) return 0;
-  std::vector<GemmArgs> args((size_t)n_ops);
-  for (int i = 0; i < n_ops; ++i)
-    if (int rc = build_args(*v, *cfg, ops[i], &args[(size_t)i])) return rc;
-  const int grid = grid_of(*v, *cfg);
   // a stream of this call's own (default priority), so that the capture sees nothing else
   hipStream_t s = nullptr;
   AG_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
@@ -909,16 +923,20 @@ int astergemm_bench_graph(const astergemm_config* cfg, const astergemm_operands*
   int le = (int)ev.create();
   {
     LaunchScope scope(s);
-    // one eager launch first: function attributes, and the partial-sum workspace of this stream
-    // where the config has one, are one-time steps that may not happen inside a capture
+    // one eager launch of every kernel first: function attributes, and the partial-sum workspace of this
+    // stream where the config has one, are one-time steps that may not happen inside a capture
     (void)hipGetLastError();
-    if (le == 0) le = v->launch(args[0], grid, s);
+    for (size_t i = 0; i < sets.size() && le == 0; ++i) {
+      bool seen = false;
+      for (size_t j = 0; j < i; ++j) seen = seen || sets[j].v == sets[i].v;
+      if (!seen) le = sets[i].launch(s);
+    }
     if (le == 0) le = (int)hipStreamSynchronize(s);
     if (le == 0) {
       le = (int)hipStreamBeginCapture(s, hipStreamCaptureModeGlobal);
       if (le == 0) {
         int ce = 0;
-        for (int i = 0; i < launches && ce == 0; ++i) ce = v->launch(args[(size_t)(i % n_ops)], grid, s);
+        for (int i = 0; i < launches && ce == 0; ++i) ce = sets[(size_t)(i % n_ops)].launch(s);
         le = (int)hipStreamEndCapture(s, &graph);  // always ended, also after a refused launch
         if (ce != 0) le = ce;
       }
@@ -938,7 +956,7 @@ int astergemm_bench_graph(const astergemm_config* cfg, const astergemm_operands*
   (void)hipStreamSynchronize(s);
   splitk_workspace_release(s);  // the partial-sum workspace this stream may have been given
   (void)hipStreamDestroy(s);
-  if (le != 0) return hip_fail((hipError_t)le, v->name, __FILE__, __LINE__);
+  if (le != 0) return hip_fail((hipError_t)le, sets[0].v->name, __FILE__, __LINE__);
   *total_ns = (int64_t)((double)ms * 1e6);
   return 0;
 }

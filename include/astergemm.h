@@ -282,13 +282,15 @@ int astergemm_bench(const astergemm_config* cfg, const astergemm_operands* ops,
  * distinct weight buffers (n_ops * bytes of B well above the 256 MiB last-level
  * cache) every launch streams its weights from HBM, which is what the
  * reference's FlushLLC hook is for (python/aster/execution/flush_llc.py:25-60).
- * No counterpart in the reference: its harness times every launch separately. */
+ * Each set runs what astergemm_run would launch for it.  No counterpart in the
+ * reference: its harness times every launch separately.                       */
 int astergemm_bench_rotate(const astergemm_config* cfg, const astergemm_operands* ops,
                            int n_ops, int iters, int64_t* total_ns, void* stream);
 
 /* The same launches as nodes of a HIP graph: `launches` launches (launch i on
- * ops[i % n_ops]) are captured once on a stream of the call's own, after one
- * eager launch that does the config's one-time steps, and the graph is replayed
+ * ops[i % n_ops], each what a captured astergemm_run would launch for that set)
+ * are captured once on a stream of the call's own, after one eager launch per
+ * kernel that does its one-time steps, and the graph is replayed
  * `replays` times between one event pair after one untimed replay;
  * *total_ns covers launches * replays launches.  What a serving loop that
  * replays a captured decode step pays per GEMM.  No counterpart in the

@@ -1264,6 +1264,48 @@ def test_bench_graph_replays_the_captured_launches(gpu, M, N, K):
         plan.bench_graph([], 3, 1)
 
 
+def test_timed_rotations_launch_what_a_call_with_each_set_would(gpu):
+    """bf16 130 x 1032 x 8192 has an optional split: a graph of launches without a caller's workspace holds
+    the kernel that a captured call runs, and sets with and without enough workspace in one rotation get each
+    its own.  The outputs have the bits of the two kernels run by themselves."""
+    import ctypes
+    import torch
+    M, N, K = 130, 1032, 8192
+    g = torch.Generator(device="cuda").manual_seed(9)
+    a = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    b = (torch.randn(N, K, generator=g, device="cuda") * 0.02).to(torch.bfloat16)
+    split, plain, c0, c1 = (torch.zeros(M, N, device="cuda", dtype=torch.bfloat16) for _ in range(4))
+    plan = AG.GemmPlan.create(M, N, K, "bf16", "bf16")
+    need = plan.workspace_bytes()
+    ws = torch.zeros(need, device="cuda", dtype=torch.uint8)
+    torch.cuda.synchronize()
+    plan.run(a.data_ptr(), b.data_ptr(), split.data_ptr())
+    plan.run_noalloc(a.data_ptr(), b.data_ptr(), plain.data_ptr())
+    torch.cuda.synchronize()
+    assert not torch.equal(split, plain)
+    lib, total = _capi.load(), ctypes.c_int64()
+
+    def rotation(n0, n1):
+        c0.zero_(), c1.zero_()
+        torch.cuda.synchronize()
+        return (_capi.Operands * 2)(*[
+            plan._operands(a.data_ptr(), b.data_ptr(), c.data_ptr(), None, None, None, None, None,
+                           ws.data_ptr() if n else None, n) for c, n in ((c0, n0), (c1, n1))])
+
+    cfg = ctypes.byref(plan.config)
+    for (n0, n1), eager, captured in (((0, 0), (split, split), (plain, plain)),
+                                      ((need, 16), (split, plain), (split, plain)),
+                                      ((16, need), (plain, split), (plain, split)),
+                                      ((need, 0), (split, split), (split, plain))):
+        print(f"rotation and graph, workspaces of {n0} and {n1} bytes", flush=True)
+        _capi.check(lib.astergemm_bench_rotate(cfg, rotation(n0, n1), 2, 4, ctypes.byref(total), None))
+        torch.cuda.synchronize()
+        assert torch.equal(c0, eager[0]) and torch.equal(c1, eager[1])
+        _capi.check(lib.astergemm_bench_graph(cfg, rotation(n0, n1), 2, 4, 3, ctypes.byref(total)))
+        torch.cuda.synchronize()
+        assert torch.equal(c0, captured[0]) and torch.equal(c1, captured[1])
+
+
 @pytest.mark.parametrize("ksteps", [2, 4, 6, 8, 10, 12, 14])
 @pytest.mark.parametrize("tile", [256, 128])
 def test_mxfp4_stream_kernel_every_loop_phase(gpu, ksteps, tile):

@@ -451,6 +451,26 @@ def test_mxfp4_scale_planes_on_8_byte_boundaries_are_taken(M, N, K, kernel):
         p.run(4096, 4096, 4096, mx_a=4096, mx_b=4096, workspace=4096, workspace_bytes=1 << 40)
 
 
+def test_timed_rotations_choose_for_every_operand_set():
+    """A set without a workspace of the size the split needs is timed on the kernel a call with it would
+    run, wherever it stands in the rotation; it is not refused because the first set's kernel needs more."""
+    if not _no_device():
+        pytest.skip("the pointers are made up")
+    p = gemm.GemmPlan.create(333, 4096, 14336)
+    need, lib, total = p.workspace_bytes(), _capi.load(), ctypes.c_int64()
+    assert need > 16
+    for sizes in ((need, 16), (16, need), (need, need), (0, 16)):
+        sets = (_capi.Operands * 2)(*[p._operands(4096, 4096, 4096, None, None, None, None, None,
+                                                  4096 if n else None, n) for n in sizes])
+        cfg = ctypes.byref(p.config)
+        for rc in (lib.astergemm_bench_rotate(cfg, sets, 2, 3, ctypes.byref(total), None),
+                   lib.astergemm_bench_graph(cfg, sets, 2, 3, 2, ctypes.byref(total))):
+            assert rc == -5 and "workspace of" not in _capi.last_error(), (sizes, rc, _capi.last_error())
+    for rc in (lib.astergemm_bench_rotate(ctypes.byref(p.config), sets, 0, 3, ctypes.byref(total), None),
+               lib.astergemm_bench_graph(ctypes.byref(p.config), sets, 0, 3, 2, ctypes.byref(total))):
+        assert rc == -22
+
+
 def test_reported_grid_is_the_launched_grid_of_the_k_range_kernels():
     # S K ranges x R row ranges, one workgroup per CU: the description comes from the same
     # function the launcher uses (the number of CUs is 0 without a device: one row range)
