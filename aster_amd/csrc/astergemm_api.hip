@@ -391,9 +391,17 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out, int av
       // from 128 on when rows are long (8 KiB and more: few prologues per byte streamed).
       const int64_t g128 = ((c.M + 127) / 128) * ((c.N + 127) / 128);
       const bool ragged_128 = g128 > 512 && g128 % 512 != 0 && g128 % 512 < 180;
-      // 16-bit and fp8 operands whose 256 x 128 tiles pass one per CU: 256 x 256 whatever part of the round
-      // they fill, the tiles between no longer pay (see unequal_tile_of)
-      const bool past_unequal = unequal_tiles_apply(c) && unequal == 0 && tile_grid(c, 256, 128) > chip_cus();
+      // 16-bit and fp8 operands whose 256 x 128 tiles pass one per CU and whose 128 x 128 tiles pass two:
+      // 256 x 256 whatever part of the round they fill, the tiles between no longer pay (see
+      // unequal_tile_of).  Up to two 128 x 128 tiles per CU those are ahead (an odd number of 128-row tiles;
+      // 128 x 128 / 256 x 256, bf16 600x11008x4096 53.2 / 77.0 us, 384x16640x4096 49.8 / 74.0, 600x12288x8192
+      // 108 / 151, 1100x6912x4096 56.4 / 79.1, 128x40960x4096 85.0 / 89.1; fp8 600x11008x4096 27.8 / 38.4,
+      // 860x8704x4096 28.4 / 36.9); past two they are behind (bf16 648x11008x4096, 516 tiles, 76.9 / 70.3,
+      // fp8 42.5 / 36.6), but for fp32 outputs on rows under 4 KiB (f16 -> f32 1120x10056x1024 31.9 / 34.8,
+      // 1024x11968x1024 29.7 / 31.3; the same with 4 KiB rows 0.90-0.95 of the time)
+      const bool past_unequal = unequal_tiles_apply(c) && unequal == 0 &&
+                                tile_grid(c, 256, 128) > chip_cus() && g128 > 2 * chip_cus() &&
+                                !(c.dtype_c == ASTERGEMM_F32 && row_bytes(c.dtype_ab, c.K) < 4096);
       const int thr256 = ragged_128 ? 140 : 220;
       const int thr256s = past_unequal ? 1 : thr256;
       // MXFP4: the generic tile kernels are weak next to the stream kernels, so the 128 x 128

@@ -137,6 +137,29 @@ def test_selection_of_unequal_tile_sides_bf16_and_fp8(shape, name):
     assert p.workspace_bytes() == 4 * 500 * 4096 * 4 and p.info.grid_x == 64 * 4
 
 
+@pytest.mark.parametrize("M,N,tile", [
+    (640, 11008, "128x128_w2x2"),   # 430 tiles of 128 x 128, two per CU; 258 of 256 x 128
+    (600, 11008, "128x128_w2x2"), (601, 11008, "128x128_w2x2"),
+    (641, 11008, "256x256_w2x4"),   # 516
+    (384, 16640, "128x128_w2x2"), (128, 40960, "128x128_w2x2"), (1152, 7168, "128x128_w2x2"),
+    (1153, 7168, "256x256_w2x4"),
+])
+@pytest.mark.parametrize("dtype,tag", [("bf16", "bf16"), ("fp8_e4m3", "fp8")])
+def test_two_128_tiles_per_cu_stay_ahead_of_half_a_round_of_256_tiles(M, N, tile, dtype, tag):
+    """An odd number of 128-row tiles whose 256 x 128 tiles just pass one per CU."""
+    for K in (2048, 4096, 8192):
+        name = gemm.GemmPlan.create(M, N, K, dtype, "bf16").info.name.decode()
+        assert name == f"stream_{tag}_{tile}_bf16", (K, name)
+
+
+def test_fp32_outputs_on_short_rows_keep_two_128_tiles_per_cu():
+    for K, dtype_c, tile in ((1024, "f32", "128x128_w2x2"), (2040, "f32", "128x128_w2x2"),
+                             (2048, "f32", "256x256_w2x4"), (1024, "f16", "256x256_w2x4")):
+        for M, N in ((1120, 10056), (1121, 10056), (1024, 11968)):
+            name = gemm.GemmPlan.create(M, N, K, "f16", dtype_c).info.name.decode()
+            assert name == f"stream_f16_{tile}_{dtype_c}", (M, N, K, name)
+
+
 def test_no_split_on_unequal_tiles_has_fewer_planes_than_the_square_split_it_replaces():
     """An eager call leaves its stream a workspace of the size it needed, and a captured call of the same
     config, which runs the square kernel, cannot make it larger."""
