@@ -227,6 +227,21 @@ bool unequal_split_pays(const astergemm_config& c) {
   return steps / S * 384 * 4 <= square * 3;
 }
 
+// Stages of the general 64 x 64 tile kernel: four on grids of up to two workgroups per CU, which is what
+// their 64 KiB of LDS leave room for, two (32 KiB) past it: four stages cover a K-step's memory latency by
+// themselves, the residency they cost past that covers it as well, and on short rows their prologue is the
+// longer part.  The two-stage kernel before / four stages / two, back to back, us: bf16 1024x3001x4096 (752
+// workgroups) 37.9 / 39.2 / 35.3, 532x3593x2056 (513) 24.0 / 28.5 / 21.8, fp8 333x8192x2048 (768) 11.3 / 13.8 /
+// 11.3, 383x7259x11008 (684) 47.9 / 55.6 / 45.6, MXFP4 1348x1847x4096 (638) 33.4 / 18.4 / 16.4; 18 K-steps: bf16
+// 1001x2048x1096 (512) 10.7 / 12.9 / 10.7, 978x1047x1096 (272) 10.0 / 9.6 / 8.4.  The other side of the lines: bf16
+// 459x4003x4096 (504) 34.4 / 26.1 / 32.2, 754x1349x4096 (264) 32.8 / 24.0 / 31.5, fp8 737x1981x4096 (372, 32
+// K-steps) 17.9 / 13.6 / 17.1, MXFP4 232x4443x11008 (280) 43.5 / 28.0 / 24.7 and, on buffers that no kernel has
+// read yet, 44.7 / 34.1 / 34.3.
+int tile64_stages_of(const astergemm_config& c) {
+  const bool short_rows = c.dtype_ab != ASTERGEMM_MXFP4 && row_bytes(c.dtype_ab, c.K) <= 24 * 128;
+  return tile_grid(c, 64, 64) > (short_rows ? 1 : 2) * (int64_t)chip_cus() ? 2 : 4;
+}
+
 // Split K where a kernel without K ranges (or with fewer) takes the problem too: 256 x 128 tiles, and
 // 128 x 128 tiles of a ragged M.  A call that has no scratch of its own for them -- the built-in scratch
 // or a caller's workspace too small, a stream under capture, whose graph may be replayed beside other work
@@ -329,6 +344,7 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out, int av
 
   const int unequal = unequal_tile_of(c);
   const bool unequal_split = unequal_split_pays(c);
+  const int tile64_stages = tile64_stages_of(c);
 
   const Variant* best = nullptr;
   int best_index = -1;
@@ -336,6 +352,7 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out, int av
   for (int i = 0; i < total_variants(); ++i) {
     const Variant* v = variant_at(i);
     if (v->family != family || !variant_matches_types(*v, c)) continue;
+    if (i < num_tile_variants() && v->tile_m == 64 && v->stages != tile64_stages) continue;
     if (v->rank == 5 && v->tile_m != unequal) continue;
     if (v->rank == 6 && !unequal_split) continue;
     if ((avoid & kAvoidOptionalSplits) && optional_split(*v, c)) continue;

@@ -42,22 +42,33 @@ const char* check_tile(const astergemm_config& c) {
       AG_TILE1(name "_f32", DT, ASTERGEMM_F32, BM, BN, WM, WN, S),               \
       AG_TILE1(name "_f16", DT, ASTERGEMM_F16, BM, BN, WM, WN, S)
 
-// Stages of LDS (the last number), measured back to back, S = 2 (every K-step waits for its own
-// transfers) / 3 / 4 / 5: 64 x 64 bf16 777x1001x1032 12.4 / 8.1 / 8.1 / 8.3 us, 130x4096x4096 47 / 25.5 /
-// 19.0 / 17.8, MXFP4 300x4096x11008 45 / 32.3 / 32.7 / 41.8 (five stages: one workgroup per CU);
-// 128 x 64 fp8 300x4096x11008 66 / 40.5 / 40.2 / 40.9 (six); 128 x 128 bf16 130x4096x4096 56 / 40.2 / 40.4 / 40.8.
-// 256 x 256 has room for two.
-#define AG_TILE_SET(prefix, DT)                              \
-  AG_TILE(prefix "_256x256_w2x4", DT, 256, 256, 2, 4, 2),    \
-      AG_TILE(prefix "_128x128_w2x2", DT, 128, 128, 2, 2, 4), \
-      AG_TILE(prefix "_128x64_w2x2", DT, 128, 64, 2, 2, 3),  \
+// Stages of LDS (the last number).  64 x 64 on grids of up to two workgroups per CU (past that: two stages,
+// see tile64_stages_of), S = 2
+// (every K-step waits for its own transfers) / 3 / 4 / 5: bf16 777x1001x1032 12.4 / 8.1 / 8.1 / 8.3 us,
+// 130x4096x4096 47 / 25.5 / 19.0 / 17.8, MXFP4 300x4096x11008 45 / 32.3 / 32.7 / 41.8 (five stages: one
+// workgroup per CU).  The larger tiles are taken from 448 workgroups on, where two (128 x 128) and three
+// (128 x 64) workgroups share a CU only with two stages: the two-stage kernel before / S = 3 / 4 / 2, back to
+// back, 128 x 128 bf16 2048x4097x4096 107 / 120 / 120 / 96.7, 700x10007x4096 66.6 / 81.7 / 80.6 / 61.2, fp8
+// 700x10007x4096 40.3 / 47.7 / 47.5 / 33.5, MXFP4 2048x4096x11008 87.2 / 72.9 / 71.6 / 64.8; 128 x 64, S = 3 / 2,
+// bf16 1500x4001x4096 61.7 / 63.2 / 57.4, 509x8245x8192 102 / 114 / 96.2, fp8 434x8749x8192 58.7 / 61.9 / 54.6
+// (behind on rows of 512-2048 bytes, bf16 408x8089x2048 26.3 / 22.3 / 22.4).  256 x 256 has room for two.
+#define AG_TILE_SET(prefix, DT)                                                  \
+  AG_TILE(prefix "_256x256_w2x4", DT, 256, 256, 2, 4, 2),                        \
+      AG_TILE(prefix "_128x128_w2x2", DT, 128, 128, 2, 2, 2),                    \
+      AG_TILE(prefix "_128x64_w2x2", DT, 128, 64, 2, 2, 2),                      \
       AG_TILE(prefix "_64x64_w2x2", DT, 64, 64, 2, 2, 4)
+#define AG_TILE_RING2(prefix, DT)                                                \
+  AG_TILE(prefix "_64x64_w2x2_ring2", DT, 64, 64, 2, 2, 2)
 
 const Variant kTileVariants[] = {
     AG_TILE_SET("tile_bf16", ASTERGEMM_BF16),
     AG_TILE_SET("tile_f16", ASTERGEMM_F16),
     AG_TILE_SET("tile_fp8", ASTERGEMM_FP8_E4M3),
     AG_TILE_SET("tile_mxfp4", ASTERGEMM_MXFP4),
+    AG_TILE_RING2("tile_bf16", ASTERGEMM_BF16),
+    AG_TILE_RING2("tile_f16", ASTERGEMM_F16),
+    AG_TILE_RING2("tile_fp8", ASTERGEMM_FP8_E4M3),
+    AG_TILE_RING2("tile_mxfp4", ASTERGEMM_MXFP4),
 };
 
 }  // namespace

@@ -659,6 +659,26 @@ def test_tile_kernels_every_stage_count(gpu, steps, tile, dtype_ab):
         assert np.isnan(out[:, N:]).all()
 
 
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 7])
+@pytest.mark.parametrize("dtype_ab", ["bf16", "f16", "fp8_e4m3", "mxfp4"])
+def test_two_stage_64_tile_has_the_bits_of_the_four_stage_one(gpu, steps, dtype_ab):
+    """One to several K-steps, with a K tail (none for MXFP4), odd M, N and output pitch: the same products
+    added in the same order."""
+    per = {"bf16": 64, "f16": 64, "fp8_e4m3": 128, "mxfp4": 256}[dtype_ab]
+    tag, M, N = {"fp8_e4m3": "fp8"}.get(dtype_ab, dtype_ab), 133, 71
+    for K in ((per * steps,) if dtype_ab == "mxfp4" else (per * steps, per * (steps - 1) + per // 4)):
+        a, b, extra = operands(M, N, K, dtype_ab, seed=61, b_std=0.05)
+        bias = np.random.default_rng(62).standard_normal(N).astype(np.float32)
+        outs = [run_gemm(a, b, M, N, K, dtype_ab, "f32", bias=bias, ldc=N + 2, **extra,
+                         variant=_variant_id(f"tile_{tag}_64x64_w2x2_{ring}f32"))[0] for ring in ("ring2_", "")]
+        assert np.array_equal(outs[0][:, :N], outs[1][:, :N]) and np.isnan(outs[0][:, N:]).all()
+        if dtype_ab == "fp8_e4m3":
+            want = G.gemm_fp8(a, b, extra["scale_a"], extra["scale_b"], out_dtype=G.F32, bias=bias)
+        else:
+            want = G.gemm(a, b, _DT[dtype_ab], G.F32, bias=bias, **extra)
+        check(outs[0], want, "f32", N, bar=1e-4 if dtype_ab == "fp8_e4m3" else 1e-5)
+
+
 @pytest.mark.parametrize("M", [9, 15, 129, 257, 263, 333])
 @pytest.mark.parametrize("tile", [128, 256])
 @pytest.mark.parametrize("dtype_ab,dtype_c", [("bf16", "bf16"), ("f16", "f32"), ("fp8_e4m3", "bf16"),

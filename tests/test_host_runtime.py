@@ -160,6 +160,27 @@ def test_fp32_outputs_on_short_rows_keep_two_128_tiles_per_cu():
             assert name == f"stream_f16_{tile}_{dtype_c}", (M, N, K, name)
 
 
+@pytest.mark.parametrize("M,N,K,dtype,name", [
+    (1024, 2049, 4104, "bf16", "tile_bf16_64x64_w2x2_ring2_bf16"),   # 528 workgroups
+    (1024, 2048, 4104, "bf16", "128x128"),                             # the stream kernels take it
+    (1024, 2047, 4104, "bf16", "tile_bf16_64x64_w2x2_bf16"),         # 512
+    (1024, 2047, 1536, "bf16", "tile_bf16_64x64_w2x2_ring2_bf16"),   # rows of 3 KiB
+    (1024, 2047, 1544, "bf16", "tile_bf16_64x64_w2x2_bf16"),
+    (1024, 1031, 1536, "bf16", "tile_bf16_64x64_w2x2_ring2_bf16"),   # 272
+    (1024, 1023, 1536, "bf16", "tile_bf16_64x64_w2x2_bf16"),         # 256
+    (1024, 2047, 3072, "fp8_e4m3", "tile_fp8_64x64_w2x2_ring2_bf16"),
+    (1024, 2047, 3088, "fp8_e4m3", "tile_fp8_64x64_w2x2_bf16"),
+    (1024, 2047, 4096, "mxfp4", "tile_mxfp4_64x64_w2x2_bf16"),       # MXFP4: the grid alone decides
+    (1024, 2049, 4096, "mxfp4", "tile_mxfp4_64x64_w2x2_ring2_bf16"),
+])
+def test_stages_of_the_general_64_tile(M, N, K, dtype, name):
+    got = gemm.GemmPlan.create(M, N, K, dtype, "bf16").info
+    assert name in got.name.decode(), got.name
+    named = gemm.GemmPlan.create(M, N - 1 + N % 2, K, dtype, "bf16", wg_tile=(64, 64)).info
+    assert (named.pipeline_stages == 2) == ("ring2" in named.name.decode())
+    assert named.lds_bytes == named.pipeline_stages * 128 * (136 if dtype == "mxfp4" else 128)
+
+
 def test_no_split_on_unequal_tiles_has_fewer_planes_than_the_square_split_it_replaces():
     """An eager call leaves its stream a workspace of the size it needed, and a captured call of the same
     config, which runs the square kernel, cannot make it larger."""
