@@ -297,7 +297,7 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p) {
   const int li = lane & 15, lq = lane >> 4;
   constexpr bool EARLY = TM * TN <= 16;  // the big tiles have no registers to spare for it
   float scale = 1.0f;
-  f32x4 bias_v[EARLY ? TN : 1];
+  f32x4 bias_v[TN];
   auto load_bias = [&](int n) {
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
     if (p.bias) {
@@ -403,19 +403,24 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p) {
   }
 
   // ---- epilogue: scale, bias, cast, vector store ----------------------------
+  // row by row: the 16-column pieces of a row leave one behind the other and meet in L2 as whole lines
+  // (column by column, 256 x 256 tiles: f16 -> f32 1269x22135x312 60.8 us and, on buffers that no kernel has
+  // read yet, 96.8; row by row 38.5 and 53.6; bf16 4096x4097x256 48.2 / 53.9 -> 45.4 / 46.7; 64 x 64 level)
+  if constexpr (!EARLY) {
 #pragma unroll
-  for (int n = 0; n < TN; ++n) {
-    const int col = col0 + (wn * TN + n) * 16 + 4 * lq;
-    const f32x4 b = EARLY ? bias_v[EARLY ? n : 0] : load_bias(n);
-    const int ncols = (p.N - col) < 4 ? (p.N - col) : 4;
+    for (int n = 0; n < TN; ++n) bias_v[n] = load_bias(n);
+  }
 #pragma unroll
-    for (int m = 0; m < TM; ++m) {
-      const int row = row0 + (wm * TM + m) * 16 + li;
+  for (int m = 0; m < TM; ++m) {
+    const int row = row0 + (wm * TM + m) * 16 + li;
+#pragma unroll
+    for (int n = 0; n < TN; ++n) {
+      const int col = col0 + (wn * TN + n) * 16 + 4 * lq;
       if (row < p.M && col < p.N) {
         f32x4 v = acc[m][n] * scale;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] += b[e];
-        store4<OUT>(p.C, (int64_t)row * p.ldc + col, v, ncols);
+        for (int e = 0; e < 4; ++e) v[e] += bias_v[n][e];
+        store4<OUT>(p.C, (int64_t)row * p.ldc + col, v, (p.N - col) < 4 ? (p.N - col) : 4);
       }
     }
   }
