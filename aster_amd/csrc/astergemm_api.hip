@@ -242,6 +242,27 @@ int tile64_stages_of(const astergemm_config& c) {
   return tile_grid(c, 64, 64) > (short_rows ? 1 : 2) * (int64_t)chip_cus() ? 2 : 4;
 }
 
+// A ragged M (no whole groups of 8 rows) that stays with the general tile kernels, which are ahead of the
+// unsplit stream kernels there; back to back, stream / general in us, and on buffers that no kernel has read
+// yet behind the semicolon:
+//   one 64-row tile          fp8 14x26864x3760 24.6 / 17.7; 35.7 / 29.6, 10x19472x17056 128 / 88.2, bf16
+//                            53x27056x136 6.1 / 4.2, f16 51x16328x11448 173 / 97.4, MXFP4 12x31008x1536 6.9 / 5.5;
+//                            past it they are behind: MXFP4 73x25520x1536 7.5 / 8.3, f16 83x21408x5720 60.5 / 73.4
+//   MXFP4, up to two 64 x 64 199x2904x7168 17.3 / 11.5; 30.3 / 13.4, 250x1080x22016 66.4 / 30.1; 84.1 / 41.8,
+//     tiles per CU           859x2096x6656 (462 tiles) 20.9 / 18.8, behind: 534x3872x6656 (549) 20.6 / 24.7
+//   fewer than five K-steps, bf16 391x6864x288 7.5 / 6.5; 7.6 / 6.8, fp8 181x13136x256 5.7 / 4.8, 695x4408x256
+//     64 x 64 tiles          6.0 / 5.3
+//   fewer than seven, fp32   f16 1269x22136x312 50.7 / 36.5; 53.7 / 50.4, 5671x2424x416 28.3 / 22.7, fp8
+//     outputs, 256 x 256     1705x8232x848 27.4 / 23.4, behind: bf16 724x13440x104 12.3 / 13.0
+bool ragged_stays_general(const astergemm_config& c) {
+  if (c.M % 8 == 0 || c.operand_path != ASTERGEMM_OPERAND_LDS) return false;
+  if (c.M <= 64) return true;
+  if (c.dtype_ab == ASTERGEMM_MXFP4) return tile_grid(c, 64, 64) <= 2 * (int64_t)chip_cus();
+  const int64_t rb = row_bytes(c.dtype_ab, c.K);
+  if (rb < 5 * 128 && c.M > 128 && tile_grid(c, 128, 64) < 448) return true;
+  return rb < 7 * 128 && c.dtype_c == ASTERGEMM_F32 && tile_grid(c, 256, 256) >= 220;
+}
+
 // Split K where a kernel without K ranges (or with fewer) takes the problem too: 256 x 128 tiles, and
 // 128 x 128 tiles of a ragged M.  A call that has no scratch of its own for them -- the built-in scratch
 // or a caller's workspace too small, a stream under capture, whose graph may be replayed beside other work
@@ -345,6 +366,7 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out, int av
   const int unequal = unequal_tile_of(c);
   const bool unequal_split = unequal_split_pays(c);
   const int tile64_stages = tile64_stages_of(c);
+  const bool stays_general = !c.wg_tile_m && !c.wg_tile_n && !c.waves_m && !c.waves_n && ragged_stays_general(c);
 
   const Variant* best = nullptr;
   int best_index = -1;
@@ -353,6 +375,9 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out, int av
     const Variant* v = variant_at(i);
     if (v->family != family || !variant_matches_types(*v, c)) continue;
     if (i < num_tile_variants() && v->tile_m == 64 && v->stages != tile64_stages) continue;
+    if (stays_general && family == ASTERGEMM_KERNEL_TILE && i >= num_tile_variants() && v->rank != 4 &&
+        v->rank != 6)
+      continue;
     if (v->rank == 5 && v->tile_m != unequal) continue;
     if (v->rank == 6 && !unequal_split) continue;
     if ((avoid & kAvoidOptionalSplits) && optional_split(*v, c)) continue;

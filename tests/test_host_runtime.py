@@ -181,6 +181,24 @@ def test_stages_of_the_general_64_tile(M, N, K, dtype, name):
     assert named.lds_bytes == named.pipeline_stages * 128 * (136 if dtype == "mxfp4" else 128)
 
 
+@pytest.mark.parametrize("M,N,K,dtype,dtype_c,kind", [
+    (63, 27056, 136, "bf16", "bf16", "tile"), (65, 27056, 136, "bf16", "bf16", "stream"),
+    (64, 27056, 136, "bf16", "bf16", "stream"),                       # whole groups of 8 rows
+    (14, 26864, 3760, "fp8_e4m3", "f32", "tile"), (12, 31008, 1536, "mxfp4", "f32", "tile"),
+    (73, 25520, 1536, "mxfp4", "f32", "stream"),
+    (199, 2904, 7168, "mxfp4", "f32", "tile"), (200, 2904, 7168, "mxfp4", "f32", "stream"),
+    (1025, 1912, 7168, "mxfp4", "bf16", "tile"),                      # 510 tiles of 64 x 64
+    (1025, 1928, 7168, "mxfp4", "bf16", "stream"),                    # 527
+    (391, 6864, 288, "bf16", "bf16", "tile"), (391, 6864, 320, "bf16", "bf16", "stream"),
+    (392, 6864, 288, "bf16", "bf16", "stream"), (1269, 22136, 312, "f16", "f32", "tile"),
+    (1269, 22136, 448, "f16", "f32", "stream"), (1269, 22136, 312, "f16", "f16", "stream"),
+    (1272, 22136, 312, "f16", "f32", "stream"),
+    (130, 1032, 8192, "bf16", "bf16", "splitk"), (9, 4096, 11008, "fp8_e4m3", "bf16", "splitk"),
+])
+def test_which_ragged_row_counts_stay_with_the_general_tiles(M, N, K, dtype, dtype_c, kind):
+    assert gemm.GemmPlan.create(M, N, K, dtype, dtype_c).info.name.decode().startswith(kind + "_")
+
+
 def test_no_split_on_unequal_tiles_has_fewer_planes_than_the_square_split_it_replaces():
     """An eager call leaves its stream a workspace of the size it needed, and a captured call of the same
     config, which runs the square kernel, cannot make it larger."""
