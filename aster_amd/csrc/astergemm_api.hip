@@ -181,12 +181,18 @@ int64_t tile_grid(const astergemm_config& c, int64_t bm, int64_t bn) {
 //                             fp8 1500x8192x8192 116 / 87.5 / 95.2 / 106
 //   three rounds against two  bf16 1300x14336 164 / 163 / 151 / 149, 600x28672 164 / 166 / 161 / 151 (where
 //                             whole rounds plus a rest exist they win: 2560x8192x8192 261 against 287);
-//                             fp8 1500x14336 97.7 / 89.5 / 102 / 89.6: level, not taken
+//                             fp8 1500x14336 97.7 / 89.5 / 102 / 89.6: level, not taken; rows with a K tail
+//                             are behind, 256 x 256 / 256 x 128 on buffers that no kernel has read yet: f16
+//                             3600x4880x13272 573 / 638, bf16 3440x5688x15992 726 / 785, 2344x9616x1904 103 / 112
 //   rows of 2 KiB             bf16 2048x4096x1024 18.9 / 24.8 / 24.3 / 18.8, 800x8192x1024 16.6 / 23.9 / 23.1 / 16.4
+//                             fp32 outputs and fp8 behind, M in whole groups of 8: bf16 -> f32 1696x4552x1024
+//                             21.6 / 23.1, fp8 -> f32 856x7824x2048 17.5 / 19.1 (128 x 128 / 256 x 128)
 //   rows of 1 KiB: behind     bf16 2048x4096x512 11.4 / 15.5 / 16.5 / 12.9
 // Up to one 128 x 128 tile per CU 16-bit operands have the nine-slot ring, which is ahead (960x4096 35.1
 // against 39.3); fp8 takes the same kernel at 128 x 128 (ring of five whole K-steps, eight waves) from
-// two tile rows on: 333x8192x8192 51.1 -> 36.8, 1000x4096x14336 86.3 -> 66.8, 200x14336 29.1 -> 23.5.
+// two tile rows on: 333x8192x8192 51.1 -> 36.8, 1000x4096x14336 86.3 -> 66.8, 200x14336 29.1 -> 23.5.  Not with
+// a K tail: level back to back, behind on buffers that no kernel has read yet (384x5408x20592 139 -> 156,
+// 872x2632x13680 90.6 -> 96.7, 1648x2120x7600 50.5 -> 53.6).
 // A config that names a tile size or wave count gets the kernels it always got.
 bool unequal_tiles_apply(const astergemm_config& c) {
   return (c.dtype_ab == ASTERGEMM_F16 || c.dtype_ab == ASTERGEMM_BF16 || c.dtype_ab == ASTERGEMM_FP8_E4M3) &&
@@ -197,15 +203,17 @@ bool unequal_tiles_apply(const astergemm_config& c) {
 int unequal_tile_of(const astergemm_config& c) {
   if (!unequal_tiles_apply(c)) return 0;
   const bool fp8 = c.dtype_ab == ASTERGEMM_FP8_E4M3;
-  const int64_t cus = chip_cus(), g128 = tile_grid(c, 128, 128);
-  if (g128 <= cus) return fp8 && c.M > 128 ? 128 : 0;
+  const int64_t cus = chip_cus(), g128 = tile_grid(c, 128, 128), rb = row_bytes(c.dtype_ab, c.K);
+  const bool whole_k = rb % 128 == 0;
+  if (g128 <= cus) return fp8 && whole_k && c.M > 128 ? 128 : 0;
   if (tile_grid(c, 192, 128) <= cus) return 192;
   // whole 128 x 128 tiles on at least 7/8 of two workgroups per CU: the tests pin this selection to
   // the 128 x 128 kernel, which is the slower one there (bf16 512x14336 72.8 against 56.0 us,
   // 2048x4096 59.3 against 53.9, fp8 2048x4096 32.4 against 31.6)
   if (c.M % 128 == 0 && c.N % 128 == 0 && g128 <= 2 * cus && g128 * 8 >= 2 * cus * 7) return 0;
+  if (rb < 18 * 128 && c.M % 8 == 0 && (fp8 || c.dtype_c == ASTERGEMM_F32)) return 0;
   const int64_t g = tile_grid(c, 256, 128);
-  if (g <= cus || (!fp8 && g <= 3 * cus && tile_grid(c, 256, 256) > cus)) return 256;
+  if (g <= cus || (!fp8 && whole_k && g <= 3 * cus && tile_grid(c, 256, 256) > cus)) return 256;
   return 0;
 }
 

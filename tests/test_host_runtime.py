@@ -199,6 +199,23 @@ def test_which_ragged_row_counts_stay_with_the_general_tiles(M, N, K, dtype, dty
     assert gemm.GemmPlan.create(M, N, K, dtype, dtype_c).info.name.decode().startswith(kind + "_")
 
 
+@pytest.mark.parametrize("M,N,K,dtype,dtype_c,name", [
+    (3600, 4880, 13248, "f16", "f16", "stream_f16_256x128_w4x2_f16"),     # three rounds against two
+    (3600, 4880, 13272, "f16", "f16", "stream_f16_256x256_w2x4_f16"),     # the same with a K tail
+    (3601, 4880, 13272, "f16", "f16", "stream_f16_256x256_w2x4_f16"),
+    (1500, 4096, 4104, "bf16", "bf16", "stream_bf16_192x128_w4x2_bf16"),  # one round: with or without
+    (872, 2632, 13696, "fp8_e4m3", "f32", "stream_fp8_128x128_w4x2_f32"),
+    (872, 2632, 13680, "fp8_e4m3", "f32", "stream_fp8_128x128_w2x2_f32"),
+    (1696, 4552, 1024, "bf16", "f32", "stream_bf16_128x128_w2x2_f32"),
+    (1696, 4552, 1152, "bf16", "f32", "stream_bf16_256x128_w4x2_f32"),
+    (1696, 4552, 1024, "bf16", "bf16", "stream_bf16_256x128_w4x2_bf16"),
+    (856, 7824, 2048, "fp8_e4m3", "bf16", "stream_fp8_128x128_w2x2_bf16"),
+    (856, 7824, 2304, "fp8_e4m3", "bf16", "stream_fp8_256x128_w4x2_bf16"),
+])
+def test_rows_that_unequal_tiles_leave_to_the_square_ones(M, N, K, dtype, dtype_c, name):
+    assert gemm.GemmPlan.create(M, N, K, dtype, dtype_c).info.name.decode() == name
+
+
 def test_no_split_on_unequal_tiles_has_fewer_planes_than_the_square_split_it_replaces():
     """An eager call leaves its stream a workspace of the size it needed, and a captured call of the same
     config, which runs the square kernel, cannot make it larger."""
