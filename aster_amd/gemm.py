@@ -193,6 +193,33 @@ def _read_descriptor(path: str) -> dict:
     return desc
 
 
+def _kernel_of_descriptor(cfg: WeakScaledMappedGemmInstance,
+                          desc: dict) -> Tuple[_capi.Config, _capi.KernelInfo]:
+    """The kernel a descriptor of `cfg` names.  Normally what is selected for `cfg`; a descriptor
+    written when another kernel was selected for the same label gets the one it names, as the
+    reference's code object would."""
+    c, info = select_for_instance(cfg)
+    if info.name.decode() == desc["kernel"]:
+        return c, info
+    refusal = RuntimeError(f"descriptor names kernel {desc['kernel']!r} but config selects "
+                           f"{info.name.decode()!r}")
+    path = _OPERAND_PATH_ID.get(desc.get("operand_path"))
+    if desc.get("label") != cfg.label or path is None:
+        raise refusal
+    c = config_from_instance(cfg, use_mapping=False)
+    c.operand_path = path
+    lib, named = _capi.load(), _capi.KernelInfo()
+    for i in range(lib.astergemm_variant_count()):
+        _capi.check(lib.astergemm_variant_info(i, ctypes.byref(c), ctypes.byref(named)))
+        if named.name.decode() == desc["kernel"]:
+            c.variant = named.variant
+            try:
+                return c, select(c)
+            except _capi.AsterGemmError:
+                break
+    raise refusal
+
+
 @dataclass
 class GemmPlan:
     """A selected kernel plus its C-ABI config; launches on device pointers."""
@@ -401,10 +428,7 @@ def execute_gemm_hsaco(cfg: WeakScaledMappedGemmInstance, hsaco_path: str, num_i
         pytest.skip(f"GPU {mcpu} not available, skip execution")
     desc = _read_descriptor(hsaco_path)
     hip_init()
-    c, info = select_for_instance(cfg)
-    if info.name.decode() != desc["kernel"]:
-        raise RuntimeError(f"descriptor names kernel {desc['kernel']!r} but config selects "
-                           f"{info.name.decode()!r}")
+    c, info = _kernel_of_descriptor(cfg, desc)
     M, N, K = cfg.spec.gemm_size
     out_np = _OUT_NP[cfg.spec.dtype_c]
     if c.operand_path != _capi.OPERAND_LDS:

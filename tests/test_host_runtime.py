@@ -311,6 +311,27 @@ def test_compile_gemm_writes_descriptor(tmp_path):
         gemm._read_descriptor(str(tmp_path / "bad.hsaco"))
 
 
+def test_a_descriptor_of_another_selection_runs_the_kernel_it_names(tmp_path):
+    """1536 x 4096 x 4096 with a mapping no kernel has: 192 x 128 tiles are selected; a descriptor that was
+    written when the 128 x 128 kernel was gets that kernel.  Another instance's descriptor is refused."""
+    cfg = make_instance(1536, 4096, 4096, wg_tile=(96, 128), waves=(2, 2))
+    path = str(tmp_path / "k.hsaco")
+    gemm.compile_gemm(cfg, path)
+    desc = gemm._read_descriptor(path)
+    assert desc["kernel"] == "stream_bf16_192x128_w4x2_bf16"
+    c, info = gemm._kernel_of_descriptor(cfg, desc)
+    assert c.variant == 0 and info.name.decode() == desc["kernel"]
+    old = dict(desc, kernel="stream_bf16_128x128_w2x2_bf16", variant=9999)
+    c, info = gemm._kernel_of_descriptor(cfg, old)
+    assert info.name.decode() == old["kernel"] and c.variant == info.variant
+    other = make_instance(3072, 4096, 4096, wg_tile=(96, 128), waves=(2, 2))
+    for bad, inst in ((dict(old, kernel="no_such_kernel"), cfg), (old, other),
+                      (dict(old, kernel="stream_fp8_128x128_w2x2_bf16"), cfg),
+                      (dict(old, kernel="skinny_bf16_m16_bf16"), cfg)):
+        with pytest.raises(RuntimeError, match="descriptor names kernel"):
+            gemm._kernel_of_descriptor(inst, bad)
+
+
 def test_descriptor_says_when_the_mapping_is_not_honoured(tmp_path):
     import dataclasses
 
