@@ -1041,6 +1041,29 @@ def test_whole_rounds_plus_tail_split(gpu, M, N, dtype_ab, dtype_c, K):
         assert np.array_equal(out[rows, cols], whole[rows, cols])
 
 
+@pytest.mark.parametrize("M,N,cut", [(32768 + 521, 512, True), (32768 + 9, 512, True), (511, 32768 + 520, True),
+                                     (32768 + 8, 512, True), (32768 + 7, 512, False), (32768 + 1, 512, False)])
+@pytest.mark.parametrize("dtype_ab,dtype_c,K", [("bf16", "bf16", 264), ("f16", "f32", 128),
+                                                ("fp8_e4m3", "bf16", 384), ("mxfp4", "bf16", 512)])
+def test_whole_rounds_plus_a_ragged_rest(gpu, M, N, cut, dtype_ab, dtype_c, K):
+    """The same cut with rows off the groups of 8, along M (rests of 521, 9 and 8 rows) and along N.  The last
+    row group of the rest is staged shifted up, so a rest of fewer than 8 rows is not cut off: it would reach
+    into the rows of the first part."""
+    a, b, ex = operands(M, N, K, dtype_ab, a_std=1.0, b_std=1.0 if dtype_ab != "bf16" else 0.02)
+    bias = np.random.default_rng(3).standard_normal(N).astype(np.float32)
+    out, name = run_gemm(a, b, M, N, K, dtype_ab, dtype_c, bias=bias, wg_tile=(256, 256), ldc=N + 8, **ex)
+    assert ("tail128" in name) == cut and name.startswith("stream_"), name
+    want = G.gemm(a, b, _DT[dtype_ab], _DT[dtype_c], bias=bias, **ex)
+    check(out, want, dtype_c, N)
+    pad = out[:, N:]
+    assert np.isnan(pad).all() if dtype_c == "f32" else (pad == 0x7FC1).all()
+    plain = name.replace("_tail128", "")
+    small = plain.replace("256x256_" + plain.split("_")[3], "128x128_w2x2")
+    whole, wname = run_gemm(a, b, M, N, K, dtype_ab, dtype_c, bias=bias, variant=_variant_id(small), **ex)
+    assert wname == small
+    assert np.array_equal(out[M - 300:, N - 128:N], whole[M - 300:, N - 128:N])   # both sides of the cut
+
+
 def test_identity_operand_is_exact_at_full_width(gpu):
     # B = I: every output is one product plus zeros, so C == A bit for bit.
     M, N = 512, 8192

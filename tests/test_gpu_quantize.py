@@ -333,6 +333,49 @@ def test_fp8_quantiser_one_and_two_launch_forms(n, dtype):
     assert np.array_equal(got[:n], qo) and (got[n:] == 0xAB).all()
 
 
+@pytest.mark.parametrize("case", ["zeros", "nan", "inf", "huge", "tiny", "subnormal", "2^60", "2^-60"])
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+def test_fp8_quantiser_two_launch_edges(case, dtype):
+    """Tensors past the one-launch limit whose scale is no ordinary one (absmax zero, NaN, infinite, scales on
+    either side of 2^-60 and 2^60): the codes of every path of the encoder, the special element among the
+    elements whose place holds the partial maxima, in the middle and behind the last whole group."""
+    n = 131072 + 5003
+    x = np.random.default_rng(17).standard_normal(n).astype(np.float32)
+    with np.errstate(all="ignore"):
+        if case == "zeros":
+            x[:] = 0.0
+            x[::7] = -0.0
+        elif case in ("huge", "tiny", "subnormal"):
+            x *= np.float32({"huge": 6e37, "tiny": 1e-30, "subnormal": 1e-41}[case] if dtype != "f16" else
+                            {"huge": 1e4, "tiny": 1e-5, "subnormal": 1e-7}[case])
+        elif case.startswith("2^"):
+            if dtype == "f16":
+                pytest.skip("not in the range of f16")
+            # 448 * 2^+-60 is the largest (smallest) absmax of the plain path; some tensors beyond it
+            x = x / np.abs(x).max() * np.float32(448.0 * 2.0 ** int(case[2:]) * (1.01 if case == "2^60" else 0.99))
+        src = (x if dtype == "f32" else x.astype(np.float16) if dtype == "f16"
+               else (x.view(np.uint32) >> 16).astype(np.uint16))
+    for at in ((3, n // 2, n - 1) if case in ("nan", "inf") else (0,)):
+        y = src.copy()
+        if case in ("nan", "inf"):
+            y[at] = {"f32": {"nan": np.nan, "inf": -np.inf}, "f16": {"nan": np.nan, "inf": -np.inf},
+                     "bf16": {"nan": 0x7FC0, "inf": 0xFF80}}[dtype][case]
+        wide = (y.astype(np.uint32) << 16).view(np.float32) if dtype == "bf16" else y.astype(np.float32)
+        a, q, sc = GpuBuffer(y.nbytes + 16), GpuBuffer(n), GpuBuffer(4)
+        a.copy_from_host(y)
+        print(f"quantize_fp8_tensor {dtype} {case} at {at}", flush=True)
+        Q.quantize_fp8_tensor_device(a.ptr_value, n, q.ptr_value, sc.ptr_value, src_dtype=dtype)
+        got, s = np.empty(n, np.uint8), np.empty(1, np.float32)
+        q.copy_to_host(got)
+        sc.copy_to_host(s)
+        with np.errstate(all="ignore"):
+            qo, so = F.quantize_fp8_tensor(wide)
+        assert s[0].tobytes() == np.float32(so).tobytes()
+        assert np.array_equal(got, qo)
+        for bf in (a, q, sc):
+            bf.free()
+
+
 @pytest.mark.parametrize("rows", [1, 15, 127, 128, 129, 300])
 @pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
 def test_mxfp4_quantiser_lane_order_edges(rows, dtype):

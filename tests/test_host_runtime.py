@@ -216,6 +216,13 @@ def test_rows_that_unequal_tiles_leave_to_the_square_ones(M, N, K, dtype, dtype_
     assert gemm.GemmPlan.create(M, N, K, dtype, dtype_c).info.name.decode() == name
 
 
+@pytest.mark.parametrize("dtype,tag", [("bf16", "bf16"), ("fp8_e4m3", "fp8"), ("mxfp4", "mxfp4")])
+def test_a_rest_of_fewer_than_8_rows_is_not_cut_off(dtype, tag):
+    names = {r: gemm.GemmPlan.create(2048 + r, 8192, 8192, dtype, "bf16").info.name.decode() for r in range(17)}
+    for r, name in names.items():
+        assert name.startswith(f"stream_{tag}_256x") and ("tail128" in name) == (r >= 8), (r, name)
+
+
 def test_no_split_on_unequal_tiles_has_fewer_planes_than_the_square_split_it_replaces():
     """An eager call leaves its stream a workspace of the size it needed, and a captured call of the same
     config, which runs the square kernel, cannot make it larger."""
