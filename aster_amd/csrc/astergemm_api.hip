@@ -221,7 +221,9 @@ int unequal_tile_of(const astergemm_config& c) {
 // operand rows (tile rows x K-steps) that one range here does, on rows long enough to pay for the
 // planes.  Square split or unsplit -> this, us: bf16 500x4096x14336 83.6 -> 67.1, 333x4096x14336 72.2 ->
 // 61.1, 1000x4096x14336 133 -> 113, 250x8192x28672 162 -> 136, 500x8192x28672 275 -> 238; fp8
-// 500x4096x14336 54.4 -> 46.2.  Behind: equal or fewer rows saved (bf16 256x4096x14336 56.5 -> 59.4),
+// 500x4096x14336 54.4 -> 46.2; from 112 K-steps on where the square tiles are split too: bf16 256x8192x8192
+// (128) 46.3 -> 44.9, 192x8192x8192 40.4 -> 40.9 and, on buffers that no kernel has read yet, 53.4 -> 50.5,
+// 384x4096x11008 (172) 49.9 -> 48.3.  Behind: equal or fewer rows saved (bf16 256x4096x14336 56.5 -> 59.4),
 // shorter rows against an unsplit kernel (800x4096x11008 86.3 -> 88.0), few tile columns, where every XCD
 // reads all of A (2000x1024x8192 45.3 -> 59.1).
 bool unequal_split_pays(const astergemm_config& c) {

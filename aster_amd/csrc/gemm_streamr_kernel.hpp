@@ -3,10 +3,13 @@
 // measured against the square tiles stands at the rules of selection (unequal_tile_of,
 // unequal_split_pays).
 //
-// What bounds it: the operand bytes a CU receives from its XCD's L2 (23-31 B/clk in every kernel
-// of this family), not the matrix cores.  A 256 x 128 tile brings in 384 rows for 32768 outputs,
-// two 128 x 128 tiles 512 rows for the same; where a problem has too few 256 x 256 tiles to fill
-// the chip these are the shapes between.
+// What bounds it: 16-bit operands the matrix cores, at the clock the power limit leaves (busy 73 % of a
+// busy CU's cycles on 333 x 14336 x 4096, 84 % on 800 x 8192 x 8192, at 1.65 of 2.4 GHz; 34-36 bytes of
+// operands per CU and clock from L2, above what the square kernels draw), and the CUs without a tile or on
+// padding rows (224 of 256 busy, 333 of 384 rows); fp8 the operand bytes from L2 (25-29 per CU and clock,
+// matrix cores busy 52-60 %).  A 256 x 128 tile brings in 384 rows for 32768 outputs, two 128 x 128 tiles
+// 512 rows for the same; where a problem has too few 256 x 256 tiles to fill the chip these are the shapes
+// between.
 //
 // LDS is a ring of NS stages, each one whole K-step (128 bytes of every row of A's and B's tile):
 // three of 48 KiB, four of 40 KiB or five of 32 KiB.  Unlike the ring of gemm_stream_body, whose halves trade

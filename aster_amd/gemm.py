@@ -274,9 +274,12 @@ class GemmPlan:
         _capi.check(_capi.load().astergemm_prepare(ctypes.byref(self.config)))
 
     def workspace_bytes(self) -> int:
-        """Bytes of fp32 workspace a launch of this plan needs (0 unless its rows are cut into
-        K ranges); pass a buffer of that size as `workspace` to `run`, or leave it to the
-        library's own buffer."""
+        """Bytes of fp32 workspace the kernel of this plan (`info`) needs (0 unless its rows are cut
+        into K ranges); pass a buffer of that size as `workspace` to `run`, or leave it to the
+        library's own buffer.  Some of these problems also have a kernel that needs less, and a
+        call without scratch of its own runs that one: through `run_noalloc`, with a smaller
+        `workspace`, or captured without one.  Its fp32 sums differ in the last bits; with a buffer
+        of this size `run` has the same bits eagerly and captured."""
         n = ctypes.c_size_t()
         _capi.check(_capi.load().astergemm_workspace_bytes(ctypes.byref(self.config), ctypes.byref(n)))
         return n.value
@@ -293,7 +296,8 @@ class GemmPlan:
                     mx_a: int = None, mx_b: int = None, bias: int = None,
                     stream: int = None) -> None:
         """`run` through the entry point that never allocates device memory: K-range partial
-        sums go to the library's built-in scratch (`_capi.NOALLOC_SCRATCH_BYTES` per device)."""
+        sums go to the library's built-in scratch (`_capi.NOALLOC_SCRATCH_BYTES` per device), and
+        problems that have a kernel without them get that one (see `workspace_bytes`)."""
         ops = self._operands(dA, dB, dC, scale_a, scale_b, mx_a, mx_b, bias)
         _capi.check(_capi.load().astergemm_run_noalloc(
             ctypes.byref(self.config), ctypes.byref(ops),

@@ -223,11 +223,23 @@ int astergemm_select(const astergemm_config* cfg, astergemm_kernel_info* out);
 int astergemm_variant_count(void);
 int astergemm_variant_info(int index, const astergemm_config* cfg,
                            astergemm_kernel_info* out);
-/* One asynchronous launch on `stream` (hipStream_t, NULL = null stream).    */
+/* One asynchronous launch on `stream` (hipStream_t, NULL = null stream).
+ * Some problems have two kernels: one cut into K ranges, which astergemm_select
+ * describes, and one with none (or fewer) that runs when the call has no scratch
+ * of its own for the partial sums: a dWorkspace smaller than
+ * astergemm_workspace_bytes(), or no dWorkspace while `stream` is being captured
+ * (a graph may be replayed beside other work on the library's buffer), and always
+ * through astergemm_run_noalloc.  The two add the same products in another order:
+ * their fp32 sums differ in the last bits.  The same bits eagerly and under
+ * capture: pass a workspace of that size, or name the kernel in cfg->variant.
+ * Row-major MXFP4 scale planes may lie on any 8-byte boundary; off a 16-byte one
+ * the general tile kernels run, also with other last bits.                    */
 int astergemm_run(const astergemm_config* cfg, const astergemm_operands* ops,
                   void* stream);
-/* Bytes of fp32 workspace astergemm_run needs for cfg with the variant it
- * selects (0 for most shapes: only rows cut into K ranges need one).  The
+/* Bytes of fp32 workspace the kernel that astergemm_select describes needs for
+ * cfg (0 for most shapes: only rows cut into K ranges need one).  A smaller one
+ * is refused, or where another kernel takes the problem without it (see
+ * astergemm_run) left unused.  The
  * reference's kernels have no workspace (every kernel takes exactly A, B, C:
  * test_102_gemm_python_multitile_g2s_directb_cdna4.py:150-156); this is the
  * caller-owned form of what split K adds here.                              */
@@ -242,7 +254,7 @@ int astergemm_workspace_bytes(const astergemm_config* cfg, size_t* bytes);
  * with ASTERGEMM_EINVAL, unless a kernel without K ranges (or with fewer) takes
  * it, which then runs.  Every call on a device shares that array, whatever
  * its stream: calls that overlap on one device race (calls on one stream are
- * ordered and safe).  Nothing in the array has to start at zero: every launch
+ * ordered and safe, also from several host threads).  Nothing in the array has to start at zero: every launch
  * writes all the planes it later adds.  The array's address is looked up on
  * the first call on a device, or by aster_rt_init / astergemm_prepare for the
  * current device.  A kernel's FIRST launch on a device also sets a function

@@ -106,6 +106,39 @@ def test_split_configs_without_scratch_of_their_own(gpu, M, N, K):
         check()
 
 
+@pytest.mark.parametrize("M,N,K", [(333, 4096, 14336), (130, 1032, 8192), (512, 4096, 14336)])
+def test_a_workspace_of_the_stated_size_gives_the_eager_bits_under_capture(gpu, M, N, K):
+    """Configs with an optional split: with a caller's workspace a captured call runs the kernel an eager one
+    does, several replays with eager work between them; so does a plan that names the kernel."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(M)
+    a = torch.randn(M, K, generator=g, device="cuda").to(torch.bfloat16)
+    b = (torch.randn(N, K, generator=g, device="cuda") * 0.02).to(torch.bfloat16)
+    eager, got = (torch.zeros(M, N, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    plan = AG.GemmPlan.create(M, N, K, "bf16", "bf16")
+    pinned = AG.GemmPlan.create(M, N, K, "bf16", "bf16", variant=plan.info.variant)
+    need = plan.workspace_bytes()
+    ws = torch.zeros(need, device="cuda", dtype=torch.uint8)
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    print(f"{plan.info.name.decode()} M={M} N={N} K={K}", flush=True)
+    plan.run(a.data_ptr(), b.data_ptr(), eager.data_ptr(), stream=stream.cuda_stream)
+    stream.synchronize()
+    for p, extra in ((plan, dict(workspace=ws.data_ptr(), workspace_bytes=need)), (pinned, {})):
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            p.run(a.data_ptr(), b.data_ptr(), got.data_ptr(), stream=stream.cuda_stream, **extra)
+        for _ in range(3):
+            got.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(stream):
+                graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(got, eager)
+            plan.run(a.data_ptr(), b.data_ptr(), eager.data_ptr(), stream=stream.cuda_stream)
+            torch.cuda.synchronize()
+
+
 def test_caller_workspace_matches_the_library_workspace(gpu):
     M, N, K = 96, 1000, 16384
     rng = np.random.default_rng(11)
