@@ -265,15 +265,16 @@ int astergemm_workspace_bytes(const astergemm_config* cfg, size_t* bytes);
 int astergemm_run_noalloc(const astergemm_config* cfg, const astergemm_operands* ops,
                           void* stream);
 
-/* Does, for the kernel `cfg` selects on the current device, everything a first
- * launch does apart from launching: raises the kernel's dynamic-LDS limit
+/* Does, for the kernel `cfg` selects on the current device and for those it
+ * selects without scratch or for scale planes on 8-byte boundaries (see
+ * astergemm_run), everything a first launch does apart from launching: raises the kernel's dynamic-LDS limit
  * (hipFuncSetAttribute), caches the device's compute-unit count and looks up
  * the address of the built-in scratch.  None of these is a stream operation,
  * so they must not happen inside a stream capture: astergemm_run and
  * astergemm_run_noalloc REFUSE a kernel's first launch on a device when the
  * stream is being captured (ASTERGEMM_EHIP, the message names this function).
  * Call it once per config and device before capturing (an eager launch of the
- * same config does the same).  Allocates nothing when the config's partial
+ * same config, with scale planes aligned alike, does the same).  Allocates nothing when the config's partial
  * sums fit the built-in scratch; reads no operand.  No counterpart in the
  * reference, whose kernels carry their LDS size in the code object. */
 int astergemm_prepare(const astergemm_config* cfg);
