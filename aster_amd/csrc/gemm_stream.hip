@@ -299,7 +299,9 @@ const char* check_stream_splitk(const astergemm_config& c) {
   if (const char* why = check_stream_whole_k(c)) return why;
   if (c.dtype_ab == ASTERGEMM_MXFP4 && c.K % 512 != 0) return "K must be a multiple of 512";
   const int64_t tiles = ((c.M + 127) / 128) * ((c.N + 127) / 128);
-  // a ragged M with a handful of tiles stays with the 64 x 64 kernels (pinned by the tests)
+  // a ragged M with a handful of tiles stays with the 64 x 64 kernels: the tests pin this selection, which is
+  // the slower one there (bf16 100x512x8192 31.8 against 12.4 us, 129x256x28672 102 against 22.3, fp8
+  // 250x384x14336 31.2 against 14.3, MXFP4 129x256x28672 36.0 against 13.0, 333x256x8192 12.6 against 11.6)
   if (c.M % 8 != 0 && tiles < 8) return "split K of a ragged M needs eight output tiles";
   // shorter rows: the unsplit 64 x 64 kernels are ahead (fp8 256x4096x4096: 15.2 against 19.8 us)
   const int64_t min_steps = c.dtype_ab == ASTERGEMM_MXFP4 ? 32 : 64;
