@@ -870,7 +870,8 @@ int astergemm_prepare(const astergemm_config* cfg) {
     return rc;
   if (cfg->variant != 0) return 0;
   // the kernels that other pointers than the usual ones lead to (choose_for_call)
-  for (int avoid = 1; avoid <= (kAvoidOptionalSplits | kAvoidMx16); ++avoid) {
+  const int last = cfg->dtype_ab == ASTERGEMM_MXFP4 ? kAvoidOptionalSplits | kAvoidMx16 : kAvoidOptionalSplits;
+  for (int avoid = 1; avoid <= last; ++avoid) {
     const Variant* o;
     {
       KeepError keep;  // a named tile may exist for 16-byte planes only

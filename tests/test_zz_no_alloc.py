@@ -353,6 +353,47 @@ def test_noalloc_launches_replay_from_a_graph(gpu):
             bf.free()
 
 
+_PLANES_CHILD = r"""
+import ctypes
+import torch
+from aster_amd import _capi, gemm as AG
+_capi.check(_capi.load().aster_rt_init())
+M, N, K = 333, 1032, 1024                      # AUTO: a stream kernel; planes off 16 bytes: the general tile kernel
+g = torch.Generator(device="cuda").manual_seed(1)
+draw = lambda rows: torch.randint(0, 256, (rows, K // 2), generator=g, device="cuda", dtype=torch.uint8)
+mx = lambda rows: torch.randint(118, 123, (rows * K // 32 + 8,), generator=g, device="cuda", dtype=torch.uint8)
+a, b, ma, mb = draw(M), draw(N), mx(M), mx(N)
+got, want = (torch.zeros(M, N, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+plan = AG.GemmPlan.create(M, N, K, "mxfp4", "bf16")
+plan.prepare()
+torch.cuda.synchronize()
+graph = torch.cuda.CUDAGraph()
+args = lambda c: (a.data_ptr(), b.data_ptr(), c.data_ptr())
+planes = dict(mx_a=ma.data_ptr() + 8, mx_b=mb.data_ptr() + 8)
+with torch.cuda.graph(graph):
+    plan.run(*args(got), stream=torch.cuda.current_stream().cuda_stream, **planes)
+plan.run(*args(want), **planes)
+for _ in range(3):
+    got.zero_()
+    torch.cuda.synchronize()
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(got, want) and float(want.float().abs().max()) > 0
+print("PLANES-OK", flush=True)
+"""
+
+
+def test_prepare_readies_the_kernel_of_planes_on_8_byte_boundaries(gpu):
+    # in a process of its own, where nothing has launched the general tile kernel yet
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    print("child process: prepare, capture with planes off 16 bytes, replays", flush=True)
+    proc = subprocess.run([sys.executable, "-c", _PLANES_CHILD], cwd=root, capture_output=True, text=True,
+                          timeout=110)
+    assert proc.returncode == 0 and "PLANES-OK" in proc.stdout, proc.stdout[-2000:] + proc.stderr[-2000:]
+
+
 _CAPTURE_CHILD = r"""
 import ctypes, sys
 import numpy as np
