@@ -9,6 +9,7 @@
 #include <vector>
 
 #include "astergemm_internal.h"
+#include "gemm_kwave.h"
 
 namespace astergemm {
 
@@ -252,6 +253,22 @@ int tile64_stages_of(const astergemm_config& c) {
   return tile_grid(c, 64, 64) > (short_rows ? 1 : 2) * (int64_t)chip_cus() ? 2 : 4;
 }
 
+// K split over the waves of a workgroup instead of the general 64 x 64 tile kernel (rank 8): its tiles
+// would not fill the chip, and the row is long enough for its K loop to be what the time goes on.
+bool kwave_tile_pays(const astergemm_config& c) {
+  return c.dtype_ab != ASTERGEMM_MXFP4 && c.operand_path == ASTERGEMM_OPERAND_LDS && !c.wg_tile_m &&
+         !c.wg_tile_n && !c.waves_m && !c.waves_n && row_bytes(c.dtype_ab, c.K) > 8 * 128 &&
+         tile_grid(c, 64, 64) < chip_cus();
+}
+
+// The same for decoding on rows of bytes that the kernels with resident activations do not take (rank 7).
+bool kwave_split_pays(const astergemm_config& c) {
+  return (c.dtype_ab == ASTERGEMM_FP8_E4M3 || c.dtype_ab == ASTERGEMM_MXFP4) &&
+         c.operand_path == ASTERGEMM_OPERAND_LDS && !c.wg_tile_m && !c.wg_tile_n && !c.waves_m &&
+         !c.waves_n && c.M <= 64 && c.K >= 4096 && c.N >= 1024 &&
+         kwave_decode_form(c.dtype_ab, c.M, c.N, c.K, chip_cus(), 1);
+}
+
 // A ragged M (no whole groups of 8 rows) that stays with the general tile kernels, which are ahead of the
 // unsplit stream kernels there; back to back, stream / general in us, and on buffers that no kernel has read
 // yet behind the semicolon:
@@ -376,6 +393,7 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out, int av
   const int unequal = unequal_tile_of(c);
   const bool unequal_split = unequal_split_pays(c);
   const int tile64_stages = tile64_stages_of(c);
+  const bool kwave_tile = kwave_tile_pays(c), kwave_split = kwave_split_pays(c);
   const bool stays_general = !c.wg_tile_m && !c.wg_tile_n && !c.waves_m && !c.waves_n && ragged_stays_general(c);
 
   const Variant* best = nullptr;
@@ -384,7 +402,9 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out, int av
   for (int i = 0; i < total_variants(); ++i) {
     const Variant* v = variant_at(i);
     if (v->family != family || !variant_matches_types(*v, c)) continue;
-    if (i < num_tile_variants() && v->tile_m == 64 && v->stages != tile64_stages) continue;
+    if (v->rank == 7 && !kwave_split) continue;
+    if (v->rank == 8 && !kwave_tile) continue;
+    if (i < num_tile_variants() && v->rank < 7 && v->tile_m == 64 && v->stages != tile64_stages) continue;
     if (stays_general && family == ASTERGEMM_KERNEL_TILE && i >= num_tile_variants() && v->rank != 4 &&
         v->rank != 6)
       continue;
@@ -467,6 +487,8 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out, int av
         // split K (rank 4) only passes its check where it was measured ahead of every
         // unsplit kernel: few output tiles, long rows
         if (x->rank == 4) return 3;
+        if (x->rank == 7) return 4;
+        if (x->rank == 8) return 0;
         // unequal sides: offered only where the rule took them; the whole-rounds form stays ahead
         // (fp8 on 128 x 128: the square kernel's lines)
         if (x->rank == 6 || (x->rank == 5 && x->tile_m > 128)) return 4;
@@ -549,8 +571,21 @@ void describe(const Variant& v, int index, const astergemm_config& c, astergemm_
   o->flops = 2 * c.M * c.N * c.K;
   o->bytes = algorithmic_bytes(c);
   snprintf(o->name, sizeof(o->name), "%s", v.name);
+  const void* func = v.func;
+  LaunchForm f;
+  if (v.form && !c.wg_tile_m && !c.wg_tile_n && !c.waves_m && !c.waves_n && v.form(c, device_cus(), &f)) {
+    o->grid_x = f.grid;
+    o->block_x = f.threads;
+    o->lds_bytes = f.lds_bytes;
+    o->wg_tile_m = f.tile_m;
+    o->wg_tile_n = f.tile_n;
+    o->waves_m = f.waves_m;
+    o->waves_n = f.waves_n;
+    o->pipeline_stages = f.stages;
+    func = f.func;
+  }
   hipFuncAttributes fa;
-  if (hipFuncGetAttributes(&fa, v.func) == hipSuccess) {
+  if (func && hipFuncGetAttributes(&fa, func) == hipSuccess) {
     o->vgprs = fa.numRegs;
     o->agprs = 0;
   } else {
@@ -622,6 +657,7 @@ int build_args(const Variant& v, const astergemm_config& c, const astergemm_oper
   // MXFP4 +1.5 %, bf16 -0.1 %, same process
   a->group_m = (a->tiles_m % 8 == 0 && a->tiles_n % 32 == 0) ? -1 : 8;
   a->split_k = 1;
+  a->named_tile = c.wg_tile_m || c.wg_tile_n || c.waves_m || c.waves_n;
   // rows cut into K ranges: the caller's workspace when one is given, else the library's own
   if (ops.dWorkspace) {
     const size_t need = workspace_need(v, c);

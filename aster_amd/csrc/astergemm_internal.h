@@ -28,6 +28,7 @@ struct GemmArgs {
   int32_t tiles_m, tiles_n;
   int32_t group_m;       // tile rows per rasterisation group; < 0: band order (see map_tile)
   int32_t split_k;       // skinny path: K slices per output row block
+  int32_t named_tile;    // the config names a tile or a wave count: launchers keep to their own kernels
   float* workspace;      // fp32 partials [split_k][M][N] when a row is cut into K ranges; set by
                          // the caller of a launcher = use this buffer, null = the library's own
 };
@@ -44,6 +45,13 @@ __host__ __device__ inline int64_t row_bytes(int dtype, int64_t k) {
 }
 
 inline int out_elt_bytes(int dtype) { return dtype == ASTERGEMM_F32 ? 4 : 2; }
+
+// What a launcher with several kernels launches for one problem.
+struct LaunchForm {
+  int grid = 0, tile_m = 0, tile_n = 0, waves_m = 0, waves_n = 0, stages = 0, lds_bytes = 0;
+  int threads = 0;
+  const void* func = nullptr;
+};
 
 // One entry of the variant table (filled in by gemm_tile.hip / gemm_skinny.hip).
 struct Variant {
@@ -71,6 +79,9 @@ struct Variant {
   int (*grid)(const astergemm_config& c, int cus) = nullptr;
   // Layout of A's e8m0 plane this variant reads (astergemm_mx_layout); row-major by default.
   int mx_a_layout = 0;
+  // Launchers with a second kernel for some problems: its description when this one is among them
+  // (`cus` as for grid; 0 = no device, nothing is known to fill it).  splits() stays an upper bound then.
+  bool (*form)(const astergemm_config& c, int cus, LaunchForm* o) = nullptr;
 };
 
 // Compute units of the current device (0 when there is none), cached per device ordinal.

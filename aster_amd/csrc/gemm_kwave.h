@@ -1,0 +1,34 @@
+// K split over the waves of a workgroup (gemm_kwave_kernel.hpp): which shape a problem takes, its launch
+// and its description.
+#pragma once
+#include "astergemm_internal.h"
+
+namespace astergemm {
+
+struct KwaveForm {
+  int shape = -1;  // -1: the problem stays with the other kernels
+  int per = 0;     // weight rows of a workgroup
+  int ranges = 1;  // K ranges
+  explicit operator bool() const { return shape >= 0; }
+};
+
+// M <= 64, as part of the decode kernels' launchers (`dt` operands, `cus` = compute units, 0 = no device;
+// at most `max_ranges` K ranges, what the launcher states as its workspace).
+KwaveForm kwave_decode_form(int dt, int64_t M, int64_t N, int64_t K, int cus, int max_ranges);
+// M <= 64 on rows the kernels with resident activations do not take, without dynamic LDS past the default
+// limit (the launcher it is part of sets no function attribute).
+KwaveForm kwave_small_decode_form(int dt, int64_t M, int64_t N, int64_t K, int cus);
+
+// Any M and N: the smallest tile that leaves at most one workgroup per CU, else 64 x 64.
+KwaveForm kwave_tile_form(int dt, int64_t M, int64_t N, int64_t K, int cus);
+
+int kwave_launch(int dt, int out, const GemmArgs& a, const KwaveForm& f, hipStream_t s);
+// The one-time step of every shape of `dt` on the current device (see lds_attr_once).
+int kwave_ready(int dt);
+void kwave_describe(int dt, const KwaveForm& f, int64_t M, int64_t N, LaunchForm* o);
+bool kwave_decode_describe(const astergemm_config& c, int cus, int max_ranges, LaunchForm* o);
+bool kwave_tile_describe(const astergemm_config& c, int cus, LaunchForm* o);
+bool kwave_split_describe(const astergemm_config& c, int cus, LaunchForm* o);  // decode form, else tile form
+bool kwave_small_decode_describe(const astergemm_config& c, int cus, LaunchForm* o);
+
+}  // namespace astergemm

@@ -1,0 +1,258 @@
+// Shapes, rules and launches of the kernels that split K over the waves of a workgroup
+// (device code: gemm_kwave_kernel.hpp).  Compiled once per operand type (AG_KWAVE_DT); the unit of f16
+// operands also holds what all of them share.
+#include "gemm_kwave.h"
+#include "gemm_kwave_kernel.hpp"
+
+namespace astergemm {
+
+// Tiles, waves (tile rows x tile columns x K) and stages; the second number of stages is MXFP4's, whose
+// scale bytes share the ring.  X(index, BM, BN, WM, WN, WK, S, S of MXFP4)
+#define AG_KWAVE_SHAPES(X)       \
+  X(0, 16, 16, 1, 1, 8, 5, 4)    \
+  X(1, 16, 32, 1, 1, 8, 3, 3)    \
+  X(2, 16, 48, 1, 1, 4, 5, 4)    \
+  X(3, 16, 64, 1, 1, 4, 4, 3)    \
+  X(4, 16, 16, 1, 1, 4, 4, 3)    \
+  X(5, 32, 16, 2, 1, 4, 6, 6)    \
+  X(6, 32, 32, 1, 2, 4, 4, 4)    \
+  X(7, 32, 64, 1, 2, 4, 3, 3)    \
+  X(8, 32, 128, 2, 2, 2, 4, 3)   \
+  X(9, 64, 32, 2, 1, 4, 3, 3)    \
+  X(10, 64, 48, 2, 1, 2, 5, 5)   \
+  X(11, 64, 64, 2, 2, 2, 3, 3)   \
+  X(12, 64, 128, 2, 2, 2, 3, 3)
+
+struct KwaveShape {
+  int bm, bn, wm, wn, wk, stages, lds;
+  const void* func;
+  int (*launch)(const KwaveArgs& q, int grid, hipStream_t s);
+};
+constexpr int kKwaveShapes = 13;
+const KwaveShape* kwave_shapes_f16();
+const KwaveShape* kwave_shapes_bf16();
+const KwaveShape* kwave_shapes_fp8();
+const KwaveShape* kwave_shapes_mxfp4();
+
+namespace {
+
+template <int DT, int BM, int BN, int WM, int WN, int WK, int S>
+int launch_kwave(const KwaveArgs& q, int grid, hipStream_t s) {
+  constexpr int lds = S * WK * kwave_step_bytes(DT, BM, BN);
+  AG_LAUNCH_KERNEL((gemm_kwave_kernel<DT, BM, BN, WM, WN, WK, S>), dim3(grid), dim3(WM * WN * WK * 64), lds, s,
+                   q);
+  return (int)hipGetLastError();
+}
+
+template <int DT, int BM, int BN, int WM, int WN, int WK, int S>
+constexpr KwaveShape kwave_shape() {
+  return KwaveShape{BM, BN, WM, WN, WK, S, S * WK * kwave_step_bytes(DT, BM, BN),
+                    (const void*)gemm_kwave_kernel<DT, BM, BN, WM, WN, WK, S>,
+                    launch_kwave<DT, BM, BN, WM, WN, WK, S>};
+}
+
+#define AG_KWAVE_ENTRY(I, BM, BN, WM, WN, WK, S, S4) \
+  kwave_shape<AG_KWAVE_DT, BM, BN, WM, WN, WK, AG_KWAVE_DT == ASTERGEMM_MXFP4 ? S4 : S>(),
+const KwaveShape kShapes[kKwaveShapes] = {AG_KWAVE_SHAPES(AG_KWAVE_ENTRY)};
+
+}  // namespace
+
+#if AG_KWAVE_DT == 0
+const KwaveShape* kwave_shapes_f16() { return kShapes; }
+#elif AG_KWAVE_DT == 1
+const KwaveShape* kwave_shapes_bf16() { return kShapes; }
+#elif AG_KWAVE_DT == 2
+const KwaveShape* kwave_shapes_fp8() { return kShapes; }
+#else
+const KwaveShape* kwave_shapes_mxfp4() { return kShapes; }
+#endif
+
+#if AG_KWAVE_DT == 0
+namespace {
+
+const KwaveShape* shapes_of(int dt) {
+  switch (dt) {
+    case ASTERGEMM_F16: return kwave_shapes_f16();
+    case ASTERGEMM_BF16: return kwave_shapes_bf16();
+    case ASTERGEMM_FP8_E4M3: return kwave_shapes_fp8();
+    default: return kwave_shapes_mxfp4();
+  }
+}
+
+// Weight rows of a workgroup when `tiles_m` tile rows share the chip: one round, groups of 8 rows.
+int rows_per(int64_t N, int tiles_m, int cus) {
+  const int slots = cus / tiles_m > 0 ? cus / tiles_m : 1;
+  return (int)(((N + slots - 1) / slots + 7) / 8 * 8);
+}
+
+int kwave_blocks(int tiles_m, int tiles_n) { return tiles_m * ((tiles_n + 7) & ~7); }
+
+}  // namespace
+
+// Decoding: the tile that brings the fewest operand rows into a CU while one round covers all of N (a
+// workgroup's panel is N / CUs rows in groups of 8, not the tile's), within two limits:
+//   * panels of more than 64 rows with up to 16 activation rows stay with the resident kernels, whose
+//     activations are then read once for many weight rows (bf16 16x28672x4096 37.3 us against 40.2 for
+//     16 x 128 tiles, fp8 21.6 / 23.4, MXFP4 11.5 / 13.2); MXFP4 on rows of 2, 4 or 8 KiB already from
+//     32 on (16x14336x4096 7.3 / 7.5).
+//   * a workgroup's own rows over all of K, (bm + per) * rb bytes, come from L2 at about 60 GB/s.  Where K
+//     ranges on 64-row panels take half a megabyte off that (two ranges, whose planes weigh more: three
+//     quarters), they pay for the planes and the kernel that adds them: bf16 64x4096x14336 37.2 -> 28.4
+//     (resident 32.9), 32x4096x11008 22.7 -> 20.2, fp8 64x8192x28672 54.6 -> 48.5 (55.9); behind: fp8
+//     64x4096x14336 14.3 / 17.5, bf16 64x8192x8192 29.4 / 30.7.  MXFP4 of more than 48 rows on such
+//     rows stays resident (64x8192x28672 39.6 / 42.2).
+// Resident kernel / this, us, over rotating weights (three sets):
+//   M       bf16 4096x4096  14336x4096   28672x4096   4096x14336   4096x11008   8192x8192    1024x8192
+//   8       8.1 / 7.4       19.8 / 18.7  resident     24.4 / 19.8  19.5 / 16.8  28.6 / 21.9  10.0 / 6.9
+//   16      8.4 / 7.4       20.1 / 18.9  resident     25.4 / 22.8  20.0 / 18.3  28.7 / 21.9  10.3 / 7.4
+//   32      11.6 / 8.0      22.5 / 19.6  40.2 / 36.6  28.0 / 24.0  22.6 / 20.2  30.7 / 22.9  13.7 / 7.6
+//   64      15.1 / 8.9      27.7 / 23.4  50.7 / 38.3  32.9 / 28.4  28.7 / 24.2  34.1 / 29.4  13.2 / 8.9
+//   fp8 16  6.1 / 5.4       12.3 / 11.1  resident     15.0 / 11.3  28.0 / 10.0  19.4 / 12.1  6.9 / 5.6
+//   fp8 64  9.4 / 6.7       17.6 / 12.3  26.9 / 22.2  21.8 / 14.3  28.7 / 12.5  18.2 / 13.2  9.7 / 6.1
+//   fp4 16  4.8 / 4.6       resident     resident     10.9 / 7.4   14.6 / 7.4   10.2 / 7.9   5.9 / 4.7
+//   fp4 64  6.5 / 5.4       11.6 / 9.4   19.0 / 14.5  16.9 / 11.0  17.0 / 9.1   14.5 / 10.9  8.6 / 4.8
+// (fp8 and MXFP4 4096x11008, no whole 512 bytes: against the tile kernels.)
+KwaveForm kwave_decode_form(int dt, int64_t M, int64_t N, int64_t K, int cus, int max_ranges) {
+  KwaveForm f;
+  const int64_t rb = row_bytes(dt, K);
+  if (cus <= 0 || M < 1 || M > 64 || N < 1 || N > INT32_MAX / 2 || rb % 16 != 0) return f;
+  const int t16 = (int)((M + 15) / 16), per = rows_per(N, 1, cus);
+  auto take = [&](int shape, int bm, int rows) {
+    const int64_t t64 = (N + 63) / 64;
+    int r = (int)(cus / t64);
+    r = r > 4 ? 4 : r;
+    r = r > max_ranges ? max_ranges : r;
+    const int64_t own = (bm + rows) * rb, cut = r > 1 ? (bm + 64) * rb / r : own;
+    if (M > 16 && own - cut > (r == 2 ? 768 << 10 : 512000)) {
+      f.shape = M <= 32 ? 7 : 11;
+      f.per = 64;
+      f.ranges = r;
+    } else if (!(dt == ASTERGEMM_MXFP4 && M > 48 && own > 1300000)) {
+      f.shape = shape;
+      f.per = rows;
+    }
+    return f;
+  };
+  if (const int p16 = rows_per(N, t16, cus); p16 <= 16) return take(0, 16, p16);
+  if (M <= 16) {
+    const bool resident = dt == ASTERGEMM_MXFP4 && (K == 4096 || K == 8192 || K == 16384);
+    if (per > (resident ? 32 : 64)) return f;
+    return per <= 32 ? take(1, 16, per) : per <= 48 ? take(2, 16, per) : take(3, 16, per);
+  }
+  if (per > 128) return f;
+  if (M <= 32)
+    return per <= 16 ? take(5, 32, per) : per <= 32 ? take(6, 32, per) : per <= 64 ? take(7, 32, per)
+                                                                                  : take(8, 32, per);
+  if (const int half = rows_per(N, 2, cus); half <= 32) return take(6, 32, half);
+  return per <= 32 ? take(9, 64, per) : per <= 48 ? take(10, 64, per) : per <= 64 ? take(11, 64, per)
+                                                                                 : take(12, 64, per);
+}
+
+// Rows the resident kernels do not take (K a multiple of 32 below 2048, or no whole 512 bytes), one round of
+// 16 x 16 tiles: against gemm_skinny_kernel, us: bf16 16x1000x1504 6.0 -> 3.8, 40x300x1984 15.8 -> 4.0,
+// 64x1000x992 9.9 -> 3.7, 62x592x352 5.5 -> 3.8 (3.7 is what a launch takes here).
+KwaveForm kwave_small_decode_form(int dt, int64_t M, int64_t N, int64_t K, int cus) {
+  KwaveForm f;
+  if (cus <= 0 || M < 1 || M > 64 || N < 1 || N > INT32_MAX / 2 || row_bytes(dt, K) % 16 != 0) return f;
+  const int per = rows_per(N, (int)((M + 15) / 16), cus);
+  if (per <= 16) f.shape = 4, f.per = per;
+  return f;
+}
+
+// Small products, general 64 x 64 tile kernel / this, us: bf16 300x300x2048 10.0 / 5.4 (32 x 32),
+// 500x500x1024 6.7 / 4.0, 207x28x1440 8.0 / 3.9 (16 x 16), 600x600x2048 10.2 / 7.3 (32 x 64), 1000x1000x512
+// 5.5 / 4.6 (64 x 64), 777x1001x1032 8.1 / 7.9 (bound by rows that start off the 128-byte lines:
+// 777x1001x1024 7.0 / 6.4); fp8 100x4096x4096 11.0 / 7.5.  From one 64 x 64 tile per CU on the general kernel
+// is level or ahead (1200x1200x1000 11.6 / 13.3).
+KwaveForm kwave_tile_form(int dt, int64_t M, int64_t N, int64_t K, int cus) {
+  (void)dt, (void)K;
+  static const struct { int shape, bm, bn; } kOrder[] = {{0, 16, 16}, {6, 32, 32}, {7, 32, 64}};
+  KwaveForm f;
+  f.shape = 11;
+  f.per = 64;
+  for (const auto& t : kOrder) {
+    const int64_t g = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+    if (g < cus || (g == cus && t.bn <= 32)) {
+      f.shape = t.shape, f.per = t.bn;
+      break;
+    }
+  }
+  return f;
+}
+
+int kwave_ready(int dt) {
+  static std::atomic<uint64_t> all[4], devs[4][kKwaveShapes];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess) return (int)hipGetLastError();
+  const uint64_t bit = (uint64_t)1 << (dev & 63);
+  if (all[dt & 3].load(std::memory_order_acquire) & bit) return 0;
+  const KwaveShape* shapes = shapes_of(dt);
+  for (int i = 0; i < kKwaveShapes; ++i) {
+    if (shapes[i].lds <= 65536) continue;  // within the default limit
+    if (int e = lds_attr_once(devs[dt & 3][i], shapes[i].func, shapes[i].lds)) return e;
+  }
+  all[dt & 3].fetch_or(bit, std::memory_order_release);
+  return 0;
+}
+
+int kwave_launch(int dt, int out, const GemmArgs& a, const KwaveForm& f, hipStream_t s) {
+  const KwaveShape& sh = shapes_of(dt)[f.shape];
+  KwaveArgs q;
+  q.g = a;
+  q.g.tiles_m = (a.M + sh.bm - 1) / sh.bm;
+  q.g.tiles_n = (a.N + f.per - 1) / f.per;
+  q.per = f.per;
+  q.ranges = f.ranges;
+  q.range_steps = (a.ksteps + f.ranges - 1) / f.ranges;
+  q.out = out;
+  // Past the last-level cache where that is no use: a matrix of more than 64 MiB is not found there again
+  // after a few others; up to 8 activation rows the loop is the weight stream and little else, from 30 MiB
+  // on.  Through the cache / past it, us, three sets in turn and cold: bf16 8x4096x11008 16.0 / 15.7 and 18.1 /
+  // 16.4, fp8 8x14336x4096 10.3 / 10.2 and 11.9 / 10.8; the other side: fp8 64x14336x4096 12.1 / 13.7 and 15.9 /
+  // 14.0.  Not where two tile rows share a panel in L2 (bf16 64x4096x11008 25.6 / 28.1).
+  const int64_t weights = (int64_t)a.N * row_bytes(dt, a.K);
+  q.nt = a.M <= 64 && q.g.tiles_m == 1 && weights > ((int64_t)(a.M <= 8 ? 30 : 64) << 20);
+  q.blocks = kwave_blocks(q.g.tiles_m, q.g.tiles_n);
+  const int grid = q.blocks * f.ranges;
+  if (f.ranges == 1) return sh.launch(q, grid, s);
+  std::unique_lock<std::mutex> order(splitk_order());
+  if (!q.g.workspace)
+    if (int rc = splitk_workspace_for((size_t)f.ranges * a.M * a.N * sizeof(float), s, &q.g.workspace)) return rc;
+  if (int e = sh.launch(q, grid, s)) return e;
+  return splitk_reduce(out, q.g, f.ranges, s);
+}
+
+void kwave_describe(int dt, const KwaveForm& f, int64_t M, int64_t N, LaunchForm* o) {
+  const KwaveShape& sh = shapes_of(dt)[f.shape];
+  o->grid = kwave_blocks((int)((M + sh.bm - 1) / sh.bm), (int)((N + f.per - 1) / f.per)) * f.ranges;
+  o->tile_m = sh.bm;
+  o->tile_n = sh.bn;
+  o->waves_m = sh.wm;
+  o->waves_n = sh.wn * sh.wk;
+  o->stages = sh.stages;
+  o->lds_bytes = sh.lds;
+  o->threads = sh.wm * sh.wn * sh.wk * 64;
+  o->func = sh.func;
+}
+
+bool kwave_tile_describe(const astergemm_config& c, int cus, LaunchForm* o) {
+  kwave_describe(c.dtype_ab, kwave_tile_form(c.dtype_ab, c.M, c.N, c.K, cus > 0 ? cus : 256), c.M, c.N, o);
+  return true;
+}
+bool kwave_split_describe(const astergemm_config& c, int cus, LaunchForm* o) {
+  if (!kwave_decode_describe(c, cus > 0 ? cus : 256, 1, o)) return kwave_tile_describe(c, cus, o);
+  return true;
+}
+bool kwave_decode_describe(const astergemm_config& c, int cus, int max_ranges, LaunchForm* o) {
+  const KwaveForm f = kwave_decode_form(c.dtype_ab, c.M, c.N, c.K, cus, max_ranges);
+  if (f) kwave_describe(c.dtype_ab, f, c.M, c.N, o);
+  return (bool)f;
+}
+bool kwave_small_decode_describe(const astergemm_config& c, int cus, LaunchForm* o) {
+  const KwaveForm f = kwave_small_decode_form(c.dtype_ab, c.M, c.N, c.K, cus);
+  if (f) kwave_describe(c.dtype_ab, f, c.M, c.N, o);
+  return (bool)f;
+}
+#endif  // AG_KWAVE_DT == 0
+
+}  // namespace astergemm

@@ -18,6 +18,7 @@
 #include <vector>
 
 #include "astergemm_internal.h"
+#include "gemm_kwave.h"
 
 namespace astergemm {
 namespace {
@@ -415,14 +416,29 @@ __global__ __launch_bounds__(512) void gemm_skinny_reg_kernel(const GemmArgs p) 
   }
 }
 
+// The kernels that split K over the waves (gemm_kwave.h) where they are ahead of the resident ones.  Both
+// are readied by either's first launch, so that a config that is captured later finds its kernel ready
+// whichever of the two an earlier one ran; inside a capture only the one that runs has to be.
+inline KwaveForm kwave_instead(int dt, const GemmArgs& a, int cus, int max_ranges) {
+  return a.named_tile ? KwaveForm{} : kwave_decode_form(dt, a.M, a.N, a.K, cus, max_ranges);
+}
+template <int (*SPLITS)(const astergemm_config&)>
+bool kwave_form_of(const astergemm_config& c, int cus, LaunchForm* o) {
+  return kwave_decode_describe(c, cus, SPLITS(c), o);
+}
+inline int one_range(const astergemm_config&) { return 1; }
+
 template <int DT, int OUT, int SPB>
 int launch_skinny_reg_t(const GemmArgs& a, hipStream_t s) {
   auto k = gemm_skinny_reg_kernel<DT, OUT, SPB>;
   constexpr int lds = 8 * 8192 + 2 * 4 * 8 * 64 * 16;
   static std::atomic<uint64_t> attr_devs{0};
-  if (int e = lds_attr_once(attr_devs, (const void*)k, lds)) return e;
   const int cus = device_cus();
+  const KwaveForm f = kwave_instead(DT, a, cus, 1);
+  if (const int e = lds_attr_once(attr_devs, (const void*)k, lds); e && !f) return e;
+  if (const int e = kwave_ready(DT); e && f) return e;
   if (cus <= 0) return (int)hipErrorNoDevice;
+  if (f) return kwave_launch(DT, OUT, a, f, s);
   const int nblocks = (int)((a.N + 15) / 16);
   const int g = nblocks < cus ? nblocks : cus;
   AG_LAUNCH_KERNEL(k, dim3(g), dim3(512), lds, s, a);
@@ -651,9 +667,12 @@ int launch_skinny_fp4_t(const GemmArgs& a, hipStream_t s) {
   auto k = gemm_skinny_fp4_kernel<OUT, SPB, SU>;
   constexpr int lds = 8 * 8192 + 2 * 4 * 8 * 64 * 16;
   static std::atomic<uint64_t> attr_devs{0};
-  if (int e = lds_attr_once(attr_devs, (const void*)k, lds)) return e;
   const int cus = device_cus();
+  const KwaveForm f = kwave_instead(ASTERGEMM_MXFP4, a, cus, 1);
+  if (const int e = lds_attr_once(attr_devs, (const void*)k, lds); e && !f) return e;
+  if (const int e = kwave_ready(ASTERGEMM_MXFP4); e && f) return e;
   if (cus <= 0) return (int)hipErrorNoDevice;
+  if (f) return kwave_launch(ASTERGEMM_MXFP4, OUT, a, f, s);
   const int nblocks = (int)((a.N + 15) / 16);
   const int g = nblocks < cus ? nblocks : cus;
   AG_LAUNCH_KERNEL(k, dim3(g), dim3(512), lds, s, a);
@@ -682,7 +701,8 @@ const char* check_skinny_fp4(const astergemm_config& c) {
   Variant {                                                                                \
     name, ASTERGEMM_KERNEL_SKINNY, ASTERGEMM_MXFP4, OUT, 16, 16, 512, 1, 8, 1, 3,           \
         8 * 8192 + 65536, (const void*)gemm_skinny_fp4_kernel<OUT, 2, 2>,                  \
-        launch_skinny_fp4<OUT>, check_skinny_fp4                                           \
+        launch_skinny_fp4<OUT>, check_skinny_fp4, ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0, \
+        kwave_form_of<one_range>                                                           \
   }
 
 // ---- rows cut into K ranges: partial sums, their workspace and the kernel that adds them ---
@@ -765,6 +785,23 @@ int splitk_workspace(size_t bytes, hipStream_t stream, float** out) {
   }
   *out = w.ptr;
   return 0;
+}
+
+// For a problem that is cut into K ranges by one kernel and not by the one that runs: the stream's buffer is
+// as large as if it had been, so that a later capture of another problem finds it.  Never inside a capture.
+void splitk_workspace_touch(size_t bytes, hipStream_t stream) {
+  int dev = 0;
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipGetDevice(&dev) != hipSuccess) return (void)hipGetLastError();
+  {
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    auto it = g_ws.find({dev, stream});
+    if (it != g_ws.end() && it->second.bytes >= bytes) return;
+  }
+  if ((stream && hipStreamIsCapturing(stream, &st) != hipSuccess) || st != hipStreamCaptureStatusNone)
+    return (void)hipGetLastError();
+  float* unused = nullptr;
+  if (splitk_workspace(bytes, stream, &unused) != 0) (void)hipGetLastError();
 }
 
 // Gives back the workspace of a stream that is about to be destroyed.  The caller has
@@ -1059,9 +1096,16 @@ int launch_skinny_fp4m_t(const GemmArgs& a0, int S, hipStream_t s) {
   auto k = gemm_skinny_fp4m_kernel<OUT, SPB, SU, MT, MH>;
   constexpr int lds = 8 * 8192 + 2 * 2 * MT * 8 * 64 * 16;
   static std::atomic<uint64_t> attr_devs{0};
-  if (int e = lds_attr_once(attr_devs, (const void*)k, lds)) return e;
   const int cus = device_cus();
+  const KwaveForm f = kwave_instead(ASTERGEMM_MXFP4, a0, cus, S);
+  if (const int e = lds_attr_once(attr_devs, (const void*)k, lds); e && !f) return e;
+  if (const int e = kwave_ready(ASTERGEMM_MXFP4); e && f) return e;
   if (cus <= 0) return (int)hipErrorNoDevice;
+  if (f) {
+    if (S > f.ranges && !a0.workspace && !launch_context().prepare_only)
+      splitk_workspace_touch((size_t)S * a0.M * a0.N * sizeof(float), s);
+    return kwave_launch(ASTERGEMM_MXFP4, OUT, a0, f, s);
+  }
   GemmArgs a = a0;
   const KRangeGrid kg = krange_grid(MH, a.N, S, cus);
   a.tiles_n = kg.rows;
@@ -1117,7 +1161,7 @@ int grid_skinny_fp4m(const astergemm_config& c, int cus) {
     name, ASTERGEMM_KERNEL_SKINNY, ASTERGEMM_MXFP4, OUT, 64, 16, 512, 1, 8, 1, 2,           \
         8 * 8192 + 65536, (const void*)gemm_skinny_fp4m_kernel<OUT, 2, 2, 2, 2>,           \
         launch_skinny_fp4m<OUT>, check_skinny_fp4m, ASTERGEMM_OPERAND_LDS,                 \
-        splits_skinny_fp4m, grid_skinny_fp4m                                               \
+        splits_skinny_fp4m, grid_skinny_fp4m, 0, kwave_form_of<splits_skinny_fp4m>         \
   }
 
 // ---- 16 < M <= 64: the same persistent kernel with two activation tiles per wave --------
@@ -1403,9 +1447,16 @@ int launch_skinny_regm_t(const GemmArgs& a0, int S, hipStream_t s) {
   auto k = gemm_skinny_regm_kernel<DT, OUT, SPB, MT, MH>;
   constexpr int lds = 8 * 8192 + 2 * (MT >= 4 ? 1 : 2) * MT * 8 * 64 * 16;
   static std::atomic<uint64_t> attr_devs{0};
-  if (int e = lds_attr_once(attr_devs, (const void*)k, lds)) return e;
   const int cus = device_cus();
+  const KwaveForm f = kwave_instead(DT, a0, cus, S);
+  if (const int e = lds_attr_once(attr_devs, (const void*)k, lds); e && !f) return e;
+  if (const int e = kwave_ready(DT); e && f) return e;
   if (cus <= 0) return (int)hipErrorNoDevice;
+  if (f) {
+    if (S > f.ranges && !a0.workspace && !launch_context().prepare_only)
+      splitk_workspace_touch((size_t)S * a0.M * a0.N * sizeof(float), s);
+    return kwave_launch(DT, OUT, a0, f, s);
+  }
   GemmArgs a = a0;
   const KRangeGrid kg = krange_grid(MH, a.N, S, cus);
   a.tiles_n = kg.rows;
@@ -1463,7 +1514,8 @@ int grid_skinny_regm(const astergemm_config& c, int cus) {
   Variant {                                                                                \
     name, ASTERGEMM_KERNEL_SKINNY, DT, OUT, 64, 16, 512, 1, 8, 1, 2, 8 * 8192 + 65536,      \
         (const void*)gemm_skinny_regm_kernel<DT, OUT, 8, 2, 2>, launch_skinny_regm<DT, OUT>, \
-        check_skinny_regm, ASTERGEMM_OPERAND_LDS, splits_skinny_regm, grid_skinny_regm     \
+        check_skinny_regm, ASTERGEMM_OPERAND_LDS, splits_skinny_regm, grid_skinny_regm, 0, \
+        kwave_form_of<splits_skinny_regm>                                                            \
   }
 
 template <int DT, int OUT>
@@ -1491,7 +1543,7 @@ const char* check_skinny_reg(const astergemm_config& c) {
   Variant {                                                                                \
     name, ASTERGEMM_KERNEL_SKINNY, DT, OUT, 16, 16, 512, 1, 8, 1, 3, 8 * 8192 + 65536,      \
         (const void*)gemm_skinny_reg_kernel<DT, OUT, 8>, launch_skinny_reg<DT, OUT>,       \
-        check_skinny_reg                                                                   \
+        check_skinny_reg, ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0, kwave_form_of<one_range> \
   }
 
 // ---- M <= 16, B pre-shuffled (operand path "direct B") ---------------------------------
@@ -1922,6 +1974,9 @@ const char* check_skinny_directb(const astergemm_config& c) {
 
 template <int DT, int OUT, int MT, int NB, int KW, int U>
 int launch_skinny(const GemmArgs& a, int grid, hipStream_t s) {
+  if (!a.named_tile)
+    if (const KwaveForm f = kwave_small_decode_form(DT, a.M, a.N, a.K, device_cus()))
+      return kwave_launch(DT, OUT, a, f, s);
   AG_LAUNCH_KERNEL((gemm_skinny_kernel<DT, OUT, MT, NB, KW, U>), dim3(grid), dim3(KW * 64), 0,
                      s, a);
   return (int)hipGetLastError();
@@ -1938,7 +1993,8 @@ const char* check_skinny(const astergemm_config& c) {
   Variant {                                                                               \
     name, ASTERGEMM_KERNEL_SKINNY, DT, OUT, 16 * MT, 16 * NB, 64 * U, 1, KW, 1, 0,        \
         KW * MT * NB * 1024, (const void*)gemm_skinny_kernel<DT, OUT, MT, NB, KW, U>,      \
-        launch_skinny<DT, OUT, MT, NB, KW, U>, check_skinny                               \
+        launch_skinny<DT, OUT, MT, NB, KW, U>, check_skinny, ASTERGEMM_OPERAND_LDS, nullptr, \
+        nullptr, 0, kwave_small_decode_describe                                           \
   }
 
 #define AG_SKINNY_SET(prefix, DT, OUTN, OUT)                                      \
@@ -1953,7 +2009,8 @@ const char* check_skinny(const astergemm_config& c) {
   Variant {                                                                               \
     name, ASTERGEMM_KERNEL_SKINNY, DT, OUT, 16 * MT, 16 * NB, 64 * U, 1, KW, 1, 1,        \
         KW * MT * NB * 1024, (const void*)gemm_skinny_kernel<DT, OUT, MT, NB, KW, U>,      \
-        launch_skinny<DT, OUT, MT, NB, KW, U>, check_skinny                               \
+        launch_skinny<DT, OUT, MT, NB, KW, U>, check_skinny, ASTERGEMM_OPERAND_LDS, nullptr, \
+        nullptr, 0, kwave_small_decode_describe                                           \
   }
 #define AG_SKINNY_WIDE_SET(prefix, DT, OUTN, OUT)                                 \
   AG_SKINNY_WIDE(prefix "_m32n64_" OUTN, DT, OUT, 2, 4, 4, 2),                    \

@@ -1,6 +1,7 @@
 // Variant table and launchers of the LDS-staged MFMA tile kernels
 // (device code: gemm_tile_kernel.hpp).
 #include "gemm_tile_kernel.hpp"
+#include "gemm_kwave.h"
 
 namespace astergemm {
 namespace {
@@ -11,13 +12,35 @@ constexpr int tile_lds_bytes(int dt, int bm, int bn, int stages) {
 }
 
 template <int DT, int OUT, int BM, int BN, int WM, int WN, int S>
-int launch_tile(const GemmArgs& a, int grid, hipStream_t s) {
-  constexpr int lds = tile_lds_bytes(DT, BM, BN, S);
-  auto k = gemm_tile_kernel<DT, OUT, BM, BN, WM, WN, S>;
+int tile_ready() {
   static std::atomic<uint64_t> attr_devs{0};
-  if (int e = lds_attr_once(attr_devs, (const void*)k, lds)) return e;
-  AG_LAUNCH_KERNEL(k, dim3(grid), dim3(WM * WN * 64), lds, s, a);
+  return lds_attr_once(attr_devs, (const void*)gemm_tile_kernel<DT, OUT, BM, BN, WM, WN, S>,
+                       tile_lds_bytes(DT, BM, BN, S));
+}
+
+template <int DT, int OUT, int BM, int BN, int WM, int WN, int S>
+int launch_tile(const GemmArgs& a, int grid, hipStream_t s) {
+  if (int e = tile_ready<DT, OUT, BM, BN, WM, WN, S>()) return e;
+  // the kernels that stand in for this one on small grids: a config captured later finds either ready
+  if constexpr (BM == 64) (void)kwave_ready(DT);
+  AG_LAUNCH_KERNEL((gemm_tile_kernel<DT, OUT, BM, BN, WM, WN, S>), dim3(grid), dim3(WM * WN * 64),
+                   tile_lds_bytes(DT, BM, BN, S), s, a);
   return (int)hipGetLastError();
+}
+
+// K split over the waves (gemm_kwave.h): SPLIT = false for small products, true for decoding on byte
+// rows that the kernels with resident activations do not take.
+template <int DT, int OUT, bool SPLIT>
+int launch_kwave_tile(const GemmArgs& a, int grid, hipStream_t s) {
+  (void)grid;
+  (void)tile_ready<DT, OUT, 64, 64, 2, 2, 4>();
+  if (int e = kwave_ready(DT)) return e;
+  const int cus = device_cus();
+  if (cus <= 0) return (int)hipErrorNoDevice;
+  KwaveForm f;
+  if (SPLIT) f = kwave_decode_form(DT, a.M, a.N, a.K, cus, 1);
+  if (!f) f = kwave_tile_form(DT, a.M, a.N, a.K, cus);
+  return kwave_launch(DT, OUT, a, f, s);
 }
 
 const char* check_tile(const astergemm_config& c) {
@@ -57,6 +80,17 @@ const char* check_tile(const astergemm_config& c) {
       AG_TILE(prefix "_128x128_w2x2", DT, 128, 128, 2, 2, 2),                    \
       AG_TILE(prefix "_128x64_w2x2", DT, 128, 64, 2, 2, 2),                      \
       AG_TILE(prefix "_64x64_w2x2", DT, 64, 64, 2, 2, 4)
+#define AG_KWAVE1(name, DT, OUT, SPLIT, RANK)                                    \
+  Variant {                                                                      \
+    name, ASTERGEMM_KERNEL_TILE, DT, OUT, 64, 64, kRowBytes, 2, 4, 3, RANK,      \
+        0, nullptr, launch_kwave_tile<DT, OUT, SPLIT>, check_tile,               \
+        ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0,                              \
+        SPLIT ? kwave_split_describe : kwave_tile_describe                       \
+  }
+#define AG_KWAVE(name, DT, SPLIT, RANK)                                          \
+  AG_KWAVE1(name "_bf16", DT, ASTERGEMM_BF16, SPLIT, RANK),                      \
+      AG_KWAVE1(name "_f32", DT, ASTERGEMM_F32, SPLIT, RANK),                    \
+      AG_KWAVE1(name "_f16", DT, ASTERGEMM_F16, SPLIT, RANK)
 #define AG_TILE_RING2(prefix, DT)                                                \
   AG_TILE(prefix "_64x64_w2x2_ring2", DT, 64, 64, 2, 2, 2)
 
@@ -69,6 +103,11 @@ const Variant kTileVariants[] = {
     AG_TILE_RING2("tile_f16", ASTERGEMM_F16),
     AG_TILE_RING2("tile_fp8", ASTERGEMM_FP8_E4M3),
     AG_TILE_RING2("tile_mxfp4", ASTERGEMM_MXFP4),
+    AG_KWAVE("tile_bf16_kwave", ASTERGEMM_BF16, false, 8),
+    AG_KWAVE("tile_f16_kwave", ASTERGEMM_F16, false, 8),
+    AG_KWAVE("tile_fp8_kwave", ASTERGEMM_FP8_E4M3, false, 8),
+    AG_KWAVE("splitk_fp8_kwave", ASTERGEMM_FP8_E4M3, true, 7),
+    AG_KWAVE("tile_mxfp4_kwave", ASTERGEMM_MXFP4, true, 7),
 };
 
 }  // namespace

@@ -1,0 +1,104 @@
+"""The kernels that split K over the waves of a workgroup, at the edges of their tiles, panels and K
+loops: against the CPU oracle, with the bars of test_gpu_parity."""
+import numpy as np
+import pytest
+
+from aster_amd import _capi, gemm as AG
+from oracle import formats as F, gemm as G
+from test_gpu_parity import _DT, REL_L2_BAR, check, operands, run_gemm
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M,N,K,dtype_ab,tile", [
+    # decoding: one panel per CU, panels of 8 ... 128 rows, short last panels, two tile rows, K ranges
+    (1, 4096, 4096, "bf16", (16, 16)), (16, 520, 14336, "f16", (16, 16)), (7, 4104, 11008, "bf16", (16, 32)),
+    (16, 11009, 4096, "bf16", (16, 48)), (15, 14336, 2048, "f16", (16, 64)), (17, 4096, 2304, "bf16", (32, 16)),
+    (31, 7000, 4096, "f16", (32, 32)), (24, 14337, 2048, "bf16", (32, 64)), (32, 28672, 2560, "bf16", (32, 128)),
+    (48, 1000, 8192, "f16", (16, 16)), (33, 4096, 4096, "bf16", (32, 32)), (64, 8191, 4096, "bf16", (64, 32)),
+    (50, 11008, 4096, "f16", (64, 48)), (64, 14336, 4352, "bf16", (64, 64)), (63, 20000, 2048, "bf16", (64, 128)),
+    (64, 4096, 14336, "bf16", (64, 64)), (29, 4100, 11008, "f16", (32, 64)), (33, 2700, 16384, "bf16", (64, 64)),
+    (16, 14336, 4096, "fp8_e4m3", (16, 64)), (3, 1000, 12288, "fp8_e4m3", (16, 16)),
+    (50, 4100, 4608, "fp8_e4m3", (64, 32)), (64, 8192, 28672, "fp8_e4m3", (64, 64)),
+    (16, 4096, 14336, "mxfp4", (16, 16)), (9, 7000, 4608, "mxfp4", (16, 32)), (33, 8200, 4096, "mxfp4", (64, 48)),
+    (64, 4100, 8192, "mxfp4", (64, 32)),
+    # rows that the kernels with resident activations do not take
+    (9, 4096, 11008, "fp8_e4m3", (16, 16)), (1, 1024, 4112, "fp8_e4m3", (16, 16)),
+    (64, 2056, 4208, "fp8_e4m3", (32, 32)), (5, 1030, 4352, "mxfp4", (16, 16)), (64, 4096, 11008, "mxfp4", (32, 32)),
+    (40, 300, 1984, "bf16", (16, 16)), (64, 1000, 992, "f16", (16, 16)), (1, 17, 32, "bf16", (16, 16)),
+    # small products: the smallest tile in one round, K tails of 1 and 7 granules, fewer steps than stages
+    (100, 100, 520, "bf16", (16, 16)), (300, 300, 2048, "f16", (32, 32)), (65, 130, 1080, "bf16", (16, 16)),
+    (600, 599, 1544, "bf16", (32, 64)), (777, 1001, 1032, "bf16", (64, 64)), (1200, 33, 2040, "f16", (16, 16)),
+    (100, 4095, 4096, "fp8_e4m3", (64, 64)), (70, 1000, 2064, "fp8_e4m3", (32, 32)),
+])
+@pytest.mark.parametrize("dtype_c", ["f32", "bf16"])
+def test_k_over_waves(gpu, M, N, K, dtype_ab, dtype_c, tile):
+    a, b, extra = operands(M, N, K, dtype_ab, seed=M + K, b_std=0.05)
+    if dtype_ab == "mxfp4":      # spread the block scales: a wrong byte must not go unnoticed
+        rng = np.random.default_rng(M)
+        for key in extra:
+            extra[key] = (extra[key].astype(np.int32) + rng.integers(-3, 4, extra[key].shape)).astype(np.uint8)
+    bias = np.random.default_rng(N).standard_normal(N).astype(np.float32)
+    info = AG.GemmPlan.create(M, N, K, dtype_ab, dtype_c, has_bias=True).info
+    assert (info.wg_tile_m, info.wg_tile_n) == tile, (info.name, info.wg_tile_m, info.wg_tile_n)
+    out, _ = run_gemm(a, b, M, N, K, dtype_ab, dtype_c, bias=bias, ldc=N + 3, **extra)
+    want = G.gemm(a, b, _DT[dtype_ab], _DT[dtype_c], bias=bias, **extra)
+    f32_bar = 1e-4 if dtype_ab == "fp8_e4m3" else 1e-5
+    if dtype_c == "f32" or M * N >= 4096:
+        check(out, want, dtype_c, N, bar=f32_bar if dtype_c == "f32" else REL_L2_BAR)
+    else:                        # few outputs: two units of the bf16 output each, and the sums' own bar
+        got, ref = G.output_to_f32(out[:, :N], _DT[dtype_c]), G.output_to_f32(want, _DT[dtype_c])
+        assert np.all(np.abs(got - ref) <= 2.0 ** -6 * np.abs(ref) + f32_bar * np.abs(ref).max())
+    pad = out[:, N:]
+    assert np.isnan(pad).all() if dtype_c == "f32" else (pad == 0x7FC1).all()
+    again, _ = run_gemm(a, b, M, N, K, dtype_ab, dtype_c, bias=bias, ldc=N + 3, **extra)
+    assert np.array_equal(out.view(np.uint8), again.view(np.uint8))
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 4096, 14336), (50, 1000, 2304), (100, 200, 1032)])
+def test_non_finite_rows_stay_in_their_row(gpu, M, N, K):
+    """The rows past M and N repeat the last one; a NaN there, and an infinity, reach their own row only."""
+    a, b, _ = operands(M, N, K, "bf16", seed=5, b_std=0.05)
+    a = np.array(a, copy=True)
+    a[M - 1, K - 1], a[0, 0] = 0x7FC0, 0x7F80       # NaN, +inf
+    out, _ = run_gemm(a, b, M, N, K, "bf16", "f32")
+    assert np.isnan(out[M - 1]).all() and not np.isfinite(out[0]).any()
+    assert np.isfinite(out[1:M - 1]).all()
+
+
+@pytest.mark.parametrize("first,then", [((16, 14336, 4096), (48, 4096, 4096)), ((16, 60000, 4096), (8, 4096, 4096)),
+                                        ((8, 4096, 4096), (16, 60000, 4096)), ((1000, 1000, 2048), (100, 100, 2048))])
+def test_a_captured_config_finds_its_kernel_ready(gpu, first, then):
+    """One eager call of a decode (small) problem of the same types readies the kernels of all of them, those
+    with resident activations included; several replays with eager work between them have the eager bits."""
+    import torch
+    torch.manual_seed(3)
+    stream = torch.cuda.Stream()
+    plans = [AG.GemmPlan.create(*s, "f16", "f16") for s in (first, then)]
+    sets = [[(torch.randn(r, s[2], device="cuda") * 0.1).half() for r in s[:2]]
+            + [torch.zeros(s[0], s[1], device="cuda", dtype=torch.float16)] for s in (first, then)]
+    torch.cuda.synchronize()
+    call = lambda i, c=None: plans[i].run(sets[i][0].data_ptr(), sets[i][1].data_ptr(),
+                                          (sets[i][2] if c is None else c).data_ptr(), stream=stream.cuda_stream)
+    print(first, then, flush=True)
+    call(0)
+    stream.synchronize()
+    graph, got = torch.cuda.CUDAGraph(), torch.zeros_like(sets[1][2])
+    with torch.cuda.graph(graph, stream=stream):
+        call(1, got)
+    call(1)
+    torch.cuda.synchronize()
+    for _ in range(3):
+        got.zero_()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, sets[1][2])
+        call(0)
+
+
+def test_a_named_tile_keeps_the_kernels_it_had():
+    for (M, N, K), wg in (((300, 300, 2048), (64, 64)), ((16, 4096, 4096), (16, 16))):
+        info = AG.GemmPlan.create(M, N, K, "bf16", "bf16", wg_tile=wg).info
+        assert (info.wg_tile_m, info.wg_tile_n) == wg and b"kwave" not in info.name
