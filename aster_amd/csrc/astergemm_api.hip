@@ -166,6 +166,12 @@ int chip_cus() {
   return cus > 0 ? cus : 256;  // no device to ask: describe the MI355X
 }
 
+// A config that names a tile size or a wave count (1) or a kernel (2) gets that kernel, not one that stands in
+// for it.
+int own_kernel(const astergemm_config& c) {
+  return c.wg_tile_m || c.wg_tile_n || c.waves_m || c.waves_n ? 1 : c.variant ? 2 : 0;
+}
+
 int64_t tile_grid(const astergemm_config& c, int64_t bm, int64_t bn) {
   return ((c.M + bm - 1) / bm) * ((c.N + bn - 1) / bn);
 }
@@ -253,19 +259,21 @@ int tile64_stages_of(const astergemm_config& c) {
   return tile_grid(c, 64, 64) > (short_rows ? 1 : 2) * (int64_t)chip_cus() ? 2 : 4;
 }
 
-// K split over the waves of a workgroup instead of the general 64 x 64 tile kernel (rank 8): its tiles
-// would not fill the chip, and the row is long enough for its K loop to be what the time goes on.
+// K split over the waves of a workgroup instead of the general 64 x 64 tile kernel (rank 8): 32 x 64 tiles or
+// smaller fit one round, and the row is long enough for the K loop to be what the time goes on (fp8 600x600x1040
+// with the quantiser before it, 32 x 64 tiles, 13.1 / 14.3).  Past that,
+// with 64 x 64 tiles of its own, it is behind on short rows (general / this: bf16 777x1001x1032 8.0 / 8.8,
+// 1200x640x1024 6.8 / 7.8, fp8 1200x640x2064 8.4 / 9.7, ahead: bf16 777x1001x4096 17.5 / 16.3).
 bool kwave_tile_pays(const astergemm_config& c) {
-  return c.dtype_ab != ASTERGEMM_MXFP4 && c.operand_path == ASTERGEMM_OPERAND_LDS && !c.wg_tile_m &&
-         !c.wg_tile_n && !c.waves_m && !c.waves_n && row_bytes(c.dtype_ab, c.K) > 8 * 128 &&
-         tile_grid(c, 64, 64) < chip_cus();
+  return c.dtype_ab != ASTERGEMM_MXFP4 && c.operand_path == ASTERGEMM_OPERAND_LDS && !own_kernel(c) &&
+         row_bytes(c.dtype_ab, c.K) > (tile_grid(c, 32, 32) <= chip_cus() ? 8 * 128 : 2047) &&
+         tile_grid(c, 32, 64) <= chip_cus();
 }
 
 // The same for decoding on rows of bytes that the kernels with resident activations do not take (rank 7).
 bool kwave_split_pays(const astergemm_config& c) {
   return (c.dtype_ab == ASTERGEMM_FP8_E4M3 || c.dtype_ab == ASTERGEMM_MXFP4) &&
-         c.operand_path == ASTERGEMM_OPERAND_LDS && !c.wg_tile_m && !c.wg_tile_n && !c.waves_m &&
-         !c.waves_n && c.M <= 64 && c.K >= 4096 && c.N >= 1024 &&
+         c.operand_path == ASTERGEMM_OPERAND_LDS && !own_kernel(c) && c.M <= 64 && c.K >= 4096 && c.N >= 1024 &&
          kwave_decode_form(c.dtype_ab, c.M, c.N, c.K, chip_cus(), 1);
 }
 
@@ -573,7 +581,10 @@ void describe(const Variant& v, int index, const astergemm_config& c, astergemm_
   snprintf(o->name, sizeof(o->name), "%s", v.name);
   const void* func = v.func;
   LaunchForm f;
-  if (v.form && !c.wg_tile_m && !c.wg_tile_n && !c.waves_m && !c.waves_n && v.form(c, device_cus(), &f)) {
+  // (a split kernel by name is what AUTO runs under that name, scratch or not)
+  const bool split_tile = v.family == ASTERGEMM_KERNEL_TILE && v.splits;
+  const int own = own_kernel(c);
+  if (v.form && (v.rank >= 7 || !own || (own == 2 && split_tile)) && v.form(c, device_cus(), &f)) {
     o->grid_x = f.grid;
     o->block_x = f.threads;
     o->lds_bytes = f.lds_bytes;
@@ -657,7 +668,7 @@ int build_args(const Variant& v, const astergemm_config& c, const astergemm_oper
   // MXFP4 +1.5 %, bf16 -0.1 %, same process
   a->group_m = (a->tiles_m % 8 == 0 && a->tiles_n % 32 == 0) ? -1 : 8;
   a->split_k = 1;
-  a->named_tile = c.wg_tile_m || c.wg_tile_n || c.waves_m || c.waves_n;
+  a->own_kernel = own_kernel(c);
   // rows cut into K ranges: the caller's workspace when one is given, else the library's own
   if (ops.dWorkspace) {
     const size_t need = workspace_need(v, c);

@@ -28,7 +28,7 @@ struct GemmArgs {
   int32_t tiles_m, tiles_n;
   int32_t group_m;       // tile rows per rasterisation group; < 0: band order (see map_tile)
   int32_t split_k;       // skinny path: K slices per output row block
-  int32_t named_tile;    // the config names a tile or a wave count: launchers keep to their own kernels
+  int32_t own_kernel;    // the config names a tile or a wave count (1) or a kernel (2): the launcher runs its own
   float* workspace;      // fp32 partials [split_k][M][N] when a row is cut into K ranges; set by
                          // the caller of a launcher = use this buffer, null = the library's own
 };
@@ -165,6 +165,9 @@ inline int streamr_split_of(int64_t tiles, int64_t ksteps) {
 // workspace of a (device, stream), and the kernel that adds `splits` planes [M][N] of
 // a.workspace in index order, applies a's scales and bias and stores a.C in `out_dtype`.
 int splitk_workspace_for(size_t bytes, hipStream_t stream, float** out);
+// A launcher whose K ranges another kernel stands in for: the stream's buffer is made as large as the ranges
+// would have, so that a later capture finds it (never inside a capture; a failure is nobody's).
+void splitk_workspace_touch(size_t bytes, hipStream_t stream);
 // Held by a launcher from the lookup of the workspace to the launch of the kernel that adds it up, whoever
 // owns that memory (the library's buffer of the stream, the built-in scratch, the caller): two host threads
 // on one stream that share it would otherwise enqueue product, product, sum, sum.

@@ -19,16 +19,21 @@ KwaveForm kwave_decode_form(int dt, int64_t M, int64_t N, int64_t K, int cus, in
 // limit (the launcher it is part of sets no function attribute).
 KwaveForm kwave_small_decode_form(int dt, int64_t M, int64_t N, int64_t K, int cus);
 
-// Any M and N: the smallest tile that leaves at most one workgroup per CU, else 64 x 64.
+// 64 < M <= 512 against at most about a round of panels, as part of the launchers of 128 x 128 tiles.
+KwaveForm kwave_prompt_form(int dt, int64_t M, int64_t N, int64_t K, int cus);
+// Any M and N: the smallest tile that leaves at most one workgroup per CU, else (and without a device) 64 x 64.
 KwaveForm kwave_tile_form(int dt, int64_t M, int64_t N, int64_t K, int cus);
+// The decode form where there is one, else the prompt form, else the tile form.
+KwaveForm kwave_any_form(int dt, int64_t M, int64_t N, int64_t K, int cus);
 
 int kwave_launch(int dt, int out, const GemmArgs& a, const KwaveForm& f, hipStream_t s);
 // The one-time step of every shape of `dt` on the current device (see lds_attr_once).
 int kwave_ready(int dt);
-void kwave_describe(int dt, const KwaveForm& f, int64_t M, int64_t N, LaunchForm* o);
+void kwave_describe(int dt, const KwaveForm& f, int64_t M, int64_t N, int cus, LaunchForm* o);
 bool kwave_decode_describe(const astergemm_config& c, int cus, int max_ranges, LaunchForm* o);
+bool kwave_prompt_describe(const astergemm_config& c, int cus, LaunchForm* o);
 bool kwave_tile_describe(const astergemm_config& c, int cus, LaunchForm* o);
-bool kwave_split_describe(const astergemm_config& c, int cus, LaunchForm* o);  // decode form, else tile form
+bool kwave_any_describe(const astergemm_config& c, int cus, LaunchForm* o);
 bool kwave_small_decode_describe(const astergemm_config& c, int cus, LaunchForm* o);
 
 }  // namespace astergemm

@@ -21,14 +21,17 @@ namespace astergemm {
   X(9, 64, 32, 2, 1, 4, 3, 3)    \
   X(10, 64, 48, 2, 1, 2, 5, 5)   \
   X(11, 64, 64, 2, 2, 2, 3, 3)   \
-  X(12, 64, 128, 2, 2, 2, 3, 3)
+  X(12, 64, 128, 2, 2, 2, 3, 3)  \
+  X(13, 96, 64, 2, 2, 2, 4, 3)   \
+  X(14, 128, 64, 2, 2, 2, 3, 3)  \
+  X(15, 128, 128, 2, 4, 1, 5, 4)
 
 struct KwaveShape {
   int bm, bn, wm, wn, wk, stages, lds;
   const void* func;
   int (*launch)(const KwaveArgs& q, int grid, hipStream_t s);
 };
-constexpr int kKwaveShapes = 13;
+constexpr int kKwaveShapes = 16;
 const KwaveShape* kwave_shapes_f16();
 const KwaveShape* kwave_shapes_bf16();
 const KwaveShape* kwave_shapes_fp8();
@@ -79,13 +82,21 @@ const KwaveShape* shapes_of(int dt) {
   }
 }
 
-// Weight rows of a workgroup when `tiles_m` tile rows share the chip: one round, groups of 8 rows.
+// Weight rows of a workgroup when `tiles_m` tile rows share the chip: one round, groups of 8 rows.  The tile
+// rows of a panel are on one XCD, so a round is what fits every XCD's eighth of the CUs (a few panels more
+// put a second round on some XCDs: bf16 400x4096x4096 26.7 -> 41.4 us).
 int rows_per(int64_t N, int tiles_m, int cus) {
-  const int slots = cus / tiles_m > 0 ? cus / tiles_m : 1;
-  return (int)(((N + slots - 1) / slots + 7) / 8 * 8);
+  const int per_xcd = cus / 8 / tiles_m, panels = per_xcd > 0 ? per_xcd * 8 : 1;
+  return (int)(((N + panels - 1) / panels + 7) / 8 * 8);
 }
 
-int kwave_blocks(int tiles_m, int tiles_n) { return tiles_m * ((tiles_n + 7) & ~7); }
+// Workgroups of a K range: by panels on one XCD each, in whole groups of 8 panels, while that is one round;
+// else tile after tile.
+int kwave_blocks(int tiles_m, int tiles_n, int cus, int* by_panel) {
+  const int64_t grouped = (int64_t)tiles_m * ((tiles_n + 7) & ~7);
+  *by_panel = grouped <= cus;
+  return *by_panel ? (int)grouped : tiles_m * tiles_n;
+}
 
 }  // namespace
 
@@ -93,8 +104,10 @@ int kwave_blocks(int tiles_m, int tiles_n) { return tiles_m * ((tiles_n + 7) & ~
 // workgroup's panel is N / CUs rows in groups of 8, not the tile's), within two limits:
 //   * panels of more than 64 rows with up to 16 activation rows stay with the resident kernels, whose
 //     activations are then read once for many weight rows (bf16 16x28672x4096 37.3 us against 40.2 for
-//     16 x 128 tiles, fp8 21.6 / 23.4, MXFP4 11.5 / 13.2); MXFP4 on rows of 2, 4 or 8 KiB already from
-//     32 on (16x14336x4096 7.3 / 7.5).
+//     16 x 128 tiles, fp8 21.6 / 23.4, MXFP4 11.5 / 13.2); MXFP4 on rows that the resident kernel takes
+//     without K ranges already from 32 on (16x14336x4096 7.3 / 7.5), with more than 16 activation rows from
+//     40 on: ahead while the weights are found in the last-level cache, behind where they are not
+//     (64x14336x4096 11.6 / 9.4 and 11.9 / 14.1, 32x28672x4096 14.3 / 12.3 and 14.6 / 17.6).
 //   * a workgroup's own rows over all of K, (bm + per) * rb bytes, come from L2 at about 60 GB/s.  Where K
 //     ranges on 64-row panels take half a megabyte off that (two ranges, whose planes weigh more: three
 //     quarters), they pay for the planes and the kernel that adds them: bf16 64x4096x14336 37.2 -> 28.4
@@ -110,7 +123,7 @@ int kwave_blocks(int tiles_m, int tiles_n) { return tiles_m * ((tiles_n + 7) & ~
 //   fp8 16  6.1 / 5.4       12.3 / 11.1  resident     15.0 / 11.3  28.0 / 10.0  19.4 / 12.1  6.9 / 5.6
 //   fp8 64  9.4 / 6.7       17.6 / 12.3  26.9 / 22.2  21.8 / 14.3  28.7 / 12.5  18.2 / 13.2  9.7 / 6.1
 //   fp4 16  4.8 / 4.6       resident     resident     10.9 / 7.4   14.6 / 7.4   10.2 / 7.9   5.9 / 4.7
-//   fp4 64  6.5 / 5.4       11.6 / 9.4   19.0 / 14.5  16.9 / 11.0  17.0 / 9.1   14.5 / 10.9  8.6 / 4.8
+//   fp4 64  6.5 / 5.4       resident     resident     16.9 / 11.0  17.0 / 9.1   14.5 / 10.9  8.6 / 4.8
 // (fp8 and MXFP4 4096x11008, no whole 512 bytes: against the tile kernels.)
 KwaveForm kwave_decode_form(int dt, int64_t M, int64_t N, int64_t K, int cus, int max_ranges) {
   KwaveForm f;
@@ -139,7 +152,7 @@ KwaveForm kwave_decode_form(int dt, int64_t M, int64_t N, int64_t K, int cus, in
     if (per > (resident ? 32 : 64)) return f;
     return per <= 32 ? take(1, 16, per) : per <= 48 ? take(2, 16, per) : take(3, 16, per);
   }
-  if (per > 128) return f;
+  if (per > 128 || (dt == ASTERGEMM_MXFP4 && (K == 4096 || K == 8192) && per > 40)) return f;
   if (M <= 32)
     return per <= 16 ? take(5, 32, per) : per <= 32 ? take(6, 32, per) : per <= 64 ? take(7, 32, per)
                                                                                   : take(8, 32, per);
@@ -159,25 +172,81 @@ KwaveForm kwave_small_decode_form(int dt, int64_t M, int64_t N, int64_t K, int c
   return f;
 }
 
+namespace {
+
+// The tile and panel that bring the fewest operand rows into a CU in one round, among those of a tile's
+// exact rows or less; shape -1 where none covers N.
+KwaveForm fewest_rows(int64_t M, int64_t N, int cus, int* rows) {
+  static const struct { int bm, bn, shape; } kTiles[] = {{32, 16, 5}, {32, 32, 6}, {32, 64, 7}, {64, 32, 9},
+                                                         {64, 48, 10}, {64, 64, 11}, {64, 128, 12},
+                                                         {96, 64, 13}, {128, 64, 14}, {128, 128, 15}};
+  KwaveForm f;
+  int bm = 0, best = INT32_MAX;
+  for (const auto& t : kTiles) {
+    const int64_t tm = (M + t.bm - 1) / t.bm;
+    if (tm > cus / 8 || t.bm == bm) continue;  // (the first panel that fits a tile height is its best)
+    const int per = rows_per(N, (int)tm, cus);
+    if (per > t.bn) continue;
+    bm = t.bm;
+    // one tile row reads every weight once: worth a sixteenth (bf16 128x14336x4096, 184 rows on 128 x 64 tiles
+    // 32.5 us, 176 on 64 x 128 33.9)
+    // and a panel of less than three quarters of the tile pays for those
+    const int loaded = t.bm + (per * 4 > t.bn * 3 ? per : t.bn * 3 / 4);
+    const int cost = loaded - (tm == 1 ? loaded / 16 : 0);
+    if (cost < best) best = cost, *rows = t.bm + per, f.shape = t.shape, f.per = per;
+  }
+  return f;
+}
+
+}  // namespace
+
+// Prompts of a few hundred tokens, 128 x 128 tiles (split K, or one K loop) / this, us:
+//   M          bf16 4096x4096  14336x4096   11008x4096   8192x8192    28672x4096
+//   80         14.8 / 11.3     41.7 / 28.0  33.9 / 22.6  42.5 / 36.9  57.8 / 49.4
+//   128        16.4 / 11.8     44.0 / 32.5  37.2 / 27.0  45.4 / 41.6  59.2 / 53.5
+//   256        19.4 / 16.8     46.6 / 45.2  42.0 / 40.6  53.3 / 54.1  80.1 / 87.2
+//   512        27.3 / 24.4     72.8 / 81.1  52.0 / 79.0  77.2 / 82.4
+//   fp8 128    11.0 / 7.9      -            -            21.7 / 19.5  34.2 / 29.8
+//   MXFP4 128  13.8 / 6.8      14.6 / 12.5  14.4 / 11.7  17.1 / 13.5  15.6 / 17.7
+//   MXFP4 256  14.1 / 8.3      15.1 / 17.3  14.6 / 16.7  23.2 / 19.8  21.3 / 32.3
+// The lines: operand rows per CU times their bytes, against tiles that read 256 rows or split K further
+// (bf16 128x4096x14336, 2.8 MB here: 37.4 / 50.0; fp8 200x4096x14336 24.8 / 30.2; MXFP4 333x8192x8192 24.3 / 26.8).
+KwaveForm kwave_prompt_form(int dt, int64_t M, int64_t N, int64_t K, int cus) {
+  const int64_t rb = row_bytes(dt, K);
+  if (cus <= 0 || M <= 64 || M > 512 || N < 1 || N > INT32_MAX / 2 || rb % 16 != 0) return KwaveForm{};
+  int rows = 0;
+  const KwaveForm f = fewest_rows(M, N, cus, &rows);
+  if (!f) return f;
+  const int64_t own = rows * rb;
+  bool pays;
+  if (dt == ASTERGEMM_MXFP4) pays = rows <= 192 && own <= 800000;
+  else if (dt == ASTERGEMM_FP8_E4M3) pays = M <= 128 ? own <= 1400000 : rows <= 128 && own <= 900000;
+  else pays = M <= 128 ? own <= 2200000 : rows <= 192 && own <= 1600000;
+  return pays ? f : KwaveForm{};
+}
+
 // Small products, general 64 x 64 tile kernel / this, us: bf16 300x300x2048 10.0 / 5.4 (32 x 32),
-// 500x500x1024 6.7 / 4.0, 207x28x1440 8.0 / 3.9 (16 x 16), 600x600x2048 10.2 / 7.3 (32 x 64), 1000x1000x512
-// 5.5 / 4.6 (64 x 64), 777x1001x1032 8.1 / 7.9 (bound by rows that start off the 128-byte lines:
-// 777x1001x1024 7.0 / 6.4); fp8 100x4096x4096 11.0 / 7.5.  From one 64 x 64 tile per CU on the general kernel
-// is level or ahead (1200x1200x1000 11.6 / 13.3).
+// 500x500x1024 6.7 / 4.6, 207x28x1440 8.0 / 3.9 (16 x 16), 600x600x2056 12.2 / 10.1 (32 x 64), 600x600x4104
+// 21.0 / 17.2, 2000x200x1032 7.5 / 7.1; fp8 300x300x4096 11.1 / 6.4, 600x600x4096 11.3 / 9.2.  The 64 x 64 form is
+// for configs that name the kernel.
 KwaveForm kwave_tile_form(int dt, int64_t M, int64_t N, int64_t K, int cus) {
   (void)dt, (void)K;
   static const struct { int shape, bm, bn; } kOrder[] = {{0, 16, 16}, {6, 32, 32}, {7, 32, 64}};
   KwaveForm f;
   f.shape = 11;
   f.per = 64;
-  for (const auto& t : kOrder) {
-    const int64_t g = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
-    if (g < cus || (g == cus && t.bn <= 32)) {
+  for (const auto& t : kOrder)
+    if (((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn) <= cus) {
       f.shape = t.shape, f.per = t.bn;
       break;
     }
-  }
   return f;
+}
+
+KwaveForm kwave_any_form(int dt, int64_t M, int64_t N, int64_t K, int cus) {
+  KwaveForm f = kwave_decode_form(dt, M, N, K, cus, 1);
+  if (!f) f = kwave_prompt_form(dt, M, N, K, cus);
+  return f ? f : kwave_tile_form(dt, M, N, K, cus);
 }
 
 int kwave_ready(int dt) {
@@ -206,13 +275,15 @@ int kwave_launch(int dt, int out, const GemmArgs& a, const KwaveForm& f, hipStre
   q.range_steps = (a.ksteps + f.ranges - 1) / f.ranges;
   q.out = out;
   // Past the last-level cache where that is no use: a matrix of more than 64 MiB is not found there again
-  // after a few others; up to 8 activation rows the loop is the weight stream and little else, from 30 MiB
-  // on.  Through the cache / past it, us, three sets in turn and cold: bf16 8x4096x11008 16.0 / 15.7 and 18.1 /
-  // 16.4, fp8 8x14336x4096 10.3 / 10.2 and 11.9 / 10.8; the other side: fp8 64x14336x4096 12.1 / 13.7 and 15.9 /
-  // 14.0.  Not where two tile rows share a panel in L2 (bf16 64x4096x11008 25.6 / 28.1).
-  const int64_t weights = (int64_t)a.N * row_bytes(dt, a.K);
-  q.nt = a.M <= 64 && q.g.tiles_m == 1 && weights > ((int64_t)(a.M <= 8 ? 30 : 64) << 20);
-  q.blocks = kwave_blocks(q.g.tiles_m, q.g.tiles_n);
+  // after a few others; with few activation rows for the panel's the loop is the weight stream and little
+  // else, from 30 MiB on.  Through the cache / past it, us, three sets in turn and sets that no kernel has
+  // read for 700 MB: bf16 8x4096x11008 16.8 / 16.6 and 19.3 / 17.4, 64x14336x4096 25.9 / 23.3 and 26.5 / 24.2,
+  // fp8 16x14336x4096 11.1 / 10.8 and 13.1 / 11.4; the other side: fp8 16x4096x14336 11.3 / 12.8 and 14.5 / 13.3,
+  // 64x14336x4096 12.3 / 14.1 and 16.7 / 14.7, 16x1024x8192 5.7 / 6.5 and 5.8 / 6.9.  Not where two tile rows
+  // share a panel in L2 (bf16 64x4096x4096 8.9 / 11.8 and 12.5 / 12.2).
+  const int64_t mib = (int64_t)a.N * row_bytes(dt, a.K) >> 20;
+  q.nt = a.M <= 64 && q.g.tiles_m == 1 && (mib > 64 || (mib >= 30 && (a.M <= 8 || (a.M <= 16 && f.per >= 48))));
+  q.blocks = kwave_blocks(q.g.tiles_m, q.g.tiles_n, device_cus(), &q.by_panel);
   const int grid = q.blocks * f.ranges;
   if (f.ranges == 1) return sh.launch(q, grid, s);
   std::unique_lock<std::mutex> order(splitk_order());
@@ -222,9 +293,10 @@ int kwave_launch(int dt, int out, const GemmArgs& a, const KwaveForm& f, hipStre
   return splitk_reduce(out, q.g, f.ranges, s);
 }
 
-void kwave_describe(int dt, const KwaveForm& f, int64_t M, int64_t N, LaunchForm* o) {
+void kwave_describe(int dt, const KwaveForm& f, int64_t M, int64_t N, int cus, LaunchForm* o) {
   const KwaveShape& sh = shapes_of(dt)[f.shape];
-  o->grid = kwave_blocks((int)((M + sh.bm - 1) / sh.bm), (int)((N + f.per - 1) / f.per)) * f.ranges;
+  int by_panel;
+  o->grid = kwave_blocks((int)((M + sh.bm - 1) / sh.bm), (int)((N + f.per - 1) / f.per), cus, &by_panel) * f.ranges;
   o->tile_m = sh.bm;
   o->tile_n = sh.bn;
   o->waves_m = sh.wm;
@@ -235,22 +307,27 @@ void kwave_describe(int dt, const KwaveForm& f, int64_t M, int64_t N, LaunchForm
   o->func = sh.func;
 }
 
+bool kwave_prompt_describe(const astergemm_config& c, int cus, LaunchForm* o) {
+  const KwaveForm f = kwave_prompt_form(c.dtype_ab, c.M, c.N, c.K, cus);
+  if (f) kwave_describe(c.dtype_ab, f, c.M, c.N, cus, o);
+  return (bool)f;
+}
 bool kwave_tile_describe(const astergemm_config& c, int cus, LaunchForm* o) {
-  kwave_describe(c.dtype_ab, kwave_tile_form(c.dtype_ab, c.M, c.N, c.K, cus > 0 ? cus : 256), c.M, c.N, o);
+  kwave_describe(c.dtype_ab, kwave_tile_form(c.dtype_ab, c.M, c.N, c.K, cus), c.M, c.N, cus, o);
   return true;
 }
-bool kwave_split_describe(const astergemm_config& c, int cus, LaunchForm* o) {
-  if (!kwave_decode_describe(c, cus > 0 ? cus : 256, 1, o)) return kwave_tile_describe(c, cus, o);
+bool kwave_any_describe(const astergemm_config& c, int cus, LaunchForm* o) {
+  kwave_describe(c.dtype_ab, kwave_any_form(c.dtype_ab, c.M, c.N, c.K, cus), c.M, c.N, cus, o);
   return true;
 }
 bool kwave_decode_describe(const astergemm_config& c, int cus, int max_ranges, LaunchForm* o) {
   const KwaveForm f = kwave_decode_form(c.dtype_ab, c.M, c.N, c.K, cus, max_ranges);
-  if (f) kwave_describe(c.dtype_ab, f, c.M, c.N, o);
+  if (f) kwave_describe(c.dtype_ab, f, c.M, c.N, cus, o);
   return (bool)f;
 }
 bool kwave_small_decode_describe(const astergemm_config& c, int cus, LaunchForm* o) {
   const KwaveForm f = kwave_small_decode_form(c.dtype_ab, c.M, c.N, c.K, cus);
-  if (f) kwave_describe(c.dtype_ab, f, c.M, c.N, o);
+  if (f) kwave_describe(c.dtype_ab, f, c.M, c.N, cus, o);
   return (bool)f;
 }
 #endif  // AG_KWAVE_DT == 0

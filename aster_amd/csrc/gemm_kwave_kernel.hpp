@@ -30,7 +30,8 @@ struct KwaveArgs {
   int32_t per;          // weight rows of a workgroup (a multiple of 8, at most BN)
   int32_t ranges;       // K ranges (1: the result; more: fp32 planes in g.workspace)
   int32_t range_steps;  // K-steps of a range
-  int32_t blocks;       // workgroups of a range: tile rows x tile columns, these in whole groups of 8
+  int32_t blocks;       // workgroups of a range
+  int32_t by_panel;     // the tile rows of a panel on one XCD (else tile after tile, whatever the XCD)
   int32_t out;          // output type
   int32_t nt;           // weights are fetched past the last-level cache
 };
@@ -57,7 +58,7 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_kwave_kernel(const Kwave
   constexpr int TPW = (NT + NW - 1) / NW;       // of them finished by one wave
   static_assert(G % GW == 0, "whole transfers per wave");
   static_assert(S >= 2 && (S - 2) * L <= 63, "the counted wait fits the vmcnt field");
-  static_assert(WK > 1 && S * STAGE <= 160 * 1024 && WK * NT * 1024 <= S * STAGE, "LDS of a CU");
+  static_assert(S * STAGE <= 160 * 1024 && WK * NT * 1024 <= S * STAGE, "LDS of a CU");
 
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
   const GemmArgs& p = q.g;
@@ -70,8 +71,8 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_kwave_kernel(const Kwave
   // that start at the same K-step are then a large power of two apart)
   const int blocks = q.blocks;                  // of one K range
   const int range = blockIdx.x / blocks, bid = blockIdx.x - range * blocks;
-  const int idx = bid >> 3, panel = idx / p.tiles_m;
-  const int tile_m = idx - panel * p.tiles_m, tile_n = panel * 8 + (bid & 7);
+  const int idx = q.by_panel ? bid >> 3 : bid, panel = idx / p.tiles_m;
+  const int tile_m = idx - panel * p.tiles_m, tile_n = q.by_panel ? panel * 8 + (bid & 7) : panel;
   if (tile_n >= p.tiles_n) return;
   const int row0 = tile_m * BM, col0 = tile_n * q.per;
   const int col1 = (col0 + q.per) < p.N ? (col0 + q.per) : p.N;

@@ -420,7 +420,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_reg_kernel(const GemmArgs p) 
 // are readied by either's first launch, so that a config that is captured later finds its kernel ready
 // whichever of the two an earlier one ran; inside a capture only the one that runs has to be.
 inline KwaveForm kwave_instead(int dt, const GemmArgs& a, int cus, int max_ranges) {
-  return a.named_tile ? KwaveForm{} : kwave_decode_form(dt, a.M, a.N, a.K, cus, max_ranges);
+  return a.own_kernel ? KwaveForm{} : kwave_decode_form(dt, a.M, a.N, a.K, cus, max_ranges);
 }
 template <int (*SPLITS)(const astergemm_config&)>
 bool kwave_form_of(const astergemm_config& c, int cus, LaunchForm* o) {
@@ -789,7 +789,7 @@ int splitk_workspace(size_t bytes, hipStream_t stream, float** out) {
 
 // For a problem that is cut into K ranges by one kernel and not by the one that runs: the stream's buffer is
 // as large as if it had been, so that a later capture of another problem finds it.  Never inside a capture.
-void splitk_workspace_touch(size_t bytes, hipStream_t stream) {
+void workspace_touch(size_t bytes, hipStream_t stream) {
   int dev = 0;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
   if (hipGetDevice(&dev) != hipSuccess) return (void)hipGetLastError();
@@ -1103,7 +1103,7 @@ int launch_skinny_fp4m_t(const GemmArgs& a0, int S, hipStream_t s) {
   if (cus <= 0) return (int)hipErrorNoDevice;
   if (f) {
     if (S > f.ranges && !a0.workspace && !launch_context().prepare_only)
-      splitk_workspace_touch((size_t)S * a0.M * a0.N * sizeof(float), s);
+      workspace_touch((size_t)S * a0.M * a0.N * sizeof(float), s);
     return kwave_launch(ASTERGEMM_MXFP4, OUT, a0, f, s);
   }
   GemmArgs a = a0;
@@ -1454,7 +1454,7 @@ int launch_skinny_regm_t(const GemmArgs& a0, int S, hipStream_t s) {
   if (cus <= 0) return (int)hipErrorNoDevice;
   if (f) {
     if (S > f.ranges && !a0.workspace && !launch_context().prepare_only)
-      splitk_workspace_touch((size_t)S * a0.M * a0.N * sizeof(float), s);
+      workspace_touch((size_t)S * a0.M * a0.N * sizeof(float), s);
     return kwave_launch(DT, OUT, a0, f, s);
   }
   GemmArgs a = a0;
@@ -1974,7 +1974,7 @@ const char* check_skinny_directb(const astergemm_config& c) {
 
 template <int DT, int OUT, int MT, int NB, int KW, int U>
 int launch_skinny(const GemmArgs& a, int grid, hipStream_t s) {
-  if (!a.named_tile)
+  if (!a.own_kernel)
     if (const KwaveForm f = kwave_small_decode_form(DT, a.M, a.N, a.K, device_cus()))
       return kwave_launch(DT, OUT, a, f, s);
   AG_LAUNCH_KERNEL((gemm_skinny_kernel<DT, OUT, MT, NB, KW, U>), dim3(grid), dim3(KW * 64), 0,
@@ -2077,6 +2077,8 @@ const Variant* skinny_variants() { return kSkinnyVariants; }
 int splitk_workspace_for(size_t bytes, hipStream_t stream, float** out) {
   return splitk_workspace(bytes, stream, out);
 }
+
+void splitk_workspace_touch(size_t bytes, hipStream_t stream) { workspace_touch(bytes, stream); }
 
 std::mutex& splitk_order() {
   static std::mutex m;

@@ -4,6 +4,7 @@
 #include <mutex>
 #include <vector>
 
+#include "gemm_kwave.h"
 #include "gemm_stream_kernel.hpp"
 #include "gemm_streamr_kernel.hpp"
 #include "gemm_stream8_kernel.hpp"
@@ -17,12 +18,34 @@
 namespace astergemm {
 namespace {
 
+// Prompts of few tokens: the kernels that split K over the waves stand in for the 128 x 128 tiles of a config
+// that names no kernel (kwave_prompt_form).  Either's first launch readies both, so that a config that
+// is captured later finds its kernel ready; inside a capture only the one that runs has to be.
+inline KwaveForm kwave_instead(int dt, const GemmArgs& a) {
+  return a.own_kernel ? KwaveForm{} : kwave_prompt_form(dt, a.M, a.N, a.K, device_cus());
+}
+// 0 and *taken = false: the launcher's own kernel is to run
+inline int kwave_prompt(int dt, int out, const GemmArgs& a, int own_ready, hipStream_t s, bool* taken) {
+  const KwaveForm f = kwave_instead(dt, a);
+  *taken = (bool)f;
+  if (own_ready != 0 && !f) return own_ready;
+  const int e = kwave_ready(dt);
+  if (!f) return 0;
+  return e != 0 ? e : kwave_launch(dt, out, a, f, s);
+}
+
 template <int DT, int OUT, int BM, int BN, int WM, int WN, int NSLOT = 5>
 int launch_stream(const GemmArgs& a, int grid, hipStream_t s) {
   constexpr int lds = NSLOT * BM * kRowBytes;
   auto k = gemm_stream_kernel<DT, OUT, BM, BN, WM, WN, NSLOT>;
   static std::atomic<uint64_t> attr_devs{0};
-  if (int e = lds_attr_once(attr_devs, (const void*)k, lds)) return e;
+  if constexpr (BM == 128) {
+    bool taken = false;
+    if (const int e = kwave_prompt(DT, OUT, a, lds_attr_once(attr_devs, (const void*)k, lds), s, &taken); e || taken)
+      return e;
+  } else if (int e = lds_attr_once(attr_devs, (const void*)k, lds)) {
+    return e;
+  }
   AG_LAUNCH_KERNEL(k, dim3(grid), dim3(WM * WN * 64), lds, s, a);
   return (int)hipGetLastError();
 }
@@ -53,7 +76,9 @@ const char* check_stream_whole_k(const astergemm_config& c) {
         (WM * WN == 8 || BM == 128) ? 2 : 0, 5 * BM * kRowBytes,                \
         (const void*)gemm_stream_kernel<DT, OUT, BM, BN, WM, WN>,                \
         launch_stream<DT, OUT, BM, BN, WM, WN>,                                  \
-        (WM * WN == 8 || BM == 128) ? check_stream : check_stream_whole_k        \
+        (WM * WN == 8 || BM == 128) ? check_stream : check_stream_whole_k,       \
+        ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0,                              \
+        BM == 128 ? kwave_prompt_describe : nullptr                              \
   }
 
 // The 128 x 128 kernel with a ring of nine slots (144 KiB of LDS, one workgroup per CU): four
@@ -77,7 +102,8 @@ const char* check_stream_ring9(const astergemm_config& c) {
     name, ASTERGEMM_KERNEL_TILE, DT, OUT, 128, 128, kRowBytes, 2, 2, 5, 3,       \
         9 * 128 * kRowBytes,                                                     \
         (const void*)gemm_stream_kernel<DT, OUT, 128, 128, 2, 2, 9>,             \
-        launch_stream<DT, OUT, 128, 128, 2, 2, 9>, check_stream_ring9            \
+        launch_stream<DT, OUT, 128, 128, 2, 2, 9>, check_stream_ring9,           \
+        ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0, kwave_prompt_describe        \
   }
 #define AG_STREAM_RING9_SET(prefix, DT)                                          \
   AG_STREAM_RING9(prefix "_128x128_w2x2_ring9_bf16", DT, ASTERGEMM_BF16),        \
@@ -90,7 +116,13 @@ int launch_streamr(const GemmArgs& a, int grid, hipStream_t s) {
   constexpr int lds = NS * (BM + BN) * kRowBytes;
   auto k = gemm_streamr_kernel<DT, OUT, BM, BN, WM, WN, NS>;
   static std::atomic<uint64_t> attr_devs{0};
-  if (int e = lds_attr_once(attr_devs, (const void*)k, lds)) return e;
+  if constexpr (BM == 128) {
+    bool taken = false;
+    if (const int e = kwave_prompt(DT, OUT, a, lds_attr_once(attr_devs, (const void*)k, lds), s, &taken); e || taken)
+      return e;
+  } else if (int e = lds_attr_once(attr_devs, (const void*)k, lds)) {
+    return e;
+  }
   AG_LAUNCH_KERNEL(k, dim3(grid), dim3(WM * WN * 64), lds, s, a);
   return (int)hipGetLastError();
 }
@@ -100,7 +132,9 @@ int launch_streamr(const GemmArgs& a, int grid, hipStream_t s) {
     name, ASTERGEMM_KERNEL_TILE, DT, OUT, BM, BN, kRowBytes, WM, WN, NS, 5,      \
         NS * (BM + BN) * kRowBytes,                                              \
         (const void*)gemm_streamr_kernel<DT, OUT, BM, BN, WM, WN, NS>,           \
-        launch_streamr<DT, OUT, BM, BN, WM, WN, NS>, check_stream                \
+        launch_streamr<DT, OUT, BM, BN, WM, WN, NS>, check_stream,               \
+        ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0,                              \
+        BM == 128 ? kwave_prompt_describe : nullptr                              \
   }
 #define AG_STREAMR_SET(prefix, DT, BM, BN, WM, WN, NS)                     \
   AG_STREAMR(prefix "_bf16", DT, ASTERGEMM_BF16, BM, BN, WM, WN, NS),      \
@@ -270,7 +304,17 @@ int launch_stream_splitk(const GemmArgs& a0, int grid, hipStream_t s) {
   else if constexpr (KIND == 1) k = gemm_stream8_splitk_kernel<DT, 128, 128, 2, 2>;
   else k = gemm_stream4_splitk_kernel<DT, 128, 128, 2, 2>;
   static std::atomic<uint64_t> attr_devs{0};
-  if (int e = lds_attr_once(attr_devs, (const void*)k, lds)) return e;
+  bool taken = false;
+  // the same kernel whether AUTO chose this launcher or the config names it: a plan of the chosen variant
+  // gives the bits of the plan it was read from
+  GemmArgs by_name = a0;
+  by_name.own_kernel = a0.own_kernel == 1;
+  if (const int e = kwave_prompt(DT, OUT, by_name, lds_attr_once(attr_devs, (const void*)k, lds), s, &taken); e || taken) {
+    const int ranges = stream_split_of((int64_t)a0.tiles_m * a0.tiles_n, a0.ksteps, KIND == 2);
+    if (!e && !a0.workspace && !launch_context().prepare_only)
+      splitk_workspace_touch((size_t)ranges * a0.M * a0.N * sizeof(float), s);
+    return e;
+  }
   if constexpr (KIND == 2) {
     if ((((uintptr_t)a0.mx_a | (uintptr_t)a0.mx_b) & 15) != 0 || a0.mx_ld % 16 != 0)
       return (int)hipErrorInvalidValue;
@@ -326,7 +370,8 @@ int splits_stream_splitk(const astergemm_config& c) {
   Variant {                                                                      \
     name, ASTERGEMM_KERNEL_TILE, DT, OUT, 128, 128, kRowBytes, 2, 2, 3, 4, LDS,  \
         (const void*)FUNC<DT, 128, 128, 2, 2>, launch_stream_splitk<KIND, DT, OUT>, \
-        check_stream_splitk, ASTERGEMM_OPERAND_LDS, splits_stream_splitk         \
+        check_stream_splitk, ASTERGEMM_OPERAND_LDS, splits_stream_splitk,        \
+        nullptr, 0, kwave_prompt_describe                                        \
   }
 #define AG_STREAM_SPLITK_SET(prefix, KIND, DT, LDS, FUNC)                        \
   AG_STREAM_SPLITK(prefix "_128x128_w2x2_bf16", KIND, DT, ASTERGEMM_BF16, LDS, FUNC),   \
@@ -391,7 +436,13 @@ int launch_stream8(const GemmArgs& a, int grid, hipStream_t s) {
   constexpr int lds = 5 * BM * kRowBytes;
   auto k = gemm_stream8_kernel<DT, OUT, BM, BN, WM, WN>;
   static std::atomic<uint64_t> attr_devs{0};
-  if (int e = lds_attr_once(attr_devs, (const void*)k, lds)) return e;
+  if constexpr (BM == 128) {
+    bool taken = false;
+    if (const int e = kwave_prompt(DT, OUT, a, lds_attr_once(attr_devs, (const void*)k, lds), s, &taken); e || taken)
+      return e;
+  } else if (int e = lds_attr_once(attr_devs, (const void*)k, lds)) {
+    return e;
+  }
   AG_LAUNCH_KERNEL(k, dim3(grid), dim3(WM * WN * 64), lds, s, a);
   return (int)hipGetLastError();
 }
@@ -452,7 +503,8 @@ int grid_stream_walk(const astergemm_config& c, int cus) {
     name, ASTERGEMM_KERNEL_TILE, DT, OUT, 128, 128, kRowBytes, 2, 2, 3, 2,       \
         5 * 128 * kRowBytes,                                                     \
         (const void*)gemm_stream8_kernel<DT, OUT, 128, 128, 2, 2>,               \
-        launch_stream8<DT, OUT, 128, 128, 2, 2>, check_stream                    \
+        launch_stream8<DT, OUT, 128, 128, 2, 2>, check_stream,                   \
+        ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0, kwave_prompt_describe        \
   }
 
 template <int DT, int OUT, int BM, int BN, int WM, int WN>
@@ -463,7 +515,13 @@ int launch_stream4(const GemmArgs& a, int grid, hipStream_t s) {
     return (int)hipErrorInvalidValue;
   auto k = gemm_stream4_kernel<DT, OUT, BM, BN, WM, WN>;
   static std::atomic<uint64_t> attr_devs{0};
-  if (int e = lds_attr_once(attr_devs, (const void*)k, lds)) return e;
+  if constexpr (BM == 128) {
+    bool taken = false;
+    if (const int e = kwave_prompt(DT, OUT, a, lds_attr_once(attr_devs, (const void*)k, lds), s, &taken); e || taken)
+      return e;
+  } else if (int e = lds_attr_once(attr_devs, (const void*)k, lds)) {
+    return e;
+  }
   AG_LAUNCH_KERNEL(k, dim3(grid), dim3(WM * WN * 64), lds, s, a);
   return (int)hipGetLastError();
 }
@@ -547,7 +605,8 @@ int grid_stream4_walk(const astergemm_config& c, int cus) {
     name, ASTERGEMM_KERNEL_TILE, DT, OUT, 128, 128, kRowBytes, 2, 2, 2, 2,       \
         4 * 128 * kRowBytes + 4 * 128 * 16,                                      \
         (const void*)gemm_stream4_kernel<DT, OUT, 128, 128, 2, 2>,               \
-        launch_stream4<DT, OUT, 128, 128, 2, 2>, check_stream4                   \
+        launch_stream4<DT, OUT, 128, 128, 2, 2>, check_stream4,                  \
+        ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0, kwave_prompt_describe        \
   }
 
 // ---- whole rounds of 256 x 256 tiles, the rest in 128 x 128 tiles ---------------------------
@@ -599,6 +658,7 @@ inline void tail_parts(const GemmArgs& a, const TailSplit& ts, int out_bytes, Ge
                        GemmArgs* part2) {
   *part1 = a;
   *part2 = a;
+  part1->own_kernel = part2->own_kernel = 1;   // the bits of the tile kernels, whatever the parts' sizes
   if (ts.along == 1) {
     part1->N = (int32_t)ts.first;
     part2->N = a.N - (int32_t)ts.first;

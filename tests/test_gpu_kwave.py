@@ -26,10 +26,17 @@ pytestmark = pytest.mark.gpu
     (9, 4096, 11008, "fp8_e4m3", (16, 16)), (1, 1024, 4112, "fp8_e4m3", (16, 16)),
     (64, 2056, 4208, "fp8_e4m3", (32, 32)), (5, 1030, 4352, "mxfp4", (16, 16)), (64, 4096, 11008, "mxfp4", (32, 32)),
     (40, 300, 1984, "bf16", (16, 16)), (64, 1000, 992, "f16", (16, 16)), (1, 17, 32, "bf16", (16, 16)),
+    # prompts of few tokens: panels of exact rows under every tile height, ragged M, short last panels
+    (65, 4096, 4096, "bf16", (32, 64)), (128, 14336, 4096, "f16", (128, 64)), (96, 11008, 4096, "bf16", (96, 64)),
+    (100, 28672, 2304, "bf16", (128, 128)), (330, 4096, 4096, "f16", (96, 64)), (511, 4096, 4096, "bf16", (64, 128)),
+    (400, 4096, 4096, "bf16", (64, 128)),
+    (128, 1024, 8192, "f16", (32, 16)), (72, 8, 4096, "bf16", (32, 16)), (128, 8192, 8192, "fp8_e4m3", (64, 64)),
+    (250, 1032, 8192, "fp8_e4m3", (32, 64)), (128, 4096, 4096, "mxfp4", (32, 64)),
+    (256, 8192, 8192, "mxfp4", (64, 128)), (80, 14336, 4096, "mxfp4", (96, 64)), (304, 1000, 8192, "mxfp4", (32, 64)),
     # small products: the smallest tile in one round, K tails of 1 and 7 granules, fewer steps than stages
     (100, 100, 520, "bf16", (16, 16)), (300, 300, 2048, "f16", (32, 32)), (65, 130, 1080, "bf16", (16, 16)),
-    (600, 599, 1544, "bf16", (32, 64)), (777, 1001, 1032, "bf16", (64, 64)), (1200, 33, 2040, "f16", (16, 16)),
-    (100, 4095, 4096, "fp8_e4m3", (64, 64)), (70, 1000, 2064, "fp8_e4m3", (32, 32)),
+    (600, 599, 1544, "bf16", (32, 64)), (780, 599, 1032, "bf16", (32, 64)), (1200, 33, 2040, "f16", (16, 16)),
+    (100, 4095, 4096, "fp8_e4m3", (32, 64)), (70, 1000, 2064, "fp8_e4m3", (32, 32)),
 ])
 @pytest.mark.parametrize("dtype_c", ["f32", "bf16"])
 def test_k_over_waves(gpu, M, N, K, dtype_ab, dtype_c, tile):
