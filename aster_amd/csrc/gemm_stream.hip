@@ -34,11 +34,61 @@ inline int kwave_prompt(int dt, int out, const GemmArgs& a, int own_ready, hipSt
   return e != 0 ? e : kwave_launch(dt, out, a, f, s);
 }
 
+// Whole 128 x 128 tiles, two to a CU, of a config that names no kernel: each two as one tile of 256 x 128, whose
+// 384 operand rows replace their 512 and whose ring runs two K-steps ahead for the CU's eight waves together.
+// From 7/8 of the chip's CUs on in pairs: below, unequal_tile_of has taken the 256 x 128 kernel already.  One
+// round only: past it a second round of pairs is as long as the first.  128 x 128 / pairs, us (rows of 4096 / 11008 / 1024
+// elements): bf16 2048x4096 57.9 / 52.8, 180 / 159, 18.4 / 18.0; 512x14336 73.1 / 57.5, 184 / 157, 16.9 / 15.8;
+// 1024x8192 57.3 / 52.1, 185 / 155, 18.0 / 17.4; with a K tail 2048x4096x4104 79.0 / 67.0.  fp32 outputs on rows
+// of 2 KiB are behind (f16 2048x4096x1024 21.2 / 21.9).  The same sums in the same order, so the same bits.
+inline bool pairs_tiles(int out, int64_t M, int64_t N, int64_t row_bytes, int cus) {
+  const int64_t g128 = M / 128 * (N / 128);
+  return M % 128 == 0 && N % 128 == 0 && row_bytes >= (out == ASTERGEMM_F32 ? 18 * 128 : 2048) && g128 * 8 >= (int64_t)2 * cus * 7 &&
+         (M + 255) / 256 * (N / 128) <= cus;
+}
+
+template <int DT, int OUT>
+int launch_pairs(GemmArgs a, hipStream_t s) {
+  a.tiles_m = (a.M + 255) / 256;
+  a.group_m = (a.tiles_m % 8 == 0 && a.tiles_n % 32 == 0) ? -1 : 8;
+  auto k = gemm_streamr_kernel<DT, OUT, 256, 128, 4, 2, 3>;
+  AG_LAUNCH_KERNEL(k, dim3(a.tiles_m * a.tiles_n), dim3(512), 3 * 384 * kRowBytes, s, a);
+  return (int)hipGetLastError();
+}
+
+template <int DT, int OUT>
+bool pairs_describe(const astergemm_config& c, int cus, LaunchForm* o) {
+  if (kwave_prompt_describe(c, cus, o)) return true;
+  if (cus <= 0 || !pairs_tiles(OUT, c.M, c.N, row_bytes(DT, c.K), cus)) return false;
+  o->grid = (int)((c.M + 255) / 256 * (c.N / 128));
+  o->tile_m = 256;
+  o->tile_n = 128;
+  o->waves_m = 4;
+  o->waves_n = 2;
+  o->stages = 3;
+  o->lds_bytes = 3 * 384 * kRowBytes;
+  o->threads = 512;
+  o->func = (const void*)gemm_streamr_kernel<DT, OUT, 256, 128, 4, 2, 3>;
+  return true;
+}
+
 template <int DT, int OUT, int BM, int BN, int WM, int WN, int NSLOT = 5>
 int launch_stream(const GemmArgs& a, int grid, hipStream_t s) {
   constexpr int lds = NSLOT * BM * kRowBytes;
   auto k = gemm_stream_kernel<DT, OUT, BM, BN, WM, WN, NSLOT>;
   static std::atomic<uint64_t> attr_devs{0};
+  if constexpr (BM == 128 && NSLOT == 5) {
+    static std::atomic<uint64_t> pair_devs{0};
+    const bool pairs = !a.own_kernel && pairs_tiles(OUT, a.M, a.N, row_bytes(DT, a.K), device_cus());
+    const int pair_ready = lds_attr_once(
+        pair_devs, (const void*)gemm_streamr_kernel<DT, OUT, 256, 128, 4, 2, 3>, 3 * 384 * kRowBytes);
+    const int own_ready = lds_attr_once(attr_devs, (const void*)k, lds);
+    bool taken = false;
+    if (const int e = kwave_prompt(DT, OUT, a, pairs ? pair_ready : own_ready, s, &taken); e || taken) return e;
+    if (pairs) return launch_pairs<DT, OUT>(a, s);
+    AG_LAUNCH_KERNEL(k, dim3(grid), dim3(WM * WN * 64), lds, s, a);
+    return (int)hipGetLastError();
+  }
   if constexpr (BM == 128) {
     bool taken = false;
     if (const int e = kwave_prompt(DT, OUT, a, lds_attr_once(attr_devs, (const void*)k, lds), s, &taken); e || taken)
@@ -78,7 +128,7 @@ const char* check_stream_whole_k(const astergemm_config& c) {
         launch_stream<DT, OUT, BM, BN, WM, WN>,                                  \
         (WM * WN == 8 || BM == 128) ? check_stream : check_stream_whole_k,       \
         ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0,                              \
-        BM == 128 ? kwave_prompt_describe : nullptr                              \
+        BM == 128 ? pairs_describe<DT, OUT> : nullptr                            \
   }
 
 // The 128 x 128 kernel with a ring of nine slots (144 KiB of LDS, one workgroup per CU): four
