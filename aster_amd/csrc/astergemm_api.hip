@@ -167,7 +167,7 @@ int chip_cus() {
 }
 
 // A config that names a tile size or a wave count (1) or a kernel (2) gets that kernel, not one that stands in
-// for it.
+// for it (by name but for Variant::form_by_name).
 int own_kernel(const astergemm_config& c) {
   return c.wg_tile_m || c.wg_tile_n || c.waves_m || c.waves_n ? 1 : c.variant ? 2 : 0;
 }
@@ -200,6 +200,8 @@ int64_t tile_grid(const astergemm_config& c, int64_t bm, int64_t bn) {
 // two tile rows on: 333x8192x8192 51.1 -> 36.8, 1000x4096x14336 86.3 -> 66.8, 200x14336 29.1 -> 23.5.  Not with
 // a K tail: level back to back, behind on buffers that no kernel has read yet (384x5408x20592 139 -> 156,
 // 872x2632x13680 90.6 -> 96.7, 1648x2120x7600 50.5 -> 53.6).
+// (All with K loops from step 0; started apart by XCD, first_step_of_xcd, the 192 x 128, 256 x 128 and nine-slot
+// kernels take 1 to 12 % less, the others as long as here.)
 // A config that names a tile size or wave count gets the kernels it always got.
 bool unequal_tiles_apply(const astergemm_config& c) {
   return (c.dtype_ab == ASTERGEMM_F16 || c.dtype_ab == ASTERGEMM_BF16 || c.dtype_ab == ASTERGEMM_FP8_E4M3) &&
@@ -215,8 +217,8 @@ int unequal_tile_of(const astergemm_config& c) {
   if (g128 <= cus) return fp8 && whole_k && c.M > 128 ? 128 : 0;
   if (tile_grid(c, 192, 128) <= cus) return 192;
   // whole 128 x 128 tiles on at least 7/8 of two workgroups per CU: the tests pin this selection to
-  // the 128 x 128 kernel, which is the slower one there (bf16 512x14336 72.8 against 56.0 us,
-  // 2048x4096 59.3 against 53.9, fp8 2048x4096 32.4 against 31.6)
+  // the name of the 128 x 128 kernel; 16-bit operands run it as pairs of tiles (pairs_tiles), fp8 as it is (2048x4096
+  // 32.4 us against 31.6)
   if (c.M % 128 == 0 && c.N % 128 == 0 && g128 <= 2 * cus && g128 * 8 >= 2 * cus * 7) return 0;
   if (rb < 18 * 128 && c.M % 8 == 0 && (fp8 || c.dtype_c == ASTERGEMM_F32)) return 0;
   const int64_t g = tile_grid(c, 256, 128);
@@ -581,10 +583,8 @@ void describe(const Variant& v, int index, const astergemm_config& c, astergemm_
   snprintf(o->name, sizeof(o->name), "%s", v.name);
   const void* func = v.func;
   LaunchForm f;
-  // (a split kernel by name is what AUTO runs under that name, scratch or not)
-  const bool split_tile = v.family == ASTERGEMM_KERNEL_TILE && v.splits;
   const int own = own_kernel(c);
-  if (v.form && (v.rank >= 7 || !own || (own == 2 && split_tile)) && v.form(c, device_cus(), &f)) {
+  if (v.form && (v.rank >= 7 || !own || (own == 2 && v.form_by_name)) && v.form(c, device_cus(), &f)) {
     o->grid_x = f.grid;
     o->block_x = f.threads;
     o->lds_bytes = f.lds_bytes;

@@ -34,17 +34,18 @@ inline int kwave_prompt(int dt, int out, const GemmArgs& a, int own_ready, hipSt
   return e != 0 ? e : kwave_launch(dt, out, a, f, s);
 }
 
-// Whole 128 x 128 tiles, two to a CU, of a config that names no kernel: each two as one tile of 256 x 128, whose
+// Whole 128 x 128 tiles, two to a CU, of a config that names no tile or waves: each two as one of 256 x 128, whose
 // 384 operand rows replace their 512 and whose ring runs two K-steps ahead for the CU's eight waves together.
 // From 7/8 of the chip's CUs on in pairs: below, unequal_tile_of has taken the 256 x 128 kernel already.  One
-// round only: past it a second round of pairs is as long as the first.  128 x 128 / pairs, us (rows of 4096 / 11008 / 1024
-// elements): bf16 2048x4096 57.9 / 52.8, 180 / 159, 18.4 / 18.0; 512x14336 73.1 / 57.5, 184 / 157, 16.9 / 15.8;
+// round only: past it a second round of pairs is as long as the first.  128 x 128 / pairs, us (rows of 4096 / 11008 /
+// 1024 elements): bf16 2048x4096 57.9 / 52.8, 180 / 159, 18.4 / 18.0; 512x14336 73.1 / 57.5, 184 / 157, 16.9 / 15.8;
 // 1024x8192 57.3 / 52.1, 185 / 155, 18.0 / 17.4; with a K tail 2048x4096x4104 79.0 / 67.0.  fp32 outputs on rows
-// of 2 KiB are behind (f16 2048x4096x1024 21.2 / 21.9).  The same sums in the same order, so the same bits.
+// of 2 KiB are behind (f16 2048x4096x1024 21.2 / 21.9).  K loops from step 0 in both; see first_step_of_xcd.  A
+// config that names the 128 x 128 kernel gets the pairs too, with its bits: the same sums in the same order.
 inline bool pairs_tiles(int out, int64_t M, int64_t N, int64_t row_bytes, int cus) {
   const int64_t g128 = M / 128 * (N / 128);
-  return M % 128 == 0 && N % 128 == 0 && row_bytes >= (out == ASTERGEMM_F32 ? 18 * 128 : 2048) && g128 * 8 >= (int64_t)2 * cus * 7 &&
-         (M + 255) / 256 * (N / 128) <= cus;
+  return M % 128 == 0 && N % 128 == 0 && row_bytes >= (out == ASTERGEMM_F32 ? 18 * 128 : 2048) &&
+         g128 * 8 >= (int64_t)2 * cus * 7 && (M + 255) / 256 * (N / 128) <= cus;
 }
 
 template <int DT, int OUT>
@@ -58,7 +59,7 @@ int launch_pairs(GemmArgs a, hipStream_t s) {
 
 template <int DT, int OUT>
 bool pairs_describe(const astergemm_config& c, int cus, LaunchForm* o) {
-  if (kwave_prompt_describe(c, cus, o)) return true;
+  if (!c.variant && kwave_prompt_describe(c, cus, o)) return true;
   if (cus <= 0 || !pairs_tiles(OUT, c.M, c.N, row_bytes(DT, c.K), cus)) return false;
   o->grid = (int)((c.M + 255) / 256 * (c.N / 128));
   o->tile_m = 256;
@@ -79,7 +80,7 @@ int launch_stream(const GemmArgs& a, int grid, hipStream_t s) {
   static std::atomic<uint64_t> attr_devs{0};
   if constexpr (BM == 128 && NSLOT == 5) {
     static std::atomic<uint64_t> pair_devs{0};
-    const bool pairs = !a.own_kernel && pairs_tiles(OUT, a.M, a.N, row_bytes(DT, a.K), device_cus());
+    const bool pairs = a.own_kernel != 1 && pairs_tiles(OUT, a.M, a.N, row_bytes(DT, a.K), device_cus());
     const int pair_ready = lds_attr_once(
         pair_devs, (const void*)gemm_streamr_kernel<DT, OUT, 256, 128, 4, 2, 3>, 3 * 384 * kRowBytes);
     const int own_ready = lds_attr_once(attr_devs, (const void*)k, lds);
@@ -128,7 +129,7 @@ const char* check_stream_whole_k(const astergemm_config& c) {
         launch_stream<DT, OUT, BM, BN, WM, WN>,                                  \
         (WM * WN == 8 || BM == 128) ? check_stream : check_stream_whole_k,       \
         ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0,                              \
-        BM == 128 ? pairs_describe<DT, OUT> : nullptr                            \
+        BM == 128 ? pairs_describe<DT, OUT> : nullptr, true                      \
   }
 
 // The 128 x 128 kernel with a ring of nine slots (144 KiB of LDS, one workgroup per CU): four
@@ -136,7 +137,8 @@ const char* check_stream_whole_k(const astergemm_config& c) {
 // more tile rows, where nothing else covers a workgroup's waits (bf16, five -> nine slots:
 // 256 x 14336 x 4096 37.7-38.7 -> 33.7-34.4 us, 384 x 8192 x 4096 34.4 -> 31.0, 2048^3 23.3 ->
 // 21.2, 1024 x 4096 x 4096 36.9 -> 35.5; one tile row, which is HBM-bound on B alone, loses:
-// 128 x 28672 x 4096 39.8 -> 41.8; eight waves instead of four: level).
+// 128 x 28672 x 4096 39.8 -> 41.8; eight waves instead of four: level).  With K loops that start at different
+// steps on different XCDs: 200 x 14336 x 4096 41.4 -> 39.2, 333 x 8192 x 8192 68.4 -> 64.4.
 const char* check_stream_ring9(const astergemm_config& c) {
   if (const char* why = check_stream(c)) return why;
   int cus = device_cus();
@@ -421,7 +423,7 @@ int splits_stream_splitk(const astergemm_config& c) {
     name, ASTERGEMM_KERNEL_TILE, DT, OUT, 128, 128, kRowBytes, 2, 2, 3, 4, LDS,  \
         (const void*)FUNC<DT, 128, 128, 2, 2>, launch_stream_splitk<KIND, DT, OUT>, \
         check_stream_splitk, ASTERGEMM_OPERAND_LDS, splits_stream_splitk,        \
-        nullptr, 0, kwave_prompt_describe                                        \
+        nullptr, 0, kwave_prompt_describe, true                                  \
   }
 #define AG_STREAM_SPLITK_SET(prefix, KIND, DT, LDS, FUNC)                        \
   AG_STREAM_SPLITK(prefix "_128x128_w2x2_bf16", KIND, DT, ASTERGEMM_BF16, LDS, FUNC),   \
@@ -446,6 +448,7 @@ int launch_streamr_splitk(const GemmArgs& a0, int grid, hipStream_t s) {
       return rc;
   }
   GemmArgs part = a;
+  part.own_kernel = 0;         // by name or not, the same starts of the K loops
   part.split_k = S;
   part.ksteps = a.ksteps / S;
   part.ldc = a.N;

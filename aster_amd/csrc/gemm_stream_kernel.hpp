@@ -263,6 +263,19 @@ __device__ __forceinline__ void stream_mma(const i32x4& a, const i32x4& b, f32x4
   }
 }
 
+// K-step at which a workgroup's loop starts, of nk: an eighth of the row apart from XCD to XCD, so that the eight
+// caches do not ask the same memory channels for the same step of all rows at once (rows a large power
+// of two apart lie on few of them).  Not by tile: the workgroups of an XCD share operand rows in its L2 as
+// long as they walk in step (by tile column bf16 500x4096x14336 68 -> 92 us).  The loop wraps at nk.  A config that
+// names a kernel or a tile starts at step 0, so that all of those add in the same order.
+__device__ __forceinline__ int first_step_of_xcd(const GemmArgs& p, int nk) {
+  return p.own_kernel ? 0 : (int)(blockIdx.x & 7) * nk >> 3;
+}
+__device__ __forceinline__ int step_from(int first, int k, int nk) {
+  const int j = k + first;
+  return j >= nk ? j - nk : j;
+}
+
 template <int DT, int OUT, int BM, int BN, int WM, int WN, int NSLOT = 5>
 __device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, int bid) {
   constexpr int NW = WM * WN;
@@ -309,6 +322,9 @@ __device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, int bid) {
   group_bases<Plan>(p.B, p.ldb_bytes, col0, wave, p.N, b_base);
   const int nk = p.ksteps - (p.tail_granules ? 1 : 0);  // whole 128-byte steps
 
+  // the nine-slot ring only: the five-slot kernels give the bits of the tile walk and of the whole-rounds form
+  const int first = NSLOT == 9 ? first_step_of_xcd(p, nk) : 0;
+  auto at = [&](int k) { return NSLOT == 9 ? step_from(first, k, nk) : k; };
   // 64 lanes x 16 bytes from (scalar base + per-lane offset) to LDS at M0 + lane*16.
   // Written as asm to keep the scalar-base form; vmcnt is tracked by hand.
   auto g2s = [&](const uint8_t* base, unsigned voff, uint8_t* dst) {
@@ -320,11 +336,11 @@ __device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, int bid) {
   };
   // transfer j (0..LH-1) of this wave for the A / B half of K-step k
   auto issue_a1 = [&](int k, int slot, int j) {
-    g2s(a_base[j] + (int64_t)k * kRowBytes, a_off,
+    g2s(a_base[j] + (int64_t)at(k) * kRowBytes, a_off,
         lds + slot * SLOT + Plan::lds_offset(wave, j));
   };
   auto issue_b1 = [&](int k, int slot, int j) {
-    g2s(b_base[j] + (int64_t)k * kRowBytes, b_off,
+    g2s(b_base[j] + (int64_t)at(k) * kRowBytes, b_off,
         lds + slot * SLOT + Plan::lds_offset(wave, j));
   };
   auto issue_a = [&](int k, int slot) {

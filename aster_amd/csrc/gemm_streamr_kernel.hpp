@@ -15,7 +15,10 @@
 // three of 48 KiB, four of 40 KiB or five of 32 KiB.  Unlike the ring of gemm_stream_body, whose halves trade
 // places and must be equal, a stage is refilled as a whole: when K-step k is in registers its stage
 // is requested for K-step k + NS, so NS - 1 K-steps are on their way at any time.  Swizzle, staging
-// plan, fragment order, sums and epilogue are those of gemm_stream_body, so the bits are too.
+// plan, fragment order and epilogue are those of gemm_stream_body.  The K loops of different XCDs start at
+// different steps (first_step_of_xcd): bf16 333x14336x4096 50.5 -> 47.9 us, 1400x4096x14336 161 -> 144,
+// 333x4096x14336 (split K) 63.1 -> 58.3, 136x28672x4096 59.7 -> 52.3, fp8 200x28672x4096 44.5 -> 40.9; on
+// buffers that no kernel has read yet as much.
 #pragma once
 #include "gemm_stream_kernel.hpp"
 
@@ -62,6 +65,7 @@ __device__ __forceinline__ void gemm_streamr_body(const GemmArgs& p, int bid) {
   group_bases<PlanB>(p.B, p.ldb_bytes, col0, wave, p.N, b_base);
   const int nk = p.ksteps - (p.tail_granules ? 1 : 0);  // whole 128-byte steps
 
+  const int first = first_step_of_xcd(p, nk);
   auto g2s = [&](const uint8_t* base, unsigned voff, uint8_t* dst) {
     const unsigned m0v = (unsigned)(size_t)AG_LDS(dst);
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
@@ -70,10 +74,10 @@ __device__ __forceinline__ void gemm_streamr_body(const GemmArgs& p, int bid) {
                  : "memory", "m0");
   };
   auto issue_a1 = [&](int k, int stage, int j) {
-    g2s(a_base[j] + (int64_t)k * kRowBytes, a_off, lds + stage * STAGE + PlanA::lds_offset(wave, j));
+    g2s(a_base[j] + (int64_t)step_from(first, k, nk) * kRowBytes, a_off, lds + stage * STAGE + PlanA::lds_offset(wave, j));
   };
   auto issue_b1 = [&](int k, int stage, int j) {
-    g2s(b_base[j] + (int64_t)k * kRowBytes, b_off,
+    g2s(b_base[j] + (int64_t)step_from(first, k, nk) * kRowBytes, b_off,
         lds + stage * STAGE + B_AT + PlanB::lds_offset(wave, j));
   };
 
@@ -226,6 +230,7 @@ __device__ __forceinline__ void gemm_stream8r_body(const GemmArgs& p, int bid) {
   group_bases<PlanB>(p.B, p.ldb_bytes, col0, wave, p.N, b_base);
   const int nk = p.ksteps - (p.tail_granules ? 1 : 0);
 
+  const int first = first_step_of_xcd(p, nk);
   auto g2s = [&](const uint8_t* base, unsigned voff, uint8_t* dst) {
     const unsigned m0v = (unsigned)(size_t)AG_LDS(dst);
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
@@ -237,10 +242,10 @@ __device__ __forceinline__ void gemm_stream8r_body(const GemmArgs& p, int bid) {
   auto issue1 = [&](int k, int stage, auto jc) {
     constexpr int J = decltype(jc)::value;
     if constexpr (J < LB)
-      g2s(b_base[J] + (int64_t)k * kRowBytes, b_off,
+      g2s(b_base[J] + (int64_t)step_from(first, k, nk) * kRowBytes, b_off,
           lds + stage * STAGE + B_AT + PlanB::lds_offset(wave, J));
     else
-      g2s(a_base[J - LB] + (int64_t)k * kRowBytes, a_off,
+      g2s(a_base[J - LB] + (int64_t)step_from(first, k, nk) * kRowBytes, a_off,
           lds + stage * STAGE + PlanA::lds_offset(wave, J - LB));
   };
 
