@@ -237,7 +237,8 @@ int astergemm_variant_info(int index, const astergemm_config* cfg,
 int astergemm_run(const astergemm_config* cfg, const astergemm_operands* ops,
                   void* stream);
 /* Bytes of fp32 workspace the kernel that astergemm_select describes needs for
- * cfg (0 for most shapes: only rows cut into K ranges need one).  A smaller one
+ * cfg (0 for most shapes: only rows cut into K ranges need one), or more: an upper
+ * bound where a kernel with fewer ranges runs in its place.  A smaller one
  * is refused, or where another kernel takes the problem without it (see
  * astergemm_run) left unused.  The
  * reference's kernels have no workspace (every kernel takes exactly A, B, C:
