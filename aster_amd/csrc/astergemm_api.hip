@@ -856,7 +856,9 @@ int astergemm_variant_info(int index, const astergemm_config* cfg, astergemm_ker
     set_error("astergemm_variant_info: index %d out of range", index);
     return ASTERGEMM_EINVAL;
   }
-  describe(*v, index, *cfg, out);
+  astergemm_config c = *cfg;  // as the id runs it, not as AUTO does
+  c.variant = index + 1;
+  describe(*v, index, c, out);
   return 0;
 }
 

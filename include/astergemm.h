@@ -219,7 +219,8 @@ const char* astergemm_last_error(void);
 /* Replaces compile_fn: pick the kernel variant for cfg and describe it.     */
 int astergemm_select(const astergemm_config* cfg, astergemm_kernel_info* out);
 /* Number of built variants and a description of variant `index`
- * (0 <= index < count) instantiated for cfg's problem.                      */
+ * (0 <= index < count) instantiated for cfg's problem: what a config that names
+ * it (cfg->variant = index + 1) launches, whatever cfg itself names.          */
 int astergemm_variant_count(void);
 int astergemm_variant_info(int index, const astergemm_config* cfg,
                            astergemm_kernel_info* out);
