@@ -1095,6 +1095,8 @@ int astergemm_tune(const astergemm_config* cfg, const astergemm_operands* ops, i
     // every variant that can run the config: right types, family if one is asked for, shape
     // check passed, activation tile covering M on the weight-streaming path
     if (!variant_matches_types(*v, *cfg) || v->check(*cfg)) continue;
+    astergemm_config c = *cfg;  // as a plan of the id launches it
+    c.variant = i + 1;
     if (cfg->family != ASTERGEMM_KERNEL_AUTO && cfg->family != v->family) continue;
     if (v->family == ASTERGEMM_KERNEL_SKINNY && v->tile_m < cfg->M) continue;
     if (cfg->M == 0 || cfg->N == 0) {
@@ -1103,11 +1105,11 @@ int astergemm_tune(const astergemm_config* cfg, const astergemm_operands* ops, i
     }
     // a caller's workspace too small for this variant's K ranges: the variant is skipped, the
     // tune goes on with the others
-    if (ops->dWorkspace && ops->workspace_bytes < workspace_need(*v, *cfg)) continue;
-    if (needs_mx16(*v) && planes_off_16(*cfg, *ops)) continue;
+    if (ops->dWorkspace && ops->workspace_bytes < workspace_need(*v, c)) continue;
+    if (needs_mx16(*v) && planes_off_16(c, *ops)) continue;
     GemmArgs a;
-    if ((rc = build_args(*v, *cfg, *ops, &a)) != 0) break;
-    const int grid = grid_of(*v, *cfg);
+    if ((rc = build_args(*v, c, *ops, &a)) != 0) break;
+    const int grid = grid_of(*v, c);
     (void)hipGetLastError();
     int le = 0;
     for (int w = 0; w < 2 && le == 0; ++w) le = v->launch(a, grid, s);  // warm-up
