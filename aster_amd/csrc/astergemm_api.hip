@@ -108,6 +108,36 @@ const Variant* variant_at(int index) {
   return nullptr;
 }
 
+// AUTO's forms of the variants that have one (Variant::auto_form), numbered behind the table.
+struct AutoForms {
+  static constexpr int kMax = 1024;
+  int count = 0;
+  int16_t variant[kMax];  // form -> variant
+  int16_t form[kMax];     // variant -> form, or -1
+  AutoForms() {
+    for (int i = 0; i < kMax; ++i) {
+      const Variant* v = variant_at(i);
+      form[i] = -1;
+      if (v && v->auto_form) variant[count] = (int16_t)i, form[i] = (int16_t)count++;
+    }
+  }
+};
+const AutoForms& auto_forms() {
+  static const AutoForms forms;
+  return forms;
+}
+// The id's index of AUTO's form of a variant; the variant's own where there is no such form.
+int auto_id(int index) {
+  const int form = index < AutoForms::kMax ? auto_forms().form[index] : -1;
+  return form < 0 ? index : total_variants() + form;
+}
+int total_ids() { return total_variants() + auto_forms().count; }
+// The variant of an id's index: of the table, or the one whose AUTO form has the id.
+int variant_of_id(int index) {
+  const int form = index - total_variants();
+  return form < 0 ? index : form < auto_forms().count ? auto_forms().variant[form] : -1;
+}
+
 bool variant_matches_types(const Variant& v, const astergemm_config& c) {
   return v.dtype_ab == c.dtype_ab && v.dtype_c == c.dtype_c && v.operand_path == c.operand_path &&
          v.mx_a_layout == c.mx_a_layout;
@@ -166,10 +196,11 @@ int chip_cus() {
   return cus > 0 ? cus : 256;  // no device to ask: describe the MI355X
 }
 
-// A config that names a tile size or a wave count (1) or a kernel (2) gets that kernel, not one that stands in
-// for it (by name but for Variant::form_by_name).
-int own_kernel(const astergemm_config& c) {
-  return c.wg_tile_m || c.wg_tile_n || c.waves_m || c.waves_n ? 1 : c.variant ? 2 : 0;
+// A config that names a variant, a tile size or a wave count gets the launcher's own kernel; one that names
+// nothing, or AUTO's form by its id, AUTO's form (Variant::auto_form).
+bool own_kernel(const astergemm_config& c) {
+  if (c.variant != 0) return c.variant <= total_variants();
+  return c.wg_tile_m || c.wg_tile_n || c.waves_m || c.waves_n;
 }
 
 int64_t tile_grid(const astergemm_config& c, int64_t bm, int64_t bn) {
@@ -261,15 +292,10 @@ int tile64_stages_of(const astergemm_config& c) {
   return tile_grid(c, 64, 64) > (short_rows ? 1 : 2) * (int64_t)chip_cus() ? 2 : 4;
 }
 
-// K split over the waves of a workgroup instead of the general 64 x 64 tile kernel (rank 8): 32 x 64 tiles or
-// smaller fit one round, and the row is long enough for the K loop to be what the time goes on (fp8 600x600x1040
-// with the quantiser before it, 32 x 64 tiles, 13.1 / 14.3).  Past that,
-// with 64 x 64 tiles of its own, it is behind on short rows (general / this: bf16 777x1001x1032 8.0 / 8.8,
-// 1200x640x1024 6.8 / 7.8, fp8 1200x640x2064 8.4 / 9.7, ahead: bf16 777x1001x4096 17.5 / 16.3).
+// K split over the waves of a workgroup instead of the general 64 x 64 tile kernel (rank 8).
 bool kwave_tile_pays(const astergemm_config& c) {
-  return c.dtype_ab != ASTERGEMM_MXFP4 && c.operand_path == ASTERGEMM_OPERAND_LDS && !own_kernel(c) &&
-         row_bytes(c.dtype_ab, c.K) > (tile_grid(c, 32, 32) <= chip_cus() ? 8 * 128 : 2047) &&
-         tile_grid(c, 32, 64) <= chip_cus();
+  return c.operand_path == ASTERGEMM_OPERAND_LDS && !own_kernel(c) &&
+         kwave_small_product(c.dtype_ab, c.M, c.N, c.K, chip_cus());
 }
 
 // The same for decoding on rows of bytes that the kernels with resident activations do not take (rank 7).
@@ -331,7 +357,7 @@ const Variant* choose(const astergemm_config& c, int* index_out, int avoid = 0) 
     const ChoiceCacheEntry& e = g_choice_cache[i];
     if (e.dev == dev && e.avoid == avoid && memcmp(&e.cfg, &c, sizeof(c)) == 0) {
       if (index_out) *index_out = e.index;
-      return variant_at(e.index);
+      return variant_at(variant_of_id(e.index));
     }
   }
   int index = -1;
@@ -356,7 +382,7 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out, int av
     return nullptr;
   }
   if (c.variant != 0) {
-    const Variant* v = variant_at(c.variant - 1);
+    const Variant* v = variant_at(variant_of_id(c.variant - 1));
     if (!v || !variant_matches_types(*v, c)) {
       set_error("astergemm: variant %d does not exist for these dtypes", c.variant);
       return nullptr;
@@ -533,7 +559,7 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out, int av
     set_error("astergemm: skinny path covers M <= %d, got M=%lld", best->tile_m, (long long)c.M);
     return nullptr;
   }
-  if (index_out) *index_out = best_index;
+  if (index_out) *index_out = own_kernel(c) ? best_index : auto_id(best_index);
   return best;
 }
 
@@ -580,11 +606,15 @@ void describe(const Variant& v, int index, const astergemm_config& c, astergemm_
   o->pipeline_stages = v.stages;
   o->flops = 2 * c.M * c.N * c.K;
   o->bytes = algorithmic_bytes(c);
-  snprintf(o->name, sizeof(o->name), "%s", v.name);
+  // by its id AUTO's form has a name of its own, "..._auto_<output>"; a selection reports the variant's
+  const char* out = strrchr(v.name, '_');
+  if (c.variant != 0 && index >= total_variants() && out)
+    snprintf(o->name, sizeof(o->name), "%.*s_auto%s", (int)(out - v.name), v.name, out);
+  else
+    snprintf(o->name, sizeof(o->name), "%s", v.name);
   const void* func = v.func;
   LaunchForm f;
-  const int own = own_kernel(c);
-  if (v.form && (v.rank >= 7 || !own || (own == 2 && v.form_by_name)) && v.form(c, device_cus(), &f)) {
+  if (v.form && !(v.auto_form && own_kernel(c)) && v.form(c, device_cus(), &f)) {
     o->grid_x = f.grid;
     o->block_x = f.threads;
     o->lds_bytes = f.lds_bytes;
@@ -741,8 +771,8 @@ int index_of(const Variant& v) {
 
 // A config with an optional split has two kernels: an eager launch of one readies the other, so that a
 // later capture finds either of them ready.  (The stream's workspace is: the kernel a capture runs has no
-// more K ranges than the split it stands in for, by the lines of unequal_split_pays.)  Once per kernel and
-// device (these launchers have one kernel each whatever the config); done on every call it cost such a
+// more K ranges than the split it stands in for, by the lines of unequal_split_pays.)  Once per launcher
+// and device (a launcher with several kernels readies all of them, whichever the config runs); done on every call it cost such a
 // call 0.5-0.7 of 8.3 us of host time.  A failure is that later launch's to report, not the call's that has just succeeded.
 void ready_other(const Variant* other, const astergemm_config& c, void* stream) {
   if (!other) return;
@@ -844,14 +874,14 @@ extern "C" {
 int astergemm_abi_version(void) { return ASTERGEMM_ABI_VERSION; }
 const char* astergemm_last_error(void) { return g_err; }
 
-int astergemm_variant_count(void) { return total_variants(); }
+int astergemm_variant_count(void) { return total_ids(); }
 
 int astergemm_variant_info(int index, const astergemm_config* cfg, astergemm_kernel_info* out) {
   if (!cfg || !out) {
     set_error("astergemm_variant_info: null argument");
     return ASTERGEMM_EINVAL;
   }
-  const Variant* v = variant_at(index);
+  const Variant* v = variant_at(variant_of_id(index));
   if (!v) {
     set_error("astergemm_variant_info: index %d out of range", index);
     return ASTERGEMM_EINVAL;
@@ -1090,8 +1120,8 @@ int astergemm_tune(const astergemm_config* cfg, const astergemm_operands* ops, i
   hipEvent_t e0 = ev.e0, e1 = ev.e1;
   double best = 0.0;
   int rc = 0;
-  for (int i = 0; i < total_variants() && rc == 0; ++i) {
-    const Variant* v = variant_at(i);
+  for (int i = 0; i < total_ids() && rc == 0; ++i) {
+    const Variant* v = variant_at(variant_of_id(i));
     // every variant that can run the config: right types, family if one is asked for, shape
     // check passed, activation tile covering M on the weight-streaming path
     if (!variant_matches_types(*v, *cfg) || v->check(*cfg)) continue;

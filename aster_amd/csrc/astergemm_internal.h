@@ -28,7 +28,7 @@ struct GemmArgs {
   int32_t tiles_m, tiles_n;
   int32_t group_m;       // tile rows per rasterisation group; < 0: band order (see map_tile)
   int32_t split_k;       // skinny path: K slices per output row block
-  int32_t own_kernel;    // the config names a tile or a wave count (1) or a kernel (2)
+  int32_t own_kernel;    // not AUTO's form: the launcher's own kernel, K loops from step 0 (Variant::auto_form)
   float* workspace;      // fp32 partials [split_k][M][N] when a row is cut into K ranges; set by
                          // the caller of a launcher = use this buffer, null = the library's own
 };
@@ -82,8 +82,11 @@ struct Variant {
   // Launchers with a second kernel for some problems: its description when this one is among them
   // (`cus` as for grid; 0 = no device, nothing is known to fill it).  splits() stays an upper bound then.
   bool (*form)(const astergemm_config& c, int cus, LaunchForm* o) = nullptr;
-  // form() holds for a config that names the variant too, so that a plan of it gives AUTO's bits
-  bool form_by_name = false;
+  // Where AUTO takes this variant the launcher may run another kernel (form) or start its K loops elsewhere
+  // (first_step_of_xcd).  AUTO's form has an id and a name of its own, behind those of the table, which are the
+  // launcher's own kernel: a plan of either gives the bits of what reported the id.  false: one form, `form`
+  // if set.
+  bool auto_form = false;
 };
 
 // Compute units of the current device (0 when there is none), cached per device ordinal.

@@ -23,8 +23,11 @@ KwaveForm kwave_small_decode_form(int dt, int64_t M, int64_t N, int64_t K, int c
 KwaveForm kwave_prompt_form(int dt, int64_t M, int64_t N, int64_t K, int cus);
 // Any M and N: the smallest tile that leaves at most one workgroup per CU, else (and without a device) 64 x 64.
 KwaveForm kwave_tile_form(int dt, int64_t M, int64_t N, int64_t K, int cus);
-// The decode form where there is one, else the prompt form, else the tile form.
-KwaveForm kwave_any_form(int dt, int64_t M, int64_t N, int64_t K, int cus);
+// Small products that AUTO takes the tile form for, where it takes the general tile kernels otherwise.
+bool kwave_small_product(int dt, int64_t M, int64_t N, int64_t K, int cus);
+// What the variants of these kernels run, by AUTO or by name: the tile form for small products (split: never),
+// else the decode form where there is one, else the prompt form, else the tile form.
+KwaveForm kwave_variant_form(bool split, int dt, int64_t M, int64_t N, int64_t K, int cus);
 
 int kwave_launch(int dt, int out, const GemmArgs& a, const KwaveForm& f, hipStream_t s);
 // The one-time step of every shape of `dt` on the current device (see lds_attr_once).
@@ -32,8 +35,6 @@ int kwave_ready(int dt);
 void kwave_describe(int dt, const KwaveForm& f, int64_t M, int64_t N, int cus, LaunchForm* o);
 bool kwave_decode_describe(const astergemm_config& c, int cus, int max_ranges, LaunchForm* o);
 bool kwave_prompt_describe(const astergemm_config& c, int cus, LaunchForm* o);
-bool kwave_tile_describe(const astergemm_config& c, int cus, LaunchForm* o);
-bool kwave_any_describe(const astergemm_config& c, int cus, LaunchForm* o);
 bool kwave_small_decode_describe(const astergemm_config& c, int cus, LaunchForm* o);
 
 }  // namespace astergemm

@@ -243,7 +243,18 @@ KwaveForm kwave_tile_form(int dt, int64_t M, int64_t N, int64_t K, int cus) {
   return f;
 }
 
-KwaveForm kwave_any_form(int dt, int64_t M, int64_t N, int64_t K, int cus) {
+// 32 x 64 tiles or smaller fit one round, and the row is long enough for the K loop to be what the time goes on
+// (fp8 600x600x1040 with the quantiser before it, 32 x 64 tiles, general 64 x 64 kernel / this 13.1 / 14.3).  Past
+// that, with 64 x 64 tiles of its own, it is behind on short rows (bf16 777x1001x1032 8.0 / 8.8, 1200x640x1024
+// 6.8 / 7.8, fp8 1200x640x2064 8.4 / 9.7, ahead: bf16 777x1001x4096 17.5 / 16.3).
+bool kwave_small_product(int dt, int64_t M, int64_t N, int64_t K, int cus) {
+  const int64_t m32 = (M + 31) / 32;
+  return dt != ASTERGEMM_MXFP4 && row_bytes(dt, K) > (m32 * ((N + 31) / 32) <= cus ? 8 * 128 : 2047) &&
+         m32 * ((N + 63) / 64) <= cus;
+}
+
+KwaveForm kwave_variant_form(bool split, int dt, int64_t M, int64_t N, int64_t K, int cus) {
+  if (!split && kwave_small_product(dt, M, N, K, cus)) return kwave_tile_form(dt, M, N, K, cus);
   KwaveForm f = kwave_decode_form(dt, M, N, K, cus, 1);
   if (!f) f = kwave_prompt_form(dt, M, N, K, cus);
   return f ? f : kwave_tile_form(dt, M, N, K, cus);
@@ -311,14 +322,6 @@ bool kwave_prompt_describe(const astergemm_config& c, int cus, LaunchForm* o) {
   const KwaveForm f = kwave_prompt_form(c.dtype_ab, c.M, c.N, c.K, cus);
   if (f) kwave_describe(c.dtype_ab, f, c.M, c.N, cus, o);
   return (bool)f;
-}
-bool kwave_tile_describe(const astergemm_config& c, int cus, LaunchForm* o) {
-  kwave_describe(c.dtype_ab, kwave_tile_form(c.dtype_ab, c.M, c.N, c.K, cus), c.M, c.N, cus, o);
-  return true;
-}
-bool kwave_any_describe(const astergemm_config& c, int cus, LaunchForm* o) {
-  kwave_describe(c.dtype_ab, kwave_any_form(c.dtype_ab, c.M, c.N, c.K, cus), c.M, c.N, cus, o);
-  return true;
 }
 bool kwave_decode_describe(const astergemm_config& c, int cus, int max_ranges, LaunchForm* o) {
   const KwaveForm f = kwave_decode_form(c.dtype_ab, c.M, c.N, c.K, cus, max_ranges);

@@ -702,7 +702,7 @@ const char* check_skinny_fp4(const astergemm_config& c) {
     name, ASTERGEMM_KERNEL_SKINNY, ASTERGEMM_MXFP4, OUT, 16, 16, 512, 1, 8, 1, 3,           \
         8 * 8192 + 65536, (const void*)gemm_skinny_fp4_kernel<OUT, 2, 2>,                  \
         launch_skinny_fp4<OUT>, check_skinny_fp4, ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0, \
-        kwave_form_of<one_range>                                                           \
+        kwave_form_of<one_range>, true                                                     \
   }
 
 // ---- rows cut into K ranges: partial sums, their workspace and the kernel that adds them ---
@@ -1161,7 +1161,7 @@ int grid_skinny_fp4m(const astergemm_config& c, int cus) {
     name, ASTERGEMM_KERNEL_SKINNY, ASTERGEMM_MXFP4, OUT, 64, 16, 512, 1, 8, 1, 2,           \
         8 * 8192 + 65536, (const void*)gemm_skinny_fp4m_kernel<OUT, 2, 2, 2, 2>,           \
         launch_skinny_fp4m<OUT>, check_skinny_fp4m, ASTERGEMM_OPERAND_LDS,                 \
-        splits_skinny_fp4m, grid_skinny_fp4m, 0, kwave_form_of<splits_skinny_fp4m>         \
+        splits_skinny_fp4m, grid_skinny_fp4m, 0, kwave_form_of<splits_skinny_fp4m>, true   \
   }
 
 // ---- 16 < M <= 64: the same persistent kernel with two activation tiles per wave --------
@@ -1515,7 +1515,7 @@ int grid_skinny_regm(const astergemm_config& c, int cus) {
     name, ASTERGEMM_KERNEL_SKINNY, DT, OUT, 64, 16, 512, 1, 8, 1, 2, 8 * 8192 + 65536,      \
         (const void*)gemm_skinny_regm_kernel<DT, OUT, 8, 2, 2>, launch_skinny_regm<DT, OUT>, \
         check_skinny_regm, ASTERGEMM_OPERAND_LDS, splits_skinny_regm, grid_skinny_regm, 0, \
-        kwave_form_of<splits_skinny_regm>                                                            \
+        kwave_form_of<splits_skinny_regm>, true                                            \
   }
 
 template <int DT, int OUT>
@@ -1543,7 +1543,8 @@ const char* check_skinny_reg(const astergemm_config& c) {
   Variant {                                                                                \
     name, ASTERGEMM_KERNEL_SKINNY, DT, OUT, 16, 16, 512, 1, 8, 1, 3, 8 * 8192 + 65536,      \
         (const void*)gemm_skinny_reg_kernel<DT, OUT, 8>, launch_skinny_reg<DT, OUT>,       \
-        check_skinny_reg, ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0, kwave_form_of<one_range> \
+        check_skinny_reg, ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0, \
+        kwave_form_of<one_range>, true                                                     \
   }
 
 // ---- M <= 16, B pre-shuffled (operand path "direct B") ---------------------------------
@@ -1994,7 +1995,7 @@ const char* check_skinny(const astergemm_config& c) {
     name, ASTERGEMM_KERNEL_SKINNY, DT, OUT, 16 * MT, 16 * NB, 64 * U, 1, KW, 1, 0,        \
         KW * MT * NB * 1024, (const void*)gemm_skinny_kernel<DT, OUT, MT, NB, KW, U>,      \
         launch_skinny<DT, OUT, MT, NB, KW, U>, check_skinny, ASTERGEMM_OPERAND_LDS, nullptr, \
-        nullptr, 0, kwave_small_decode_describe                                           \
+        nullptr, 0, kwave_small_decode_describe, true                                     \
   }
 
 #define AG_SKINNY_SET(prefix, DT, OUTN, OUT)                                      \
@@ -2010,7 +2011,7 @@ const char* check_skinny(const astergemm_config& c) {
     name, ASTERGEMM_KERNEL_SKINNY, DT, OUT, 16 * MT, 16 * NB, 64 * U, 1, KW, 1, 1,        \
         KW * MT * NB * 1024, (const void*)gemm_skinny_kernel<DT, OUT, MT, NB, KW, U>,      \
         launch_skinny<DT, OUT, MT, NB, KW, U>, check_skinny, ASTERGEMM_OPERAND_LDS, nullptr, \
-        nullptr, 0, kwave_small_decode_describe                                           \
+        nullptr, 0, kwave_small_decode_describe, true                                     \
   }
 #define AG_SKINNY_WIDE_SET(prefix, DT, OUTN, OUT)                                 \
   AG_SKINNY_WIDE(prefix "_m32n64_" OUTN, DT, OUT, 2, 4, 4, 2),                    \

@@ -18,8 +18,8 @@
 namespace astergemm {
 namespace {
 
-// Prompts of few tokens: the kernels that split K over the waves stand in for the 128 x 128 tiles of a config
-// that names no kernel (kwave_prompt_form).  Either's first launch readies both, so that a config that
+// Prompts of few tokens: the kernels that split K over the waves stand in for the 128 x 128 tiles in AUTO's form
+// of their variants (kwave_prompt_form).  Either's first launch readies both, so that a config that
 // is captured later finds its kernel ready; inside a capture only the one that runs has to be.
 inline KwaveForm kwave_instead(int dt, const GemmArgs& a) {
   return a.own_kernel ? KwaveForm{} : kwave_prompt_form(dt, a.M, a.N, a.K, device_cus());
@@ -34,14 +34,14 @@ inline int kwave_prompt(int dt, int out, const GemmArgs& a, int own_ready, hipSt
   return e != 0 ? e : kwave_launch(dt, out, a, f, s);
 }
 
-// Whole 128 x 128 tiles, two to a CU, of a config that names no tile or waves: each two as one of 256 x 128, whose
+// Whole 128 x 128 tiles, two to a CU, in AUTO's form of the variant: each two as one of 256 x 128, whose
 // 384 operand rows replace their 512 and whose ring runs two K-steps ahead for the CU's eight waves together.
 // From 7/8 of the chip's CUs on in pairs: below, unequal_tile_of has taken the 256 x 128 kernel already.  One
 // round only: past it a second round of pairs is as long as the first.  128 x 128 / pairs, us (rows of 4096 / 11008 /
 // 1024 elements): bf16 2048x4096 57.9 / 52.8, 180 / 159, 18.4 / 18.0; 512x14336 73.1 / 57.5, 184 / 157, 16.9 / 15.8;
 // 1024x8192 57.3 / 52.1, 185 / 155, 18.0 / 17.4; with a K tail 2048x4096x4104 79.0 / 67.0.  fp32 outputs on rows
-// of 2 KiB are behind (f16 2048x4096x1024 21.2 / 21.9).  K loops from step 0 in both; see first_step_of_xcd.  A
-// config that names the 128 x 128 kernel gets the pairs too, with its bits: the same sums in the same order.
+// of 2 KiB are behind (f16 2048x4096x1024 21.2 / 21.9).  K loops from step 0 in both for these figures; as AUTO
+// runs them they start by XCD (first_step_of_xcd).
 inline bool pairs_tiles(int out, int64_t M, int64_t N, int64_t row_bytes, int cus) {
   const int64_t g128 = M / 128 * (N / 128);
   return M % 128 == 0 && N % 128 == 0 && row_bytes >= (out == ASTERGEMM_F32 ? 18 * 128 : 2048) &&
@@ -59,7 +59,7 @@ int launch_pairs(GemmArgs a, hipStream_t s) {
 
 template <int DT, int OUT>
 bool pairs_describe(const astergemm_config& c, int cus, LaunchForm* o) {
-  if (!c.variant && kwave_prompt_describe(c, cus, o)) return true;
+  if (kwave_prompt_describe(c, cus, o)) return true;
   if (cus <= 0 || !pairs_tiles(OUT, c.M, c.N, row_bytes(DT, c.K), cus)) return false;
   o->grid = (int)((c.M + 255) / 256 * (c.N / 128));
   o->tile_m = 256;
@@ -80,7 +80,7 @@ int launch_stream(const GemmArgs& a, int grid, hipStream_t s) {
   static std::atomic<uint64_t> attr_devs{0};
   if constexpr (BM == 128 && NSLOT == 5) {
     static std::atomic<uint64_t> pair_devs{0};
-    const bool pairs = a.own_kernel != 1 && pairs_tiles(OUT, a.M, a.N, row_bytes(DT, a.K), device_cus());
+    const bool pairs = !a.own_kernel && pairs_tiles(OUT, a.M, a.N, row_bytes(DT, a.K), device_cus());
     const int pair_ready = lds_attr_once(
         pair_devs, (const void*)gemm_streamr_kernel<DT, OUT, 256, 128, 4, 2, 3>, 3 * 384 * kRowBytes);
     const int own_ready = lds_attr_once(attr_devs, (const void*)k, lds);
@@ -129,7 +129,7 @@ const char* check_stream_whole_k(const astergemm_config& c) {
         launch_stream<DT, OUT, BM, BN, WM, WN>,                                  \
         (WM * WN == 8 || BM == 128) ? check_stream : check_stream_whole_k,       \
         ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0,                              \
-        BM == 128 ? pairs_describe<DT, OUT> : nullptr, true                      \
+        BM == 128 ? pairs_describe<DT, OUT> : nullptr, BM == 128                 \
   }
 
 // The 128 x 128 kernel with a ring of nine slots (144 KiB of LDS, one workgroup per CU): four
@@ -155,7 +155,7 @@ const char* check_stream_ring9(const astergemm_config& c) {
         9 * 128 * kRowBytes,                                                     \
         (const void*)gemm_stream_kernel<DT, OUT, 128, 128, 2, 2, 9>,             \
         launch_stream<DT, OUT, 128, 128, 2, 2, 9>, check_stream_ring9,           \
-        ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0, kwave_prompt_describe        \
+        ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0, kwave_prompt_describe, true  \
   }
 #define AG_STREAM_RING9_SET(prefix, DT)                                          \
   AG_STREAM_RING9(prefix "_128x128_w2x2_ring9_bf16", DT, ASTERGEMM_BF16),        \
@@ -186,7 +186,7 @@ int launch_streamr(const GemmArgs& a, int grid, hipStream_t s) {
         (const void*)gemm_streamr_kernel<DT, OUT, BM, BN, WM, WN, NS>,           \
         launch_streamr<DT, OUT, BM, BN, WM, WN, NS>, check_stream,               \
         ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0,                              \
-        BM == 128 ? kwave_prompt_describe : nullptr                              \
+        BM == 128 ? kwave_prompt_describe : nullptr, true                        \
   }
 #define AG_STREAMR_SET(prefix, DT, BM, BN, WM, WN, NS)                     \
   AG_STREAMR(prefix "_bf16", DT, ASTERGEMM_BF16, BM, BN, WM, WN, NS),      \
@@ -357,11 +357,7 @@ int launch_stream_splitk(const GemmArgs& a0, int grid, hipStream_t s) {
   else k = gemm_stream4_splitk_kernel<DT, 128, 128, 2, 2>;
   static std::atomic<uint64_t> attr_devs{0};
   bool taken = false;
-  // the same kernel whether AUTO chose this launcher or the config names it: a plan of the chosen variant
-  // gives the bits of the plan it was read from
-  GemmArgs by_name = a0;
-  by_name.own_kernel = a0.own_kernel == 1;
-  if (const int e = kwave_prompt(DT, OUT, by_name, lds_attr_once(attr_devs, (const void*)k, lds), s, &taken); e || taken) {
+  if (const int e = kwave_prompt(DT, OUT, a0, lds_attr_once(attr_devs, (const void*)k, lds), s, &taken); e || taken) {
     const int ranges = stream_split_of((int64_t)a0.tiles_m * a0.tiles_n, a0.ksteps, KIND == 2);
     if (!e && !a0.workspace && !launch_context().prepare_only)
       splitk_workspace_touch((size_t)ranges * a0.M * a0.N * sizeof(float), s);
@@ -448,7 +444,6 @@ int launch_streamr_splitk(const GemmArgs& a0, int grid, hipStream_t s) {
       return rc;
   }
   GemmArgs part = a;
-  part.own_kernel = 0;         // by name or not, the same starts of the K loops
   part.split_k = S;
   part.ksteps = a.ksteps / S;
   part.ldc = a.N;
@@ -477,7 +472,7 @@ const char* check_streamr_splitk(const astergemm_config& c) {
         3 * (256 + 128) * kRowBytes,                                             \
         (const void*)gemm_streamr_splitk_kernel<DT, 256, 128, 4, 2, 3>,          \
         launch_streamr_splitk<DT, OUT>, check_streamr_splitk,                    \
-        ASTERGEMM_OPERAND_LDS, splits_streamr_splitk                             \
+        ASTERGEMM_OPERAND_LDS, splits_streamr_splitk, nullptr, 0, nullptr, true  \
   }
 #define AG_STREAMR_SPLITK_SET(prefix, DT)                                        \
   AG_STREAMR_SPLITK(prefix "_256x128_w4x2_bf16", DT, ASTERGEMM_BF16),            \
@@ -557,7 +552,7 @@ int grid_stream_walk(const astergemm_config& c, int cus) {
         5 * 128 * kRowBytes,                                                     \
         (const void*)gemm_stream8_kernel<DT, OUT, 128, 128, 2, 2>,               \
         launch_stream8<DT, OUT, 128, 128, 2, 2>, check_stream,                   \
-        ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0, kwave_prompt_describe        \
+        ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0, kwave_prompt_describe, true  \
   }
 
 template <int DT, int OUT, int BM, int BN, int WM, int WN>
@@ -659,7 +654,7 @@ int grid_stream4_walk(const astergemm_config& c, int cus) {
         4 * 128 * kRowBytes + 4 * 128 * 16,                                      \
         (const void*)gemm_stream4_kernel<DT, OUT, 128, 128, 2, 2>,               \
         launch_stream4<DT, OUT, 128, 128, 2, 2>, check_stream4,                  \
-        ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0, kwave_prompt_describe        \
+        ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0, kwave_prompt_describe, true  \
   }
 
 // ---- whole rounds of 256 x 256 tiles, the rest in 128 x 128 tiles ---------------------------

@@ -266,8 +266,10 @@ __device__ __forceinline__ void stream_mma(const i32x4& a, const i32x4& b, f32x4
 // K-step at which a workgroup's loop starts, of nk: an eighth of the row apart from XCD to XCD, so that the eight
 // caches do not ask the same memory channels for the same step of all rows at once (rows a large power
 // of two apart lie on few of them).  Not by tile: the workgroups of an XCD share operand rows in its L2 as
-// long as they walk in step (by tile column bf16 500x4096x14336 68 -> 92 us).  The loop wraps at nk.  A config that
-// names a kernel or a tile starts at step 0, so that all of those add in the same order.
+// long as they walk in step (by tile column bf16 500x4096x14336 68 -> 92 us).  The loop wraps at nk.  In AUTO's
+// form only: a launcher's own kernel starts at step 0, so that all of those add in the same order.  Which XCD a
+// tile is on decides the order of its fp32 sums then, so equal rows of A may differ in the last bits from one row
+// of tiles to another; the bits of a config are the same on every run.
 __device__ __forceinline__ int first_step_of_xcd(const GemmArgs& p, int nk) {
   return p.own_kernel ? 0 : (int)(blockIdx.x & 7) * nk >> 3;
 }

@@ -37,10 +37,7 @@ int launch_kwave_tile(const GemmArgs& a, int grid, hipStream_t s) {
   if (int e = kwave_ready(DT)) return e;
   const int cus = device_cus();
   if (cus <= 0) return (int)hipErrorNoDevice;
-  // named by its number, the best form it has
-  const KwaveForm f = SPLIT || a.own_kernel ? kwave_any_form(DT, a.M, a.N, a.K, cus)
-                                            : kwave_tile_form(DT, a.M, a.N, a.K, cus);
-  return kwave_launch(DT, OUT, a, f, s);
+  return kwave_launch(DT, OUT, a, kwave_variant_form(SPLIT, DT, a.M, a.N, a.K, cus), s);
 }
 
 const char* check_tile(const astergemm_config& c) {
@@ -80,8 +77,10 @@ const char* check_tile(const astergemm_config& c) {
       AG_TILE(prefix "_128x128_w2x2", DT, 128, 128, 2, 2, 2),                    \
       AG_TILE(prefix "_128x64_w2x2", DT, 128, 64, 2, 2, 2),                      \
       AG_TILE(prefix "_64x64_w2x2", DT, 64, 64, 2, 2, 4)
-bool kwave_tile_any_describe(const astergemm_config& c, int cus, LaunchForm* o) {
-  return c.variant ? kwave_any_describe(c, cus, o) : kwave_tile_describe(c, cus, o);
+template <bool SPLIT>
+bool kwave_variant_describe(const astergemm_config& c, int cus, LaunchForm* o) {
+  kwave_describe(c.dtype_ab, kwave_variant_form(SPLIT, c.dtype_ab, c.M, c.N, c.K, cus), c.M, c.N, cus, o);
+  return true;
 }
 
 #define AG_KWAVE1(name, DT, OUT, SPLIT, RANK)                                    \
@@ -89,7 +88,7 @@ bool kwave_tile_any_describe(const astergemm_config& c, int cus, LaunchForm* o) 
     name, ASTERGEMM_KERNEL_TILE, DT, OUT, 64, 64, kRowBytes, 2, 4, 3, RANK,      \
         0, nullptr, launch_kwave_tile<DT, OUT, SPLIT>, check_tile,               \
         ASTERGEMM_OPERAND_LDS, nullptr, nullptr, 0,                              \
-        SPLIT ? kwave_any_describe : kwave_tile_any_describe                     \
+        kwave_variant_describe<SPLIT>                                            \
   }
 #define AG_KWAVE(name, DT, SPLIT, RANK)                                          \
   AG_KWAVE1(name "_bf16", DT, ASTERGEMM_BF16, SPLIT, RANK),                      \

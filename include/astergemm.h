@@ -151,7 +151,7 @@ typedef struct astergemm_config {
   int32_t waves_m;       /* num_waves_per_workgroup[M]                      */
   int32_t waves_n;       /* num_waves_per_workgroup[N]                      */
   int32_t variant;       /* explicit variant id from astergemm_variant_*,
-                            or 0                                             */
+                            astergemm_select or astergemm_tune, or 0         */
   int32_t operand_path;  /* astergemm_operand_path: how B (DIRECT_AB: and A)
                             is stored                                       */
   int32_t mx_a_layout;   /* astergemm_mx_layout: how A's e8m0 plane is stored
@@ -163,7 +163,9 @@ typedef struct astergemm_config {
  * parsing the generated asm (`parse_asm_kernel_resources`,
  * python/aster/compiler/metadata.py) and from cfg.num_workgroups/num_threads. */
 typedef struct astergemm_kernel_info {
-  int32_t variant;        /* id usable in astergemm_config.variant           */
+  int32_t variant;        /* id usable in astergemm_config.variant: a config
+                             that names it launches what is described here, and
+                             gives the same bits                             */
   int32_t family;
   int32_t grid_x;         /* 1-D grid, like every reference GEMM             */
   int32_t block_x;
@@ -175,7 +177,11 @@ typedef struct astergemm_kernel_info {
   int32_t pipeline_stages;
   int64_t flops;          /* 2*M*N*K                                         */
   int64_t bytes;          /* algorithmic bytes: A + B (+ scales) + C         */
-  char name[64];
+  char name[64];          /* of the selected variant.  Where AUTO runs another
+                             kernel in its place, or starts its K loops
+                             elsewhere, `variant` is the id of that form, which
+                             astergemm_variant_info names "..._auto_<output>",
+                             and the fields above describe it                */
 } astergemm_kernel_info;
 
 /* Device operands of one GEMM call. Unused pointers are NULL. */
@@ -218,9 +224,11 @@ const char* astergemm_last_error(void);
 /* ---- GEMM path ---------------------------------------------------------- */
 /* Replaces compile_fn: pick the kernel variant for cfg and describe it.     */
 int astergemm_select(const astergemm_config* cfg, astergemm_kernel_info* out);
-/* Number of built variants and a description of variant `index`
- * (0 <= index < count) instantiated for cfg's problem: what a config that names
- * it (cfg->variant = index + 1) launches, whatever cfg itself names.          */
+/* Number of variant ids and a description of id `index` + 1 (0 <= index < count)
+ * for cfg's problem: what a config that names it (cfg->variant = index + 1)
+ * launches, whatever cfg itself names.  First the built variants, each its own
+ * kernel; behind them, as "..._auto_<output>", what AUTO runs where it selects
+ * one of them and the two differ for some problems.                          */
 int astergemm_variant_count(void);
 int astergemm_variant_info(int index, const astergemm_config* cfg,
                            astergemm_kernel_info* out);
@@ -232,7 +240,8 @@ int astergemm_variant_info(int index, const astergemm_config* cfg,
  * (a graph may be replayed beside other work on the library's buffer), and always
  * through astergemm_run_noalloc.  The two add the same products in another order:
  * their fp32 sums differ in the last bits.  The same bits eagerly and under
- * capture: pass a workspace of that size, or name the kernel in cfg->variant.
+ * capture: pass a workspace of that size, or put the id that astergemm_select
+ * reports into cfg->variant.
  * Row-major MXFP4 scale planes may lie on any 8-byte boundary; off a 16-byte one
  * the general tile kernels run, also with other last bits.                    */
 int astergemm_run(const astergemm_config* cfg, const astergemm_operands* ops,
@@ -313,9 +322,10 @@ int astergemm_bench_rotate(const astergemm_config* cfg, const astergemm_operands
 int astergemm_bench_graph(const astergemm_config* cfg, const astergemm_operands* ops,
                           int n_ops, int launches, int replays, int64_t* total_ns);
 
-/* Measures every variant that can run cfg on the given operands (`iters`
+/* Measures every id that can run cfg on the given operands, AUTO's own forms
+ * among them, each as a config that names it launches it (`iters`
  * back-to-back launches between one event pair each, after two warm-up
- * launches) and returns the fastest: *best_variant is what cfg->variant takes
+ * launches), and returns the fastest: *best_variant is what cfg->variant takes
  * to pin it, *best_ns (may be NULL) its time per launch.  cfg->family
  * restricts the candidates when it is not AUTO; cfg->variant is ignored.  dC
  * is overwritten by every candidate.  This is the reference's sweep step

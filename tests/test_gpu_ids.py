@@ -1,5 +1,5 @@
-"""Variant ids and what runs under them: astergemm_variant_info describes what a plan of its id launches, and
-astergemm_tune times that."""
+"""Variant ids and what runs under them: a plan of the id that AUTO reports runs AUTO's kernel with AUTO's bits,
+astergemm_variant_info describes what a plan of its id launches, and astergemm_tune times that."""
 import ctypes
 import re
 
@@ -65,6 +65,22 @@ def test_every_id_is_described_as_a_plan_of_it_is(gpu, M, N, K, dtype):
         seen += 1
         assert facts(info) == facts(named.info)
     assert seen > 0
+
+
+@pytest.mark.parametrize("M,N,K,dtype", PROBLEMS)
+def test_a_plan_of_the_selected_id_is_the_selected_kernel(gpu, M, N, K, dtype):
+    """The same launch and the same bits, whatever AUTO runs in place of the kernel its variant is named for; the
+    name alone says that it is AUTO's form."""
+    import torch
+    auto = AG.GemmPlan.create(M, N, K, dtype, "f32")
+    named = AG.GemmPlan.create(M, N, K, dtype, "f32", variant=auto.info.variant)
+    a, n = facts(auto.info), facts(named.info)
+    stem, out = a.pop("name").decode().rsplit("_", 1)
+    assert n.pop("name").decode() in (f"{stem}_{out}", f"{stem}_auto_{out}") and a == n
+    assert auto.workspace_bytes() == named.workspace_bytes()
+    ptrs, kw, keep = device_operands(M, N, K, dtype)
+    want, got = bits(auto, ptrs, kw, M, N), bits(named, ptrs, kw, M, N)
+    assert bool((got == want).all()) and bool(want.view(torch.float32).isfinite().all())
 
 
 @pytest.mark.parametrize("M,N,K,dtype", PROBLEMS)

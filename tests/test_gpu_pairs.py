@@ -1,12 +1,12 @@
 """Two 128 x 128 tiles of a CU run as one of 256 x 128, and K loops that start at different steps on different
-XCDs: against the CPU oracle; the same bits on a second run, and from a plan of the variant the bits of the
-128 x 128 kernel."""
+XCDs: against the CPU oracle; the same bits on a second run and from a plan of the selected id; the kernel by its
+name has the bits of the 128 x 128 one."""
 import numpy as np
 import pytest
 
 from aster_amd import gemm as AG
 from oracle import gemm as G
-from test_gpu_parity import _DT, REL_L2_BAR, check, operands, run_gemm
+from test_gpu_parity import _DT, REL_L2_BAR, _variant_id, check, operands, run_gemm
 
 pytestmark = pytest.mark.gpu
 
@@ -30,10 +30,12 @@ def test_pairs_of_tiles(gpu, M, N, K, dtype_ab, dtype_c, tile):
     out, _ = run_gemm(a, b, M, N, K, dtype_ab, dtype_c, bias=bias, ldc=N + 8, **extra)
     again, _ = run_gemm(a, b, M, N, K, dtype_ab, dtype_c, bias=bias, ldc=N + 8, **extra)
     assert np.array_equal(out.view(np.uint8), again.view(np.uint8))
+    pinned, _ = run_gemm(a, b, M, N, K, dtype_ab, dtype_c, bias=bias, ldc=N + 8, variant=info.variant, **extra)
+    assert np.array_equal(out.view(np.uint8), pinned.view(np.uint8))
     want = G.gemm(a, b, _DT[dtype_ab], _DT[dtype_c], bias=bias, **extra)
     check(out, want, dtype_c, N, bar=(1e-4 if dtype_ab == "fp8_e4m3" else 1e-5) if dtype_c == "f32" else REL_L2_BAR)
-    if dtype_ab != "fp8_e4m3":  # by name the K loops start at step 0, pairs or not; by tile size there are no pairs
+    if dtype_ab != "fp8_e4m3":  # by name and by tile size: no pairs, and the K loops start at step 0
         named, square = (run_gemm(a, b, M, N, K, dtype_ab, dtype_c, bias=bias, ldc=N + 8, **how)[0]
-                         for how in (dict(variant=info.variant), dict(wg_tile=(128, 128))))
+                         for how in (dict(variant=_variant_id(info.name.decode())), dict(wg_tile=(128, 128))))
         assert np.array_equal(named.view(np.uint8), square.view(np.uint8))
         check(named, want, dtype_c, N, bar=1e-5 if dtype_c == "f32" else REL_L2_BAR)

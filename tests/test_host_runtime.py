@@ -270,6 +270,34 @@ def test_explicit_variant_and_enumeration():
     assert lib.astergemm_variant_info(n, ctypes.byref(c), ctypes.byref(info)) == -22
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f16", "fp8_e4m3", "mxfp4"])
+def test_the_selected_id_names_the_selected_kernel(dtype):
+    """A config with the id that a selection reports is accepted wherever the selection is, with the same launch
+    and workspace; a config that names a tile is reported the kernel of that tile, never AUTO's form of it."""
+    facts = lambda info: {f: getattr(info, f) for f, _ in info._fields_ if f != "name"}
+    forms, ks = 0, (4096, 14336, 11008, 256) + (() if dtype == "mxfp4" else (1032 if dtype != "fp8_e4m3" else 1040,))
+    for M in (1, 16, 33, 64, 65, 128, 333, 512, 777, 2048, 4100):
+        for N in (8, 300, 1001, 4096, 14336):
+            for K in ks:
+                for kw in ({}, dict(has_bias=True, lda=K + 256, ldb=K + 512, ldc=N + 3),
+                           dict(family=_capi.KERNEL_TILE)):
+                    auto = gemm.GemmPlan.create(M, N, K, dtype, "f32", **kw)
+                    named = gemm.GemmPlan.create(M, N, K, dtype, "f32", variant=auto.info.variant, **kw)
+                    assert facts(auto.info) == facts(named.info), (M, N, K, kw)
+                    assert auto.workspace_bytes() == named.workspace_bytes()
+                    stem, out = auto.info.name.decode().rsplit("_", 1)
+                    form = named.info.name.decode() == f"{stem}_auto_{out}"
+                    assert form or named.info.name == auto.info.name
+                    forms += form
+                try:
+                    tile = gemm.GemmPlan.create(M, N, K, dtype, "f32", wg_tile=(128, 128))
+                except _capi.AsterGemmError:
+                    continue
+                named = gemm.GemmPlan.create(M, N, K, dtype, "f32", variant=tile.info.variant)
+                assert named.info.name == tile.info.name and "_auto_" not in named.info.name.decode()
+    assert forms > 100
+
+
 @pytest.mark.parametrize("kw,msg", [
     (dict(M=128, N=128, K=0), "K > 0"),
     (dict(M=-1, N=128, K=64), ">= 0"),
