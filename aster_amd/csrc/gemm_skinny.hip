@@ -764,6 +764,7 @@ void launch_splitk_reduce(const GemmArgs& a, int S, hipStream_t s) {
 struct SplitWorkspace {
   float* ptr = nullptr;
   size_t bytes = 0;
+  size_t refused = 0;  // smallest size workspace_touch could not get (0: none)
 };
 std::mutex g_ws_mutex;
 std::map<std::pair<int, hipStream_t>, SplitWorkspace> g_ws;
@@ -782,13 +783,15 @@ int splitk_workspace(size_t bytes, hipStream_t stream, float** out) {
     if (w.ptr) g_ws_retired.push_back(w.ptr);
     w.ptr = fresh;
     w.bytes = want;
+    w.refused = 0;
   }
   *out = w.ptr;
   return 0;
 }
 
 // For a problem that is cut into K ranges by one kernel and not by the one that runs: the stream's buffer is
-// as large as if it had been, so that a later capture of another problem finds it.  Never inside a capture.
+// as large as if it had been, so that a later capture of another problem finds it.  Never inside a capture.  A
+// size that the device had no memory for is not asked for again on every call: the running kernel needs none.
 void workspace_touch(size_t bytes, hipStream_t stream) {
   int dev = 0;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
@@ -796,12 +799,20 @@ void workspace_touch(size_t bytes, hipStream_t stream) {
   {
     std::lock_guard<std::mutex> lock(g_ws_mutex);
     auto it = g_ws.find({dev, stream});
-    if (it != g_ws.end() && it->second.bytes >= bytes) return;
+    if (it != g_ws.end() &&
+        (it->second.bytes >= bytes || (it->second.refused && bytes >= it->second.refused)))
+      return;
   }
   if ((stream && hipStreamIsCapturing(stream, &st) != hipSuccess) || st != hipStreamCaptureStatusNone)
     return (void)hipGetLastError();
   float* unused = nullptr;
-  if (splitk_workspace(bytes, stream, &unused) != 0) (void)hipGetLastError();
+  const int rc = splitk_workspace(bytes, stream, &unused);
+  if (rc == 0) return;
+  (void)hipGetLastError();
+  if (rc != (int)hipErrorOutOfMemory) return;
+  std::lock_guard<std::mutex> lock(g_ws_mutex);
+  size_t& refused = g_ws[{dev, stream}].refused;
+  if (!refused || bytes < refused) refused = bytes;
 }
 
 // Gives back the workspace of a stream that is about to be destroyed.  The caller has
