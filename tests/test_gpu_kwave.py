@@ -5,9 +5,23 @@ import pytest
 
 from aster_amd import _capi, gemm as AG
 from oracle import formats as F, gemm as G
+from test_gpu_ids import PROBLEMS, device_operands
 from test_gpu_parity import _DT, REL_L2_BAR, check, operands, run_gemm
 
 pytestmark = pytest.mark.gpu
+
+
+# waves over a tile's rows and columns: the others of a workgroup share K
+_TILE_WAVES = {(16, 16): 1, (16, 32): 1, (16, 48): 1, (16, 64): 1, (32, 16): 2, (32, 32): 2, (32, 64): 2, (32, 128): 4,
+               (64, 32): 2, (64, 48): 2, (64, 64): 4, (64, 128): 4, (96, 64): 4, (128, 64): 4, (128, 128): 8}
+
+
+def ring_bytes(info, dtype_ab):
+    """LDS of the kernel that splits K over waves: the ring of every wave group.  The kernels it stands in for have
+    other sizes (resident activations 128 KiB, 128 x 128 tiles 80 or 144 KiB in rings of whole tiles)."""
+    tile = (info.wg_tile_m, info.wg_tile_n)
+    scales = (sum(tile) + 31) // 32 * 256 if dtype_ab == "mxfp4" else 0
+    return info.pipeline_stages * (info.block_x // 64 // _TILE_WAVES[tile]) * (sum(tile) * 128 + scales)
 
 
 @pytest.mark.parametrize("M,N,K,dtype_ab,tile", [
@@ -48,6 +62,7 @@ def test_k_over_waves(gpu, M, N, K, dtype_ab, dtype_c, tile):
     bias = np.random.default_rng(N).standard_normal(N).astype(np.float32)
     info = AG.GemmPlan.create(M, N, K, dtype_ab, dtype_c, has_bias=True).info
     assert (info.wg_tile_m, info.wg_tile_n) == tile, (info.name, info.wg_tile_m, info.wg_tile_n)
+    assert info.lds_bytes == ring_bytes(info, dtype_ab)
     out, _ = run_gemm(a, b, M, N, K, dtype_ab, dtype_c, bias=bias, ldc=N + 3, **extra)
     want = G.gemm(a, b, _DT[dtype_ab], _DT[dtype_c], bias=bias, **extra)
     f32_bar = 1e-4 if dtype_ab == "fp8_e4m3" else 1e-5
@@ -109,3 +124,32 @@ def test_a_named_tile_keeps_the_kernels_it_had():
     for (M, N, K), wg in (((300, 300, 2048), (64, 64)), ((16, 4096, 4096), (16, 16))):
         info = AG.GemmPlan.create(M, N, K, "bf16", "bf16", wg_tile=wg).info
         assert (info.wg_tile_m, info.wg_tile_n) == wg and b"kwave" not in info.name
+    assert info.lds_bytes == 128 * 1024 != ring_bytes(info, "bf16")      # resident activations
+
+
+@pytest.mark.parametrize("dtype_c", ["f16", "bf16", "f32"])
+@pytest.mark.parametrize("M,N,K,dtype_ab", PROBLEMS + [(100, 100, 520, "bf16"), (70, 1000, 2064, "fp8_e4m3"),
+                                                       (1000, 4096, 2080, "f16"), (1000, 7048, 1032, "bf16")])
+def test_row_pitches_above_k(gpu, M, N, K, dtype_ab, dtype_c):
+    """A and B with pitches of their own, the gaps full of NaN codes (MXFP4: -6): the bits of packed
+    operands, and nothing written past column N."""
+    import torch
+    (pa, pb), kw, keep = device_operands(M, N, K, dtype_ab)
+    per = {"mxfp4": 2, "fp8_e4m3": 1}.get(dtype_ab, 0.5)          # elements of a byte
+    row = int(K / per)
+    wide = [torch.full((r, row + pad), 0xFF, dtype=torch.uint8, device="cuda") for r, pad in ((M, 16), (N, 144))]
+    for w, t in zip(wide, keep):
+        w[:, :row] = t.view(torch.uint8)
+    ldc, out = N + (3 if M <= 64 else 8), {"f16": torch.float16, "bf16": torch.bfloat16, "f32": torch.float32}[dtype_c]
+    lda, ldb = K + int(16 * per), K + int(144 * per)
+    packed = AG.GemmPlan.create(M, N, K, dtype_ab, dtype_c, ldc=ldc)
+    padded = AG.GemmPlan.create(M, N, K, dtype_ab, dtype_c, lda=lda, ldb=ldb, ldc=ldc)
+    want, got = (torch.full((M, ldc), float("nan"), dtype=out, device="cuda") for _ in range(2))
+    torch.cuda.synchronize()
+    print(f"{padded.info.name.decode()} M={M} N={N} K={K}", flush=True)
+    packed.run(pa, pb, want.data_ptr(), **kw)
+    padded.run(wide[0].data_ptr(), wide[1].data_ptr(), got.data_ptr(), **kw)
+    torch.cuda.synchronize()
+    assert padded.info.variant == packed.info.variant
+    assert torch.equal(got[:, :N], want[:, :N]) and bool(torch.isfinite(want[:, :N]).all())
+    assert bool(torch.isnan(got[:, N:]).all())

@@ -139,13 +139,14 @@ def test_a_workspace_of_the_stated_size_gives_the_eager_bits_under_capture(gpu, 
             torch.cuda.synchronize()
 
 
-def test_caller_workspace_matches_the_library_workspace(gpu):
-    M, N, K = 96, 1000, 16384
+@pytest.mark.parametrize("M,N,K", [(96, 1000, 16384),      # one launch: K over waves, the workspace left unused
+                                   (128, 4096, 14336)])    # 128 x 128 tiles in eight K ranges
+def test_caller_workspace_matches_the_library_workspace(gpu, M, N, K):
     rng = np.random.default_rng(11)
     a, b = _bf16(rng, (M, K), 1.0), _bf16(rng, (N, K), 0.02)
     plan = AG.GemmPlan.create(M, N, K, "bf16", "bf16")
     need = plan.workspace_bytes()
-    assert need > 0
+    assert need > 0 and ((plan.info.wg_tile_m, plan.info.wg_tile_n) == (128, 128)) == (N == 4096)
     bufs = [GpuBuffer(a.nbytes), GpuBuffer(b.nbytes), GpuBuffer(M * N * 2), GpuBuffer(need)]
     bufs[0].copy_from_host(a)
     bufs[1].copy_from_host(b)
@@ -161,6 +162,58 @@ def test_caller_workspace_matches_the_library_workspace(gpu):
                  workspace=bufs[3].ptr_value, workspace_bytes=need - 4)
     for bf in bufs:
         bf.free()
+
+
+@pytest.mark.parametrize("M,N,K,dtype,kernel,planes", [
+    # AUTO: K over waves in fewer ranges than the kernel it stands in for, whose planes the workspace is sized for
+    (64, 4096, 14336, "bf16", None, 4), (29, 4100, 11008, "f16", None, 3), (64, 8192, 28672, "fp8_e4m3", None, 2),
+    # by name: the kernels with K ranges themselves
+    (96, 1000, 16384, "bf16", "splitk_bf16_128x128_w2x2_bf16", 0), (128, 1024, 8192, "f16", "splitk_f16_128x128_w2x2_bf16", 0),
+    (50, 1032, 28672, "bf16", "skinnyx_bf16_m64_bf16", 0), (16, 4096, 14336, "fp8_e4m3", "skinnyx_fp8_m64_bf16", 0)])
+def test_partial_sums_go_to_the_memory_of_the_call(gpu, M, N, K, dtype, kernel, planes):
+    """The library's buffer, a caller's, the built-in scratch, each eagerly and captured (several replays with eager
+    work between): the same bits; of a caller's buffer the planes are written and nothing else."""
+    import torch
+    from test_gpu_ids import device_operands
+    from test_gpu_parity import _variant_id
+    plan = AG.GemmPlan.create(M, N, K, dtype, "bf16", variant=_variant_id(kernel) if kernel else 0)
+    need, own = plan.workspace_bytes(), planes or plan.workspace_bytes() // (4 * M * N)
+    assert (planes or 2) * 4 * M * N <= need <= _capi.NOALLOC_SCRATCH_BYTES
+    (pa, pb), kw, keep = device_operands(M, N, K, dtype)
+    want, got = (torch.zeros(M, N, device="cuda", dtype=torch.bfloat16) for _ in range(2))
+    ws = torch.full((need // 4 + 64,), float("nan"), device="cuda")
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    print(f"{plan.info.name.decode()} M={M} N={N} K={K}", flush=True)
+    plan.run(pa, pb, want.data_ptr(), stream=stream.cuda_stream, **kw)
+    stream.synchronize()
+    ref = keep[0].float() @ keep[1].float().T * (0.125 if dtype == "fp8_e4m3" else 1.0)
+    assert float((want.float() - ref).norm() / ref.norm()) <= 4e-3   # bf16 rounding, 1.7e-3, and the sums' order
+    small = dict(workspace=ws.data_ptr(), workspace_bytes=need - 4)
+    with pytest.raises(_capi.AsterGemmError, match="workspace of"):
+        plan.run(pa, pb, got.data_ptr(), **kw, **small)
+    for call, extra in ((plan.run, {}), (plan.run, dict(workspace=ws.data_ptr(), workspace_bytes=need)),
+                        (plan.run_noalloc, {})):
+        ws.fill_(float("nan"))
+        got.zero_()
+        torch.cuda.synchronize()
+        call(pa, pb, got.data_ptr(), stream=stream.cuda_stream, **kw, **extra)
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+        written = ~torch.isnan(ws)
+        assert int(written.sum()) == (own * M * N if extra else 0) and (not extra or bool(written[:own * M * N].all()))
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            call(pa, pb, got.data_ptr(), stream=stream.cuda_stream, **kw, **extra)
+        for _ in range(3):
+            got.zero_()
+            torch.cuda.synchronize()
+            with torch.cuda.stream(stream):
+                graph.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(got, want)
+            plan.run(pa, pb, want.data_ptr(), stream=stream.cuda_stream, **kw)
+            torch.cuda.synchronize()
 
 
 def test_an_eager_split_call_readies_its_stream_for_a_capture_of_the_same_config(gpu):
@@ -210,7 +263,8 @@ def test_an_eager_split_call_readies_its_stream_for_a_capture_of_the_same_config
 @pytest.mark.parametrize("M,N,K,dtype,kernel", [
     (128, 1024, 8192, "bf16", "splitk_bf16_128x128_w2x2_bf16"),
     (129, 1032, 8192, "bf16", "splitk_bf16_256x128_w4x2_bf16"),
-    (50, 1032, 28672, "bf16", "skinnyx_bf16_m64_bf16"), (16, 520, 14336, "mxfp4", "skinnyx_mxfp4_m64_bf16")])
+    (50, 1032, 28672, "bf16", "skinnyx_bf16_m64_bf16"), (16, 520, 14336, "mxfp4", "skinnyx_mxfp4_m64_bf16"),
+    (64, 2048, 14336, "bf16", None), (64, 4096, 14336, "bf16", None)])    # AUTO: K over waves in four ranges
 def test_two_host_threads_on_one_stream_keep_products_and_sums_in_pairs(gpu, M, N, K, dtype, kernel):
     """Split K and the K ranges of the decode kernels: two threads enqueue different activations on one
     stream and share the partial sums' memory (the library's buffer, the built-in scratch, a caller's
@@ -233,7 +287,10 @@ def test_two_host_threads_on_one_stream_keep_products_and_sums_in_pairs(gpu, M, 
         _capi.check(lib.astergemm_variant_info(i, ctypes.byref(plan.config), ctypes.byref(info)))
         if info.name.decode() == kernel:
             plan = AG.GemmPlan.create(M, N, K, dtype, "bf16", variant=info.variant)
-    assert plan.info.name.decode() == kernel
+    if kernel is None:
+        assert (plan.info.wg_tile_m, plan.info.wg_tile_n) == (64, 64) and plan.info.grid_x == N // 64 * 4
+    else:
+        assert plan.info.name.decode() == kernel
     need = plan.workspace_bytes()
     assert 0 < need <= _capi.NOALLOC_SCRATCH_BYTES
     own = torch.zeros(need, device="cuda", dtype=torch.uint8)
