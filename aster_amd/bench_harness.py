@@ -343,7 +343,7 @@ def bench_perf_sweep(configs, compile_fn, execute_fn, repro_cmd_fn=None, *, mcpu
             failed.append((cfg, f"compile: {str(exc).splitlines()[0][:200]}"))
             continue
         selected[f"{cfg.label}|{cfg.mapping.operand_path.value}"] = desc["kernel"]
-        key = (desc["kernel"], tuple(cfg.spec.gemm_size))
+        key = (desc.get("launches", desc["kernel"]), tuple(cfg.spec.gemm_size))
         groups.setdefault(key, []).append((cfg, path, desc))
     print(f"Sweep: {len(configs)} configs -> {len(groups)} distinct kernels, "
           f"{len(failed)} refused, {iterations} iterations each", file=out)
@@ -351,10 +351,11 @@ def bench_perf_sweep(configs, compile_fn, execute_fn, repro_cmd_fn=None, *, mcpu
     have_gpu = system_has_gpu(mcpu)
     if not have_gpu:
         print("No GPUs detected -- execution skipped.", file=out)
-    for (kernel, size), members in (groups.items() if have_gpu else ()):
+    for (launched, size), members in (groups.items() if have_gpu else ()):
         # the mapping the kernel honours stands for the group; the others ran the same code
         members.sort(key=lambda m: not m[2].get("mapping_honoured", False))
         cfg, path, desc = members[0]
+        kernel = desc["kernel"]
         try:
             A, B = make_inputs(cfg, init_mode)
             _, times_ns = execute_fn(cfg, path, iterations, A, B, skip_gpu_check=True)
@@ -374,7 +375,7 @@ def bench_perf_sweep(configs, compile_fn, execute_fn, repro_cmd_fn=None, *, mcpu
             with open(results_file, "a") as rs:
                 emit_one_result(rs, bench, cfg, s, label=label)
         aliases = [m[0].label for m in members[1:]]
-        print(f"  {s.p50_tf:8.1f} TF p50 ({s.p50_pct:5.1f} % peak)  {kernel}  <- {label}"
+        print(f"  {s.p50_tf:8.1f} TF p50 ({s.p50_pct:5.1f} % peak)  {launched}  <- {label}"
               + (f"  (+{len(aliases)} mappings that select the same kernel)" if aliases else ""), file=out)
     results.sort(key=lambda r: -r[1].p50_tf)
     for cfg, why in failed:

@@ -67,6 +67,14 @@ def select(c: _capi.Config) -> _capi.KernelInfo:
     return info
 
 
+def launched_kernel(c: _capi.Config, info: _capi.KernelInfo) -> str:
+    """The name of what the selection `info` of `c` launches: `info.name`, or where AUTO runs another kernel
+    than the one it names, the name of that form ("..._auto_<output>")."""
+    named = _capi.KernelInfo()
+    _capi.check(_capi.load().astergemm_variant_info(info.variant - 1, ctypes.byref(c), ctypes.byref(named)))
+    return named.name.decode()
+
+
 @dataclass
 class MappingReport:
     """How much of a GemmMappingSpec the selected pre-built kernel follows.
@@ -153,7 +161,9 @@ def compile_gemm(cfg: WeakScaledMappedGemmInstance, output_hsaco_path: str, **kw
     The descriptor and the summary say whether the mapping was honoured
     (`mapping_honoured`, `mapping_not_honoured`) and which of its knobs cannot
     change a pre-built kernel (`mapping_fixed_by_kernel`), so that a sweep over
-    mappings can tell labels that ran the same kernel apart from real variants.
+    mappings can tell labels that ran the same kernel apart from real variants:
+    `launches` names what runs, which for a selection of the library's own may
+    be another form of `kernel`.
     """
     c, info = select_for_instance(cfg)
     rep = mapping_report(cfg, c, info)
@@ -161,6 +171,7 @@ def compile_gemm(cfg: WeakScaledMappedGemmInstance, output_hsaco_path: str, **kw
         "format": "astergemm-descriptor-v1",
         "label": cfg.label,
         "kernel": info.name.decode(),
+        "launches": launched_kernel(c, info),
         "variant": info.variant,
         "grid": info.grid_x,
         "block": info.block_x,

@@ -346,6 +346,30 @@ def test_compile_gemm_writes_descriptor(tmp_path):
         gemm._read_descriptor(str(tmp_path / "bad.hsaco"))
 
 
+def test_a_sweep_times_a_named_tile_and_what_auto_runs_under_its_name():
+    """2048 x 4096 x 4096: 128 x 128 tiles by their mapping, and the library's selection for a mapping that no
+    kernel has, which keeps that kernel's name and launches another form."""
+    import io
+
+    from aster_amd import bench_harness as BH
+    cfgs = [make_instance(2048, 4096, 4096, wg_tile=t, waves=w)
+            for t, w in (((128, 128), (2, 2)), ((128, 256), (1, 4)), ((64, 256), (1, 4)))]
+    descs, out = [], io.StringIO()
+
+    def compile_fn(cfg, path):
+        gemm.compile_gemm(cfg, path)
+        descs.append(gemm._read_descriptor(path))
+
+    def execute_fn(cfg, path, iterations, A, B, skip_gpu_check):
+        raise RuntimeError("not timed here")
+
+    _, selected = BH.bench_perf_sweep(cfgs, compile_fn, execute_fn, None, bench="t", out=out)
+    name = "stream_bf16_128x128_w2x2_bf16"
+    assert set(selected.values()) == {name} and [d["mapping_honoured"] for d in descs] == [True, False, False]
+    assert [d["launches"] for d in descs] == [name] + ["stream_bf16_128x128_w2x2_auto_bf16"] * 2
+    assert "3 configs -> 2 distinct kernels" in out.getvalue()
+
+
 def test_a_descriptor_of_another_selection_runs_the_kernel_it_names(tmp_path):
     """1536 x 4096 x 4096 with a mapping no kernel has: 192 x 128 tiles are selected; a descriptor that was
     written when the 128 x 128 kernel was gets that kernel.  Another instance's descriptor is refused."""
