@@ -22,7 +22,7 @@ KwaveForm kwave_small_decode_form(int dt, int64_t M, int64_t N, int64_t K, int c
 // 64 < M <= 512 against at most about a round of panels, as part of the launchers of 128 x 128 tiles.
 KwaveForm kwave_prompt_form(int dt, int64_t M, int64_t N, int64_t K, int cus);
 // Any M and N: the smallest tile that leaves at most one workgroup per CU, else (and without a device) 64 x 64.
-KwaveForm kwave_tile_form(int dt, int64_t M, int64_t N, int64_t K, int cus);
+KwaveForm kwave_tile_form(int64_t M, int64_t N, int cus);
 // Small products that AUTO takes the tile form for, where it takes the general tile kernels otherwise.
 bool kwave_small_product(int dt, int64_t M, int64_t N, int64_t K, int cus);
 // What the variants of these kernels run, by AUTO or by name: the tile form for small products (split: never),

@@ -125,6 +125,8 @@ int kwave_blocks(int tiles_m, int tiles_n, int cus, int* by_panel) {
 //   fp4 16  4.8 / 4.6       resident     resident     10.9 / 7.4   14.6 / 7.4   10.2 / 7.9   5.9 / 4.7
 //   fp4 64  6.5 / 5.4       resident     resident     16.9 / 11.0  17.0 / 9.1   14.5 / 10.9  8.6 / 4.8
 // (fp8 and MXFP4 4096x11008, no whole 512 bytes: against the tile kernels.)
+// The byte limits are what one of 256 CUs reads in the time the other side's extra launch or planes take on this
+// chip: another CU count moves `per` with it, the limits were measured at this one only.
 KwaveForm kwave_decode_form(int dt, int64_t M, int64_t N, int64_t K, int cus, int max_ranges) {
   KwaveForm f;
   const int64_t rb = row_bytes(dt, K);
@@ -209,7 +211,8 @@ KwaveForm fewest_rows(int64_t M, int64_t N, int cus, int* rows) {
 //   fp8 128    11.0 / 7.9      -            -            21.7 / 19.5  34.2 / 29.8
 //   MXFP4 128  13.8 / 6.8      14.6 / 12.5  14.4 / 11.7  17.1 / 13.5  15.6 / 17.7
 //   MXFP4 256  14.1 / 8.3      15.1 / 17.3  14.6 / 16.7  23.2 / 19.8  21.3 / 32.3
-// The lines: operand rows per CU times their bytes, against tiles that read 256 rows or split K further
+// The lines, measured on 256 CUs: operand rows per CU times their bytes, against tiles that read 256 rows or
+// split K further
 // (bf16 128x4096x14336, 2.8 MB here: 37.4 / 50.0; fp8 200x4096x14336 24.8 / 30.2; MXFP4 333x8192x8192 24.3 / 26.8).
 KwaveForm kwave_prompt_form(int dt, int64_t M, int64_t N, int64_t K, int cus) {
   const int64_t rb = row_bytes(dt, K);
@@ -229,8 +232,7 @@ KwaveForm kwave_prompt_form(int dt, int64_t M, int64_t N, int64_t K, int cus) {
 // 500x500x1024 6.7 / 4.6, 207x28x1440 8.0 / 3.9 (16 x 16), 600x600x2056 12.2 / 10.1 (32 x 64), 600x600x4104
 // 21.0 / 17.2, 2000x200x1032 7.5 / 7.1; fp8 300x300x4096 11.1 / 6.4, 600x600x4096 11.3 / 9.2.  The 64 x 64 form is
 // for configs that name the kernel.
-KwaveForm kwave_tile_form(int dt, int64_t M, int64_t N, int64_t K, int cus) {
-  (void)dt, (void)K;
+KwaveForm kwave_tile_form(int64_t M, int64_t N, int cus) {
   static const struct { int shape, bm, bn; } kOrder[] = {{0, 16, 16}, {6, 32, 32}, {7, 32, 64}};
   KwaveForm f;
   f.shape = 11;
@@ -254,10 +256,10 @@ bool kwave_small_product(int dt, int64_t M, int64_t N, int64_t K, int cus) {
 }
 
 KwaveForm kwave_variant_form(bool split, int dt, int64_t M, int64_t N, int64_t K, int cus) {
-  if (!split && kwave_small_product(dt, M, N, K, cus)) return kwave_tile_form(dt, M, N, K, cus);
+  if (!split && kwave_small_product(dt, M, N, K, cus)) return kwave_tile_form(M, N, cus);
   KwaveForm f = kwave_decode_form(dt, M, N, K, cus, 1);
   if (!f) f = kwave_prompt_form(dt, M, N, K, cus);
-  return f ? f : kwave_tile_form(dt, M, N, K, cus);
+  return f ? f : kwave_tile_form(M, N, cus);
 }
 
 int kwave_ready(int dt) {

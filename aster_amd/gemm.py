@@ -328,7 +328,8 @@ class GemmPlan:
     def tune(self, dA: int, dB: int, dC: int, iters: int = 10, *, scale_a: int = None,
              scale_b: int = None, mx_a: int = None, mx_b: int = None, bias: int = None,
              stream: int = None) -> "GemmPlan":
-        """Times every variant that can run this plan's problem on the given operands and
+        """Times every id that can run this plan's problem on the given operands, what the library
+        would choose among them, each as a plan of it launches it, and
         returns a plan pinned to the fastest (`plan.tuned_ns` = its time per launch).  dC is
         overwritten by every candidate."""
         ops = self._operands(dA, dB, dC, scale_a, scale_b, mx_a, mx_b, bias)
