@@ -772,8 +772,9 @@ int index_of(const Variant& v) {
 // A config with an optional split has two kernels: an eager launch of one readies the other, so that a
 // later capture finds either of them ready.  (The stream's workspace is: the kernel a capture runs has no
 // more K ranges than the split it stands in for, by the lines of unequal_split_pays.)  Once per launcher
-// and device (a launcher with several kernels readies all of them, whichever the config runs); done on every call it cost such a
-// call 0.5-0.7 of 8.3 us of host time.  A failure is that later launch's to report, not the call's that has just succeeded.
+// and device (a launcher with several kernels readies all of them, whichever the config runs); done on every
+// call it cost such a call 0.5-0.7 of 8.3 us of host time.  A failure is that later launch's to report, not the
+// call's that has just succeeded.
 void ready_other(const Variant* other, const astergemm_config& c, void* stream) {
   if (!other) return;
   static std::vector<std::atomic<uint64_t>> ready((size_t)total_variants());

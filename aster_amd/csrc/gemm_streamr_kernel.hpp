@@ -16,9 +16,9 @@
 // places and must be equal, a stage is refilled as a whole: when K-step k is in registers its stage
 // is requested for K-step k + NS, so NS - 1 K-steps are on their way at any time.  Swizzle, staging
 // plan, fragment order and epilogue are those of gemm_stream_body.  As AUTO runs it the K loops of different XCDs
-// start at different steps (first_step_of_xcd), by name at step 0 with the bits of gemm_stream_body: bf16 333x14336x4096 50.5 -> 47.9 us, 1400x4096x14336 161 -> 144,
-// 333x4096x14336 (split K) 63.1 -> 58.3, 136x28672x4096 59.7 -> 52.3, fp8 200x28672x4096 44.5 -> 40.9; on
-// buffers that no kernel has read yet as much.
+// start at different steps (first_step_of_xcd), by name at step 0 with the bits of gemm_stream_body: bf16
+// 333x14336x4096 50.5 -> 47.9 us, 1400x4096x14336 161 -> 144, 333x4096x14336 (split K) 63.1 -> 58.3, 136x28672x4096
+// 59.7 -> 52.3, fp8 200x28672x4096 44.5 -> 40.9; on buffers that no kernel has read yet as much.
 #pragma once
 #include "gemm_stream_kernel.hpp"
 

@@ -168,7 +168,8 @@ def test_caller_workspace_matches_the_library_workspace(gpu, M, N, K):
     # AUTO: K over waves in fewer ranges than the kernel it stands in for, whose planes the workspace is sized for
     (64, 4096, 14336, "bf16", None, 4), (29, 4100, 11008, "f16", None, 3), (64, 8192, 28672, "fp8_e4m3", None, 2),
     # by name: the kernels with K ranges themselves
-    (96, 1000, 16384, "bf16", "splitk_bf16_128x128_w2x2_bf16", 0), (128, 1024, 8192, "f16", "splitk_f16_128x128_w2x2_bf16", 0),
+    (96, 1000, 16384, "bf16", "splitk_bf16_128x128_w2x2_bf16", 0),
+    (128, 1024, 8192, "f16", "splitk_f16_128x128_w2x2_bf16", 0),
     (50, 1032, 28672, "bf16", "skinnyx_bf16_m64_bf16", 0), (16, 4096, 14336, "fp8_e4m3", "skinnyx_fp8_m64_bf16", 0)])
 def test_partial_sums_go_to_the_memory_of_the_call(gpu, M, N, K, dtype, kernel, planes):
     """The library's buffer, a caller's, the built-in scratch, each eagerly and captured (several replays with eager
