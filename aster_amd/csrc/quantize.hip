@@ -140,8 +140,11 @@ __device__ __forceinline__ unsigned block_max(unsigned m) {
 }
 
 // This thread's share of max |src[0..n)|: groups first, first + stride, ..., U loads in flight,
-// and the elements behind the last whole group.
-template <int SRC, int U>
+// and the elements behind the last whole group.  BATCHED: what is left of less than U groups is requested together
+// too (one by one each waits for the one before: bf16 500 x 4096 10.8 -> 9.9 us for the two launches, 333 x 4096
+// 9.7 -> 8.7); a workgroup that reads the whole of a small tensor has U groups or few (16 x 4096 3.56 against
+// 3.62 us) and does without.
+template <int SRC, int U, bool BATCHED>
 __device__ __forceinline__ unsigned absmax_share(const void* __restrict__ src, int64_t n, int64_t first,
                                                  int64_t stride) {
   constexpr int NE = Src<SRC>::kPer;
@@ -156,7 +159,18 @@ __device__ __forceinline__ unsigned absmax_share(const void* __restrict__ src, i
 #pragma unroll
     for (int u = 0; u < U; ++u) am.fold(v[u]);
   }
-  for (; i < ng; i += stride) am.fold(g[i]);
+  if constexpr (!BATCHED) {
+    for (; i < ng; i += stride) am.fold(g[i]);
+  } else if (i < ng) {
+    i32x4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      v[u] = i32x4{0, 0, 0, 0};
+      if (i + u * stride < ng) v[u] = g[i + u * stride];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) am.fold(v[u]);
+  }
   unsigned m = am.bits();
   for (int64_t j = ng * NE + first; j < n; j += stride) {
     const unsigned b = __float_as_uint(load1<SRC>(src, j)) & 0x7FFFFFFFu;
@@ -170,7 +184,7 @@ __device__ __forceinline__ unsigned absmax_share(const void* __restrict__ src, i
 template <int SRC>
 __global__ __launch_bounds__(1024) void absmax_kernel(const void* __restrict__ src, int64_t n,
                                                       unsigned* __restrict__ out) {
-  const unsigned m = block_max<16>(absmax_share<SRC, 4>(
+  const unsigned m = block_max<16>(absmax_share<SRC, 4, false>(
       src, n, blockIdx.x * (int64_t)1024 + threadIdx.x, (int64_t)gridDim.x * 1024));
   if (threadIdx.x == 0 && m != 0) atomicMax(out, m);
 }
@@ -239,7 +253,7 @@ __global__ __launch_bounds__(1024) void quantize_fp8_small_kernel(const void* __
   const int i = blockIdx.x * 1024 + threadIdx.x;
   i32x4 mine = {0, 0, 0, 0};
   if (i < ng) mine = ((const i32x4*)src)[i];
-  const Fp8Scale sc(block_max<16>(absmax_share<SRC, 8>(src, n, threadIdx.x, 1024)));
+  const Fp8Scale sc(block_max<16>(absmax_share<SRC, 8, false>(src, n, threadIdx.x, 1024)));
   if (i == 0) *scale = sc.s;
   if (i < ng) fp8_store_group<SRC>(mine, i, sc, dst);
   if (blockIdx.x == 0)
@@ -250,13 +264,17 @@ __global__ __launch_bounds__(1024) void quantize_fp8_small_kernel(const void* __
 // (clear, absmax, scale, encode): bf16 500 x 14336 37.4 -> 13.4 us, 4096 x 4096 47.8 -> 19.4, 8192 x
 // 8192 97.4 -> 62.4 (the source is read twice, the second time from the last-level cache; 40 us at
 // the rate of a large copy).  The first leaves one maximum per workgroup in the first 4 * gridDim.x bytes
-// of dst (written over by the codes in the end) and clears *scale, which the second uses as a
-// counter.
+// of dst (written over by the codes in the end) and clears the counters of the second: *scale, and
+// kFp8Counters of them behind the partial maxima.
+constexpr int kFp8Counters = 16, kFp8CounterPitch = 32;  // a counter every 128 bytes of dst
+constexpr int kFp8CounterBytes = kFp8Counters * kFp8CounterPitch * 4;
+
 template <int SRC>
 __global__ __launch_bounds__(256) void fp8_absmax_kernel(const void* __restrict__ src, int64_t n,
                                                          unsigned* __restrict__ partial,
                                                          unsigned* __restrict__ counter) {
-  const unsigned m = block_max<4>(absmax_share<SRC, 8>(
+  if (blockIdx.x == 0 && threadIdx.x < kFp8Counters) partial[gridDim.x + threadIdx.x * kFp8CounterPitch] = 0u;
+  const unsigned m = block_max<4>(absmax_share<SRC, 8, true>(
       src, n, blockIdx.x * (int64_t)256 + threadIdx.x, (int64_t)gridDim.x * 256));
   if (threadIdx.x == 0) {
     partial[blockIdx.x] = m;
@@ -265,18 +283,22 @@ __global__ __launch_bounds__(256) void fp8_absmax_kernel(const void* __restrict_
 }
 
 // Every workgroup takes the maximum of the `np` partial ones, counts itself in and encodes its
-// part of the tensor behind the first 4 * np elements; the last one to have counted itself in --
-// everybody has read the partial maxima by then -- encodes those and stores the scale over the
-// counter.  Nobody waits for anybody.  256 workgroups at most: the counter's atomics are taken
-// one at a time (2048 workgroups of 256 threads: 34.7 us instead of 13.4 on 500 x 14336).
+// part of the tensor behind the place of the partial maxima and counters; the last one to have counted itself
+// in -- everybody has read the partial maxima by then -- encodes that place and stores the scale over
+// the counter there.  Nobody waits for anybody.  Atomics on one address are taken one at a time (one counter for 256
+// workgroups kept the kernel 1.3 us longer than its bytes: bf16 500 x 4096 10.8 -> 8.0 us for the two launches,
+// 500 x 14336 13.5 -> 12.4, 4096 x 4096 20.8 -> 19.5), so past 64 workgroups each adds to one of 16 counters, a line
+// of dst apart, and the last of each of them to the one in *scale; up to 64 one counter is level or ahead (64 x 4096
+// 6.1 against 6.3).
 template <int SRC>
 __global__ __launch_bounds__(1024) void quantize_fp8_kernel(const void* __restrict__ src, int64_t n, int np,
                                                            uint8_t* __restrict__ dst,
                                                            float* __restrict__ scale) {
   constexpr int NE = Src<SRC>::kPer, U = 4;
-  __shared__ unsigned arrived;
+  __shared__ bool last;
   const i32x4* g = (const i32x4*)src;
-  const int64_t ng = n / NE, head = (int64_t)np * 4 / NE;
+  const bool two_levels = gridDim.x > 4 * kFp8Counters;
+  const int64_t ng = n / NE, head = ((int64_t)np * 4 + (two_levels ? kFp8CounterBytes : 0)) / NE;
   const int64_t stride = (int64_t)gridDim.x * 1024;
   int64_t i = head + blockIdx.x * (int64_t)1024 + threadIdx.x;
   i32x4 v[U];
@@ -292,7 +314,10 @@ __global__ __launch_bounds__(1024) void quantize_fp8_kernel(const void* __restri
     m = o > m ? o : m;
   }
   const Fp8Scale sc(block_max<16>(m));  // its barrier: the workgroup's reads of dst are over
-  if (threadIdx.x == 0) arrived = atomicAdd((unsigned*)scale, 1u);
+  const unsigned c = blockIdx.x % kFp8Counters;
+  unsigned ticket = 0;  // looked at in the end: nobody waits for the atomic
+  if (threadIdx.x == 0)
+    ticket = atomicAdd(two_levels ? (unsigned*)dst + np + c * kFp8CounterPitch : (unsigned*)scale, 1u);
   while (i < ng) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
@@ -302,8 +327,13 @@ __global__ __launch_bounds__(1024) void quantize_fp8_kernel(const void* __restri
   }
   for (int64_t j = ng * NE + blockIdx.x * (int64_t)1024 + threadIdx.x; j < n; j += stride)
     dst[j] = (uint8_t)sc.code(load1<SRC>(src, j));
+  if (threadIdx.x == 0) {
+    const unsigned of_c = (gridDim.x - c + kFp8Counters - 1) / kFp8Counters;
+    last = two_levels ? ticket == of_c - 1 && atomicAdd((unsigned*)scale, 1u) == kFp8Counters - 1
+                      : ticket == gridDim.x - 1;
+  }
   __syncthreads();
-  if (arrived != gridDim.x - 1) return;
+  if (!last) return;
   for (int64_t j = threadIdx.x; j < head; j += 1024) fp8_store_group<SRC>(g[j], j, sc, dst);
   if (threadIdx.x == 0) *scale = sc.s;
 }
@@ -542,8 +572,10 @@ extern "C" int astergemm_quantize_fp8_tensor(const void* dSrc, int src_dtype, in
     if (np > 1024) np = 1024;
     hipLaunchKernelGGL(fp8_absmax_kernel<SRC>, dim3((unsigned)np), dim3(256), 0, s, dSrc, n,
                        (unsigned*)dDst, (unsigned*)dScale);
-    const int64_t b = (ng + 1023) / 1024;
-    hipLaunchKernelGGL(quantize_fp8_kernel<SRC>, dim3((unsigned)(b < 256 ? b : 256)), dim3(1024), 0, s,
+    // a workgroup per CU, two from 2^25 elements on (bf16, one / two: 4096 x 4096 19.5 / 20.4 us, 4096 x 14336
+    // 57.5 / 55.7, 8192 x 8192 73.3 / 72.0)
+    const int64_t b = (ng + 1023) / 1024, cap = n < ((int64_t)1 << 25) ? 256 : 512;
+    hipLaunchKernelGGL(quantize_fp8_kernel<SRC>, dim3((unsigned)(b < cap ? b : cap)), dim3(1024), 0, s,
                        dSrc, n, (int)np, dDst, dScale);
   });
   AG_HIP(hipGetLastError());

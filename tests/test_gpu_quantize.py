@@ -309,10 +309,10 @@ def test_preshuffle_on_the_device_writes_the_bytes_of_the_host_functions(gpu, dt
         bf.free()
 
 
-@pytest.mark.parametrize("n", [7, 8, 9, 8191, 131072, 131073, 131080, 300007])
+@pytest.mark.parametrize("n", [7, 8, 9, 8191, 131072, 131073, 131080, 262144, 262149, 300007, 524288, 524296, 2097159])
 @pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
 def test_fp8_quantiser_one_and_two_launch_forms(n, dtype):
-    """Both sides of the one-launch limit, whole and broken 16-byte groups, every source type, with
+    """Both sides of the one-launch limit and of 64 workgroups (65 count on two levels), whole and broken 16-byte groups, every source type, with
     signed zeros and the maximum in the last element; nothing behind the n codes is written."""
     rng = np.random.default_rng(n)
     x = rng.standard_normal(n).astype(np.float32)
