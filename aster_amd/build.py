@@ -26,17 +26,16 @@ OBJ_DIR = os.path.join(ROOT, "build", "obj")
 
 # (object stem, source file, extra flags).  gemm_stream.hip holds the variant table of the stream
 # kernels in five parts (bf16, fp8, MXFP4, f16 operands, unequal tile sides) and is compiled once
-# per part, gemm_kwave.hip once per operand type.
+# per part, gemm_kwave.hip once per operand type and order
+# of the weights.
 UNITS = [("gemm_stream_p0", "gemm_stream.hip", ["-DAG_STREAM_PART=0"]),
          ("gemm_stream_p3", "gemm_stream.hip", ["-DAG_STREAM_PART=3"]),
          ("gemm_stream_p2", "gemm_stream.hip", ["-DAG_STREAM_PART=2"]),
          ("gemm_stream_p1", "gemm_stream.hip", ["-DAG_STREAM_PART=1"]),
          ("gemm_stream_p4", "gemm_stream.hip", ["-DAG_STREAM_PART=4"]),
          ("gemm_skinny", "gemm_skinny.hip", []),
-         ("gemm_kwave_f16", "gemm_kwave.hip", ["-DAG_KWAVE_DT=0"]),
-         ("gemm_kwave_bf16", "gemm_kwave.hip", ["-DAG_KWAVE_DT=1"]),
-         ("gemm_kwave_fp8", "gemm_kwave.hip", ["-DAG_KWAVE_DT=2"]),
-         ("gemm_kwave_mxfp4", "gemm_kwave.hip", ["-DAG_KWAVE_DT=3"]),
+         *((f"gemm_kwave_{dt}{'_k8' if k8 else ''}", "gemm_kwave.hip", [f"-DAG_KWAVE_DT={i}", f"-DAG_KWAVE_K8={k8}"])
+           for i, dt in enumerate(("f16", "bf16", "fp8", "mxfp4")) for k8 in (0, 1)),
          ("gemm_tile", "gemm_tile.hip", []),
          ("astergemm_api", "astergemm_api.hip", []),
          ("quantize", "quantize.hip", []),

@@ -9,6 +9,7 @@ struct KwaveForm {
   int shape = -1;  // -1: the problem stays with the other kernels
   int per = 0;     // weight rows of a workgroup
   int ranges = 1;  // K ranges
+  bool k8 = false; // weights (MXFP4: and both scale planes) in the order of ASTERGEMM_OPERAND_DIRECT_B_K8
   explicit operator bool() const { return shape >= 0; }
 };
 
@@ -21,6 +22,9 @@ KwaveForm kwave_small_decode_form(int dt, int64_t M, int64_t N, int64_t K, int c
 
 // 64 < M <= 512 against at most about a round of panels, as part of the launchers of 128 x 128 tiles.
 KwaveForm kwave_prompt_form(int dt, int64_t M, int64_t N, int64_t K, int cus);
+// M <= 512 on pre-shuffled weights (*rows: the operand rows of a workgroup), as part of the launchers of 128 x 256
+// tiles that load them straight into MFMA operands.
+KwaveForm kwave_k8_form(int dt, int64_t M, int64_t N, int cus, int* rows);
 // Any M and N: the smallest tile that leaves at most one workgroup per CU, else (and without a device) 64 x 64.
 KwaveForm kwave_tile_form(int64_t M, int64_t N, int cus);
 // Small products that AUTO takes the tile form for, where it takes the general tile kernels otherwise.
@@ -31,7 +35,7 @@ KwaveForm kwave_variant_form(bool split, int dt, int64_t M, int64_t N, int64_t K
 
 int kwave_launch(int dt, int out, const GemmArgs& a, const KwaveForm& f, hipStream_t s);
 // The one-time step of every shape of `dt` on the current device (see lds_attr_once).
-int kwave_ready(int dt);
+int kwave_ready(int dt, bool k8 = false);
 void kwave_describe(int dt, const KwaveForm& f, int64_t M, int64_t N, int cus, LaunchForm* o);
 bool kwave_decode_describe(const astergemm_config& c, int cus, int max_ranges, LaunchForm* o);
 bool kwave_prompt_describe(const astergemm_config& c, int cus, LaunchForm* o);

@@ -1,6 +1,6 @@
 // Shapes, rules and launches of the kernels that split K over the waves of a workgroup
-// (device code: gemm_kwave_kernel.hpp).  Compiled once per operand type (AG_KWAVE_DT); the unit of f16
-// operands also holds what all of them share.
+// (device code: gemm_kwave_kernel.hpp).  Compiled once per operand type (AG_KWAVE_DT) and order of the weights
+// (AG_KWAVE_K8); the unit of f16 operands and row-major weights also holds what all of them share.
 #include "gemm_kwave.h"
 #include "gemm_kwave_kernel.hpp"
 
@@ -32,62 +32,63 @@ struct KwaveShape {
   int (*launch)(const KwaveArgs& q, int grid, hipStream_t s);
 };
 constexpr int kKwaveShapes = 16;
-const KwaveShape* kwave_shapes_f16();
-const KwaveShape* kwave_shapes_bf16();
-const KwaveShape* kwave_shapes_fp8();
-const KwaveShape* kwave_shapes_mxfp4();
+template <int DT, bool K8>
+const KwaveShape* kwave_shapes();
 
 namespace {
 
-template <int DT, int BM, int BN, int WM, int WN, int WK, int S>
+template <int DT, bool K8, int BM, int BN, int WM, int WN, int WK, int S>
 int launch_kwave(const KwaveArgs& q, int grid, hipStream_t s) {
-  constexpr int lds = S * WK * kwave_step_bytes(DT, BM, BN);
-  AG_LAUNCH_KERNEL((gemm_kwave_kernel<DT, BM, BN, WM, WN, WK, S>), dim3(grid), dim3(WM * WN * WK * 64), lds, s,
+  constexpr int lds = S * WK * kwave_step_bytes(DT, K8, BM, BN);
+  AG_LAUNCH_KERNEL((gemm_kwave_kernel<DT, K8, BM, BN, WM, WN, WK, S>), dim3(grid), dim3(WM * WN * WK * 64), lds, s,
                    q);
   return (int)hipGetLastError();
 }
 
-template <int DT, int BM, int BN, int WM, int WN, int WK, int S>
+template <int DT, bool K8, int BM, int BN, int WM, int WN, int WK, int S>
 constexpr KwaveShape kwave_shape() {
-  return KwaveShape{BM, BN, WM, WN, WK, S, S * WK * kwave_step_bytes(DT, BM, BN),
-                    (const void*)gemm_kwave_kernel<DT, BM, BN, WM, WN, WK, S>,
-                    launch_kwave<DT, BM, BN, WM, WN, WK, S>};
+  return KwaveShape{BM, BN, WM, WN, WK, S, S * WK * kwave_step_bytes(DT, K8, BM, BN),
+                    (const void*)gemm_kwave_kernel<DT, K8, BM, BN, WM, WN, WK, S>,
+                    launch_kwave<DT, K8, BM, BN, WM, WN, WK, S>};
 }
 
 #define AG_KWAVE_ENTRY(I, BM, BN, WM, WN, WK, S, S4) \
-  kwave_shape<AG_KWAVE_DT, BM, BN, WM, WN, WK, AG_KWAVE_DT == ASTERGEMM_MXFP4 ? S4 : S>(),
+  kwave_shape<AG_KWAVE_DT, AG_KWAVE_K8 != 0, BM, BN, WM, WN, WK, AG_KWAVE_DT == ASTERGEMM_MXFP4 ? S4 : S>(),
 const KwaveShape kShapes[kKwaveShapes] = {AG_KWAVE_SHAPES(AG_KWAVE_ENTRY)};
 
 }  // namespace
 
-#if AG_KWAVE_DT == 0
-const KwaveShape* kwave_shapes_f16() { return kShapes; }
-#elif AG_KWAVE_DT == 1
-const KwaveShape* kwave_shapes_bf16() { return kShapes; }
-#elif AG_KWAVE_DT == 2
-const KwaveShape* kwave_shapes_fp8() { return kShapes; }
-#else
-const KwaveShape* kwave_shapes_mxfp4() { return kShapes; }
-#endif
+template <>
+const KwaveShape* kwave_shapes<AG_KWAVE_DT, AG_KWAVE_K8 != 0>() { return kShapes; }
 
-#if AG_KWAVE_DT == 0
+#if AG_KWAVE_DT == 0 && !AG_KWAVE_K8
+template <> const KwaveShape* kwave_shapes<ASTERGEMM_F16, true>();
+template <> const KwaveShape* kwave_shapes<ASTERGEMM_BF16, false>();
+template <> const KwaveShape* kwave_shapes<ASTERGEMM_BF16, true>();
+template <> const KwaveShape* kwave_shapes<ASTERGEMM_FP8_E4M3, false>();
+template <> const KwaveShape* kwave_shapes<ASTERGEMM_FP8_E4M3, true>();
+template <> const KwaveShape* kwave_shapes<ASTERGEMM_MXFP4, false>();
+template <> const KwaveShape* kwave_shapes<ASTERGEMM_MXFP4, true>();
+
 namespace {
 
+template <bool K8>
 const KwaveShape* shapes_of(int dt) {
   switch (dt) {
-    case ASTERGEMM_F16: return kwave_shapes_f16();
-    case ASTERGEMM_BF16: return kwave_shapes_bf16();
-    case ASTERGEMM_FP8_E4M3: return kwave_shapes_fp8();
-    default: return kwave_shapes_mxfp4();
+    case ASTERGEMM_F16: return kwave_shapes<ASTERGEMM_F16, K8>();
+    case ASTERGEMM_BF16: return kwave_shapes<ASTERGEMM_BF16, K8>();
+    case ASTERGEMM_FP8_E4M3: return kwave_shapes<ASTERGEMM_FP8_E4M3, K8>();
+    default: return kwave_shapes<ASTERGEMM_MXFP4, K8>();
   }
 }
+const KwaveShape* shapes_of(int dt, bool k8) { return k8 ? shapes_of<true>(dt) : shapes_of<false>(dt); }
 
 // Weight rows of a workgroup when `tiles_m` tile rows share the chip: one round, groups of 8 rows.  The tile
 // rows of a panel are on one XCD, so a round is what fits every XCD's eighth of the CUs (a few panels more
 // put a second round on some XCDs: bf16 400x4096x4096 26.7 -> 41.4 us).
-int rows_per(int64_t N, int tiles_m, int cus) {
+int rows_per(int64_t N, int tiles_m, int cus, int unit = 8) {
   const int per_xcd = cus / 8 / tiles_m, panels = per_xcd > 0 ? per_xcd * 8 : 1;
-  return (int)(((N + panels - 1) / panels + 7) / 8 * 8);
+  return (int)(((N + panels - 1) / panels + unit - 1) / unit * unit);
 }
 
 // Workgroups of a K range: by panels on one XCD each, in whole groups of 8 panels, while that is one round;
@@ -262,23 +263,46 @@ KwaveForm kwave_variant_form(bool split, int dt, int64_t M, int64_t N, int64_t K
   return f ? f : kwave_tile_form(M, N, cus);
 }
 
-int kwave_ready(int dt) {
-  static std::atomic<uint64_t> all[4], devs[4][kKwaveShapes];
+// Pre-shuffled weights (K8): the tile that brings the fewest operand rows into a CU in one round, panels of whole
+// 16-row blocks (MXFP4: of pairs of them, whose scale bytes are fetched together).
+KwaveForm kwave_k8_form(int dt, int64_t M, int64_t N, int cus, int* rows) {
+  static const struct { int bm, bn, shape; } kTiles[] = {
+      {16, 16, 0},  {16, 32, 1},  {16, 48, 2},  {16, 64, 3},   {32, 16, 5},  {32, 32, 6},  {32, 64, 7}, {32, 128, 8},
+      {64, 32, 9},  {64, 48, 10}, {64, 64, 11}, {64, 128, 12}, {96, 64, 13}, {128, 64, 14}, {128, 128, 15}};
+  KwaveForm f;
+  if (cus < 8 || M < 1 || M > 512 || N < 16 || N % 16 != 0 || N > INT32_MAX / 2) return f;
+  int bm = 0, best = INT32_MAX;
+  for (const auto& t : kTiles) {
+    const int64_t tm = (M + t.bm - 1) / t.bm;
+    if (tm > cus / 8 || t.bm == bm) continue;  // (the first panel that fits a tile height is its best)
+    const int per = rows_per(N, (int)tm, cus, dt == ASTERGEMM_MXFP4 && t.bn > 16 ? 32 : 16);
+    if (per > t.bn) continue;
+    bm = t.bm;
+    const int loaded = t.bm + (per * 4 > t.bn * 3 ? per : t.bn * 3 / 4);
+    const int cost = loaded - (tm == 1 ? loaded / 16 : 0);
+    if (cost < best) best = cost, *rows = t.bm + per, f.shape = t.shape, f.per = per, f.k8 = true;
+  }
+  return f;
+}
+
+int kwave_ready(int dt, bool k8) {
+  static std::atomic<uint64_t> all[8], devs[8][kKwaveShapes];
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess) return (int)hipGetLastError();
   const uint64_t bit = (uint64_t)1 << (dev & 63);
-  if (all[dt & 3].load(std::memory_order_acquire) & bit) return 0;
-  const KwaveShape* shapes = shapes_of(dt);
+  const int set = (dt & 3) + (k8 ? 4 : 0);
+  if (all[set].load(std::memory_order_acquire) & bit) return 0;
+  const KwaveShape* shapes = shapes_of(dt, k8);
   for (int i = 0; i < kKwaveShapes; ++i) {
     if (shapes[i].lds <= 65536) continue;  // within the default limit
-    if (int e = lds_attr_once(devs[dt & 3][i], shapes[i].func, shapes[i].lds)) return e;
+    if (int e = lds_attr_once(devs[set][i], shapes[i].func, shapes[i].lds)) return e;
   }
-  all[dt & 3].fetch_or(bit, std::memory_order_release);
+  all[set].fetch_or(bit, std::memory_order_release);
   return 0;
 }
 
 int kwave_launch(int dt, int out, const GemmArgs& a, const KwaveForm& f, hipStream_t s) {
-  const KwaveShape& sh = shapes_of(dt)[f.shape];
+  const KwaveShape& sh = shapes_of(dt, f.k8)[f.shape];
   KwaveArgs q;
   q.g = a;
   q.g.tiles_m = (a.M + sh.bm - 1) / sh.bm;
@@ -307,7 +331,7 @@ int kwave_launch(int dt, int out, const GemmArgs& a, const KwaveForm& f, hipStre
 }
 
 void kwave_describe(int dt, const KwaveForm& f, int64_t M, int64_t N, int cus, LaunchForm* o) {
-  const KwaveShape& sh = shapes_of(dt)[f.shape];
+  const KwaveShape& sh = shapes_of(dt, f.k8)[f.shape];
   int by_panel;
   o->grid = kwave_blocks((int)((M + sh.bm - 1) / sh.bm), (int)((N + f.per - 1) / f.per), cus, &by_panel) * f.ranges;
   o->tile_m = sh.bm;
@@ -335,6 +359,6 @@ bool kwave_small_decode_describe(const astergemm_config& c, int cus, LaunchForm*
   if (f) kwave_describe(c.dtype_ab, f, c.M, c.N, cus, o);
   return (bool)f;
 }
-#endif  // AG_KWAVE_DT == 0
+#endif  // AG_KWAVE_DT == 0 && !AG_KWAVE_K8
 
 }  // namespace astergemm

@@ -17,6 +17,10 @@
 //     columns of every weight row, and with rows a multiple of a few KiB apart those are few HBM channels:
 //     bf16 8x8192x8192 28.3 us in step, 21.4 rotated; 64x14336x4096 25.3 -> 22.9; 64x28672x4096 49.3 -> 37.7;
 //     fp8 8x8192x8192 17.6 -> 11.2.
+//   * K8: weights pre-shuffled (ASTERGEMM_OPERAND_DIRECT_B_K8), staged as they lie: 16 rows x 128 bytes are 2 KiB in
+//     one piece, lane for lane the operands of the 16 x 16 tile, so a transfer is 1 KiB of consecutive bytes and a
+//     fragment read 1 KiB of consecutive LDS.  MXFP4: both scale planes in lane order, whose bytes a lane reads
+//     are its own: two tiles' bytes are a dword per lane.
 // Sums: a K-step's products in MFMA order, a group's steps in rotated order, the groups in index order: the
 // same bits on every run of a config.
 #pragma once
@@ -36,24 +40,25 @@ struct KwaveArgs {
   int32_t nt;           // weights are fetched past the last-level cache
 };
 
-constexpr int kwave_scale_loads(int dt, int bm, int bn) {  // 32-row transfers of e8m0 bytes per K-step
-  return dt == ASTERGEMM_MXFP4 ? (bm + bn + 31) / 32 : 0;
+// 32-row transfers of e8m0 bytes per K-step (K8: of each operand by itself)
+constexpr int kwave_scale_loads(int dt, bool k8, int bm, int bn) {
+  return dt != ASTERGEMM_MXFP4 ? 0 : k8 ? (bm + 31) / 32 + (bn + 31) / 32 : (bm + bn + 31) / 32;
 }
-constexpr int kwave_step_bytes(int dt, int bm, int bn) {   // LDS of one K-step of a wave group
-  return (bm + bn) * kRowBytes + kwave_scale_loads(dt, bm, bn) * 256;
+constexpr int kwave_step_bytes(int dt, bool k8, int bm, int bn) {  // LDS of one K-step of a wave group
+  return (bm + bn) * kRowBytes + kwave_scale_loads(dt, k8, bm, bn) * 256;
 }
 
-template <int DT, int BM, int BN, int WM, int WN, int WK, int S>
+template <int DT, bool K8, int BM, int BN, int WM, int WN, int WK, int S>
 __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_kwave_kernel(const KwaveArgs q) {
   constexpr int GW = WM * WN;                   // waves of a group
   constexpr int NW = GW * WK;
   constexpr int TM = BM / WM / 16, TN = BN / WN / 16;
   constexpr int GA = BM / 8, G = GA + BN / 8;   // 8-row transfers of a K-step, A's first
   constexpr bool FP4 = DT == ASTERGEMM_MXFP4;
-  constexpr int NSX = kwave_scale_loads(DT, BM, BN);
+  constexpr int NSX = kwave_scale_loads(DT, K8, BM, BN);
   constexpr int LG = G / GW, LS = (NSX + GW - 1) / GW, L = LG + LS;  // transfers per wave and stage
   constexpr int B_AT = BM * kRowBytes, SCALES = (BM + BN) * kRowBytes;
-  constexpr int STEP = kwave_step_bytes(DT, BM, BN), STAGE = STEP * WK;
+  constexpr int STEP = kwave_step_bytes(DT, K8, BM, BN), STAGE = STEP * WK;
   constexpr int NT = (BM / 16) * (BN / 16);     // 16 x 16 tiles of the workgroup
   constexpr int TPW = (NT + NW - 1) / NW;       // of them finished by one wave
   static_assert(G % GW == 0, "whole transfers per wave");
@@ -97,9 +102,38 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_kwave_kernel(const Kwave
     const int last = is_a ? p.M - 1 - row0 : col1 - 1 - col0;
     r = r < last ? r : last;
     off[j] = (unsigned)(r * (int)(is_a ? p.lda_bytes : p.ldb_bytes) + gran[j] * 16);
+    if (K8 && !is_a) {  // half (t - GA) & 1 of a block of 16 rows (ranges of whole blocks: past the end the last one)
+      const int blk = (t - GA) >> 1, last_blk = ((col1 - col0) >> 4) - 1;
+      off[j] = (unsigned)((blk < last_blk ? blk : last_blk) * 16 * (int)p.ldb_bytes + ((t - GA) & 1) * 1024 + lane * 16);
+    }
   }
+  constexpr int B_STEP = K8 ? 16 * kRowBytes : kRowBytes;  // from one K-step of B to the next
   const uint8_t* s_src[LS ? LS : 1];            // e8m0: 8 bytes per row and K-step, A's rows first
-  if constexpr (FP4) {
+  int s_step[K8 && FP4 ? LS : 1];
+  if constexpr (FP4 && K8) {
+    // lane order: tiles t, t + 1 (t even) of lane L are 4 bytes at 16 L + 2 t of A's 128-row group (1 KiB per
+    // K-step), at 8 L + 2 t of B's 64-row group (512 bytes); pairs of tiles, A's first
+    constexpr int PA = (BM + 31) / 32;
+#pragma unroll
+    for (int j = 0; j < LS; ++j) {
+      int x = wv + j * GW;
+      x = x < NSX ? x : NSX - 1;                // a surplus transfer repeats the last one: the same bytes
+      if (x < PA) {
+        // pairs past the last group of A's plane, whose rows are never stored, repeat its last
+        int t = ((row0 >> 4) & ~1) + 2 * x;
+        const int last = ((p.M - 1) >> 7) * 8 + 6;
+        t = t < last ? t : last;
+        s_src[j] = p.mx_a + (int64_t)(t >> 3) * p.ksteps * 1024 + lane * 16 + (t & 7) * 2;
+        s_step[j] = 1024;
+      } else {
+        int t = ((col0 >> 4) & ~1) + 2 * (x - PA);
+        const int last = (p.N >> 4) - 2;
+        t = t < last ? t : last;
+        s_src[j] = p.mx_b + (int64_t)(t >> 2) * p.ksteps * 512 + lane * 8 + (t & 3) * 2;
+        s_step[j] = 512;
+      }
+    }
+  } else if constexpr (FP4) {
 #pragma unroll
     for (int j = 0; j < LS; ++j) {
       int x = wv + j * GW;
@@ -138,13 +172,17 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_kwave_kernel(const Kwave
                  : "s"(m0_of(dst)), "v"(src)
                  : "memory", "m0");
   };
+  auto s_stride = [&](int j) {
+    if constexpr (K8 && FP4) return s_step[j];
+    else return 8;
+  };
   auto issue = [&](int st, int slot) {          // this group's K-step of stage st
     int sr = st + rot;
     sr = sr < nst ? sr : sr - nst;
     const int k = k0 + sr * WK + wk;
     const uint8_t* d = lds + slot * STAGE + wk * STEP;
     const uint8_t* ga = a_base + (int64_t)k * kRowBytes;
-    const uint8_t* gb = b_base + (int64_t)k * kRowBytes;
+    const uint8_t* gb = b_base + (int64_t)k * B_STEP;
     auto dst = [&](int j) {
       const int t = wv + j * GW;
       return d + (t < GA ? t * 1024 : B_AT + (t - GA) * 1024);
@@ -170,7 +208,7 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_kwave_kernel(const Kwave
       for (int j = 0; j < LS; ++j) {
         int x = wv + j * GW;
         x = x < NSX ? x : NSX - 1;
-        g2s_dword(k < k1 ? s_src[j] + (int64_t)k * 8 : g_zero16, d + SCALES + x * 256);
+        g2s_dword(k < k1 ? s_src[j] + (int64_t)k * s_stride(j) : g_zero16, d + SCALES + x * 256);
       }
     }
   };
@@ -199,6 +237,12 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_kwave_kernel(const Kwave
 #pragma unroll
   for (int s = 0; s < 2; ++s)
     rd[s] = (unsigned)(li * kRowBytes + (((DT == ASTERGEMM_FP8_E4M3 ? 2 * lq + s : 4 * s + lq) ^ (li >> 1)) << 4));
+  unsigned rd_b[2];  // K8: granule g of row li of a block is at (g / 4) KiB, lane 16 (g mod 4) + li
+#pragma unroll
+  for (int s = 0; s < 2; ++s)
+    rd_b[s] = !K8 ? rd[s]
+              : DT == ASTERGEMM_FP8_E4M3 ? (unsigned)((lq >> 1) * 1024 + (((lq & 1) * 2 + s) * 16 + li) * 16)
+                                         : (unsigned)(s * 1024 + lane * 16);
   f32x4 acc[TM][TN];
 #pragma unroll
   for (int m = 0; m < TM; ++m)
@@ -223,10 +267,20 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_kwave_kernel(const Kwave
       for (int m = 0; m < TM; ++m) af[s][m] = *(const i32x4*)(sp + (wm * TM + m) * 16 * kRowBytes + rd[s]);
 #pragma unroll
       for (int n = 0; n < TN; ++n)
-        bf[s][n] = *(const i32x4*)(sp + B_AT + (wn * TN + n) * 16 * kRowBytes + rd[s]);
+        bf[s][n] = *(const i32x4*)(sp + B_AT + (wn * TN + n) * 16 * kRowBytes + rd_b[s]);
     }
     i32x2 sa[FP4 ? TM : 1], sb[FP4 ? TN : 1];
-    if constexpr (FP4) {
+    if constexpr (FP4 && K8) {
+      // bytes 0, 1 of a word: substeps 0, 1 of the pair's first tile, bytes 2, 3 of its second
+      constexpr int PA = (BM + 31) / 32;
+      const int ta = ((row0 >> 4) & 1) + wm * TM, tb = ((col0 >> 4) & 1) + wn * TN;
+#pragma unroll
+      for (int m = 0; m < TM; ++m)
+        sa[m][0] = *(const int*)(sp + SCALES + ((ta + m) >> 1) * 256 + lane * 4) >> (((ta + m) & 1) * 16);
+#pragma unroll
+      for (int n = 0; n < TN; ++n)
+        sb[n][0] = *(const int*)(sp + SCALES + (PA + ((tb + n) >> 1)) * 256 + lane * 4) >> (((tb + n) & 1) * 16);
+    } else if constexpr (FP4) {
 #pragma unroll
       for (int m = 0; m < TM; ++m) sa[m] = *(const i32x2*)(sp + SCALES + ((wm * TM + m) * 16 + li) * 8);
 #pragma unroll
@@ -248,7 +302,10 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_kwave_kernel(const Kwave
 #pragma unroll
           for (int n = 0; n < TN; ++n) {
             int xa = 0, xb = 0;
-            if constexpr (FP4) {
+            if constexpr (FP4 && K8) {
+              xa = (int)((unsigned)sa[m][0] >> (8 * s));
+              xb = (int)((unsigned)sb[n][0] >> (8 * s));
+            } else if constexpr (FP4) {
               xa = (int)((unsigned)sa[m][s] >> (8 * lq));
               xb = (int)((unsigned)sb[n][s] >> (8 * lq));
             }

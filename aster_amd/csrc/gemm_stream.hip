@@ -193,17 +193,128 @@ int launch_streamr(const GemmArgs& a, int grid, hipStream_t s) {
       AG_STREAMR(prefix "_f32", DT, ASTERGEMM_F32, BM, BN, WM, WN, NS),    \
       AG_STREAMR(prefix "_f16", DT, ASTERGEMM_F16, BM, BN, WM, WN, NS)
 
+// ---- pre-shuffled weights (K8 order) in AUTO's form of the kernels below -----------------------
+//
+// The kernels that load them straight into MFMA operands have 128 x 256 tiles and nothing for problems that those leave
+// half the chip without: through LDS they are as good an operand as rows (16 rows x 128 bytes are 2 KiB in one
+// piece), for K over waves (gemm_kwave_kernel) and tiles of 128, 192 or 256 x 128 (gemm_streamr_kernel).  A
+// workgroup takes as long as its operand rows, per K-step; straight into operands 384 rows weigh as much as
+// 500 here (390 in fp8; past one per CU two share it).  Own kernel / K over waves / 128 / 192 / 256 x 128,
+// us over three sets of weights (fp8 and MXFP4 with their quantiser):
+//   bf16 80x4096x4096       43.0 / 11.9 / 22.0 / 27.9 / 35.2    bf16 512x1024x8192   77.8 / 22.1 / 41.7 / 53.2 / 67.7
+//   bf16 160x14336x4096     60.3 / 49.3 / 38.9 / 44.0 / 44.4    bf16 320x4096x14336  181 / 85.5 / 101 / 128 / 123
+//   bf16 320x14336x4096     63.8 / - / 63.9 / 44.6 / 49.0       bf16 512x14336x4096  68.5 / - / 72.5 / 79.4 / 53.8
+//   bf16 640x11008x4096     63.2 / - / 68.6 / 71.8 / 82.7       bf16 1280x8192x8192  199 / - / 188 / 156 / 184
+//   bf16 640x28672x4096     165 / - / 178 / 158 / 145           bf16 4096x4096x4096  108 / - / - / 123 / 109
+//   fp8 80x14336x4096       29.3 / 20.8 / 22.6 / 23.8 / 27.6    fp8 320x28672x4096   66.2 / - / 67.9 / 55.1 / 62.3
+//   fp8 1280x4096x14336     96.3 / - / 117 / 87.6 / 96.3        fp8 944x14336x4096   60.0 / - / - / 71.9 / 63.2
+//   MXFP4 160x4096x14336    45.4 / 28.4                         MXFP4 160x14336x4096 21.5 / 23.2 (240 rows)
+// fp8 in this order adds from K-step 0 on, so the tiles have the bits of the own kernel, and K over waves, which does
+// not, is for weights of 1024 rows and more, as among row-major ones (MXFP4 too).
+struct K8Form {
+  KwaveForm kw;
+  int tile = 0;  // rows of a tile 128 columns wide; neither: the launcher's own kernel
+  explicit operator bool() const { return kw || tile; }
+};
+inline K8Form k8_form(int dt, int64_t M, int64_t N, int cus) {
+  K8Form f;
+  if (cus <= 0) return f;
+  const bool fp8 = dt == ASTERGEMM_FP8_E4M3, fp4 = dt == ASTERGEMM_MXFP4;
+  int64_t best = INT64_MAX;
+  if (!fp4) {
+    const int64_t own_grid = (M + 127) / 128 * ((N + 255) / 256);
+    if (own_grid > (fp8 ? 2 * cus : 700 * cus / 256)) return f;
+    best = own_grid <= cus ? (fp8 ? 390 : 500) : fp8 ? 700 : own_grid <= 2 * cus ? 1000 : 1200;
+    for (int bm : {128, 192, 256}) {
+      const int64_t rounds = ((M + bm - 1) / bm * ((N + 127) / 128) + cus - 1) / cus;
+      if (rounds <= 3 && rounds * (bm + 128) < best) best = rounds * (bm + 128), f.tile = bm;
+    }
+  }
+  int rows = 0;
+  if ((fp8 || fp4) && N < 1024) return f;
+  const KwaveForm kw = kwave_k8_form(dt, M, N, cus, &rows);
+  if (kw && (fp4 ? rows <= 192 : fp8 ? rows * 4 < best * 3 : rows * 4 <= best * 3)) f.kw = kw, f.tile = 0;
+  return f;
+}
+
+constexpr int k8_stages(int bm) { return bm == 128 ? 5 : bm == 192 ? 4 : 3; }
+constexpr int k8_lds(int bm) { return k8_stages(bm) * (bm + 128) * kRowBytes; }
+template <int DT, int OUT, int BM>
+constexpr auto k8_kernel() {
+  return gemm_streamr_kernel<DT, OUT, BM, 128, 4, 2, k8_stages(BM), true>;
+}
+template <int DT, int OUT, int BM>
+int launch_k8_tile(GemmArgs a, hipStream_t s) {
+  a.tiles_m = (a.M + BM - 1) / BM;
+  a.tiles_n = (a.N + 127) / 128;
+  a.group_m = (a.tiles_m % 8 == 0 && a.tiles_n % 32 == 0) ? -1 : 8;
+  auto k = k8_kernel<DT, OUT, BM>();
+  AG_LAUNCH_KERNEL(k, dim3(a.tiles_m * a.tiles_n), dim3(512), k8_lds(BM), s, a);
+  return (int)hipGetLastError();
+}
+
+// 0 and *taken = false: the launcher's own kernel is to run.  Either's first launch readies all of them.
+template <int DT, int OUT>
+int k8_instead(const GemmArgs& a, int own_ready, hipStream_t s, bool* taken) {
+  *taken = false;
+  const K8Form f = a.own_kernel ? K8Form{} : k8_form(DT, a.M, a.N, device_cus());
+  if (own_ready != 0 && !f) return own_ready;
+  if (const int e = kwave_ready(DT, true)) return e;
+  if constexpr (DT != ASTERGEMM_MXFP4) {
+    static std::atomic<uint64_t> devs[3];
+    if (const int e = lds_attr_once(devs[0], (const void*)k8_kernel<DT, OUT, 128>(), k8_lds(128))) return e;
+    if (const int e = lds_attr_once(devs[1], (const void*)k8_kernel<DT, OUT, 192>(), k8_lds(192))) return e;
+    if (const int e = lds_attr_once(devs[2], (const void*)k8_kernel<DT, OUT, 256>(), k8_lds(256))) return e;
+  }
+  if (!f) return 0;
+  *taken = true;
+  if (f.kw) return kwave_launch(DT, OUT, a, f.kw, s);
+  if constexpr (DT != ASTERGEMM_MXFP4) {
+    if (f.tile == 128) return launch_k8_tile<DT, OUT, 128>(a, s);
+    if (f.tile == 192) return launch_k8_tile<DT, OUT, 192>(a, s);
+    return launch_k8_tile<DT, OUT, 256>(a, s);
+  }
+  return 0;
+}
+
+template <int DT, int OUT>
+bool k8_describe(const astergemm_config& c, int cus, LaunchForm* o) {
+  const K8Form f = cus > 0 ? k8_form(DT, c.M, c.N, cus) : K8Form{};
+  if (f.kw) kwave_describe(DT, f.kw, c.M, c.N, cus, o);
+  if constexpr (DT != ASTERGEMM_MXFP4) {
+    if (f.tile) {
+      o->grid = (int)((c.M + f.tile - 1) / f.tile * ((c.N + 127) / 128));
+      o->tile_m = f.tile;
+      o->tile_n = 128;
+      o->waves_m = 4;
+      o->waves_n = 2;
+      o->stages = k8_stages(f.tile);
+      o->lds_bytes = k8_lds(f.tile);
+      o->threads = 512;
+      o->func = f.tile == 128   ? (const void*)k8_kernel<DT, OUT, 128>()
+                : f.tile == 192 ? (const void*)k8_kernel<DT, OUT, 192>()
+                                : (const void*)k8_kernel<DT, OUT, 256>();
+    }
+  }
+  return (bool)f;
+}
+
 // ---- B pre-shuffled, loaded straight into MFMA operands (gemm_streamdb_kernel.hpp) ---------
 template <int DT, int OUT, int NSLOT, int NBUF, int WM>
 int launch_streamdb(const GemmArgs& a, int grid, hipStream_t s) {
   constexpr int lds = 5 * 128 * WM * kRowBytes;  // the epilogue stages through the ring
   auto k = gemm_streamdb_kernel<DT, OUT, NSLOT, NBUF, WM>;
   static std::atomic<uint64_t> attr_devs{0};
-  if (int e = lds_attr_once(attr_devs, (const void*)k, lds)) return e;
-  // what the kernel's indexing assumes: whole 16-row blocks of B and whole K-steps
+  // what the kernels' indexing assumes: whole 16-row blocks of B and whole K-steps
   if (a.N % 16 != 0 || a.N < 16 || a.M < 8 || a.M % 8 != 0 || a.K % 64 != 0 || a.tail_granules != 0 ||
       a.ldb_bytes != (int64_t)a.K * 2)
     return (int)hipErrorInvalidValue;
+  const int own_ready = lds_attr_once(attr_devs, (const void*)k, lds);
+  if constexpr (WM == 1) {
+    bool taken = false;
+    if (const int e = k8_instead<DT, OUT>(a, own_ready, s, &taken); e || taken) return e;
+  }
+  if (own_ready != 0) return own_ready;
   AG_LAUNCH_KERNEL(k, dim3(grid), dim3(WM * 256), lds, s, a);
   return (int)hipGetLastError();
 }
@@ -224,7 +335,8 @@ const char* check_streamdb(const astergemm_config& c) {
         5 * 128 * WM * kRowBytes,                                                \
         (const void*)gemm_streamdb_kernel<DT, OUT, NSLOT, NBUF, WM>,             \
         launch_streamdb<DT, OUT, NSLOT, NBUF, WM>, check_streamdb,               \
-        ASTERGEMM_OPERAND_DIRECT_B_K8                                            \
+        ASTERGEMM_OPERAND_DIRECT_B_K8, nullptr, nullptr, 0,                      \
+        WM == 1 ? k8_describe<DT, OUT> : nullptr, WM == 1                        \
   }
 
 // ---- A and B pre-shuffled, both loaded straight into MFMA operands, no LDS
@@ -278,13 +390,18 @@ int launch_stream4db(const GemmArgs& a, int grid, hipStream_t s) {
   if constexpr (SAL) k = gemm_stream4dbl_kernel<DT, OUT>;
   else k = gemm_stream4db_kernel<DT, OUT>;
   static std::atomic<uint64_t> attr_devs{0};
-  if (int e = lds_attr_once(attr_devs, (const void*)k, lds)) return e;
-  // what the kernel's indexing assumes: whole 64-row groups of B, an even number of whole
+  // what the kernels' indexing assumes: whole 64-row groups of B, an even number of whole
   // K-steps, packed B, A scale rows fetched in 16-byte granules
   if (a.N % 64 != 0 || a.N < 64 || a.M < 8 || a.M % 8 != 0 || a.K % 512 != 0 || a.tail_granules != 0 ||
       a.ldb_bytes != (int64_t)a.K / 2 || (((uintptr_t)a.mx_a | (uintptr_t)a.mx_b) & 15) != 0 ||
       a.mx_ld % 16 != 0)
     return (int)hipErrorInvalidValue;
+  const int own_ready = lds_attr_once(attr_devs, (const void*)k, lds);
+  if constexpr (SAL) {
+    bool taken = false;
+    if (const int e = k8_instead<DT, OUT>(a, own_ready, s, &taken); e || taken) return e;
+  }
+  if (own_ready != 0) return own_ready;
   AG_LAUNCH_KERNEL(k, dim3(grid), dim3(256), lds, s, a);
   return (int)hipGetLastError();
 }
@@ -307,7 +424,8 @@ const char* check_stream4db(const astergemm_config& c) {
             : (const void*)gemm_stream4db_kernel<DT, OUT>,                       \
         launch_stream4db<DT, OUT, SAL>, check_stream4db,                         \
         ASTERGEMM_OPERAND_DIRECT_B_K8, nullptr, nullptr,                         \
-        SAL ? ASTERGEMM_MX_LANES128 : ASTERGEMM_MX_ROWS                          \
+        SAL ? ASTERGEMM_MX_LANES128 : ASTERGEMM_MX_ROWS,                         \
+        SAL ? k8_describe<DT, OUT> : nullptr, SAL                                \
   }
 
 // ---- fp8, B pre-shuffled into step order and loaded straight into MFMA operands: 128 x 256
@@ -317,11 +435,14 @@ int launch_stream8db(const GemmArgs& a, int grid, hipStream_t s) {
   constexpr int lds = 4 * 128 * kRowBytes;
   auto k = gemm_stream8db_kernel<DT, OUT>;
   static std::atomic<uint64_t> attr_devs{0};
-  if (int e = lds_attr_once(attr_devs, (const void*)k, lds)) return e;
-  // what the kernel's indexing assumes: whole 16-row blocks of B, whole K-steps, packed B
+  // what the kernels' indexing assumes: whole 16-row blocks of B, whole K-steps, packed B
   if (a.N % 16 != 0 || a.N < 16 || a.M < 8 || a.M % 8 != 0 || a.K % 128 != 0 || a.tail_granules != 0 ||
       a.ldb_bytes != (int64_t)a.K)
     return (int)hipErrorInvalidValue;
+  const int own_ready = lds_attr_once(attr_devs, (const void*)k, lds);
+  bool taken = false;
+  if (const int e = k8_instead<DT, OUT>(a, own_ready, s, &taken); e || taken) return e;
+  if (own_ready != 0) return own_ready;
   AG_LAUNCH_KERNEL(k, dim3(grid), dim3(256), lds, s, a);
   return (int)hipGetLastError();
 }
@@ -341,7 +462,8 @@ const char* check_stream8db(const astergemm_config& c) {
     name, ASTERGEMM_KERNEL_TILE, DT, OUT, 128, 256, kRowBytes, 1, 4, 4, 2,       \
         4 * 128 * kRowBytes,                                                     \
         (const void*)gemm_stream8db_kernel<DT, OUT>, launch_stream8db<DT, OUT>,  \
-        check_stream8db, ASTERGEMM_OPERAND_DIRECT_B_K8                           \
+        check_stream8db, ASTERGEMM_OPERAND_DIRECT_B_K8, nullptr, nullptr, 0,     \
+        k8_describe<DT, OUT>, true                                               \
   }
 
 // ---- split K on the 128x128 kernel --------------------------------------------------------

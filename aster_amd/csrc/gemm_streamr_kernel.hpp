@@ -25,7 +25,21 @@
 namespace astergemm {
 namespace {
 
-template <int DT, int OUT, int BM, int BN, int WM, int WN, int NS>
+// Bases of a wave's transfers of pre-shuffled weights (K8): 8-row group x of the tile is half x & 1 of a block of 16
+// rows; a block past the end reads the last one (products that the epilogue does not store).
+template <class Plan>
+__device__ __forceinline__ void block_bases(const uint8_t* mat, int64_t row_bytes_, int tile_row0, int wave, int rows,
+                                            const uint8_t* (&out)[Plan::LH]) {
+#pragma unroll
+  for (int j = 0; j < Plan::LH; ++j) {
+    const int x = Plan::tile(wave, j);
+    int blk = (tile_row0 >> 4) + (x >> 1);
+    blk = blk < (rows >> 4) ? blk : (rows >> 4) - 1;
+    out[j] = mat + (int64_t)blk * 16 * row_bytes_ + (x & 1) * 1024;
+  }
+}
+
+template <int DT, int OUT, int BM, int BN, int WM, int WN, int NS, bool K8>
 __device__ __forceinline__ void gemm_streamr_body(const GemmArgs& p, int bid) {
   constexpr int NW = WM * WN;
   constexpr int TM = BM / WM / 16;
@@ -58,14 +72,16 @@ __device__ __forceinline__ void gemm_streamr_body(const GemmArgs& p, int bid) {
   const int lrow = lane >> 3;
   const int g_lane = (lane & 7) ^ (((wave * 8 + lrow) >> 1) & 7);
   const unsigned a_off = (unsigned)(lrow * (int)p.lda_bytes + g_lane * 16);
-  const unsigned b_off = (unsigned)(lrow * (int)p.ldb_bytes + g_lane * 16);
+  const unsigned b_off = K8 ? lane * 16 : (unsigned)(lrow * (int)p.ldb_bytes + g_lane * 16);
   const uint8_t* a_base[LA];
   const uint8_t* b_base[LB];
+  constexpr int B_STEP = K8 ? 16 * kRowBytes : kRowBytes;  // from one K-step of B to the next
   group_bases<PlanA>(p.A, p.lda_bytes, row0, wave, p.M, a_base);
-  group_bases<PlanB>(p.B, p.ldb_bytes, col0, wave, p.N, b_base);
+  if constexpr (K8) block_bases<PlanB>(p.B, p.ldb_bytes, col0, wave, p.N, b_base);
+  else group_bases<PlanB>(p.B, p.ldb_bytes, col0, wave, p.N, b_base);
   const int nk = p.ksteps - (p.tail_granules ? 1 : 0);  // whole 128-byte steps
 
-  const int first = first_step_of_xcd(p, nk);
+  const int first = K8 && DT == ASTERGEMM_FP8_E4M3 ? 0 : first_step_of_xcd(p, nk);
   auto g2s = [&](const uint8_t* base, unsigned voff, uint8_t* dst) {
     const unsigned m0v = (unsigned)(size_t)AG_LDS(dst);
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
@@ -77,7 +93,7 @@ __device__ __forceinline__ void gemm_streamr_body(const GemmArgs& p, int bid) {
     g2s(a_base[j] + (int64_t)step_from(first, k, nk) * kRowBytes, a_off, lds + stage * STAGE + PlanA::lds_offset(wave, j));
   };
   auto issue_b1 = [&](int k, int stage, int j) {
-    g2s(b_base[j] + (int64_t)step_from(first, k, nk) * kRowBytes, b_off,
+    g2s(b_base[j] + (int64_t)step_from(first, k, nk) * B_STEP, b_off,
         lds + stage * STAGE + B_AT + PlanB::lds_offset(wave, j));
   };
 
@@ -87,6 +103,9 @@ __device__ __forceinline__ void gemm_streamr_body(const GemmArgs& p, int bid) {
 #pragma unroll
   for (int s = 0; s < 2; ++s)
     rd_off[s] = (unsigned)(li * kRowBytes + (((s * 4 + lq) ^ (li >> 1)) << 4));
+  unsigned rd_b[2];  // K8: a block of 16 rows is 2 KiB, lane for lane the fragments of its two halves
+#pragma unroll
+  for (int s = 0; s < 2; ++s) rd_b[s] = K8 ? (unsigned)(s * 1024 + lane * 16) : rd_off[s];
   const unsigned a_rd = (unsigned)(wm * TM * 16 * kRowBytes);
   const unsigned b_rd = (unsigned)(B_AT + wn * TN * 16 * kRowBytes);
   i32x4 fa[2][TM], fb[2][TN];
@@ -94,7 +113,7 @@ __device__ __forceinline__ void gemm_streamr_body(const GemmArgs& p, int bid) {
     constexpr int S = decltype(sub)::value;
     constexpr int I = decltype(idx)::value;
     const uint8_t* st = lds + decltype(stage)::value * STAGE;
-    if constexpr (I < TN) fb[S][I] = *(const i32x4*)(st + b_rd + I * 16 * kRowBytes + rd_off[S]);
+    if constexpr (I < TN) fb[S][I] = *(const i32x4*)(st + b_rd + I * 16 * kRowBytes + rd_b[S]);
     else fa[S][I - TN] = *(const i32x4*)(st + a_rd + (I - TN) * 16 * kRowBytes + rd_off[S]);
   };
 
@@ -190,7 +209,7 @@ __device__ __forceinline__ void gemm_streamr_body(const GemmArgs& p, int bid) {
 // are the same).  64 accumulators leave room for two whole sets of fragments (2 x 64 registers), so
 // trip k multiplies set k mod 2 and reads K-step k + 1 into the other one.  The stage is a scalar that
 // rotates from trip to trip: unrolled over six trips (both sets, three stages) it spilled 400 dwords.
-template <int DT, int OUT, int BM, int BN, int WM, int WN, int NS>
+template <int DT, int OUT, int BM, int BN, int WM, int WN, int NS, bool K8>
 __device__ __forceinline__ void gemm_stream8r_body(const GemmArgs& p, int bid) {
   constexpr int NW = WM * WN;
   constexpr int TM = BM / WM / 16;
@@ -223,14 +242,16 @@ __device__ __forceinline__ void gemm_stream8r_body(const GemmArgs& p, int bid) {
   const int lrow = lane >> 3;
   const int g_lane = (lane & 7) ^ (((wave * 8 + lrow) >> 1) & 7);
   const unsigned a_off = (unsigned)(lrow * (int)p.lda_bytes + g_lane * 16);
-  const unsigned b_off = (unsigned)(lrow * (int)p.ldb_bytes + g_lane * 16);
+  const unsigned b_off = K8 ? lane * 16 : (unsigned)(lrow * (int)p.ldb_bytes + g_lane * 16);
   const uint8_t* a_base[LA];
   const uint8_t* b_base[LB];
+  constexpr int B_STEP = K8 ? 16 * kRowBytes : kRowBytes;  // from one K-step of B to the next
   group_bases<PlanA>(p.A, p.lda_bytes, row0, wave, p.M, a_base);
-  group_bases<PlanB>(p.B, p.ldb_bytes, col0, wave, p.N, b_base);
+  if constexpr (K8) block_bases<PlanB>(p.B, p.ldb_bytes, col0, wave, p.N, b_base);
+  else group_bases<PlanB>(p.B, p.ldb_bytes, col0, wave, p.N, b_base);
   const int nk = p.ksteps - (p.tail_granules ? 1 : 0);
 
-  const int first = first_step_of_xcd(p, nk);
+  const int first = K8 && DT == ASTERGEMM_FP8_E4M3 ? 0 : first_step_of_xcd(p, nk);
   auto g2s = [&](const uint8_t* base, unsigned voff, uint8_t* dst) {
     const unsigned m0v = (unsigned)(size_t)AG_LDS(dst);
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2"
@@ -242,7 +263,7 @@ __device__ __forceinline__ void gemm_stream8r_body(const GemmArgs& p, int bid) {
   auto issue1 = [&](int k, int stage, auto jc) {
     constexpr int J = decltype(jc)::value;
     if constexpr (J < LB)
-      g2s(b_base[J] + (int64_t)step_from(first, k, nk) * kRowBytes, b_off,
+      g2s(b_base[J] + (int64_t)step_from(first, k, nk) * B_STEP, b_off,
           lds + stage * STAGE + B_AT + PlanB::lds_offset(wave, J));
     else
       g2s(a_base[J - LB] + (int64_t)step_from(first, k, nk) * kRowBytes, a_off,
@@ -254,6 +275,9 @@ __device__ __forceinline__ void gemm_stream8r_body(const GemmArgs& p, int bid) {
 #pragma unroll
   for (int h = 0; h < 2; ++h)
     rd_off[h] = (unsigned)(li * kRowBytes + (((h * 4 + lq) ^ (li >> 1)) << 4));
+  unsigned rd_b[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) rd_b[h] = K8 ? (unsigned)(h * 1024 + lane * 16) : rd_off[h];
   const unsigned a_rd = (unsigned)(wm * TM * 16 * kRowBytes);
   const unsigned b_rd = (unsigned)(B_AT + wn * TN * 16 * kRowBytes);
   i32x8 fa[2][TM], fb[2][TN];
@@ -262,7 +286,7 @@ __device__ __forceinline__ void gemm_stream8r_body(const GemmArgs& p, int bid) {
     constexpr int S = decltype(set)::value;
     constexpr int F = decltype(idx)::value / 2, H = decltype(idx)::value % 2;
     const unsigned at = F < TN ? b_rd + F * 16 * kRowBytes : a_rd + (F - TN) * 16 * kRowBytes;
-    const i32x4 v = *(const i32x4*)(lds + stage * STAGE + at + rd_off[H]);
+    const i32x4 v = *(const i32x4*)(lds + stage * STAGE + at + (F < TN ? rd_b[H] : rd_off[H]));
     i32x8* f;
     if constexpr (F < TN) f = &fb[S][F];
     else f = &fa[S][F - TN];
@@ -345,10 +369,10 @@ __device__ __forceinline__ void gemm_stream8r_body(const GemmArgs& p, int bid) {
   stream_epilogue<OUT, BM, BN, WM, WN, NS * STAGE>(p, acc, lds, wave, row0, col0);
 }
 
-template <int DT, int OUT, int BM, int BN, int WM, int WN, int NS>
+template <int DT, int OUT, int BM, int BN, int WM, int WN, int NS, bool K8 = false>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_streamr_kernel(const GemmArgs p) {
-  if constexpr (DT == ASTERGEMM_FP8_E4M3) gemm_stream8r_body<DT, OUT, BM, BN, WM, WN, NS>(p, blockIdx.x);
-  else gemm_streamr_body<DT, OUT, BM, BN, WM, WN, NS>(p, blockIdx.x);
+  if constexpr (DT == ASTERGEMM_FP8_E4M3) gemm_stream8r_body<DT, OUT, BM, BN, WM, WN, NS, K8>(p, blockIdx.x);
+  else gemm_streamr_body<DT, OUT, BM, BN, WM, WN, NS, K8>(p, blockIdx.x);
 }
 
 // Split K (see gemm_stream_splitk_kernel): copy s of the tile grid multiplies K steps
@@ -362,8 +386,8 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_streamr_splitk_kernel(const 
   q.A = p.A + (int64_t)ks * p.ksteps * kRowBytes;
   q.B = p.B + (int64_t)ks * p.ksteps * kRowBytes;
   q.C = p.workspace + (int64_t)ks * p.M * p.N;
-  if constexpr (DT == ASTERGEMM_FP8_E4M3) gemm_stream8r_body<DT, ASTERGEMM_F32, BM, BN, WM, WN, NS>(q, bid);
-  else gemm_streamr_body<DT, ASTERGEMM_F32, BM, BN, WM, WN, NS>(q, bid);
+  if constexpr (DT == ASTERGEMM_FP8_E4M3) gemm_stream8r_body<DT, ASTERGEMM_F32, BM, BN, WM, WN, NS, false>(q, bid);
+  else gemm_streamr_body<DT, ASTERGEMM_F32, BM, BN, WM, WN, NS, false>(q, bid);
 }
 
 }  // namespace
