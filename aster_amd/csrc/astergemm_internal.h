@@ -44,6 +44,34 @@ __host__ __device__ inline int64_t row_bytes(int dtype, int64_t k) {
   }
 }
 
+// The same in one 64-byte line, for the kernels of products that a launch is a good part of.  A launch writes its
+// arguments to device memory, across PCIe: one line costs the host 2.9 us, two 3.5, the 144 bytes of GemmArgs 3.6
+// (empty kernels).  Addresses have 48 bits, row pitches of A and B 23 (validate_problem), in units of 16 bytes 19,
+// with bits 32 ... 57 of C's above them; everything else follows from M, N and K.
+struct PackedArgs {
+  uint32_t lo[6];       // A, B, C (K ranges: the workspace), bias, scale_a or mx_a, scale_b or mx_b
+  uint16_t hi[6];
+  int32_t M, N, K;
+  uint32_t lda, ldb, ldc;
+  uint32_t form;        // the kernel's own
+};
+static_assert(sizeof(PackedArgs) == 64, "one line");
+inline PackedArgs pack_args(const GemmArgs& a, uint32_t form, const void* c) {
+  const void* ptr[6] = {a.A, a.B, c, a.bias, a.mx_a ? a.mx_a : (const void*)a.scale_a,
+                        a.mx_b ? a.mx_b : (const void*)a.scale_b};
+  PackedArgs q;
+  for (int i = 0; i < 6; ++i) {
+    q.lo[i] = (uint32_t)(uintptr_t)ptr[i];
+    q.hi[i] = (uint16_t)((uintptr_t)ptr[i] >> 32);
+  }
+  q.M = a.M, q.N = a.N, q.K = a.K;
+  q.lda = (uint32_t)(a.lda_bytes >> 4) | (uint32_t)((uint64_t)a.ldc >> 32 & 0x1FFF) << 19;
+  q.ldb = (uint32_t)(a.ldb_bytes >> 4) | (uint32_t)((uint64_t)a.ldc >> 45 & 0x1FFF) << 19;
+  q.ldc = (uint32_t)a.ldc;
+  q.form = form;
+  return q;
+}
+
 inline int out_elt_bytes(int dtype) { return dtype == ASTERGEMM_F32 ? 4 : 2; }
 
 // What a launcher with several kernels launches for one problem.

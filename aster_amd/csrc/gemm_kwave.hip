@@ -29,7 +29,7 @@ namespace astergemm {
 struct KwaveShape {
   int bm, bn, wm, wn, wk, stages, lds;
   const void* func;
-  int (*launch)(const KwaveArgs& q, int grid, hipStream_t s);
+  int (*launch)(const PackedArgs& q, int grid, hipStream_t s);
 };
 constexpr int kKwaveShapes = 16;
 template <int DT, bool K8>
@@ -38,7 +38,7 @@ const KwaveShape* kwave_shapes();
 namespace {
 
 template <int DT, bool K8, int BM, int BN, int WM, int WN, int WK, int S>
-int launch_kwave(const KwaveArgs& q, int grid, hipStream_t s) {
+int launch_kwave(const PackedArgs& q, int grid, hipStream_t s) {
   constexpr int lds = S * WK * kwave_step_bytes(DT, K8, BM, BN);
   AG_LAUNCH_KERNEL((gemm_kwave_kernel<DT, K8, BM, BN, WM, WN, WK, S>), dim3(grid), dim3(WM * WN * WK * 64), lds, s,
                    q);
@@ -303,13 +303,10 @@ int kwave_ready(int dt, bool k8) {
 
 int kwave_launch(int dt, int out, const GemmArgs& a, const KwaveForm& f, hipStream_t s) {
   const KwaveShape& sh = shapes_of(dt, f.k8)[f.shape];
-  KwaveArgs q;
-  q.g = a;
-  q.g.tiles_m = (a.M + sh.bm - 1) / sh.bm;
-  q.g.tiles_n = (a.N + f.per - 1) / f.per;
+  const int tiles_m = (a.M + sh.bm - 1) / sh.bm, tiles_n = (a.N + f.per - 1) / f.per;
+  KwaveForm32 q;
   q.per = f.per;
   q.ranges = f.ranges;
-  q.range_steps = (a.ksteps + f.ranges - 1) / f.ranges;
   q.out = out;
   // Past the last-level cache where that is no use: a matrix of more than 64 MiB is not found there again
   // after a few others; with few activation rows for the panel's the loop is the weight stream and little
@@ -319,15 +316,16 @@ int kwave_launch(int dt, int out, const GemmArgs& a, const KwaveForm& f, hipStre
   // 64x14336x4096 12.3 / 14.1 and 16.7 / 14.7, 16x1024x8192 5.7 / 6.5 and 5.8 / 6.9.  Not where two tile rows
   // share a panel in L2 (bf16 64x4096x4096 8.9 / 11.8 and 12.5 / 12.2).
   const int64_t mib = (int64_t)a.N * row_bytes(dt, a.K) >> 20;
-  q.nt = a.M <= 64 && q.g.tiles_m == 1 && (mib > 64 || (mib >= 30 && (a.M <= 8 || (a.M <= 16 && f.per >= 48))));
-  q.blocks = kwave_blocks(q.g.tiles_m, q.g.tiles_n, device_cus(), &q.by_panel);
+  q.nt = a.M <= 64 && tiles_m == 1 && (mib > 64 || (mib >= 30 && (a.M <= 8 || (a.M <= 16 && f.per >= 48))));
+  q.blocks = kwave_blocks(tiles_m, tiles_n, device_cus(), &q.by_panel);
   const int grid = q.blocks * f.ranges;
-  if (f.ranges == 1) return sh.launch(q, grid, s);
+  if (f.ranges == 1) return sh.launch(pack_args(a, q.bits(), a.C), grid, s);
   std::unique_lock<std::mutex> order(splitk_order());
-  if (!q.g.workspace)
-    if (int rc = splitk_workspace_for((size_t)f.ranges * a.M * a.N * sizeof(float), s, &q.g.workspace)) return rc;
-  if (int e = sh.launch(q, grid, s)) return e;
-  return splitk_reduce(out, q.g, f.ranges, s);
+  GemmArgs g = a;
+  if (!g.workspace)
+    if (int rc = splitk_workspace_for((size_t)f.ranges * a.M * a.N * sizeof(float), s, &g.workspace)) return rc;
+  if (int e = sh.launch(pack_args(g, q.bits(), g.workspace), grid, s)) return e;
+  return splitk_reduce(out, g, f.ranges, s);
 }
 
 void kwave_describe(int dt, const KwaveForm& f, int64_t M, int64_t N, int cus, LaunchForm* o) {

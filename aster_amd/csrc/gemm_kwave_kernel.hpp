@@ -29,15 +29,20 @@
 namespace astergemm {
 namespace {
 
-struct KwaveArgs {
-  GemmArgs g;
-  int32_t per;          // weight rows of a workgroup (a multiple of 8, at most BN)
-  int32_t ranges;       // K ranges (1: the result; more: fp32 planes in g.workspace)
-  int32_t range_steps;  // K-steps of a range
-  int32_t blocks;       // workgroups of a range
-  int32_t by_panel;     // the tile rows of a panel on one XCD (else tile after tile, whatever the XCD)
-  int32_t out;          // output type
-  int32_t nt;           // weights are fetched past the last-level cache
+// What PackedArgs::form says: weight rows of a workgroup (a multiple of 8, at most BN), K ranges (1: the result;
+// more: fp32 planes in the workspace), output type, whether weights are fetched past the last-level cache, whether the
+// tile rows of a panel are on one XCD (else tile after tile, whatever the XCD), and with K ranges the workgroups of
+// one.
+struct KwaveForm32 {
+  int per, ranges, out, nt, by_panel, blocks;
+  __host__ __device__ uint32_t bits() const {
+    return (uint32_t)(per >> 3) | (uint32_t)ranges << 5 | (uint32_t)out << 10 | (uint32_t)nt << 13 |
+           (uint32_t)by_panel << 14 | (uint32_t)(ranges > 1 ? blocks : 0) << 16;
+  }
+  __host__ __device__ static KwaveForm32 of(uint32_t b) {
+    return KwaveForm32{(int)(b & 31) << 3, (int)(b >> 5 & 31), (int)(b >> 10 & 7), (int)(b >> 13 & 1),
+                       (int)(b >> 14 & 1), (int)(b >> 16)};
+  }
 };
 
 // 32-row transfers of e8m0 bytes per K-step (K8: of each operand by itself)
@@ -49,7 +54,7 @@ constexpr int kwave_step_bytes(int dt, bool k8, int bm, int bn) {  // LDS of one
 }
 
 template <int DT, bool K8, int BM, int BN, int WM, int WN, int WK, int S>
-__global__ __launch_bounds__(WM* WN* WK * 64) void gemm_kwave_kernel(const KwaveArgs q) {
+__global__ __launch_bounds__(WM* WN* WK * 64) void gemm_kwave_kernel(const PackedArgs args) {
   constexpr int GW = WM * WN;                   // waves of a group
   constexpr int NW = GW * WK;
   constexpr int TM = BM / WM / 16, TN = BN / WN / 16;
@@ -66,7 +71,9 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_kwave_kernel(const Kwave
   static_assert(S * STAGE <= 160 * 1024 && WK * NT * 1024 <= S * STAGE, "LDS of a CU");
 
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
-  const GemmArgs& p = q.g;
+  const GemmArgs p = unpack_args<DT>(args);
+  const KwaveForm32 q = KwaveForm32::of(args.form);
+  const int tiles_m = (p.M + BM - 1) / BM;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wk = wave / GW, wv = wave % GW, wm = wv / WN, wn = wv % WN;
@@ -74,15 +81,19 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_kwave_kernel(const Kwave
   // block b runs on XCD b % 8: the tile rows of a weight panel side by side on one XCD, the panels round
   // robin over the XCDs (runs of neighbouring panels per XCD: fp8 8x8192x8192 11.0 -> 15.5 us, the panels
   // that start at the same K-step are then a large power of two apart)
-  const int blocks = q.blocks;                  // of one K range
-  const int range = blockIdx.x / blocks, bid = blockIdx.x - range * blocks;
-  const int idx = q.by_panel ? bid >> 3 : bid, panel = idx / p.tiles_m;
-  const int tile_m = idx - panel * p.tiles_m, tile_n = q.by_panel ? panel * 8 + (bid & 7) : panel;
-  if (tile_n >= p.tiles_n) return;
+  int range = 0, bid = blockIdx.x, range_steps = p.ksteps;
+  if (q.ranges > 1) {
+    range = bid / q.blocks;
+    bid -= range * q.blocks;
+    range_steps = (p.ksteps + q.ranges - 1) / q.ranges;
+  }
+  const int idx = q.by_panel ? bid >> 3 : bid, panel = idx / tiles_m;
+  const int tile_m = idx - panel * tiles_m, tile_n = q.by_panel ? panel * 8 + (bid & 7) : panel;
+  if ((int64_t)tile_n * q.per >= p.N) return;
   const int row0 = tile_m * BM, col0 = tile_n * q.per;
   const int col1 = (col0 + q.per) < p.N ? (col0 + q.per) : p.N;
-  const int k0 = range * q.range_steps;
-  const int k1 = (k0 + q.range_steps) < p.ksteps ? (k0 + q.range_steps) : p.ksteps;
+  const int k0 = range * range_steps;
+  const int k1 = (k0 + range_steps) < p.ksteps ? (k0 + range_steps) : p.ksteps;
   const int kwhole = p.tail_granules && k1 == p.ksteps ? k1 - 1 : k1;  // steps of 128 bytes
   const int nst = (k1 - k0 + WK - 1) / WK;
   const int rot = panel % nst;
@@ -349,7 +360,7 @@ __global__ __launch_bounds__(WM* WN* WK * 64) void gemm_kwave_kernel(const Kwave
     if (row >= p.M || col >= col1) continue;
     const int ncols = (col1 - col) < 4 ? (col1 - col) : 4;
     if (q.ranges > 1) {
-      store4<ASTERGEMM_F32>(p.workspace, ((int64_t)range * p.M + row) * p.N + col, v, ncols);
+      store4<ASTERGEMM_F32>(p.C, ((int64_t)range * p.M + row) * p.N + col, v, ncols);
       continue;
     }
     v *= scale;

@@ -714,14 +714,13 @@ __global__ __launch_bounds__(256) void skinny_splitk_reduce_kernel(const float* 
                                                                    int N, int64_t ldc,
                                                                    const float* scale_a,
                                                                    const float* scale_b,
-                                                                   const float* bias, void* C) {
+                                                                   const float* bias, void* C, int grid) {
   float scale = 1.0f;
   if (scale_a) scale *= *scale_a;
   if (scale_b) scale *= *scale_b;
   const int cg = (N + 3) >> 2;                     // groups of four columns per row
   const int64_t plane = (int64_t)M * N;
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < (int64_t)M * cg;
-       i += (int64_t)gridDim.x * blockDim.x) {
+  for (int64_t i = blockIdx.x * (int64_t)256 + threadIdx.x; i < (int64_t)M * cg; i += (int64_t)grid * 256) {
     const int m = (int)(i / cg), n = (int)(i - (int64_t)m * cg) * 4;
     const int ncols = (N - n) < 4 ? (N - n) : 4;
     const float* src = ws + (int64_t)m * N + n;
@@ -752,7 +751,7 @@ void launch_splitk_reduce(const GemmArgs& a, int S, hipStream_t s) {
   const int64_t total = (int64_t)a.M * ((a.N + 3) / 4);
   const int rg = (int)((total + 255) / 256 < 2048 ? (total + 255) / 256 : 2048);
   AG_LAUNCH_KERNEL(skinny_splitk_reduce_kernel<OUT>, dim3(rg), dim3(256), 0, s, a.workspace, S,
-                     a.M, a.N, a.ldc, a.scale_a, a.scale_b, a.bias, a.C);
+                     a.M, a.N, a.ldc, a.scale_a, a.scale_b, a.bias, a.C, rg);
 }
 
 // fp32 scratch for the K-split partial sums when the caller brings none: one buffer per

@@ -24,7 +24,7 @@ int launch_tile(const GemmArgs& a, int grid, hipStream_t s) {
   // the kernels that stand in for this one on small grids: a config captured later finds either ready
   if constexpr (BM == 64) (void)kwave_ready(DT);
   AG_LAUNCH_KERNEL((gemm_tile_kernel<DT, OUT, BM, BN, WM, WN, S>), dim3(grid), dim3(WM * WN * 64),
-                   tile_lds_bytes(DT, BM, BN, S), s, a);
+                   tile_lds_bytes(DT, BM, BN, S), s, pack_args(a, 0, a.C));
   return (int)hipGetLastError();
 }
 

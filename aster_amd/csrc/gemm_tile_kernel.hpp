@@ -99,6 +99,36 @@ __device__ __forceinline__ void map_tile(int bid, int tiles_m, int tiles_n,
   tn = r / rows;
 }
 
+// What a packed kernel argument says, apart from the tile grid and the workspace.
+template <int DT>
+__device__ __forceinline__ GemmArgs unpack_args(const PackedArgs& q) {
+  GemmArgs a = {};
+  auto ptr = [&](int i) {  // by way of a global pointer: loads and stores stay global ones
+    return (uint8_t*)(__attribute__((address_space(1))) uint8_t*)((uint64_t)q.hi[i] << 32 | q.lo[i]);
+  };
+  a.A = ptr(0);
+  a.B = ptr(1);
+  a.C = ptr(2);
+  a.bias = (const float*)ptr(3);
+  if constexpr (DT == ASTERGEMM_MXFP4) {
+    a.mx_a = ptr(4);
+    a.mx_b = ptr(5);
+    a.mx_ld = q.K >> 5;
+  } else {
+    a.scale_a = (const float*)ptr(4);
+    a.scale_b = (const float*)ptr(5);
+  }
+  a.M = q.M, a.N = q.N, a.K = q.K;
+  a.lda_bytes = (int64_t)(q.lda & 0x7FFFF) << 4;
+  a.ldb_bytes = (int64_t)(q.ldb & 0x7FFFF) << 4;
+  a.ldc = (int64_t)((uint64_t)(q.ldb >> 19) << 45 | (uint64_t)(q.lda >> 19) << 32 | q.ldc);
+  const unsigned rb = DT == ASTERGEMM_MXFP4 ? (unsigned)q.K >> 1 : DT == ASTERGEMM_FP8_E4M3 ? (unsigned)q.K
+                                                                                       : (unsigned)q.K * 2;
+  a.ksteps = (int)((rb + 127) >> 7);
+  a.tail_granules = (int)((rb & 127) >> 4);
+  return a;
+}
+
 template <int DT>
 struct Enc {
   // MFMA k-substeps per 128-byte row chunk and 16-byte granules per fragment.
@@ -428,7 +458,11 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p) {
 
 
 template <int DT, int OUT, int BM, int BN, int WM, int WN, int S>
-__global__ __launch_bounds__(WM* WN * 64) void gemm_tile_kernel(const GemmArgs p) {
+__global__ __launch_bounds__(WM* WN * 64) void gemm_tile_kernel(const PackedArgs q) {
+  GemmArgs p = unpack_args<DT>(q);
+  p.tiles_m = (p.M + BM - 1) / BM;
+  p.tiles_n = (p.N + BN - 1) / BN;
+  p.group_m = (p.tiles_m % 8 == 0 && p.tiles_n % 32 == 0) ? -1 : 8;
   gemm_tile_body<DT, OUT, BM, BN, WM, WN, S>(p);
 }
 

@@ -17,6 +17,8 @@
 namespace astergemm {
 namespace {
 
+// Kernels take the size of their grid as an argument: asking for it costs 256 bytes of hidden ones, and a launch
+// writes its arguments to device memory line by line (PackedArgs).
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 // Vector elements are passed by value (__float_as_uint) before their bits are taken: a bit
 // cast applied to the element expression itself read element 0 for every index.
@@ -183,9 +185,9 @@ __device__ __forceinline__ unsigned absmax_share(const void* __restrict__ src, i
 // system takes one at a time (2048 workgroups: 20 us of a 30 us call; 256: 3 us).
 template <int SRC>
 __global__ __launch_bounds__(1024) void absmax_kernel(const void* __restrict__ src, int64_t n,
-                                                      unsigned* __restrict__ out) {
+                                                      unsigned* __restrict__ out, int grid) {
   const unsigned m = block_max<16>(absmax_share<SRC, 4, false>(
-      src, n, blockIdx.x * (int64_t)1024 + threadIdx.x, (int64_t)gridDim.x * 1024));
+      src, n, blockIdx.x * (int64_t)1024 + threadIdx.x, (int64_t)grid * 1024));
   if (threadIdx.x == 0 && m != 0) atomicMax(out, m);
 }
 
@@ -272,10 +274,10 @@ constexpr int kFp8CounterBytes = kFp8Counters * kFp8CounterPitch * 4;
 template <int SRC>
 __global__ __launch_bounds__(256) void fp8_absmax_kernel(const void* __restrict__ src, int64_t n,
                                                          unsigned* __restrict__ partial,
-                                                         unsigned* __restrict__ counter) {
-  if (blockIdx.x == 0 && threadIdx.x < kFp8Counters) partial[gridDim.x + threadIdx.x * kFp8CounterPitch] = 0u;
+                                                         unsigned* __restrict__ counter, int grid) {
+  if (blockIdx.x == 0 && threadIdx.x < kFp8Counters) partial[grid + threadIdx.x * kFp8CounterPitch] = 0u;
   const unsigned m = block_max<4>(absmax_share<SRC, 8, true>(
-      src, n, blockIdx.x * (int64_t)256 + threadIdx.x, (int64_t)gridDim.x * 256));
+      src, n, blockIdx.x * (int64_t)256 + threadIdx.x, (int64_t)grid * 256));
   if (threadIdx.x == 0) {
     partial[blockIdx.x] = m;
     if (blockIdx.x == 0) *counter = 0u;
@@ -293,13 +295,13 @@ __global__ __launch_bounds__(256) void fp8_absmax_kernel(const void* __restrict_
 template <int SRC>
 __global__ __launch_bounds__(1024) void quantize_fp8_kernel(const void* __restrict__ src, int64_t n, int np,
                                                            uint8_t* __restrict__ dst,
-                                                           float* __restrict__ scale) {
+                                                           float* __restrict__ scale, int grid) {
   constexpr int NE = Src<SRC>::kPer, U = 4;
   __shared__ bool last;
   const i32x4* g = (const i32x4*)src;
-  const bool two_levels = gridDim.x > 4 * kFp8Counters;
+  const bool two_levels = grid > 4 * kFp8Counters;
   const int64_t ng = n / NE, head = ((int64_t)np * 4 + (two_levels ? kFp8CounterBytes : 0)) / NE;
-  const int64_t stride = (int64_t)gridDim.x * 1024;
+  const int64_t stride = (int64_t)grid * 1024;
   int64_t i = head + blockIdx.x * (int64_t)1024 + threadIdx.x;
   i32x4 v[U];
   auto fetch = [&]() {
@@ -328,9 +330,9 @@ __global__ __launch_bounds__(1024) void quantize_fp8_kernel(const void* __restri
   for (int64_t j = ng * NE + blockIdx.x * (int64_t)1024 + threadIdx.x; j < n; j += stride)
     dst[j] = (uint8_t)sc.code(load1<SRC>(src, j));
   if (threadIdx.x == 0) {
-    const unsigned of_c = (gridDim.x - c + kFp8Counters - 1) / kFp8Counters;
+    const unsigned of_c = (grid - c + kFp8Counters - 1) / kFp8Counters;
     last = two_levels ? ticket == of_c - 1 && atomicAdd((unsigned*)scale, 1u) == kFp8Counters - 1
-                      : ticket == gridDim.x - 1;
+                      : ticket == (unsigned)grid - 1;
   }
   __syncthreads();
   if (!last) return;
@@ -415,10 +417,10 @@ __global__ __launch_bounds__(256) void quantize_mxfp4_kernel(const void* __restr
                                                              int64_t nblocks, unsigned bpr,
                                                              int64_t ld,
                                                              uint8_t* __restrict__ packed,
-                                                             uint8_t* __restrict__ scales) {
+                                                             uint8_t* __restrict__ scales, int grid) {
   constexpr int U = 4, PB = Mx4Group<SRC>::kPB;
   const int64_t ngroups = nblocks * PB;
-  const int64_t step = (int64_t)gridDim.x * 256;
+  const int64_t step = (int64_t)grid * 256;
   for (int64_t base = blockIdx.x * (int64_t)256 + threadIdx.x; base < ngroups; base += U * step) {
     i32x4 v[U];
 #pragma unroll
@@ -542,7 +544,7 @@ extern "C" int astergemm_absmax(const void* dSrc, int src_dtype, int64_t n, floa
       constexpr int SRC = decltype(T)::value;
       const int64_t b = (n / Src<SRC>::kPer + 4 * 1024) / (4 * 1024);
       hipLaunchKernelGGL(absmax_kernel<SRC>, dim3((unsigned)(b < 256 ? b : 256)), dim3(1024), 0, s, dSrc,
-                         n, (unsigned*)dAbsmax);
+                         n, (unsigned*)dAbsmax, (int)(b < 256 ? b : 256));
     });
   AG_HIP(hipGetLastError());
   return 0;
@@ -571,12 +573,12 @@ extern "C" int astergemm_quantize_fp8_tensor(const void* dSrc, int src_dtype, in
     int64_t np = ((ng + 4 * 256 - 1) / (4 * 256) + 31) & ~(int64_t)31;
     if (np > 1024) np = 1024;
     hipLaunchKernelGGL(fp8_absmax_kernel<SRC>, dim3((unsigned)np), dim3(256), 0, s, dSrc, n,
-                       (unsigned*)dDst, (unsigned*)dScale);
+                       (unsigned*)dDst, (unsigned*)dScale, (int)np);
     // a workgroup per CU, two from 2^25 elements on (bf16, one / two: 4096 x 4096 19.5 / 20.4 us, 4096 x 14336
     // 57.5 / 55.7, 8192 x 8192 73.3 / 72.0)
     const int64_t b = (ng + 1023) / 1024, cap = n < ((int64_t)1 << 25) ? 256 : 512;
     hipLaunchKernelGGL(quantize_fp8_kernel<SRC>, dim3((unsigned)(b < cap ? b : cap)), dim3(1024), 0, s,
-                       dSrc, n, (int)np, dDst, dScale);
+                       dSrc, n, (int)np, dDst, dScale, (int)(b < cap ? b : cap));
   });
   AG_HIP(hipGetLastError());
   return 0;
@@ -615,7 +617,7 @@ extern "C" int astergemm_quantize_mxfp4_ex(const void* dSrc, int src_dtype, int6
     }
     const dim3 grid(blocks_for((nblocks * Mx4Group<SRC>::kPB + 3) / 4));  // four groups per thread
     auto go = [&](auto kern) {
-      hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, dSrc, nblocks, bpr, ld_src, dPacked, dScales);
+      hipLaunchKernelGGL(kern, grid, dim3(256), 0, st, dSrc, nblocks, bpr, ld_src, dPacked, dScales, (int)grid.x);
     };
     if (ld_src == K) go(quantize_mxfp4_kernel<SRC, true>);
     else go(quantize_mxfp4_kernel<SRC, false>);
