@@ -10,12 +10,14 @@ call fails, an exception is raised.
 from __future__ import annotations
 
 import ctypes as C
+import importlib.machinery
 import importlib.util
 import os
 import sys
 from typing import Optional
 
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libastergemm.so")
+_FASTCALL_PATH = os.path.join(os.path.dirname(_LIB_PATH), "aster_fastcall.so")
 
 # astergemm_dtype
 F16, BF16, FP8_E4M3, MXFP4, F32 = 0, 1, 2, 3, 4
@@ -180,6 +182,7 @@ SIGNATURES = {
 }
 
 _lib: Optional[C.CDLL] = None
+fast_run = None  # astergemm_run without ctypes (csrc/fastcall.c); set by load()
 
 
 def library_path() -> str:
@@ -209,13 +212,15 @@ def _bind_one_hip_runtime() -> None:
 
 def load() -> C.CDLL:
     """Load libastergemm.so and attach the prototypes. Raises if it is not built."""
-    global _lib
+    global _lib, fast_run
     if _lib is not None:
         return _lib
     _bind_one_hip_runtime()
-    if not os.path.exists(_LIB_PATH):
+    for path in (_LIB_PATH, _FASTCALL_PATH):
+        if os.path.exists(path):
+            continue
         raise FileNotFoundError(
-            f"{_LIB_PATH} is not built; run `python -m aster_amd.build` "
+            f"{path} is not built; run `python -m aster_amd.build` "
             "(needs hipcc; cross-compiles for gfx950 without a GPU)"
         )
     lib = C.CDLL(_LIB_PATH)
@@ -223,6 +228,11 @@ def load() -> C.CDLL:
         fn = getattr(lib, name)  # AttributeError if the symbol is missing
         fn.restype = restype
         fn.argtypes = argtypes
+    loader = importlib.machinery.ExtensionFileLoader("aster_fastcall", _FASTCALL_PATH)
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("aster_fastcall", loader))
+    loader.exec_module(module)
+    module.bind(C.cast(lib.astergemm_run, C.c_void_p).value)
+    fast_run = module.run
     _lib = lib
     return lib
 

@@ -12,6 +12,7 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 from concurrent.futures import ThreadPoolExecutor
 
 from .asm_scan import (MFMA_WAIT_STATES, VMEM_SGPR_WAIT_STATES, scan_mfma_hazards,  # noqa: F401
@@ -44,6 +45,7 @@ UNITS = [("gemm_stream_p0", "gemm_stream.hip", ["-DAG_STREAM_PART=0"]),
 HSACO_SOURCE = "hsaco_kernels.hip"
 HSACO_PATH = os.path.join(LIB_DIR, "astergemm_kernels.hsaco")
 REPLAY_PATH = os.path.join(LIB_DIR, "astergemm_replay")
+FASTCALL_PATH = os.path.join(LIB_DIR, "aster_fastcall.so")
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
@@ -157,6 +159,12 @@ def build_library(verbose: bool = False, only=None) -> str:
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"replay tool build failed:\n{proc.stdout}\n{proc.stderr}")
+    # the CPython binding of the launch (no GPU code, linked to nothing: _capi binds it to the library)
+    cmd = ["gcc", "-O2", "-shared", "-fPIC", "-Wall", "-I" + sysconfig.get_paths()["include"],
+           "-I" + os.path.join(ROOT, "include"), os.path.join(CSRC, "fastcall.c"), "-o", FASTCALL_PATH]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"fastcall build failed:\n{proc.stdout}\n{proc.stderr}")
     if verbose:
         print(f"built {LIB_PATH}")
     return LIB_PATH

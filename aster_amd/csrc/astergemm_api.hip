@@ -75,7 +75,7 @@ int device_cus() {
     }
   }
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) {
+  if (current_device(&dev) != hipSuccess) {
     (void)hipGetLastError();
     return 0;
   }
@@ -184,7 +184,7 @@ thread_local int g_choice_cache_used = 0, g_choice_cache_next = 0;
 
 int current_device_or_minus_one() {
   int dev = -1;
-  if (hipGetDevice(&dev) != hipSuccess) {
+  if (current_device(&dev) != hipSuccess) {
     (void)hipGetLastError();
     dev = -1;
   }
@@ -910,6 +910,8 @@ int astergemm_run(const astergemm_config* cfg, const astergemm_operands* ops, vo
     set_error("astergemm_run: null argument");
     return ASTERGEMM_EINVAL;
   }
+  LaunchScope scope(stream);
+  launch_context().dev = current_device_or_minus_one();
   const Variant* other = nullptr;
   const Variant* v = choose_for_call(*cfg, *ops, stream, &other);
   if (!v) return g_choose_rc;
@@ -917,11 +919,8 @@ int astergemm_run(const astergemm_config* cfg, const astergemm_operands* ops, vo
   GemmArgs a;
   if (int rc = build_args(*v, *cfg, *ops, &a)) return rc;
   (void)hipGetLastError();  // the launchers report hipGetLastError(): drop what an earlier call left
-  {
-    LaunchScope scope(stream);
-    const int e = v->launch(a, grid_of(*v, *cfg), (hipStream_t)stream);
-    if (e != 0) return launch_fail(e, v->name, __FILE__, __LINE__);
-  }
+  if (const int e = v->launch(a, grid_of(*v, *cfg), (hipStream_t)stream); e != 0)
+    return launch_fail(e, v->name, __FILE__, __LINE__);
   ready_other(other, *cfg, stream);
   return 0;
 }

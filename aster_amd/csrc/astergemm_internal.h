@@ -126,8 +126,18 @@ int device_cus();
 struct LaunchContext {
   hipStream_t stream = nullptr;
   bool prepare_only = false;
+  int dev = -1;  // the thread's device for the length of the call; -1: not asked for
 };
 LaunchContext& launch_context();
+// The current device: asked for once by an entry point that has set it in the context (50 ns a time, and a call
+// needs it in half a dozen places).
+inline hipError_t current_device(int* dev) {
+  if (const int d = launch_context().dev; d >= 0) {
+    *dev = d;
+    return hipSuccess;
+  }
+  return hipGetDevice(dev);
+}
 
 // Every GEMM kernel launch of the library goes through this macro.
 #define AG_LAUNCH_KERNEL(...)                                                   \
@@ -142,7 +152,7 @@ LaunchContext& launch_context();
 // of touching the runtime from inside the capture; astergemm_prepare does this step ahead of time.
 inline int lds_attr_once(std::atomic<uint64_t>& devs, const void* func, int lds_bytes) {
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return (int)hipGetLastError();
+  if (current_device(&dev) != hipSuccess) return (int)hipGetLastError();
   const uint64_t bit = (uint64_t)1 << (dev & 63);
   if (devs.load(std::memory_order_acquire) & bit) return 0;
   hipStreamCaptureStatus st = hipStreamCaptureStatusNone;

@@ -294,7 +294,7 @@ KwaveForm kwave_k8_form(int dt, int64_t M, int64_t N, int cus, int* rows) {
 int kwave_ready(int dt, bool k8) {
   static std::atomic<uint64_t> all[8], devs[8][kKwaveShapes];
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return (int)hipGetLastError();
+  if (current_device(&dev) != hipSuccess) return (int)hipGetLastError();
   const uint64_t bit = (uint64_t)1 << (dev & 63);
   const int set = (dt & 3) + (k8 ? 4 : 0);
   if (all[set].load(std::memory_order_acquire) & bit) return 0;
