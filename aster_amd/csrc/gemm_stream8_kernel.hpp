@@ -343,13 +343,13 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_stream8_walk_kernel(const Ge
 // applied by the kernel that adds the planes.
 template <int DT, int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_stream8_splitk_kernel(const GemmArgs p) {
-  const int tiles = p.tiles_m * p.tiles_n;
-  const int ks = blockIdx.x / tiles;
+  int ks, bid;
+  place_range(blockIdx.x, p.tiles_m * p.tiles_n, p.split_k, ks, bid);
   GemmArgs q = p;
   q.A = p.A + (int64_t)ks * p.ksteps * kRowBytes;
   q.B = p.B + (int64_t)ks * p.ksteps * kRowBytes;
   q.C = p.workspace + (int64_t)ks * p.M * p.N;
-  gemm_stream8_body<DT, ASTERGEMM_F32, BM, BN, WM, WN>(q, blockIdx.x - ks * tiles);
+  gemm_stream8_body<DT, ASTERGEMM_F32, BM, BN, WM, WN>(q, bid);
 }
 
 }  // namespace

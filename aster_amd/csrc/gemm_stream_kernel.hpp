@@ -518,13 +518,13 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_stream_kernel(const GemmArgs
 // For few output tiles and long rows, where the tile grid alone leaves most CUs idle.
 template <int DT, int BM, int BN, int WM, int WN, int NSLOT = 5>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_stream_splitk_kernel(const GemmArgs p) {
-  const int tiles = p.tiles_m * p.tiles_n;
-  const int ks = blockIdx.x / tiles;
+  int ks, bid;
+  place_range(blockIdx.x, p.tiles_m * p.tiles_n, p.split_k, ks, bid);
   GemmArgs q = p;
   q.A = p.A + (int64_t)ks * p.ksteps * kRowBytes;
   q.B = p.B + (int64_t)ks * p.ksteps * kRowBytes;
   q.C = p.workspace + (int64_t)ks * p.M * p.N;
-  gemm_stream_body<DT, ASTERGEMM_F32, BM, BN, WM, WN, NSLOT>(q, blockIdx.x - ks * tiles);
+  gemm_stream_body<DT, ASTERGEMM_F32, BM, BN, WM, WN, NSLOT>(q, bid);
 }
 
 }  // namespace

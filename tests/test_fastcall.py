@@ -1,0 +1,43 @@
+"""GemmPlan.run's binding of the launch (csrc/fastcall.c): what it takes, what it refuses, and that refusals are ctypes'."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from aster_amd import _capi
+from aster_amd.gemm import GemmPlan
+
+
+def empty_plan():
+    return GemmPlan.create(0, 16, 64, "bf16", "f32")   # M = 0: accepted, nothing is launched
+
+
+def test_integers_none_and_what_ctypes_takes():
+    p = empty_plan()
+    p.run(16, 32, 48)
+    p.run(16, 32, 48, bias=None, stream=0, workspace=None)
+    p.run(ctypes.c_void_p(16), 32, 48)                  # not an integer: the structure takes it
+    p.run(True, 2 ** 63 + 16, -16)                      # masked to 64 bits, as in the structure
+
+
+@pytest.mark.parametrize("bad", ["16", 1.5, np.int64(16), object()])
+def test_refusals_are_type_errors(bad):
+    p = empty_plan()
+    with pytest.raises(TypeError):
+        p.run(bad, 32, 48)
+    with pytest.raises(TypeError):
+        p.run(16, 32, 48, workspace_bytes=None)
+
+
+def test_binding_checks_its_arguments():
+    _capi.load()
+    with pytest.raises(TypeError):
+        _capi.fast_run(empty_plan().config, 1, 2, 3)
+    with pytest.raises(TypeError):
+        _capi.fast_run(ctypes.c_int(3), *[None] * 9, 0, None)
+
+
+def test_status_becomes_the_exception():
+    p = GemmPlan.create(16, 16, 64, "bf16", "f32")
+    with pytest.raises(_capi.AsterGemmError, match="non-null"):
+        p.run(0, 32, 48)

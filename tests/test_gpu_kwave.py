@@ -153,3 +153,52 @@ def test_row_pitches_above_k(gpu, M, N, K, dtype_ab, dtype_c):
     assert padded.info.variant == packed.info.variant
     assert torch.equal(got[:, :N], want[:, :N]) and bool(torch.isfinite(want[:, :N]).all())
     assert bool(torch.isnan(got[:, N:]).all())
+
+
+@pytest.mark.parametrize("M,N,K,dtype_ab,tile", [
+    # one round of small tiles whatever the row: one K-step and less, fewer than wave groups, exact rounds of them
+    (256, 256, 256, "f16", (16, 16)), (17, 26, 40, "bf16", (16, 16)), (65, 16, 8, "f16", (16, 16)),
+    (512, 500, 64, "bf16", (32, 32)), (300, 300, 512, "f16", (32, 32)), (1024, 250, 320, "bf16", (32, 32)),
+    # 32 x 64 tiles: from three K-steps on, from nine with whole panels on an XCD only
+    (500, 1000, 136, "bf16", (32, 64)), (500, 1000, 128, "bf16", (64, 64)), (2000, 200, 512, "f16", (32, 64)),
+    (256, 2000, 800, "bf16", (32, 64)), (2000, 200, 520, "bf16", (64, 64)),
+])
+@pytest.mark.parametrize("dtype_c", ["f32", "bf16"])
+def test_small_products_of_short_rows(gpu, M, N, K, dtype_ab, dtype_c, tile):
+    a, b, _ = operands(M, N, K, dtype_ab, seed=M + K, b_std=0.05)
+    bias = np.random.default_rng(K).standard_normal(N).astype(np.float32)
+    info = AG.GemmPlan.create(M, N, K, dtype_ab, dtype_c, has_bias=True).info
+    assert (info.wg_tile_m, info.wg_tile_n) == tile, (info.name, info.wg_tile_m, info.wg_tile_n)
+    out, _ = run_gemm(a, b, M, N, K, dtype_ab, dtype_c, bias=bias, ldc=N + 3)
+    check(out, G.gemm(a, b, _DT[dtype_ab], _DT[dtype_c], bias=bias), dtype_c, N,
+          bar=1e-5 if dtype_c == "f32" else REL_L2_BAR)
+    pad = out[:, N:]
+    assert np.isnan(pad).all() if dtype_c == "f32" else (pad == 0x7FC1).all()
+
+
+@pytest.mark.parametrize("wg_tile", [(0, 0), (64, 64), (128, 128)])
+@pytest.mark.parametrize("scale_mode", ["none", "tensor"])
+def test_row_pitches_past_32_bits(gpu, wg_tile, scale_mode):
+    """Everything a packed launch argument holds at its widest: rows of C 2^32 + 24 elements apart, padded rows of A
+    and B, tensor scales on 16-bit operands, bias."""
+    import torch
+    M, N, K, lda, ldb, ldc = 2, 40, 72, 4096, 88, 2 ** 32 + 24
+    a, b, _ = operands(M, N, K, "bf16", seed=9, b_std=0.05)
+    dev = torch.device("cuda:0")
+    ta, tb = torch.zeros(M, lda, dtype=torch.int16, device=dev), torch.zeros(N, ldb, dtype=torch.int16, device=dev)
+    ta[:, :K] = torch.from_numpy(a.view(np.int16)).to(dev)
+    tb[:, :K] = torch.from_numpy(b.view(np.int16)).to(dev)
+    bias = torch.arange(N, dtype=torch.float32, device=dev) * 0.25
+    scales = torch.tensor([0.5, 3.0], device=dev)
+    out = torch.empty(ldc + 64, dtype=torch.int16, device=dev)
+    plan = AG.GemmPlan.create(M, N, K, "bf16", "bf16", scale_mode=scale_mode, has_bias=True, lda=lda, ldb=ldb, ldc=ldc,
+                              wg_tile=wg_tile, family=_capi.KERNEL_TILE)
+    kw = dict(scale_a=scales.data_ptr(), scale_b=scales.data_ptr() + 4) if scale_mode == "tensor" else {}
+    torch.cuda.synchronize()
+    print("launch", plan.info.name.decode(), flush=True)
+    plan.run(ta.data_ptr(), tb.data_ptr(), out.data_ptr(), bias=bias.data_ptr(), **kw)
+    torch.cuda.synchronize()
+    got = np.stack([out[m * ldc:m * ldc + N].cpu().numpy().view(np.uint16) for m in range(M)])
+    s = dict(scale_a=0.5, scale_b=3.0) if kw else {}
+    want = F.bf16_bits_to_f32(a) @ F.bf16_bits_to_f32(b).T * (1.5 if s else 1.0) + bias.cpu().numpy()
+    assert G.rel_l2(F.bf16_bits_to_f32(got), want) <= 4e-3   # one bf16 rounding: 2^-9 of each value at most
