@@ -516,6 +516,17 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out, int av
       // stream kernel from 16 workgroups on when K >= 4096, and instead of the 256 x 256 one
       // (long prologue: two K-steps and their scales) when K < 4096
       const bool fp4 = c.dtype_ab == ASTERGEMM_MXFP4;
+      // MXFP4 by rounds, on rows of 2 KiB and more: one round of 256 x 256 tiles where the 128 x 128 ones pass two per
+      // CU (128 x 128 / 256 x 256, us, with the quantiser: 1280x11008x4096 39.3 / 31.3, 3000x4096x4096 35.4 / 31.5,
+      // 3000x4096x14336 105 / 88.7), and three rounds of two 128 x 128 tiles instead of two of 256 x 256 (1280x14336x4096
+      // 50.7 / 58.4, 1600x11008x4096 50.2 / 57.5, 640x28672x4096 50.1 / 57.2; behind from five tiles per CU on,
+      // 1792 tiles 72.2 / 62.3; a rest of fewer than eight rows stays as the tests pin it, with the 256 x 256 ones)
+      const bool fp4_rounds = fp4 && c.K >= 4096;
+      const int64_t g256 = tile_grid(c, 256, 256);
+      const bool fp4_one_round = fp4_rounds && g256 <= chip_cus() && g128 > 2 * chip_cus();
+      const bool fp4_small_tiles =
+          fp4_rounds && g256 > chip_cus() && g256 <= 2 * chip_cus() && g128 <= 5 * chip_cus() &&
+          (c.M % 256 == 0 || c.M % 256 >= 8);
       const int thr128s = fp4 ? (c.K >= 4096 ? 16 : 200)
                               : (row_bytes(c.dtype_ab, c.K) >= 8192 ? 128 : 200);
       auto tier = [&](const Variant* x) {
@@ -536,6 +547,8 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out, int av
         // against 29.8, 4096 x 6144 x 1024 24.0 against 21.8)
         const bool walk_pays = x->rank == 3 && wgs(x) * c.K >= (int64_t)512 * 2048;
         if (area >= 256 * 256 && fp4 && c.K < 4096 && c.K % 512 == 0 && !walk_pays) return -1;
+        if (area >= 256 * 256 && fp4_small_tiles && !strstr(x->name, "_tail128_")) return -1;
+        if (area >= 256 * 256 && fp4_one_round && x->rank >= 2) return 2;
         if (area >= 256 * 256) return wgs(x) >= (x->rank >= 2 ? thr256s : thr256) ? 2 : -1;
         return wgs(x) >= ((x->rank >= 2) ? thr128s : 448) ? 1 : 0;
       };

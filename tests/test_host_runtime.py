@@ -223,6 +223,17 @@ def test_a_rest_of_fewer_than_8_rows_is_not_cut_off(dtype, tag):
         assert name.startswith(f"stream_{tag}_256x") and ("tail128" in name) == (r >= 8), (r, name)
 
 
+@pytest.mark.parametrize("M,N,K,name", [
+    (1280, 11008, 4096, "256x256_w2x4"), (1024, 8192, 4096, "128x128_w2x2"),   # 215 and 128 tiles: one round past 512 small ones
+    (1056, 8192, 4096, "256x256_w2x4"), (3000, 4096, 2048, "128x128_w2x2"),    # 160; rows of 1 KiB
+    (1280, 14336, 4096, "128x128_w2x2"), (1280, 16640, 4096, "256x256_w2x4"),  # 280 tiles, 1120 small ones; 325, 1300
+    (1288, 11008, 4096, "128x128_w2x2"), (1281, 11008, 4096, "256x256_w2x4"),  # a rest of 8 rows, of 1
+])
+def test_mxfp4_tiles_by_rounds(M, N, K, name):
+    got = gemm.GemmPlan.create(M, N, K, "mxfp4", "bf16").info.name.decode()
+    assert got.startswith("stream_mxfp4_" + name), got
+
+
 def test_no_split_on_unequal_tiles_has_fewer_planes_than_the_square_split_it_replaces():
     """An eager call leaves its stream a workspace of the size it needed, and a captured call of the same
     config, which runs the square kernel, cannot make it larger."""
