@@ -219,6 +219,8 @@ int64_t tile_grid(const astergemm_config& c, int64_t bm, int64_t bn) {
 //                             fp8 1500x8192x8192 116 / 87.5 / 95.2 / 106
 //   three rounds against two  bf16 1300x14336 164 / 163 / 151 / 149, 600x28672 164 / 166 / 161 / 151 (where
 //                             whole rounds plus a rest exist they win: 2560x8192x8192 261 against 287);
+//                             (192 x 128 where it has the third round half full and 256 x 128 just begun: 1300x11008
+//                             117 / 151 / 120 / 132, f16 1290x11008 127 against 141);
 //                             fp8 1500x14336 97.7 / 89.5 / 102 / 89.6: level, not taken; rows with a K tail
 //                             are behind, 256 x 256 / 256 x 128 on buffers that no kernel has read yet: f16
 //                             3600x4880x13272 573 / 638, bf16 3440x5688x15992 726 / 785, 2344x9616x1904 103 / 112
@@ -253,7 +255,9 @@ int unequal_tile_of(const astergemm_config& c) {
   if (c.M % 128 == 0 && c.N % 128 == 0 && g128 <= 2 * cus && g128 * 8 >= 2 * cus * 7) return 0;
   if (rb < 18 * 128 && c.M % 8 == 0 && (fp8 || c.dtype_c == ASTERGEMM_F32)) return 0;
   const int64_t g = tile_grid(c, 256, 128);
-  if (g <= cus || (!fp8 && whole_k && g <= 3 * cus && tile_grid(c, 256, 256) > cus)) return 256;
+  if (g <= cus) return 256;
+  if (!fp8 && whole_k && g <= 3 * cus && tile_grid(c, 256, 256) > cus)
+    return g > 2 * cus && tile_grid(c, 192, 128) * 2 <= 5 * cus ? 192 : 256;
   return 0;
 }
 
@@ -516,16 +520,19 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out, int av
       // stream kernel from 16 workgroups on when K >= 4096, and instead of the 256 x 256 one
       // (long prologue: two K-steps and their scales) when K < 4096
       const bool fp4 = c.dtype_ab == ASTERGEMM_MXFP4;
-      // MXFP4 by rounds, on rows of 2 KiB and more: one round of 256 x 256 tiles where the 128 x 128 ones pass two per
+      // MXFP4 and fp8 by rounds, MXFP4 on rows of 2 KiB and more: one round of 256 x 256 tiles where the 128 x 128 ones pass two per
       // CU (128 x 128 / 256 x 256, us, with the quantiser: 1280x11008x4096 39.3 / 31.3, 3000x4096x4096 35.4 / 31.5,
       // 3000x4096x14336 105 / 88.7), and three rounds of two 128 x 128 tiles instead of two of 256 x 256 (1280x14336x4096
       // 50.7 / 58.4, 1600x11008x4096 50.2 / 57.5, 640x28672x4096 50.1 / 57.2; behind from five tiles per CU on,
-      // 1792 tiles 72.2 / 62.3; a rest of fewer than eight rows stays as the tests pin it, with the 256 x 256 ones)
+      // 1792 tiles 72.2 / 62.3; fp8 1300x11008x4096 56.5 / 78.2, 1300x14336x4096 72.4 / 80.2, 1700x11008x4096 72.5 / 80.6;
+      // fp8 weights of more than 64 MiB, which a large tile reads less often from memory, are behind: 600x28672x4096 with
+      // the quantiser 101 / 95, 1300x14336x8192 183 / 174); a rest of fewer than eight rows stays with the 256 x 256 ones
+      const bool fp8 = c.dtype_ab == ASTERGEMM_FP8_E4M3;
       const bool fp4_rounds = fp4 && c.K >= 4096;
       const int64_t g256 = tile_grid(c, 256, 256);
       const bool fp4_one_round = fp4_rounds && g256 <= chip_cus() && g128 > 2 * chip_cus();
-      const bool fp4_small_tiles =
-          fp4_rounds && g256 > chip_cus() && g256 <= 2 * chip_cus() && g128 <= 5 * chip_cus() &&
+      const bool small_tiles =
+          (fp4_rounds || (fp8 && past_unequal && c.N * c.K <= (int64_t)64 << 20)) && g256 > chip_cus() && g256 <= 2 * chip_cus() && g128 <= 5 * chip_cus() &&
           (c.M % 256 == 0 || c.M % 256 >= 8);
       const int thr128s = fp4 ? (c.K >= 4096 ? 16 : 200)
                               : (row_bytes(c.dtype_ab, c.K) >= 8192 ? 128 : 200);
@@ -547,9 +554,13 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out, int av
         // against 29.8, 4096 x 6144 x 1024 24.0 against 21.8)
         const bool walk_pays = x->rank == 3 && wgs(x) * c.K >= (int64_t)512 * 2048;
         if (area >= 256 * 256 && fp4 && c.K < 4096 && c.K % 512 == 0 && !walk_pays) return -1;
-        if (area >= 256 * 256 && fp4_small_tiles && !strstr(x->name, "_tail128_")) return -1;
+        if (area >= 256 * 256 && small_tiles && !strstr(x->name, "_tail128_")) return -1;
         if (area >= 256 * 256 && fp4_one_round && x->rank >= 2) return 2;
         if (area >= 256 * 256) return wgs(x) >= (x->rank >= 2 ? thr256s : thr256) ? 2 : -1;
+        // fp8, eight waves on 128 x 128: from just over half the chip on (general 64 x 64 kernel / this, with the
+        // quantiser: 600x4096x4096 30.5 / 23.8, 513x4096x4096 30.0 / 23.1, 150x11008x4096 26.3 / 22.3, 300x6144x4096, 144
+        // tiles, 24.2 / 22.1; 128 tiles level)
+        if (fp8 && x->rank == 5) return wgs(x) >= 136 ? 1 : 0;
         return wgs(x) >= ((x->rank >= 2) ? thr128s : 448) ? 1 : 0;
       };
       const int tv = tier(v), tb = tier(best);

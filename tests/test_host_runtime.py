@@ -234,6 +234,17 @@ def test_mxfp4_tiles_by_rounds(M, N, K, name):
     assert got.startswith("stream_mxfp4_" + name), got
 
 
+@pytest.mark.parametrize("M,N,K,dtype,name", [
+    (1300, 11008, 4096, "fp8_e4m3", "stream_fp8_128x128_w2x2"), (1300, 11008, 4104 + 8, "fp8_e4m3", "stream_fp8_128x128_w2x2"),
+    (1300, 14336, 8192, "fp8_e4m3", "stream_fp8_256x256"), (1281, 11008, 4096, "fp8_e4m3", "stream_fp8_256x256"),
+    (513, 4096, 4096, "fp8_e4m3", "stream_fp8_128x128_w4x2"), (512, 4096, 4096, "fp8_e4m3", "tile_fp8_64x64"),
+    (1300, 11008, 4096, "bf16", "stream_bf16_192x128_w4x2"), (1400, 11008, 4096, "bf16", "stream_bf16_256x128_w4x2"),
+])
+def test_fp8_and_16_bit_tiles_by_rounds(M, N, K, dtype, name):
+    got = gemm.GemmPlan.create(M, N, K, dtype, "bf16").info.name.decode()
+    assert got.startswith(name), got
+
+
 def test_no_split_on_unequal_tiles_has_fewer_planes_than_the_square_split_it_replaces():
     """An eager call leaves its stream a workspace of the size it needed, and a captured call of the same
     config, which runs the square kernel, cannot make it larger."""
