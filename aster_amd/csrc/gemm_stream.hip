@@ -197,10 +197,10 @@ int launch_streamr(const GemmArgs& a, int grid, hipStream_t s) {
 //
 // The kernels that load them straight into MFMA operands have 128 x 256 tiles and nothing for problems that those leave
 // half the chip without: through LDS they are as good an operand as rows (16 rows x 128 bytes are 2 KiB in one
-// piece), for K over waves (gemm_kwave_kernel) and tiles of 128, 192 or 256 x 128 (gemm_streamr_kernel).  A
-// workgroup takes as long as its operand rows, per K-step; straight into operands 384 rows weigh as much as
-// 500 here (390 in fp8; past one per CU two share it).  Own kernel / K over waves / 128 / 192 / 256 x 128,
-// us over three sets of weights (fp8 and MXFP4 with their quantiser):
+// piece), for K over waves (gemm_kwave_kernel), tiles of 128, 192 or 256 x 128 (gemm_streamr_kernel) and of 256 x 256
+// (gemm_stream_kernel).  A workgroup takes as long as its operand rows, per K-step; straight into operands 384 rows
+// weigh as much as 500 here (390 in fp8; past one per CU two share it).  Own kernel / K over waves / 128 / 192 /
+// 256 x 128, us over three sets of weights (fp8 and MXFP4 with their quantiser):
 //   bf16 80x4096x4096       43.0 / 11.9 / 22.0 / 27.9 / 35.2    bf16 512x1024x8192   77.8 / 22.1 / 41.7 / 53.2 / 67.7
 //   bf16 160x14336x4096     60.3 / 49.3 / 38.9 / 44.0 / 44.4    bf16 320x4096x14336  181 / 85.5 / 101 / 128 / 123
 //   bf16 320x14336x4096     63.8 / - / 63.9 / 44.6 / 49.0       bf16 512x14336x4096  68.5 / - / 72.5 / 79.4 / 53.8
@@ -209,31 +209,52 @@ int launch_streamr(const GemmArgs& a, int grid, hipStream_t s) {
 //   fp8 80x14336x4096       29.3 / 20.8 / 22.6 / 23.8 / 27.6    fp8 320x28672x4096   66.2 / - / 67.9 / 55.1 / 62.3
 //   fp8 1280x4096x14336     96.3 / - / 117 / 87.6 / 96.3        fp8 944x14336x4096   60.0 / - / - / 71.9 / 63.2
 //   MXFP4 160x4096x14336    45.4 / 28.4                         MXFP4 160x14336x4096 21.5 / 23.2 (240 rows)
+// and, in 16-bit, the 256 x 256 tiles of the row-major kernel: a round of them weighs as 580 rows, more by what M is
+// padded with, and two rounds and more pay where five sixths of the workgroups' places in them are filled (two from
+// 2048 columns: 1920x14336x1024 takes 57.9 / 58.9, 8192x4096x512 40.1 / 40.8).  Own / what this rule took without them /
+// these:
+//   bf16 944x14336x4096     108.9 / 97.8 / 86.9                 bf16 640x14336x4096  91.5 / 77.9 / 79.0 (M padded by 1.2)
+//   bf16 1280x8192x28672    735 / 565 / 489                     bf16 640x11008x4096  61.9 / 61.1 / 67.5
+//   bf16 8192x4096x14336    721 / 720 / 624 (2 rounds, full)    bf16 1920x11008x4096 149 / 147 / 156 (0.67 of 2)
+//   bf16 4096x14336x4096    363 / 362 / 342 (0.88 of 4)         bf16 2560x14336x4096 241 / 236 / 244 (0.73 of 3)
 // fp8 in this order adds from K-step 0 on, so the tiles have the bits of the own kernel, and K over waves, which does
 // not, is for weights of 1024 rows and more, as among row-major ones (MXFP4 too).
 struct K8Form {
   KwaveForm kw;
-  int tile = 0;  // rows of a tile 128 columns wide; neither: the launcher's own kernel
-  explicit operator bool() const { return kw || tile; }
+  int tile = 0;         // rows of a tile 128 columns wide
+  bool square = false;  // 256 x 256 tiles (16-bit); none of them: the launcher's own kernel
+  explicit operator bool() const { return kw || tile || square; }
 };
-inline K8Form k8_form(int dt, int64_t M, int64_t N, int cus) {
+// ksteps: 16-bit K-steps (of 64 columns); no other type reads it
+inline K8Form k8_form(int dt, int64_t M, int64_t N, int64_t ksteps, int cus) {
   K8Form f;
   if (cus <= 0) return f;
   const bool fp8 = dt == ASTERGEMM_FP8_E4M3, fp4 = dt == ASTERGEMM_MXFP4;
   int64_t best = INT64_MAX;
   if (!fp4) {
     const int64_t own_grid = (M + 127) / 128 * ((N + 255) / 256);
-    if (own_grid > (fp8 ? 2 * cus : 700 * cus / 256)) return f;
+    if (fp8 && own_grid > 2 * cus) return f;
+    const int64_t squares = (M + 255) / 256 * ((N + 255) / 256), sq_rounds = (squares + cus - 1) / cus;
+    if (!fp8 && sq_rounds > 1 && squares * 6 >= sq_rounds * cus * 5 && (sq_rounds > 2 || ksteps >= 32)) {
+      f.square = true;
+      return f;
+    }
+    if (own_grid > 700 * cus / 256) return f;
     best = own_grid <= cus ? (fp8 ? 390 : 500) : fp8 ? 700 : own_grid <= 2 * cus ? 1000 : 1200;
     for (int bm : {128, 192, 256}) {
       const int64_t rounds = ((M + bm - 1) / bm * ((N + 127) / 128) + cus - 1) / cus;
       if (rounds <= 3 && rounds * (bm + 128) < best) best = rounds * (bm + 128), f.tile = bm;
     }
+    const int64_t sq = 580 * ((M + 255) / 256 * 256) / M;
+    if (!fp8 && sq_rounds == 1 && sq < best) best = sq, f.tile = 0, f.square = true;
   }
   int rows = 0;
   if ((fp8 || fp4) && N < 1024) return f;
   const KwaveForm kw = kwave_k8_form(dt, M, N, cus, &rows);
-  if (kw && (fp4 ? rows <= 192 : fp8 ? rows * 4 < best * 3 : rows * 4 <= best * 3)) f.kw = kw, f.tile = 0;
+  if (kw && (fp4 ? rows <= 192 : fp8 ? rows * 4 < best * 3 : rows * 4 <= best * 3)) {
+    f.kw = kw;
+    f.tile = 0, f.square = false;
+  }
   return f;
 }
 
@@ -253,11 +274,26 @@ int launch_k8_tile(GemmArgs a, hipStream_t s) {
   return (int)hipGetLastError();
 }
 
+template <int DT, int OUT>
+constexpr auto k8_square() {
+  return gemm_stream_kernel<DT, OUT, 256, 256, 2, 4, 5, true>;
+}
+constexpr int k8_square_lds = 5 * 256 * kRowBytes;
+template <int DT, int OUT>
+int launch_k8_square(GemmArgs a, hipStream_t s) {
+  a.tiles_m = (a.M + 255) / 256;
+  a.tiles_n = (a.N + 255) / 256;
+  a.group_m = (a.tiles_m % 8 == 0 && a.tiles_n % 32 == 0) ? -1 : 8;
+  auto k = k8_square<DT, OUT>();
+  AG_LAUNCH_KERNEL(k, dim3(a.tiles_m * a.tiles_n), dim3(512), k8_square_lds, s, a);
+  return (int)hipGetLastError();
+}
+
 // 0 and *taken = false: the launcher's own kernel is to run.  Either's first launch readies all of them.
 template <int DT, int OUT>
 int k8_instead(const GemmArgs& a, int own_ready, hipStream_t s, bool* taken) {
   *taken = false;
-  const K8Form f = a.own_kernel ? K8Form{} : k8_form(DT, a.M, a.N, device_cus());
+  const K8Form f = a.own_kernel ? K8Form{} : k8_form(DT, a.M, a.N, a.ksteps, device_cus());
   if (own_ready != 0 && !f) return own_ready;
   if (const int e = kwave_ready(DT, true)) return e;
   if constexpr (DT != ASTERGEMM_MXFP4) {
@@ -266,9 +302,17 @@ int k8_instead(const GemmArgs& a, int own_ready, hipStream_t s, bool* taken) {
     if (const int e = lds_attr_once(devs[1], (const void*)k8_kernel<DT, OUT, 192>(), k8_lds(192))) return e;
     if (const int e = lds_attr_once(devs[2], (const void*)k8_kernel<DT, OUT, 256>(), k8_lds(256))) return e;
   }
+  constexpr bool SQUARE = DT == ASTERGEMM_BF16 || DT == ASTERGEMM_F16;
+  if constexpr (SQUARE) {
+    static std::atomic<uint64_t> devs{0};
+    if (const int e = lds_attr_once(devs, (const void*)k8_square<DT, OUT>(), k8_square_lds)) return e;
+  }
   if (!f) return 0;
   *taken = true;
   if (f.kw) return kwave_launch(DT, OUT, a, f.kw, s);
+  if constexpr (SQUARE) {
+    if (f.square) return launch_k8_square<DT, OUT>(a, s);
+  }
   if constexpr (DT != ASTERGEMM_MXFP4) {
     if (f.tile == 128) return launch_k8_tile<DT, OUT, 128>(a, s);
     if (f.tile == 192) return launch_k8_tile<DT, OUT, 192>(a, s);
@@ -279,8 +323,20 @@ int k8_instead(const GemmArgs& a, int own_ready, hipStream_t s, bool* taken) {
 
 template <int DT, int OUT>
 bool k8_describe(const astergemm_config& c, int cus, LaunchForm* o) {
-  const K8Form f = cus > 0 ? k8_form(DT, c.M, c.N, cus) : K8Form{};
+  const K8Form f = cus > 0 ? k8_form(DT, c.M, c.N, c.K / 64, cus) : K8Form{};
   if (f.kw) kwave_describe(DT, f.kw, c.M, c.N, cus, o);
+  if constexpr (DT == ASTERGEMM_BF16 || DT == ASTERGEMM_F16) {
+    if (f.square) {
+      o->grid = (int)((c.M + 255) / 256 * ((c.N + 255) / 256));
+      o->tile_m = o->tile_n = 256;
+      o->waves_m = 2;
+      o->waves_n = 4;
+      o->stages = 3;
+      o->lds_bytes = k8_square_lds;
+      o->threads = 512;
+      o->func = (const void*)k8_square<DT, OUT>();
+    }
+  }
   if constexpr (DT != ASTERGEMM_MXFP4) {
     if (f.tile) {
       o->grid = (int)((c.M + f.tile - 1) / f.tile * ((c.N + 127) / 128));

@@ -69,6 +69,20 @@ __device__ __forceinline__ void group_bases(const uint8_t* mat, int64_t ld_bytes
   }
 }
 
+// Bases of a wave's transfers of pre-shuffled weights (K8): 8-row group x of the tile is half x & 1 of a block of 16
+// rows; a block past the end reads the last one (products that the epilogue does not store).
+template <class Plan>
+__device__ __forceinline__ void block_bases(const uint8_t* mat, int64_t row_bytes_, int tile_row0, int wave, int rows,
+                                            const uint8_t* (&out)[Plan::LH]) {
+#pragma unroll
+  for (int j = 0; j < Plan::LH; ++j) {
+    const int x = Plan::tile(wave, j);
+    int blk = (tile_row0 >> 4) + (x >> 1);
+    blk = blk < (rows >> 4) ? blk : (rows >> 4) - 1;
+    out[j] = mat + (int64_t)blk * 16 * row_bytes_ + (x & 1) * 1024;
+  }
+}
+
 // K tail: when a row does not end on a 128-byte step, the K loop runs over the whole steps and
 // the remaining 1..7 granules (16 bytes each) are multiplied here, once per tile, straight from
 // global memory: lane (li, lq) loads the granules it would have read from LDS (s * 4 + lq for
@@ -278,7 +292,9 @@ __device__ __forceinline__ int step_from(int first, int k, int nk) {
   return j >= nk ? j - nk : j;
 }
 
-template <int DT, int OUT, int BM, int BN, int WM, int WN, int NSLOT = 5>
+// K8: B pre-shuffled, 16 rows x 128 bytes in one piece of 2 KiB, lane for lane the fragments of its two substeps; whole
+// K-steps only.
+template <int DT, int OUT, int BM, int BN, int WM, int WN, int NSLOT = 5, bool K8 = false>
 __device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, int bid) {
   constexpr int NW = WM * WN;
   constexpr int TM = BM / WM / 16;
@@ -317,11 +333,13 @@ __device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, int bid) {
   const int lrow = lane >> 3;
   const int g_lane = (lane & 7) ^ (((wave * 8 + lrow) >> 1) & 7);
   const unsigned a_off = (unsigned)(lrow * (int)p.lda_bytes + g_lane * 16);
-  const unsigned b_off = (unsigned)(lrow * (int)p.ldb_bytes + g_lane * 16);
+  const unsigned b_off = K8 ? lane * 16 : (unsigned)(lrow * (int)p.ldb_bytes + g_lane * 16);
+  constexpr int B_STEP = K8 ? 16 * kRowBytes : kRowBytes;  // from one K-step of B to the next
   const uint8_t* a_base[LH];
   const uint8_t* b_base[LH];
   group_bases<Plan>(p.A, p.lda_bytes, row0, wave, p.M, a_base);
-  group_bases<Plan>(p.B, p.ldb_bytes, col0, wave, p.N, b_base);
+  if constexpr (K8) block_bases<Plan>(p.B, p.ldb_bytes, col0, wave, p.N, b_base);
+  else group_bases<Plan>(p.B, p.ldb_bytes, col0, wave, p.N, b_base);
   const int nk = p.ksteps - (p.tail_granules ? 1 : 0);  // whole 128-byte steps
 
   // the nine-slot ring only: the five-slot kernels give the bits of the tile walk and of the whole-rounds form
@@ -342,7 +360,7 @@ __device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, int bid) {
         lds + slot * SLOT + Plan::lds_offset(wave, j));
   };
   auto issue_b1 = [&](int k, int slot, int j) {
-    g2s(b_base[j] + (int64_t)at(k) * kRowBytes, b_off,
+    g2s(b_base[j] + (int64_t)at(k) * B_STEP, b_off,
         lds + slot * SLOT + Plan::lds_offset(wave, j));
   };
   auto issue_a = [&](int k, int slot) {
@@ -362,6 +380,7 @@ __device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, int bid) {
     rd_off[s] = (unsigned)(li * kRowBytes + (((s * 4 + lq) ^ (li >> 1)) << 4));
   const unsigned a_rd = (unsigned)(wm * TM * 16 * kRowBytes);
   const unsigned b_rd = (unsigned)(wn * TN * 16 * kRowBytes);
+  auto rd_b = [&](int s) { return K8 ? s * 1024 + b_off : rd_off[s]; };
 
   // KM = k mod NSLOT fixes the ring slots of K-step k at compile time.
   i32x4 fa[2][TM], fb[2][TN];
@@ -372,7 +391,7 @@ __device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, int bid) {
     const uint8_t* sb = lds + ((2 * KM + 1) % NSLOT) * SLOT;
 #pragma unroll
     for (int n = 0; n < TN; ++n)
-      fb[S][n] = *(const i32x4*)(sb + b_rd + n * 16 * kRowBytes + rd_off[S]);
+      fb[S][n] = *(const i32x4*)(sb + b_rd + n * 16 * kRowBytes + rd_b(S));
 #pragma unroll
     for (int m = 0; m < TM; ++m)
       fa[S][m] = *(const i32x4*)(sa + a_rd + m * 16 * kRowBytes + rd_off[S]);
@@ -395,7 +414,7 @@ __device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, int bid) {
     constexpr int I = decltype(idx)::value;
     if constexpr (I < TN) {
       const uint8_t* sb = lds + ((2 * KM + 1) % NSLOT) * SLOT;
-      fb[S][I] = *(const i32x4*)(sb + b_rd + I * 16 * kRowBytes + rd_off[S]);
+      fb[S][I] = *(const i32x4*)(sb + b_rd + I * 16 * kRowBytes + rd_b(S));
     } else {
       const uint8_t* sa = lds + ((2 * KM) % NSLOT) * SLOT;
       fa[S][I - TN] = *(const i32x4*)(sa + a_rd + (I - TN) * 16 * kRowBytes + rd_off[S]);
@@ -501,15 +520,15 @@ __device__ __forceinline__ void gemm_stream_body(const GemmArgs& p, int bid) {
   __builtin_amdgcn_sched_barrier(0);
   mfmas(S1{});
 
-  if constexpr (WM * WN == 8 || BM == 128) {  // four waves on 256 x 256 have no registers to spare
+  if constexpr (!K8 && (WM * WN == 8 || BM == 128)) {  // four waves on 256 x 256 have no registers to spare
     if (p.tail_granules) stream_k_tail<DT, BM, BN, WM, WN>(p, acc, wave, row0, col0, nk);
   }
   stream_epilogue<OUT, BM, BN, WM, WN>(p, acc, lds, wave, row0, col0);
 }
 
-template <int DT, int OUT, int BM, int BN, int WM, int WN, int NSLOT = 5>
+template <int DT, int OUT, int BM, int BN, int WM, int WN, int NSLOT = 5, bool K8 = false>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_stream_kernel(const GemmArgs p) {
-  gemm_stream_body<DT, OUT, BM, BN, WM, WN, NSLOT>(p, blockIdx.x);
+  gemm_stream_body<DT, OUT, BM, BN, WM, WN, NSLOT, K8>(p, blockIdx.x);
 }
 
 // Split K: the grid is p.split_k copies of the tile grid; copy s multiplies K steps

@@ -25,20 +25,6 @@
 namespace astergemm {
 namespace {
 
-// Bases of a wave's transfers of pre-shuffled weights (K8): 8-row group x of the tile is half x & 1 of a block of 16
-// rows; a block past the end reads the last one (products that the epilogue does not store).
-template <class Plan>
-__device__ __forceinline__ void block_bases(const uint8_t* mat, int64_t row_bytes_, int tile_row0, int wave, int rows,
-                                            const uint8_t* (&out)[Plan::LH]) {
-#pragma unroll
-  for (int j = 0; j < Plan::LH; ++j) {
-    const int x = Plan::tile(wave, j);
-    int blk = (tile_row0 >> 4) + (x >> 1);
-    blk = blk < (rows >> 4) ? blk : (rows >> 4) - 1;
-    out[j] = mat + (int64_t)blk * 16 * row_bytes_ + (x & 1) * 1024;
-  }
-}
-
 template <int DT, int OUT, int BM, int BN, int WM, int WN, int NS, bool K8>
 __device__ __forceinline__ void gemm_streamr_body(const GemmArgs& p, int bid) {
   constexpr int NW = WM * WN;

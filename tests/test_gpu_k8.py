@@ -28,8 +28,12 @@ pytestmark = pytest.mark.gpu
     (640, 14320, 192, "bf16", (192, 128)), (504, 14336, 576, "f16", (256, 128)), (4096, 4112, 128, "bf16", (192, 128)),
     (200, 8208, 128, "fp8_e4m3", (128, 128)), (328, 14336, 640, "fp8_e4m3", (192, 128)),
     (1280, 4096, 1152, "fp8_e4m3", (192, 128)), (968, 8176, 256, "fp8_e4m3", (256, 128)),
-    # neither: the own kernel
+    # 256 x 256 tiles: one round, two of long rows, three; edge tiles
+    (1912, 14336, 2048, "bf16", (256, 256)),
+    (1000, 11008, 192, "bf16", (256, 256)), (4096, 11024, 64, "f16", (256, 256)), (2040, 8176, 704, "bf16", (256, 256)),
+    # none of them: the own kernel
     (320, 14336, 1024, "mxfp4", (128, 256)), (4096, 8192, 256, "fp8_e4m3", (128, 256)), (640, 11008, 128, "bf16", (128, 256)),
+    (1912, 14336, 1984, "bf16", (128, 256)),
 ])
 @pytest.mark.parametrize("dtype_c", ["f32", "bf16"])
 def test_pre_shuffled_weights_through_lds(gpu, M, N, K, dtype_ab, tile, dtype_c):
