@@ -91,7 +91,8 @@ typedef enum astergemm_operand_path {
                                      decode kernels, M <= 16                 */
   ASTERGEMM_OPERAND_DIRECT_B_K8 = 2, /* B packed [N, K] and pre-shuffled for the
                                      stream kernels that load B straight into
-                                     MFMA operands.  MXFP4: payload with
+                                     MFMA operands (many sizes take the same
+                                     bytes through LDS instead).  MXFP4: payload with
                                      astergemm_shuffle_weight_8, dMxB with
                                      astergemm_shuffle_scales_e8m0_lanes
                                      (128 x 256 tiles, N % 64 == 0,
