@@ -228,7 +228,7 @@ struct K8Form {
 // ksteps: 16-bit K-steps (of 64 columns); no other type reads it
 inline K8Form k8_form(int dt, int64_t M, int64_t N, int64_t ksteps, int cus) {
   K8Form f;
-  if (cus <= 0) return f;
+  if (cus <= 0 || M < 1 || N < 1) return f;  // (an id is described whether or not its kernel takes the sizes)
   const bool fp8 = dt == ASTERGEMM_FP8_E4M3, fp4 = dt == ASTERGEMM_MXFP4;
   int64_t best = INT64_MAX;
   if (!fp4) {

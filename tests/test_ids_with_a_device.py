@@ -1,0 +1,55 @@
+"""Every id describes every config: what the launchers' rules say with a chip's CU count in hand, on sizes that no
+kernel takes as well.  A stand-in for the two device queries gives the count, so nothing here needs a GPU; in a process
+of its own, which an arithmetic fault would end."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+QUERIES = """
+#include <hip/hip_runtime.h>
+#include <cstring>
+extern "C" hipError_t hipGetDevice(int* d) { *d = 0; return hipSuccess; }
+extern "C" hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600* p, int) {
+  memset(p, 0, sizeof(*p));
+  p->multiProcessorCount = 256;
+  return hipSuccess;
+}
+"""
+
+WALK = """
+import ctypes
+from aster_amd import _capi
+lib, info, c, n = _capi.load(), _capi.KernelInfo(), _capi.Config(), 0
+c.M, c.N, c.K = 80, 4096, 4096                 # the stand-in is heard: K over waves on 256 CUs
+c.dtype_ab = c.dtype_c = _capi.BF16
+c.operand_path = _capi.OPERAND_DIRECT_B_K8
+assert lib.astergemm_select(ctypes.byref(c), ctypes.byref(info)) == 0 and info.wg_tile_m < 128, info.wg_tile_m
+for M, N, K in ((0, 0, 64), (0, 4096, 4096), (4096, 0, 4096), (-8, 16, 64), (16, -16, 64), (1, 1, 1), (8, 16, 0),
+                (0, 1 << 31, 512), (1 << 40, 16, 512)):
+    c = _capi.Config()
+    c.M, c.N, c.K = M, N, K
+    for i in range(lib.astergemm_variant_count()):
+        print(i, M, N, K, flush=True)
+        assert lib.astergemm_variant_info(i, ctypes.byref(c), ctypes.byref(info)) == 0
+        n += 1
+print("described", n)
+"""
+
+
+@pytest.fixture(scope="module")
+def queries(tmp_path_factory):
+    where = tmp_path_factory.mktemp("queries")
+    (where / "queries.cpp").write_text(QUERIES)
+    subprocess.run(["g++", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    str(where / "queries.cpp"), "-o", str(where / "queries.so")], check=True)
+    return str(where / "queries.so")
+
+
+def test_every_id_describes_sizes_that_no_kernel_takes(queries):
+    p = subprocess.run([sys.executable, "-c", WALK], cwd=ROOT, env=dict(os.environ, LD_PRELOAD=queries),
+                       capture_output=True, text=True, timeout=300)
+    assert p.returncode == 0 and "described" in p.stdout, (p.returncode, p.stdout[-200:], p.stderr[-2000:])
