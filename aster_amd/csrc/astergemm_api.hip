@@ -557,10 +557,11 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out, int av
         if (area >= 256 * 256 && small_tiles && !strstr(x->name, "_tail128_")) return -1;
         if (area >= 256 * 256 && fp4_one_round && x->rank >= 2) return 2;
         if (area >= 256 * 256) return wgs(x) >= (x->rank >= 2 ? thr256s : thr256) ? 2 : -1;
-        // fp8, eight waves on 128 x 128: from just over half the chip on (general 64 x 64 kernel / this, with the
-        // quantiser: 600x4096x4096 30.5 / 23.8, 513x4096x4096 30.0 / 23.1, 150x11008x4096 26.3 / 22.3, 300x6144x4096, 144
-        // tiles, 24.2 / 22.1; 128 tiles level)
-        if (fp8 && x->rank == 5) return wgs(x) >= 136 ? 1 : 0;
+        // fp8, eight waves on 128 x 128: from just over half the chip on where the rows are shorter than 8 KiB
+        // (general 64 x 64 kernel / this, with the quantiser: 600x4096x4096 30.5 / 23.8, 513x4096x4096 30.0 / 23.1,
+        // 150x11008x4096 26.3 / 22.3, 300x6144x4096, 144 tiles, 24.2 / 22.1; 128 tiles level), from the line of the
+        // other 128 x 128 kernels on longer ones: below it the four waves of theirs would take the problem
+        if (fp8 && x->rank == 5) return wgs(x) >= (thr128s < 136 ? thr128s : 136) ? 1 : 0;
         return wgs(x) >= ((x->rank >= 2) ? thr128s : 448) ? 1 : 0;
       };
       const int tv = tier(v), tb = tier(best);

@@ -245,6 +245,12 @@ def test_fp8_and_16_bit_tiles_by_rounds(M, N, K, dtype, name):
     assert got.startswith(name), got
 
 
+@pytest.mark.parametrize("M,N,K", [(1536, 1408, 8192), (640, 3328, 8192), (1152, 1920, 16384), (1024, 2176, 8192)])
+def test_fp8_on_long_rows_keeps_its_eight_waves(M, N, K):
+    # 132, 130, 135 and 136 tiles of 128 x 128
+    assert gemm.GemmPlan.create(M, N, K, "fp8_e4m3", "bf16").info.name.decode() == "stream_fp8_128x128_w4x2_bf16"
+
+
 def test_no_split_on_unequal_tiles_has_fewer_planes_than_the_square_split_it_replaces():
     """An eager call leaves its stream a workspace of the size it needed, and a captured call of the same
     config, which runs the square kernel, cannot make it larger."""
