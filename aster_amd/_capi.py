@@ -17,7 +17,8 @@ import sys
 from typing import Optional
 
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "lib", "libastergemm.so")
-_FASTCALL_PATH = os.path.join(os.path.dirname(_LIB_PATH), "aster_fastcall.so")
+# of this interpreter: another one finds none of its own and calls the library through ctypes
+_FASTCALL_PATH = os.path.join(os.path.dirname(_LIB_PATH), "aster_fastcall" + importlib.machinery.EXTENSION_SUFFIXES[0])
 
 # astergemm_dtype
 F16, BF16, FP8_E4M3, MXFP4, F32 = 0, 1, 2, 3, 4
@@ -182,7 +183,7 @@ SIGNATURES = {
 }
 
 _lib: Optional[C.CDLL] = None
-fast_run = None  # astergemm_run without ctypes (csrc/fastcall.c); set by load()
+fast_run = None  # astergemm_run without ctypes (csrc/fastcall.c) where that is built; set by load()
 
 
 def library_path() -> str:
@@ -216,11 +217,9 @@ def load() -> C.CDLL:
     if _lib is not None:
         return _lib
     _bind_one_hip_runtime()
-    for path in (_LIB_PATH, _FASTCALL_PATH):
-        if os.path.exists(path):
-            continue
+    if not os.path.exists(_LIB_PATH):
         raise FileNotFoundError(
-            f"{path} is not built; run `python -m aster_amd.build` "
+            f"{_LIB_PATH} is not built; run `python -m aster_amd.build` "
             "(needs hipcc; cross-compiles for gfx950 without a GPU)"
         )
     lib = C.CDLL(_LIB_PATH)
@@ -228,11 +227,12 @@ def load() -> C.CDLL:
         fn = getattr(lib, name)  # AttributeError if the symbol is missing
         fn.restype = restype
         fn.argtypes = argtypes
-    loader = importlib.machinery.ExtensionFileLoader("aster_fastcall", _FASTCALL_PATH)
-    module = importlib.util.module_from_spec(importlib.util.spec_from_loader("aster_fastcall", loader))
-    loader.exec_module(module)
-    module.bind(C.cast(lib.astergemm_run, C.c_void_p).value)
-    fast_run = module.run
+    if os.path.exists(_FASTCALL_PATH):
+        loader = importlib.machinery.ExtensionFileLoader("aster_fastcall", _FASTCALL_PATH)
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("aster_fastcall", loader))
+        loader.exec_module(module)
+        module.bind(C.cast(lib.astergemm_run, C.c_void_p).value)
+        fast_run = module.run
     _lib = lib
     return lib
 

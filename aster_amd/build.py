@@ -9,7 +9,9 @@ tree.  `python -m aster_amd.build` rebuilds it.
 
 from __future__ import annotations
 
+import importlib.machinery
 import os
+import shutil
 import subprocess
 import sys
 import sysconfig
@@ -45,7 +47,7 @@ UNITS = [("gemm_stream_p0", "gemm_stream.hip", ["-DAG_STREAM_PART=0"]),
 HSACO_SOURCE = "hsaco_kernels.hip"
 HSACO_PATH = os.path.join(LIB_DIR, "astergemm_kernels.hsaco")
 REPLAY_PATH = os.path.join(LIB_DIR, "astergemm_replay")
-FASTCALL_PATH = os.path.join(LIB_DIR, "aster_fastcall.so")
+FASTCALL_PATH = os.path.join(LIB_DIR, "aster_fastcall" + importlib.machinery.EXTENSION_SUFFIXES[0])
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
@@ -128,6 +130,23 @@ def _genco(src: str) -> str:
     return HSACO_PATH
 
 
+def build_fastcall() -> bool:
+    """The CPython binding of the launch, for the interpreter that runs this (no GPU code, linked to nothing: _capi binds
+    it to the library).  False where there is no C compiler or no Python.h: calls then go through ctypes."""
+    cc, include = shutil.which(os.environ.get("CC", "gcc")), sysconfig.get_paths()["include"]
+    if cc is None or not os.path.exists(os.path.join(include, "Python.h")):
+        print("aster_fastcall: no C compiler or no Python.h, launches go through ctypes (0.5 us more each)", file=sys.stderr)
+        if os.path.exists(FASTCALL_PATH):
+            os.remove(FASTCALL_PATH)
+        return False
+    cmd = [cc, "-O2", "-shared", "-fPIC", "-Wall", "-I" + include,
+           "-I" + os.path.join(ROOT, "include"), os.path.join(CSRC, "fastcall.c"), "-o", FASTCALL_PATH]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"fastcall build failed:\n{proc.stdout}\n{proc.stderr}")
+    return True
+
+
 def build_library(verbose: bool = False, only=None) -> str:
     """Compile every HIP source, link libastergemm.so and build the code object
     astergemm_kernels.hsaco; returns the library path.  `only` (a list of unit names, for work
@@ -159,12 +178,7 @@ def build_library(verbose: bool = False, only=None) -> str:
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(f"replay tool build failed:\n{proc.stdout}\n{proc.stderr}")
-    # the CPython binding of the launch (no GPU code, linked to nothing: _capi binds it to the library)
-    cmd = ["gcc", "-O2", "-shared", "-fPIC", "-Wall", "-I" + sysconfig.get_paths()["include"],
-           "-I" + os.path.join(ROOT, "include"), os.path.join(CSRC, "fastcall.c"), "-o", FASTCALL_PATH]
-    proc = subprocess.run(cmd, capture_output=True, text=True)
-    if proc.returncode != 0:
-        raise RuntimeError(f"fastcall build failed:\n{proc.stdout}\n{proc.stderr}")
+    build_fastcall()
     if verbose:
         print(f"built {LIB_PATH}")
     return LIB_PATH

@@ -298,15 +298,18 @@ class GemmPlan:
     def run(self, dA: int, dB: int, dC: int, *, scale_a: int = None, scale_b: int = None,
             mx_a: int = None, mx_b: int = None, bias: int = None, stream: int = None,
             workspace: int = None, workspace_bytes: int = 0) -> None:
-        _capi.load()
-        try:
-            rc = _capi.fast_run(self.config, dA, dB, dC, scale_a, scale_b, mx_a, mx_b, bias, workspace,
-                                workspace_bytes, stream or None)
-        except TypeError:  # not integers: what ctypes makes of them (nothing has been launched)
+        lib, rc = _capi.load(), None
+        if _capi.fast_run is not None:
+            try:
+                rc = _capi.fast_run(self.config, dA, dB, dC, scale_a, scale_b, mx_a, mx_b, bias, workspace,
+                                    workspace_bytes, stream or None)
+            except TypeError:  # not integers: what ctypes makes of them (nothing has been launched)
+                pass
+        if rc is None:
             ops = self._operands(dA, dB, dC, scale_a, scale_b, mx_a, mx_b, bias, workspace,
                                  workspace_bytes)
-            rc = _capi.load().astergemm_run(ctypes.byref(self.config), ctypes.byref(ops),
-                                            ctypes.c_void_p(stream) if stream else None)
+            rc = lib.astergemm_run(ctypes.byref(self.config), ctypes.byref(ops),
+                                   ctypes.c_void_p(stream) if stream else None)
         if rc != 0:
             _capi.check(rc)
 

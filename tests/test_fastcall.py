@@ -1,10 +1,11 @@
 """GemmPlan.run's binding of the launch (csrc/fastcall.c): what it takes, what it refuses, and that refusals are ctypes'."""
 import ctypes
+import importlib.machinery
 
 import numpy as np
 import pytest
 
-from aster_amd import _capi
+from aster_amd import _capi, build
 from aster_amd.gemm import GemmPlan
 
 
@@ -41,3 +42,24 @@ def test_status_becomes_the_exception():
     p = GemmPlan.create(16, 16, 64, "bf16", "f32")
     with pytest.raises(_capi.AsterGemmError, match="non-null"):
         p.run(0, 32, 48)
+
+
+def test_without_the_binding_launches_go_through_ctypes(monkeypatch, tmp_path):
+    monkeypatch.setattr(_capi, "_lib", None)
+    monkeypatch.setattr(_capi, "fast_run", None)
+    monkeypatch.setattr(_capi, "_FASTCALL_PATH", str(tmp_path / "none.so"))
+    p = empty_plan()
+    p.run(16, 32, 48, stream=0)
+    assert _capi.fast_run is None
+    with pytest.raises(TypeError):
+        p.run("16", 32, 48)
+    p = GemmPlan.create(16, 16, 64, "bf16", "f32")
+    with pytest.raises(_capi.AsterGemmError, match="non-null"):
+        p.run(0, 32, 48)
+
+
+def test_the_binding_belongs_to_one_interpreter(monkeypatch, tmp_path):
+    assert any(_capi._FASTCALL_PATH.endswith(s) and len(s) > 3 for s in importlib.machinery.EXTENSION_SUFFIXES)
+    monkeypatch.setattr(build, "FASTCALL_PATH", str(tmp_path / "aster_fastcall.so"))
+    monkeypatch.setenv("CC", str(tmp_path / "no-such-compiler"))
+    assert not build.build_fastcall() and not list(tmp_path.iterdir())
