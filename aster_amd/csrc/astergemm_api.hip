@@ -710,6 +710,14 @@ int build_args(const Variant& v, const astergemm_config& c, const astergemm_oper
   a->lda_bytes = row_bytes(c.dtype_ab, c.lda ? c.lda : c.K);
   a->ldb_bytes = row_bytes(c.dtype_ab, c.ldb ? c.ldb : c.K);
   a->ldc = c.ldc ? c.ldc : c.N;
+  // what PackedArgs holds; beyond it lies no device memory (a single row never moves by its pitch)
+  const uintptr_t any = (uintptr_t)a->A | (uintptr_t)a->B | (uintptr_t)a->C | (uintptr_t)a->bias | (uintptr_t)a->scale_a |
+                        (uintptr_t)a->scale_b | (uintptr_t)a->mx_a | (uintptr_t)a->mx_b;
+  auto refuse = [] {
+    set_error("astergemm: device addresses have 48 bits, ldc at most 58");
+    return ASTERGEMM_EINVAL;
+  };
+  if (any >> 48 || (c.M > 1 && a->ldc >> 58)) return refuse();
   a->M = (int32_t)c.M;
   a->N = (int32_t)c.N;
   a->K = (int32_t)c.K;
@@ -736,6 +744,7 @@ int build_args(const Variant& v, const astergemm_config& c, const astergemm_oper
       set_error("astergemm: dWorkspace must be 16-byte aligned");
       return ASTERGEMM_EINVAL;
     }
+    if (need && (uintptr_t)ops.dWorkspace >> 48) return refuse();
     if (need) a->workspace = (float*)ops.dWorkspace;
   }
   return 0;

@@ -63,3 +63,26 @@ def test_the_binding_belongs_to_one_interpreter(monkeypatch, tmp_path):
     monkeypatch.setattr(build, "FASTCALL_PATH", str(tmp_path / "aster_fastcall.so"))
     monkeypatch.setenv("CC", str(tmp_path / "no-such-compiler"))
     assert not build.build_fastcall() and not list(tmp_path.iterdir())
+
+
+@pytest.mark.parametrize("where", ["dA", "dB", "dC", "scale_a", "scale_b", "bias"])
+def test_addresses_past_48_bits_are_refused(where):
+    """Kernels take theirs in 48 bits (PackedArgs): one more would be another address."""
+    p = GemmPlan.create(16, 16, 64, "fp8_e4m3", "f32", has_bias=True)
+    ops = dict(dA=16, dB=32, dC=48, scale_a=64, scale_b=64, bias=64)
+    ops[where] = 1 << 48
+    with pytest.raises(_capi.AsterGemmError, match="48 bits"):
+        p.run(**ops)
+
+
+def test_workspaces_past_48_bits_are_refused_where_they_are_used():
+    p = GemmPlan.create(500, 4096, 14336, "bf16", "bf16")
+    with pytest.raises(_capi.AsterGemmError, match="48 bits"):
+        p.run(16, 32, 48, workspace=1 << 48, workspace_bytes=p.workspace_bytes() or 1)
+    assert p.workspace_bytes() > 0
+
+
+def test_pitches_of_c_past_58_bits_are_refused():
+    p = GemmPlan.create(2, 16, 64, "bf16", "f32", ldc=1 << 58)
+    with pytest.raises(_capi.AsterGemmError, match="58"):
+        p.run(16, 32, 48)
