@@ -725,11 +725,7 @@ int build_args(const Variant& v, const astergemm_config& c, const astergemm_oper
   a->tail_granules = (int32_t)((row_bytes(c.dtype_ab, c.K) % 128) / 16);
   a->tiles_m = (int32_t)((c.M + v.tile_m - 1) / v.tile_m);
   a->tiles_n = (int32_t)((c.N + v.tile_n - 1) / v.tile_n);
-  // tile order (map_tile): groups of 8 tile rows inside one contiguous run per XCD; where the
-  // tile grid divides, band order instead (all XCDs on one band of 8 tile rows, 8 x 4 tiles per
-  // XCD and round as before): 8192^3 bf16 +0.5 %, fp8 +1.3 %, 16384 x 16384 x 4096 fp8 +1.2 %,
-  // MXFP4 +1.5 %, bf16 -0.1 %, same process
-  a->group_m = (a->tiles_m % 8 == 0 && a->tiles_n % 32 == 0) ? -1 : 8;
+  a->group_m = tile_order(a->tiles_m, a->tiles_n);
   a->split_k = 1;
   a->own_kernel = own_kernel(c);
   // rows cut into K ranges: the caller's workspace when one is given, else the library's own

@@ -33,6 +33,13 @@ struct GemmArgs {
                          // the caller of a launcher = use this buffer, null = the library's own
 };
 
+// Tile order (map_tile): groups of 8 tile rows inside one contiguous run per XCD; where the tile grid divides, band order
+// instead (all XCDs on one band of 8 tile rows, 8 x 4 tiles per XCD and round as before): 8192^3 bf16 +0.5 %, fp8
+// +1.3 %, 16384 x 16384 x 4096 fp8 +1.2 %, MXFP4 +1.5 %, bf16 -0.1 %, same process.
+__host__ __device__ inline int tile_order(int tiles_m, int tiles_n) {
+  return (tiles_m % 8 == 0 && tiles_n % 32 == 0) ? -1 : 8;
+}
+
 // Bytes of one operand row covering `k` elements.
 __host__ __device__ inline int64_t row_bytes(int dtype, int64_t k) {
   switch (dtype) {

@@ -51,7 +51,7 @@ inline bool pairs_tiles(int out, int64_t M, int64_t N, int64_t row_bytes, int cu
 template <int DT, int OUT>
 int launch_pairs(GemmArgs a, hipStream_t s) {
   a.tiles_m = (a.M + 255) / 256;
-  a.group_m = (a.tiles_m % 8 == 0 && a.tiles_n % 32 == 0) ? -1 : 8;
+  a.group_m = tile_order(a.tiles_m, a.tiles_n);
   auto k = gemm_streamr_kernel<DT, OUT, 256, 128, 4, 2, 3>;
   AG_LAUNCH_KERNEL(k, dim3(a.tiles_m * a.tiles_n), dim3(512), 3 * 384 * kRowBytes, s, a);
   return (int)hipGetLastError();
@@ -268,7 +268,7 @@ template <int DT, int OUT, int BM>
 int launch_k8_tile(GemmArgs a, hipStream_t s) {
   a.tiles_m = (a.M + BM - 1) / BM;
   a.tiles_n = (a.N + 127) / 128;
-  a.group_m = (a.tiles_m % 8 == 0 && a.tiles_n % 32 == 0) ? -1 : 8;
+  a.group_m = tile_order(a.tiles_m, a.tiles_n);
   auto k = k8_kernel<DT, OUT, BM>();
   AG_LAUNCH_KERNEL(k, dim3(a.tiles_m * a.tiles_n), dim3(512), k8_lds(BM), s, a);
   return (int)hipGetLastError();
@@ -283,7 +283,7 @@ template <int DT, int OUT>
 int launch_k8_square(GemmArgs a, hipStream_t s) {
   a.tiles_m = (a.M + 255) / 256;
   a.tiles_n = (a.N + 255) / 256;
-  a.group_m = (a.tiles_m % 8 == 0 && a.tiles_n % 32 == 0) ? -1 : 8;
+  a.group_m = tile_order(a.tiles_m, a.tiles_n);
   auto k = k8_square<DT, OUT>();
   AG_LAUNCH_KERNEL(k, dim3(a.tiles_m * a.tiles_n), dim3(512), k8_square_lds, s, a);
   return (int)hipGetLastError();
@@ -904,8 +904,8 @@ inline void tail_parts(const GemmArgs& a, const TailSplit& ts, int out_bytes, Ge
   part2->tiles_m = (part2->M + 127) / 128;
   part2->tiles_n = (part2->N + 127) / 128;
   // the tile order is a property of each part's own tile grid (see map_tile)
-  part1->group_m = (part1->tiles_m % 8 == 0 && part1->tiles_n % 32 == 0) ? -1 : 8;
-  part2->group_m = (part2->tiles_m % 8 == 0 && part2->tiles_n % 32 == 0) ? -1 : 8;
+  part1->group_m = tile_order(part1->tiles_m, part1->tiles_n);
+  part2->group_m = tile_order(part2->tiles_m, part2->tiles_n);
 }
 
 // KIND 0: 16-bit operands, 1: fp8, 2: MXFP4

@@ -11,11 +11,31 @@ constexpr int tile_lds_bytes(int dt, int bm, int bn, int stages) {
   return stages * (bm + bn) * (kRowBytes + (dt == ASTERGEMM_MXFP4 ? 8 : 0));
 }
 
+// 64 x 64 tiles, operands of bytes: the arguments in one line whatever the size (in one line / as GemmArgs, us: MXFP4
+// 512x512x1024 4.28 / 4.6, 256x256x4096 7.50 / 7.95, fp8 512x512x512 with the quantiser 10.5 / 11.2).  16-bit ones where a
+// launch is as long as the kernel (bf16 500x1000x40 3.34 / 3.8, f16 1200x1200x64, 361 tiles, 3.69 / 4.35; bf16
+// 1000x1000x256, 256 tiles of 4 K-steps, level at 4.5); past that the launch is hidden and unpacking stands in front of
+// the K loop (f16 1100x1003x200, 288 tiles of 4, 5.00 / 4.83, bf16 391x6864x288 6.50 / 6.43, 777x1001x1032 8.11 / 8.07).
+// Larger tiles have no such sizes: GemmArgs (bf16 1269x22136x312 49.3 / 48.8).
+template <int DT, int BM>
+constexpr bool kTileAlwaysPacks = BM == 64 && (DT == ASTERGEMM_FP8_E4M3 || DT == ASTERGEMM_MXFP4);
+inline bool packs_16_bit(int64_t grid, int ksteps) { return ksteps <= 4 && grid <= 512 && grid * ksteps <= 1024; }
+
+template <int DT, int OUT, int BM, int BN, int WM, int WN, int S>
+constexpr auto tile_kernel() {
+  if constexpr (kTileAlwaysPacks<DT, BM>) return gemm_tile_packed_kernel<DT, OUT, BM, BN, WM, WN, S>;
+  else return gemm_tile_kernel<DT, OUT, BM, BN, WM, WN, S>;
+}
+
 template <int DT, int OUT, int BM, int BN, int WM, int WN, int S>
 int tile_ready() {
-  static std::atomic<uint64_t> attr_devs{0};
-  return lds_attr_once(attr_devs, (const void*)gemm_tile_kernel<DT, OUT, BM, BN, WM, WN, S>,
-                       tile_lds_bytes(DT, BM, BN, S));
+  static std::atomic<uint64_t> attr_devs{0}, packed_devs{0};
+  constexpr int lds = tile_lds_bytes(DT, BM, BN, S);
+  if constexpr (BM == 64)
+    if (int e = lds_attr_once(packed_devs, (const void*)gemm_tile_packed_kernel<DT, OUT, BM, BN, WM, WN, S>, lds)) return e;
+  if constexpr (!kTileAlwaysPacks<DT, BM>)
+    return lds_attr_once(attr_devs, (const void*)gemm_tile_kernel<DT, OUT, BM, BN, WM, WN, S>, lds);
+  return 0;
 }
 
 template <int DT, int OUT, int BM, int BN, int WM, int WN, int S>
@@ -23,8 +43,16 @@ int launch_tile(const GemmArgs& a, int grid, hipStream_t s) {
   if (int e = tile_ready<DT, OUT, BM, BN, WM, WN, S>()) return e;
   // the kernels that stand in for this one on small grids: a config captured later finds either ready
   if constexpr (BM == 64) (void)kwave_ready(DT);
-  AG_LAUNCH_KERNEL((gemm_tile_kernel<DT, OUT, BM, BN, WM, WN, S>), dim3(grid), dim3(WM * WN * 64),
-                   tile_lds_bytes(DT, BM, BN, S), s, pack_args(a, 0, a.C));
+  constexpr int lds = tile_lds_bytes(DT, BM, BN, S);
+  if constexpr (BM == 64) {
+    if (kTileAlwaysPacks<DT, BM> || packs_16_bit(grid, a.ksteps)) {
+      AG_LAUNCH_KERNEL((gemm_tile_packed_kernel<DT, OUT, BM, BN, WM, WN, S>), dim3(grid), dim3(WM * WN * 64), lds, s,
+                       pack_args(a, 0, a.C));
+      return (int)hipGetLastError();
+    }
+  }
+  if constexpr (!kTileAlwaysPacks<DT, BM>)
+    AG_LAUNCH_KERNEL((gemm_tile_kernel<DT, OUT, BM, BN, WM, WN, S>), dim3(grid), dim3(WM * WN * 64), lds, s, a);
   return (int)hipGetLastError();
 }
 
@@ -54,7 +82,7 @@ const char* check_tile(const astergemm_config& c) {
   Variant {                                                                      \
     name, ASTERGEMM_KERNEL_TILE, DT, OUT, BM, BN, kRowBytes, WM, WN, S, 1,       \
         tile_lds_bytes(DT, BM, BN, S),                                           \
-        (const void*)gemm_tile_kernel<DT, OUT, BM, BN, WM, WN, S>,               \
+        (const void*)tile_kernel<DT, OUT, BM, BN, WM, WN, S>(),                  \
         launch_tile<DT, OUT, BM, BN, WM, WN, S>, check_tile                      \
   }
 #define AG_TILE(name, DT, BM, BN, WM, WN, S)                                     \

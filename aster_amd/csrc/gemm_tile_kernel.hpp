@@ -483,11 +483,17 @@ __device__ __forceinline__ void gemm_tile_body(const GemmArgs& p) {
 
 
 template <int DT, int OUT, int BM, int BN, int WM, int WN, int S>
-__global__ __launch_bounds__(WM* WN * 64) void gemm_tile_kernel(const PackedArgs q) {
+__global__ __launch_bounds__(WM* WN * 64) void gemm_tile_kernel(const GemmArgs p) {
+  gemm_tile_body<DT, OUT, BM, BN, WM, WN, S>(p);
+}
+
+// The same with its arguments in one line (gemm_tile.hip says which of the two a launch takes).
+template <int DT, int OUT, int BM, int BN, int WM, int WN, int S>
+__global__ __launch_bounds__(WM* WN * 64) void gemm_tile_packed_kernel(const PackedArgs q) {
   GemmArgs p = unpack_args<DT>(q);
   p.tiles_m = (p.M + BM - 1) / BM;
   p.tiles_n = (p.N + BN - 1) / BN;
-  p.group_m = (p.tiles_m % 8 == 0 && p.tiles_n % 32 == 0) ? -1 : 8;
+  p.group_m = tile_order(p.tiles_m, p.tiles_n);
   gemm_tile_body<DT, OUT, BM, BN, WM, WN, S>(p);
 }
 

@@ -202,3 +202,21 @@ def test_row_pitches_past_32_bits(gpu, wg_tile, scale_mode):
     s = dict(scale_a=0.5, scale_b=3.0) if kw else {}
     want = F.bf16_bits_to_f32(a) @ F.bf16_bits_to_f32(b).T * (1.5 if s else 1.0) + bias.cpu().numpy()
     assert G.rel_l2(F.bf16_bits_to_f32(got), want) <= 4e-3   # one bf16 rounding: 2^-9 of each value at most
+
+
+@pytest.mark.parametrize("M,N,K,dtype_ab", [
+    (1000, 1000, 256, "bf16"), (1000, 1030, 256, "f16"),      # 256 and 272 tiles of four K-steps
+    (1024, 1000, 264, "bf16"), (1001, 1000, 200, "f16"),      # five, and four with a tail
+    (2040, 1000, 40, "bf16"), (2060, 1000, 40, "f16"),        # 512 and 528 tiles of one
+    (520, 1000, 72, "bf16"),
+])
+@pytest.mark.parametrize("dtype_c", ["f32", "bf16"])
+def test_either_form_of_the_general_kernels_arguments(gpu, M, N, K, dtype_ab, dtype_c):
+    """64 x 64 tiles on both sides of the line up to which 16-bit operands have their arguments packed."""
+    a, b, _ = operands(M, N, K, dtype_ab, seed=M + K, b_std=0.05)
+    bias = np.random.default_rng(K).standard_normal(N).astype(np.float32)
+    out, info = run_gemm(a, b, M, N, K, dtype_ab, dtype_c, bias=bias, ldc=N + 3, wg_tile=(64, 64))
+    check(out, G.gemm(a, b, _DT[dtype_ab], _DT[dtype_c], bias=bias), dtype_c, N,
+          bar=1e-5 if dtype_c == "f32" else REL_L2_BAR)
+    pad = out[:, N:]
+    assert np.isnan(pad).all() if dtype_c == "f32" else (pad == 0x7FC1).all()
