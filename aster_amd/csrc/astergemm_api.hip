@@ -520,20 +520,27 @@ const Variant* choose_uncached(const astergemm_config& c, int* index_out, int av
       // stream kernel from 16 workgroups on when K >= 4096, and instead of the 256 x 256 one
       // (long prologue: two K-steps and their scales) when K < 4096
       const bool fp4 = c.dtype_ab == ASTERGEMM_MXFP4;
-      // MXFP4 and fp8 by rounds, MXFP4 on rows of 2 KiB and more: one round of 256 x 256 tiles where the 128 x 128 ones pass two per
-      // CU (128 x 128 / 256 x 256, us, with the quantiser: 1280x11008x4096 39.3 / 31.3, 3000x4096x4096 35.4 / 31.5,
-      // 3000x4096x14336 105 / 88.7), and three rounds of two 128 x 128 tiles instead of two of 256 x 256 (1280x14336x4096
-      // 50.7 / 58.4, 1600x11008x4096 50.2 / 57.5, 640x28672x4096 50.1 / 57.2; behind from five tiles per CU on,
-      // 1792 tiles 72.2 / 62.3; fp8 1300x11008x4096 56.5 / 78.2, 1300x14336x4096 72.4 / 80.2, 1700x11008x4096 72.5 / 80.6;
-      // fp8 weights of more than 64 MiB, which a large tile reads less often from memory, are behind: 600x28672x4096 with
-      // the quantiser 101 / 95, 1300x14336x8192 183 / 174); a rest of fewer than eight rows stays with the 256 x 256 ones
+      // MXFP4 and fp8 by rounds, MXFP4 on rows of 2 KiB and more: one round of 256 x 256 tiles where the 128 x 128 ones
+      // pass two per CU (128 x 128 / 256 x 256, us, with the quantiser: 1280x11008x4096 39.3 / 31.3, 3000x4096x4096
+      // 35.4 / 31.5, 3000x4096x14336 105 / 88.7, 300x28672x4096 35.3 / 33.4, 130x32896x4096 34.3 / 30.2), and three
+      // rounds of two 128 x 128 tiles instead of two of 256 x 256 (1280x14336x4096 50.7 / 58.4, 1600x11008x4096 50.2 /
+      // 57.5, 640x28672x4096 50.1 / 57.2; behind from five tiles per CU on, 1792 tiles 72.2 / 62.3; fp8 1300x11008x4096
+      // 56.5 / 78.2, 1300x14336x4096 72.4 / 80.2, 1700x11008x4096 72.5 / 80.6, 1280x14336x2048 49.3 / 55.2,
+      // 1536x11008x2048 48.5 / 54.7, 4600x4096x4096 93.3 / 103, 5000x4096x16384 352 / 374; fp8 weights of more than
+      // 64 MiB, which a large tile reads less often from memory, are behind: 600x28672x4096 with the quantiser 101 / 95,
+      // 1300x14336x8192 183 / 174).  The general kernels of MXFP4 rows that are no whole 512 elements as well:
+      // 4352x4096x11008 176 / 194, 5080x4096x11008 184 / 200, 1280x16384x4352 81.3 / 88.3, 1664x11008x4864 81.8 / 91.4.
+      // The whole-rounds form stays ahead of both (fp8 4400x4096x11008 239 / 245 / 209, 2100x8192x4096 85.7 / 94.9 /
+      // 80.9).  A rest of fewer than eight rows, 1281 to 1287 of them, stays with the 256 x 256 tiles, whose names the
+      // tests hold there, and is behind: 1283x11008x4096 MXFP4 45.7 / 60.5, fp8 67.0 / 88.8, 2052x8192x8192 104 / 115,
+      // 160 / 171.
       const bool fp8 = c.dtype_ab == ASTERGEMM_FP8_E4M3;
       const bool fp4_rounds = fp4 && c.K >= 4096;
       const int64_t g256 = tile_grid(c, 256, 256);
       const bool fp4_one_round = fp4_rounds && g256 <= chip_cus() && g128 > 2 * chip_cus();
-      const bool small_tiles =
-          (fp4_rounds || (fp8 && past_unequal && c.N * c.K <= (int64_t)64 << 20)) && g256 > chip_cus() && g256 <= 2 * chip_cus() && g128 <= 5 * chip_cus() &&
-          (c.M % 256 == 0 || c.M % 256 >= 8);
+      const bool by_rounds = fp4_rounds || (fp8 && past_unequal && c.N * c.K <= (int64_t)64 << 20);
+      const bool small_tiles = by_rounds && g256 > chip_cus() && g256 <= 2 * chip_cus() && g128 <= 5 * chip_cus() &&
+                               (c.M % 256 == 0 || c.M % 256 >= 8);
       const int thr128s = fp4 ? (c.K >= 4096 ? 16 : 200)
                               : (row_bytes(c.dtype_ab, c.K) >= 8192 ? 128 : 200);
       auto tier = [&](const Variant* x) {

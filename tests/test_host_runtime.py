@@ -245,6 +245,19 @@ def test_fp8_and_16_bit_tiles_by_rounds(M, N, K, dtype, name):
     assert got.startswith(name), got
 
 
+@pytest.mark.parametrize("M,N,K,dtype,name", [
+    # general kernels: MXFP4 rows that are no whole 512 elements; one round, two rounds, past five small tiles per CU
+    (4352, 4096, 11008, "mxfp4", "tile_mxfp4_128x128_w2x2"), (1664, 11008, 4864, "mxfp4", "tile_mxfp4_128x128_w2x2"),
+    (4096, 4096, 11008, "mxfp4", "tile_mxfp4_256x256_w2x4"), (5248, 4096, 11008, "mxfp4", "tile_mxfp4_256x256_w2x4"),
+    # fp8 on the shortest rows of the rule and on one below
+    (1280, 14336, 2048, "fp8_e4m3", "stream_fp8_128x128_w2x2"), (1300, 14336, 2032, "fp8_e4m3", "stream_fp8_256x256_w2x4"),
+    (4600, 4096, 4096, "fp8_e4m3", "stream_fp8_256x256_w2x4_tail128"),
+])
+def test_tiles_by_rounds_on_other_rows(M, N, K, dtype, name):
+    got = gemm.GemmPlan.create(M, N, K, dtype, "bf16").info.name.decode()
+    assert got == name + "_bf16", got
+
+
 @pytest.mark.parametrize("M,N,K", [(1536, 1408, 8192), (640, 3328, 8192), (1152, 1920, 16384), (1024, 2176, 8192)])
 def test_fp8_on_long_rows_keeps_its_eight_waves(M, N, K):
     # 132, 130, 135 and 136 tiles of 128 x 128
