@@ -333,6 +333,13 @@ def test_fp8_quantiser_one_and_two_launch_forms(n, dtype):
     assert np.array_equal(got[:n], qo) and (got[n:] == 0xAB).all()
 
 
+@pytest.mark.parametrize("n", [2 ** 25 - 1, 2 ** 25, 2 ** 25 + 1029])
+@pytest.mark.parametrize("dtype", ["f32", "bf16"])
+def test_fp8_quantiser_with_two_workgroups_per_cu(n, dtype):
+    """2^25 elements and more: 512 workgroups, 32 on each counter; one below, 256."""
+    test_fp8_quantiser_one_and_two_launch_forms(n, dtype)
+
+
 @pytest.mark.parametrize("case", ["zeros", "nan", "inf", "huge", "tiny", "subnormal", "2^60", "2^-60"])
 @pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
 def test_fp8_quantiser_two_launch_edges(case, dtype):
