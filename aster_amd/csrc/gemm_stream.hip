@@ -209,6 +209,16 @@ int launch_streamr(const GemmArgs& a, int grid, hipStream_t s) {
 //   fp8 80x14336x4096       29.3 / 20.8 / 22.6 / 23.8 / 27.6    fp8 320x28672x4096   66.2 / - / 67.9 / 55.1 / 62.3
 //   fp8 1280x4096x14336     96.3 / - / 117 / 87.6 / 96.3        fp8 944x14336x4096   60.0 / - / - / 71.9 / 63.2
 //   MXFP4 160x4096x14336    45.4 / 28.4                         MXFP4 160x14336x4096 21.5 / 23.2 (240 rows)
+// A third round is not what the count of rows says; own / these:
+//   128 x 128 (up to 128 rows, more than 65536 columns) from 1024 columns of K on: bf16 128x73728x4096 156 / 129,
+//     128x66048x1024 45.2 / 38.9, 128x73728x512 20.6 / 22.8
+//   192 x 128 where the own kernel needs one too (more than two per CU): bf16 1472x11008x4096 135 / 124, 4512x4096x4096
+//     132 / 122, 2184x8192x8192 274 / 246, 560x28672x4096 160 / 137; not 1392x11008x4096 (473 of its tiles) 111 / 117,
+//     1648x9920x4096 110 / 121, 4984x3328x1024 30.8 / 37.1
+//   256 x 128, which reads weights less often: past 132 MiB of them on up to 2048 rows, 720x28672x4096 166 / 153,
+//     1224x17024x4096 160 / 151, 976x20672x14336 (f16) 572 / 528; not 1664x13120x3584 129 / 139, 1288x14336x4096 (f16)
+//     149 / 154, 5264x4096x4096 139 / 144, 2552x7360x8192 268 / 279, 656x28224x1024 40.5 / 42.7, 2552x8192x28672 (f16)
+//     1077 / 1100
 // and, in 16-bit, the 256 x 256 tiles of the row-major kernel: a round of them weighs as 580 rows, more by what M is
 // padded with, and two rounds and more pay where five sixths of the workgroups' places in them are filled (two from
 // 2048 columns: 1920x14336x1024 takes 57.9 / 58.9, 8192x4096x512 40.1 / 40.8).  Own / what this rule took without them /
@@ -241,9 +251,10 @@ inline K8Form k8_form(int dt, int64_t M, int64_t N, int64_t ksteps, int cus) {
     }
     if (own_grid > 700 * cus / 256) return f;
     best = own_grid <= cus ? (fp8 ? 390 : 500) : fp8 ? 700 : own_grid <= 2 * cus ? 1000 : 1200;
+    const bool third[] = {ksteps >= 16, own_grid > 2 * cus, M <= 2048 && N * ksteps * 64 > (int64_t)66 << 20};
     for (int bm : {128, 192, 256}) {
       const int64_t rounds = ((M + bm - 1) / bm * ((N + 127) / 128) + cus - 1) / cus;
-      if (rounds <= 3 && rounds * (bm + 128) < best) best = rounds * (bm + 128), f.tile = bm;
+      if ((rounds <= 2 || (rounds == 3 && third[bm / 64 - 2])) && rounds * (bm + 128) < best) best = rounds * (bm + 128), f.tile = bm;
     }
     const int64_t sq = 580 * ((M + 255) / 256 * 256) / M;
     if (!fp8 && sq_rounds == 1 && sq < best) best = sq, f.tile = 0, f.square = true;

@@ -53,3 +53,29 @@ def test_every_id_describes_sizes_that_no_kernel_takes(queries):
     p = subprocess.run([sys.executable, "-c", WALK], cwd=ROOT, env=dict(os.environ, LD_PRELOAD=queries),
                        capture_output=True, text=True, timeout=300)
     assert p.returncode == 0 and "described" in p.stdout, (p.returncode, p.stdout[-200:], p.stderr[-2000:])
+
+
+TILES = """
+import ctypes
+from aster_amd import _capi
+lib, info = _capi.load(), _capi.KernelInfo()
+for M, N, K, tile in %r:
+    c = _capi.Config()
+    c.M, c.N, c.K = M, N, K
+    c.dtype_ab = c.dtype_c = _capi.BF16
+    c.operand_path = _capi.OPERAND_DIRECT_B_K8
+    assert lib.astergemm_select(ctypes.byref(c), ctypes.byref(info)) == 0
+    assert (info.wg_tile_m, info.wg_tile_n) == tile, (M, N, K, info.wg_tile_m, info.wg_tile_n)
+print("selected")
+"""
+
+
+def test_a_third_round_of_tiles_on_pre_shuffled_weights(queries):
+    own = (128, 256)
+    cases = [(128, 73728, 1024, (128, 128)), (128, 73728, 960, own),
+             (1416, 11008, 4096, (192, 128)), (1400, 11008, 4096, own),           # 516 and 473 tiles of the own kernel
+             (720, 28672, 4096, (256, 128)), (1664, 13120, 3584, own), (2552, 8192, 28672, own),
+             (1288, 14336, 4096, own), (872, 11008, 4096, (192, 128))]            # four rounds and two of 192 x 128
+    p = subprocess.run([sys.executable, "-c", TILES % cases], cwd=ROOT, env=dict(os.environ, LD_PRELOAD=queries),
+                       capture_output=True, text=True, timeout=300)
+    assert p.returncode == 0 and "selected" in p.stdout, (p.returncode, p.stderr[-2000:])
