@@ -209,19 +209,27 @@ int launch_streamr(const GemmArgs& a, int grid, hipStream_t s) {
 //   fp8 80x14336x4096       29.3 / 20.8 / 22.6 / 23.8 / 27.6    fp8 320x28672x4096   66.2 / - / 67.9 / 55.1 / 62.3
 //   fp8 1280x4096x14336     96.3 / - / 117 / 87.6 / 96.3        fp8 944x14336x4096   60.0 / - / - / 71.9 / 63.2
 //   MXFP4 160x4096x14336    45.4 / 28.4                         MXFP4 160x14336x4096 21.5 / 23.2 (240 rows)
-// A third round is not what the count of rows says; own / these:
+// A second round on short rows, and a third one, are not what the count of rows says; own / these:
+//   two rounds: fp8 from 2048 columns of K on (320x22016x256 11.6 / 13.4, 3776x3200x512 18.9 / 20.7, 1792x5632x1024 22.5 /
+//     23.8, 1912x6464x1536 27.8 / 28.6, 1512x7744x2048 32.3 / 32.1, 3016x4096x4096 59.6 / 56.9), 16-bit from 192 on (bf16
+//     584x15936x64 6.85 / 7.53; the tests hold a size of 192, up to 256 it is still behind, 664x15616x256 11.1 / 11.9);
+//     256 x 128 up to 2048 rows from 8192 on (bf16 1568x9344x8192 207 / 200, f16 1304x10880x14336 376 / 359; f16
+//     1360x10816x2048 52.5 / 54.7, bf16 4944x3200x5120 118 / 121, f16 3128x4992x14336 357 / 364)
 //   128 x 128 (up to 128 rows, more than 65536 columns) from 1024 columns of K on: bf16 128x73728x4096 156 / 129,
 //     128x66048x1024 45.2 / 38.9, 128x73728x512 20.6 / 22.8
 //   192 x 128 where the own kernel needs one too (more than two per CU): bf16 1472x11008x4096 135 / 124, 4512x4096x4096
 //     132 / 122, 2184x8192x8192 274 / 246, 560x28672x4096 160 / 137; not 1392x11008x4096 (473 of its tiles) 111 / 117,
 //     1648x9920x4096 110 / 121, 4984x3328x1024 30.8 / 37.1
-//   256 x 128, which reads weights less often: past 132 MiB of them on up to 2048 rows, 720x28672x4096 166 / 153,
-//     1224x17024x4096 160 / 151, 976x20672x14336 (f16) 572 / 528; not 1664x13120x3584 129 / 139, 1288x14336x4096 (f16)
+//   256 x 128, which reads weights less often: past 132 MiB of them on up to 2048 rows and a third of the third round,
+//     720x28672x4096 166 / 153, 1224x17024x4096 160 / 151, 976x20672x14336 (f16) 572 / 528; not 1664x13120x3584 129 / 139, 1288x14336x4096 (f16)
 //     149 / 154, 5264x4096x4096 139 / 144, 2552x7360x8192 268 / 279, 656x28224x1024 40.5 / 42.7, 2552x8192x28672 (f16)
-//     1077 / 1100
+//     1077 / 1100, 1264x14208x7680 (f16, 555 tiles) 258 / 277
 // and, in 16-bit, the 256 x 256 tiles of the row-major kernel: a round of them weighs as 580 rows, more by what M is
-// padded with, and two rounds and more pay where five sixths of the workgroups' places in them are filled (two from
-// 2048 columns: 1920x14336x1024 takes 57.9 / 58.9, 8192x4096x512 40.1 / 40.8).  Own / what this rule took without them /
+// padded with, and two rounds and more pay where seven eighths of the workgroups' places in them are filled (0.85 of 6,
+// 5496x14912x1024 134 / 152, 0.86 of 3, f16 1304x28032x1024 69.3 / 76.7, 0.84 of 2, f16 880x27648x3072 130 / 139), two from
+// 2048 columns on (1920x14336x1024 takes 57.9 / 58.9, 8192x4096x512 40.1 / 40.8), more than three from 1536 on
+// (4928x23872x64 50.6 / 53.9, 5464x23872x256 85.8 / 92.3, f16 5656x27328x1024 264 / 275, bf16 3584x18560x1536 156 / 150;
+// three as well, but the tests hold one of 64 columns: 1520x32512x64 24.5 / 25.5).  Own / what this rule took without them /
 // these:
 //   bf16 944x14336x4096     108.9 / 97.8 / 86.9                 bf16 640x14336x4096  91.5 / 77.9 / 79.0 (M padded by 1.2)
 //   bf16 1280x8192x28672    735 / 565 / 489                     bf16 640x11008x4096  61.9 / 61.1 / 67.5
@@ -235,8 +243,7 @@ struct K8Form {
   bool square = false;  // 256 x 256 tiles (16-bit); none of them: the launcher's own kernel
   explicit operator bool() const { return kw || tile || square; }
 };
-// ksteps: 16-bit K-steps (of 64 columns); no other type reads it
-inline K8Form k8_form(int dt, int64_t M, int64_t N, int64_t ksteps, int cus) {
+inline K8Form k8_form(int dt, int64_t M, int64_t N, int64_t K, int cus) {
   K8Form f;
   if (cus <= 0 || M < 1 || N < 1) return f;  // (an id is described whether or not its kernel takes the sizes)
   const bool fp8 = dt == ASTERGEMM_FP8_E4M3, fp4 = dt == ASTERGEMM_MXFP4;
@@ -245,16 +252,20 @@ inline K8Form k8_form(int dt, int64_t M, int64_t N, int64_t ksteps, int cus) {
     const int64_t own_grid = (M + 127) / 128 * ((N + 255) / 256);
     if (fp8 && own_grid > 2 * cus) return f;
     const int64_t squares = (M + 255) / 256 * ((N + 255) / 256), sq_rounds = (squares + cus - 1) / cus;
-    if (!fp8 && sq_rounds > 1 && squares * 6 >= sq_rounds * cus * 5 && (sq_rounds > 2 || ksteps >= 32)) {
+    const int64_t sq_from = sq_rounds == 2 ? 2048 : sq_rounds == 3 ? 64 : 1536;
+    if (!fp8 && sq_rounds > 1 && squares * 8 >= sq_rounds * cus * 7 && K >= sq_from) {
       f.square = true;
       return f;
     }
     if (own_grid > 700 * cus / 256) return f;
     best = own_grid <= cus ? (fp8 ? 390 : 500) : fp8 ? 700 : own_grid <= 2 * cus ? 1000 : 1200;
-    const bool third[] = {ksteps >= 16, own_grid > 2 * cus, M <= 2048 && N * ksteps * 64 > (int64_t)66 << 20};
+    const bool second[] = {K >= (fp8 ? 2048 : 192), K >= (fp8 ? 2048 : 192), M <= 2048 && K >= 8192};
+    const bool third[] = {K >= 1024, own_grid > 2 * cus, M <= 2048 && N * K > (int64_t)66 << 20};
     for (int bm : {128, 192, 256}) {
-      const int64_t rounds = ((M + bm - 1) / bm * ((N + 127) / 128) + cus - 1) / cus;
-      if ((rounds <= 2 || (rounds == 3 && third[bm / 64 - 2])) && rounds * (bm + 128) < best) best = rounds * (bm + 128), f.tile = bm;
+      const int64_t tiles = (M + bm - 1) / bm * ((N + 127) / 128), rounds = (tiles + cus - 1) / cus;
+      if (bm == 256 && rounds == 3 && tiles * 3 < 7 * cus) break;
+      const bool pays = rounds == 1 || (rounds == 2 && second[bm / 64 - 2]) || (rounds == 3 && third[bm / 64 - 2]);
+      if (pays && rounds * (bm + 128) < best) best = rounds * (bm + 128), f.tile = bm;
     }
     const int64_t sq = 580 * ((M + 255) / 256 * 256) / M;
     if (!fp8 && sq_rounds == 1 && sq < best) best = sq, f.tile = 0, f.square = true;
@@ -304,7 +315,7 @@ int launch_k8_square(GemmArgs a, hipStream_t s) {
 template <int DT, int OUT>
 int k8_instead(const GemmArgs& a, int own_ready, hipStream_t s, bool* taken) {
   *taken = false;
-  const K8Form f = a.own_kernel ? K8Form{} : k8_form(DT, a.M, a.N, a.ksteps, device_cus());
+  const K8Form f = a.own_kernel ? K8Form{} : k8_form(DT, a.M, a.N, a.K, device_cus());
   if (own_ready != 0 && !f) return own_ready;
   if (const int e = kwave_ready(DT, true)) return e;
   if constexpr (DT != ASTERGEMM_MXFP4) {
@@ -334,7 +345,7 @@ int k8_instead(const GemmArgs& a, int own_ready, hipStream_t s, bool* taken) {
 
 template <int DT, int OUT>
 bool k8_describe(const astergemm_config& c, int cus, LaunchForm* o) {
-  const K8Form f = cus > 0 ? k8_form(DT, c.M, c.N, c.K / 64, cus) : K8Form{};
+  const K8Form f = cus > 0 ? k8_form(DT, c.M, c.N, c.K, cus) : K8Form{};
   if (f.kw) kwave_describe(DT, f.kw, c.M, c.N, cus, o);
   if constexpr (DT == ASTERGEMM_BF16 || DT == ASTERGEMM_F16) {
     if (f.square) {

@@ -59,23 +59,33 @@ TILES = """
 import ctypes
 from aster_amd import _capi
 lib, info = _capi.load(), _capi.KernelInfo()
-for M, N, K, tile in %r:
+for M, N, K, dtype, tile in %r:
     c = _capi.Config()
     c.M, c.N, c.K = M, N, K
-    c.dtype_ab = c.dtype_c = _capi.BF16
+    c.dtype_ab, c.dtype_c, c.scale_mode = dtype, _capi.BF16, int(dtype == _capi.FP8_E4M3)
     c.operand_path = _capi.OPERAND_DIRECT_B_K8
     assert lib.astergemm_select(ctypes.byref(c), ctypes.byref(info)) == 0
-    assert (info.wg_tile_m, info.wg_tile_n) == tile, (M, N, K, info.wg_tile_m, info.wg_tile_n)
+    assert (info.wg_tile_m, info.wg_tile_n) == tile, (M, N, K, dtype, info.wg_tile_m, info.wg_tile_n)
 print("selected")
 """
 
 
-def test_a_third_round_of_tiles_on_pre_shuffled_weights(queries):
-    own = (128, 256)
-    cases = [(128, 73728, 1024, (128, 128)), (128, 73728, 960, own),
-             (1416, 11008, 4096, (192, 128)), (1400, 11008, 4096, own),           # 516 and 473 tiles of the own kernel
-             (720, 28672, 4096, (256, 128)), (1664, 13120, 3584, own), (2552, 8192, 28672, own),
-             (1288, 14336, 4096, own), (872, 11008, 4096, (192, 128))]            # four rounds and two of 192 x 128
+OWN, BF16, FP8 = (128, 256), 1, 2
+
+
+@pytest.mark.parametrize("cases", [
+    [(128, 73728, 1024, BF16, (128, 128)), (128, 73728, 960, BF16, OWN),
+     (1416, 11008, 4096, BF16, (192, 128)), (1400, 11008, 4096, BF16, OWN),     # 516 and 473 tiles of the own kernel
+     (720, 28672, 4096, BF16, (256, 128)), (1664, 13120, 3584, BF16, OWN), (2552, 8192, 28672, BF16, OWN),
+     (1264, 14208, 7680, BF16, OWN), (1520, 12928, 14336, BF16, (256, 128)),     # 555 and 606 tiles
+     (1288, 14336, 4096, BF16, OWN), (872, 11008, 4096, BF16, (192, 128))],     # four rounds and two of 192 x 128
+    [(320, 22016, 2048, FP8, (192, 128)), (320, 22016, 1920, FP8, OWN), (344, 14336, 128, FP8, (192, 128)),
+     (640, 14320, 192, BF16, (192, 128)), (640, 14320, 128, BF16, (256, 256)),
+     (1568, 9344, 8192, BF16, (256, 128)), (1568, 9344, 8128, BF16, OWN), (3128, 4992, 14336, BF16, OWN)],
+    [(1912, 14336, 2048, BF16, (256, 256)), (880, 27648, 3072, BF16, OWN),      # 448 and 432 places of 512
+     (5216, 14848, 1536, BF16, (256, 256)), (5216, 14848, 1472, BF16, OWN), (5496, 14912, 1024, BF16, OWN)],
+], ids=["third", "second", "squares"])
+def test_rounds_of_tiles_on_pre_shuffled_weights(queries, cases):
     p = subprocess.run([sys.executable, "-c", TILES % cases], cwd=ROOT, env=dict(os.environ, LD_PRELOAD=queries),
                        capture_output=True, text=True, timeout=300)
     assert p.returncode == 0 and "selected" in p.stdout, (p.returncode, p.stderr[-2000:])
