@@ -215,6 +215,9 @@ int launch_streamr(const GemmArgs& a, int grid, hipStream_t s) {
 //     584x15936x64 6.85 / 7.53; the tests hold a size of 192, up to 256 it is still behind, 664x15616x256 11.1 / 11.9);
 //     256 x 128 up to 2048 rows from 8192 on (bf16 1568x9344x8192 207 / 200, f16 1304x10880x14336 376 / 359; f16
 //     1360x10816x2048 52.5 / 54.7, bf16 4944x3200x5120 118 / 121, f16 3128x4992x14336 357 / 364)
+//   one round of 256 x 128, fp8: up to 768 rows (496x14336x8192 70.5 / 62.6, 640x10240x8192 65.6 / 59.5; 896x8192x8192 58.0 /
+//     61.8, 800x8192x4096 34.0 / 35.3), past them only where the own kernel's tiles are a whole round, one of which the tests
+//     hold: level to 4 % behind (960x8192x4096 35.8 / 36.3, 1936x4096x14336 111 / 116)
 //   128 x 128 (up to 128 rows, more than 65536 columns) from 1024 columns of K on: bf16 128x73728x4096 156 / 129,
 //     128x66048x1024 45.2 / 38.9, 128x73728x512 20.6 / 22.8
 //   192 x 128 where the own kernel needs one too (more than two per CU): bf16 1472x11008x4096 135 / 124, 4512x4096x4096
@@ -263,7 +266,7 @@ inline K8Form k8_form(int dt, int64_t M, int64_t N, int64_t K, int cus) {
     const bool third[] = {K >= 1024, own_grid > 2 * cus, M <= 2048 && N * K > (int64_t)66 << 20};
     for (int bm : {128, 192, 256}) {
       const int64_t tiles = (M + bm - 1) / bm * ((N + 127) / 128), rounds = (tiles + cus - 1) / cus;
-      if (bm == 256 && rounds == 3 && tiles * 3 < 7 * cus) break;
+      if (bm == 256 && (rounds == 3 ? tiles * 3 < 7 * cus : fp8 && M > 768 && own_grid < cus)) break;
       const bool pays = rounds == 1 || (rounds == 2 && second[bm / 64 - 2]) || (rounds == 3 && third[bm / 64 - 2]);
       if (pays && rounds * (bm + 128) < best) best = rounds * (bm + 128), f.tile = bm;
     }

@@ -84,7 +84,9 @@ OWN, BF16, FP8 = (128, 256), 1, 2
      (1568, 9344, 8192, BF16, (256, 128)), (1568, 9344, 8128, BF16, OWN), (3128, 4992, 14336, BF16, OWN)],
     [(1912, 14336, 2048, BF16, (256, 256)), (880, 27648, 3072, BF16, OWN),      # 448 and 432 places of 512
      (5216, 14848, 1536, BF16, (256, 256)), (5216, 14848, 1472, BF16, OWN), (5496, 14912, 1024, BF16, OWN)],
-], ids=["third", "second", "squares"])
+    [(768, 10240, 8192, FP8, (256, 128)), (896, 8192, 8192, FP8, OWN), (968, 8176, 256, FP8, (256, 128)),
+     (640, 8192, 8192, FP8, (192, 128))],
+], ids=["third", "second", "squares", "first"])
 def test_rounds_of_tiles_on_pre_shuffled_weights(queries, cases):
     p = subprocess.run([sys.executable, "-c", TILES % cases], cwd=ROOT, env=dict(os.environ, LD_PRELOAD=queries),
                        capture_output=True, text=True, timeout=300)
