@@ -29,8 +29,7 @@ OBJ_DIR = os.path.join(ROOT, "build", "obj")
 
 # (object stem, source file, extra flags).  gemm_stream.hip holds the variant table of the stream
 # kernels in five parts (bf16, fp8, MXFP4, f16 operands, unequal tile sides) and is compiled once
-# per part, gemm_kwave.hip once per operand type and order
-# of the weights.
+# per part, gemm_kwave.hip once per operand type and order of the weights.
 UNITS = [("gemm_stream_p0", "gemm_stream.hip", ["-DAG_STREAM_PART=0"]),
          ("gemm_stream_p3", "gemm_stream.hip", ["-DAG_STREAM_PART=3"]),
          ("gemm_stream_p2", "gemm_stream.hip", ["-DAG_STREAM_PART=2"]),
@@ -135,7 +134,8 @@ def build_fastcall() -> bool:
     it to the library).  False where there is no C compiler or no Python.h: calls then go through ctypes."""
     cc, include = shutil.which(os.environ.get("CC", "gcc")), sysconfig.get_paths()["include"]
     if cc is None or not os.path.exists(os.path.join(include, "Python.h")):
-        print("aster_fastcall: no C compiler or no Python.h, launches go through ctypes (0.5 us more each)", file=sys.stderr)
+        print("aster_fastcall: no C compiler or no Python.h, launches go through ctypes (0.5 us more each)",
+              file=sys.stderr)
         if os.path.exists(FASTCALL_PATH):
             os.remove(FASTCALL_PATH)
         return False

@@ -54,7 +54,8 @@ __host__ __device__ inline int64_t row_bytes(int dtype, int64_t k) {
 // The same in one 64-byte line, for the kernels of products that a launch is a good part of.  A launch writes its
 // arguments to device memory, across PCIe: one line costs the host 2.9 us, two 3.5, the 144 bytes of GemmArgs 3.6
 // (empty kernels).  Addresses have 48 bits and C's pitch 58 (build_args refuses others), row pitches of A and B 23
-// (validate_problem), in units of 16 bytes 19, with bits 32 ... 57 of C's above them; everything else follows from M, N and K.
+// (validate_problem), in units of 16 bytes 19, with bits 32 ... 57 of C's above them; everything else follows from M,
+// N and K.
 struct PackedArgs {
   uint32_t lo[6];       // A, B, C (K ranges: the workspace), bias, scale_a or mx_a, scale_b or mx_b
   uint16_t hi[6];

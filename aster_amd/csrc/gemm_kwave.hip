@@ -247,13 +247,14 @@ KwaveForm kwave_tile_form(int64_t M, int64_t N, int cus) {
 }
 
 // Tiles of up to 32 x 64 fit one round.  Up to 32 x 32 whatever the row, 16-bit operands: a launch is most of the
-// time, and a K-step per wave group takes less of it than a chain of K-steps in 64 x 64 tiles (general kernel / this, captured
-// and replayed, us: f16 256x256x256 3.7 / 2.75, bf16 17x26x40 2.9 / 2.6, 100x100x384 4.1 / 2.7, 512x500x40 3.1 / 3.1,
-// 512x500x520 4.9 / 3.7).  32 x 64 from three K-steps on (500x1000x40 3.3 / 3.5, x136 3.8 / 3.5, x384 4.35 / 3.85,
-// 2000x200x384 4.3 / 3.8), from nine to sixteen of them only with the tile rows of a panel on one XCD (256x2000x800 5.9 / 4.9;
-// not 800x600x800 5.96 / 6.14).  fp8 on 32 x 32 from nine K-steps on, 32 x 64 from sixteen (600x600x1040 with the
-// quantiser before it 13.1 / 14.3).  Past one round, with 64 x 64 tiles of its own, it is behind on short rows (bf16
-// 777x1001x1032 8.0 / 8.8, 1200x640x1024 6.8 / 7.8, fp8 1200x640x2064 8.4 / 9.7, ahead: bf16 777x1001x4096 17.5 / 16.3).
+// time, and a K-step per wave group takes less of it than a chain of K-steps in 64 x 64 tiles (general kernel / this,
+// captured and replayed, us: f16 256x256x256 3.7 / 2.75, bf16 17x26x40 2.9 / 2.6, 100x100x384 4.1 / 2.7, 512x500x40
+// 3.1 / 3.1, 512x500x520 4.9 / 3.7).  32 x 64 from three K-steps on (500x1000x40 3.3 / 3.5, x136 3.8 / 3.5, x384 4.35
+// / 3.85, 2000x200x384 4.3 / 3.8), from nine to sixteen of them only with the tile rows of a panel on one XCD
+// (256x2000x800 5.9 / 4.9; not 800x600x800 5.96 / 6.14).  fp8 on 32 x 32 from nine K-steps on, 32 x 64 from sixteen
+// (600x600x1040 with the quantiser before it 13.1 / 14.3).  Past one round, with 64 x 64 tiles of its own, it is
+// behind on short rows (bf16 777x1001x1032 8.0 / 8.8, 1200x640x1024 6.8 / 7.8, fp8 1200x640x2064 8.4 / 9.7, ahead:
+// bf16 777x1001x4096 17.5 / 16.3).
 bool kwave_small_product(int dt, int64_t M, int64_t N, int64_t K, int cus) {
   const int64_t m32 = (M + 31) / 32, n64 = (N + 63) / 64, rb = row_bytes(dt, K);
   if (dt == ASTERGEMM_MXFP4 || m32 * n64 > cus) return false;

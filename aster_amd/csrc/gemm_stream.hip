@@ -210,30 +210,31 @@ int launch_streamr(const GemmArgs& a, int grid, hipStream_t s) {
 //   fp8 1280x4096x14336     96.3 / - / 117 / 87.6 / 96.3        fp8 944x14336x4096   60.0 / - / - / 71.9 / 63.2
 //   MXFP4 160x4096x14336    45.4 / 28.4                         MXFP4 160x14336x4096 21.5 / 23.2 (240 rows)
 // A second round on short rows, and a third one, are not what the count of rows says; own / these:
-//   two rounds: fp8 from 2048 columns of K on (320x22016x256 11.6 / 13.4, 3776x3200x512 18.9 / 20.7, 1792x5632x1024 22.5 /
-//     23.8, 1912x6464x1536 27.8 / 28.6, 1512x7744x2048 32.3 / 32.1, 3016x4096x4096 59.6 / 56.9), 16-bit from 192 on (bf16
-//     584x15936x64 6.85 / 7.53; the tests hold a size of 192, up to 256 it is still behind, 664x15616x256 11.1 / 11.9);
-//     256 x 128 up to 2048 rows from 8192 on (bf16 1568x9344x8192 207 / 200, f16 1304x10880x14336 376 / 359; f16
-//     1360x10816x2048 52.5 / 54.7, bf16 4944x3200x5120 118 / 121, f16 3128x4992x14336 357 / 364)
-//   one round of 256 x 128, fp8: up to 768 rows (496x14336x8192 70.5 / 62.6, 640x10240x8192 65.6 / 59.5; 896x8192x8192 58.0 /
-//     61.8, 800x8192x4096 34.0 / 35.3), past them only where the own kernel's tiles are a whole round, one of which the tests
-//     hold: level to 4 % behind (960x8192x4096 35.8 / 36.3, 1936x4096x14336 111 / 116)
+//   two rounds: fp8 from 2048 columns of K on (320x22016x256 11.6 / 13.4, 3776x3200x512 18.9 / 20.7, 1792x5632x1024
+//     22.5 / 23.8, 1912x6464x1536 27.8 / 28.6, 1512x7744x2048 32.3 / 32.1, 3016x4096x4096 59.6 / 56.9), 16-bit from
+//     192 on (bf16 584x15936x64 6.85 / 7.53; the tests hold a size of 192, up to 256 it is still behind,
+//     664x15616x256 11.1 / 11.9); 256 x 128 up to 2048 rows from 8192 on (bf16 1568x9344x8192 207 / 200, f16
+//     1304x10880x14336 376 / 359; f16 1360x10816x2048 52.5 / 54.7, bf16 4944x3200x5120 118 / 121, f16 3128x4992x14336
+//     357 / 364)
+//   one round of 256 x 128, fp8: up to 768 rows (496x14336x8192 70.5 / 62.6, 640x10240x8192 65.6 / 59.5;
+//     896x8192x8192 58.0 / 61.8, 800x8192x4096 34.0 / 35.3), past them only where the own kernel's tiles are a whole
+//     round, one of which the tests hold: level to 4 % behind (960x8192x4096 35.8 / 36.3, 1936x4096x14336 111 / 116)
 //   128 x 128 (up to 128 rows, more than 65536 columns) from 1024 columns of K on: bf16 128x73728x4096 156 / 129,
 //     128x66048x1024 45.2 / 38.9, 128x73728x512 20.6 / 22.8
-//   192 x 128 where the own kernel needs one too (more than two per CU): bf16 1472x11008x4096 135 / 124, 4512x4096x4096
-//     132 / 122, 2184x8192x8192 274 / 246, 560x28672x4096 160 / 137; not 1392x11008x4096 (473 of its tiles) 111 / 117,
-//     1648x9920x4096 110 / 121, 4984x3328x1024 30.8 / 37.1
-//   256 x 128, which reads weights less often: past 132 MiB of them on up to 2048 rows and a third of the third round,
-//     720x28672x4096 166 / 153, 1224x17024x4096 160 / 151, 976x20672x14336 (f16) 572 / 528; not 1664x13120x3584 129 / 139, 1288x14336x4096 (f16)
-//     149 / 154, 5264x4096x4096 139 / 144, 2552x7360x8192 268 / 279, 656x28224x1024 40.5 / 42.7, 2552x8192x28672 (f16)
-//     1077 / 1100, 1264x14208x7680 (f16, 555 tiles) 258 / 277
+//   192 x 128 where the own kernel needs one too (more than two per CU): bf16 1472x11008x4096 135 / 124,
+//     4512x4096x4096 132 / 122, 2184x8192x8192 274 / 246, 560x28672x4096 160 / 137; not 1392x11008x4096 (473 of its
+//     tiles) 111 / 117, 1648x9920x4096 110 / 121, 4984x3328x1024 30.8 / 37.1
+//   256 x 128, which reads weights less often: past 132 MiB of them on up to 2048 rows and a third of the third
+//     round, 720x28672x4096 166 / 153, 1224x17024x4096 160 / 151, 976x20672x14336 (f16) 572 / 528; not
+//     1664x13120x3584 129 / 139, 1288x14336x4096 (f16) 149 / 154, 5264x4096x4096 139 / 144, 2552x7360x8192 268 / 279,
+//     656x28224x1024 40.5 / 42.7, 2552x8192x28672 (f16) 1077 / 1100, 1264x14208x7680 (f16, 555 tiles) 258 / 277
 // and, in 16-bit, the 256 x 256 tiles of the row-major kernel: a round of them weighs as 580 rows, more by what M is
-// padded with, and two rounds and more pay where seven eighths of the workgroups' places in them are filled (0.85 of 6,
-// 5496x14912x1024 134 / 152, 0.86 of 3, f16 1304x28032x1024 69.3 / 76.7, 0.84 of 2, f16 880x27648x3072 130 / 139), two from
-// 2048 columns on (1920x14336x1024 takes 57.9 / 58.9, 8192x4096x512 40.1 / 40.8), more than three from 1536 on
-// (4928x23872x64 50.6 / 53.9, 5464x23872x256 85.8 / 92.3, f16 5656x27328x1024 264 / 275, bf16 3584x18560x1536 156 / 150;
-// three as well, but the tests hold one of 64 columns: 1520x32512x64 24.5 / 25.5).  Own / what this rule took without them /
-// these:
+// padded with, and two rounds and more pay where seven eighths of the workgroups' places in them are filled (0.85 of
+// 6, 5496x14912x1024 134 / 152, 0.86 of 3, f16 1304x28032x1024 69.3 / 76.7, 0.84 of 2, f16 880x27648x3072 130 / 139),
+// two from 2048 columns on (1920x14336x1024 takes 57.9 / 58.9, 8192x4096x512 40.1 / 40.8), more than three from 1536
+// on (4928x23872x64 50.6 / 53.9, 5464x23872x256 85.8 / 92.3, f16 5656x27328x1024 264 / 275, bf16 3584x18560x1536 156
+// / 150; three as well, but the tests hold one of 64 columns: 1520x32512x64 24.5 / 25.5).  Own / what this rule took
+// without them / these:
 //   bf16 944x14336x4096     108.9 / 97.8 / 86.9                 bf16 640x14336x4096  91.5 / 77.9 / 79.0 (M padded by 1.2)
 //   bf16 1280x8192x28672    735 / 565 / 489                     bf16 640x11008x4096  61.9 / 61.1 / 67.5
 //   bf16 8192x4096x14336    721 / 720 / 624 (2 rounds, full)    bf16 1920x11008x4096 149 / 147 / 156 (0.67 of 2)

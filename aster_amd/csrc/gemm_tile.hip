@@ -12,11 +12,11 @@ constexpr int tile_lds_bytes(int dt, int bm, int bn, int stages) {
 }
 
 // 64 x 64 tiles, operands of bytes: the arguments in one line whatever the size (in one line / as GemmArgs, us: MXFP4
-// 512x512x1024 4.28 / 4.6, 256x256x4096 7.50 / 7.95, fp8 512x512x512 with the quantiser 10.5 / 11.2).  16-bit ones where a
-// launch is as long as the kernel (bf16 500x1000x40 3.34 / 3.8, f16 1200x1200x64, 361 tiles, 3.69 / 4.35; bf16
-// 1000x1000x256, 256 tiles of 4 K-steps, level at 4.5); past that the launch is hidden and unpacking stands in front of
-// the K loop (f16 1100x1003x200, 288 tiles of 4, 5.00 / 4.83, bf16 391x6864x288 6.50 / 6.43, 777x1001x1032 8.11 / 8.07).
-// Larger tiles have no such sizes: GemmArgs (bf16 1269x22136x312 49.3 / 48.8).
+// 512x512x1024 4.28 / 4.6, 256x256x4096 7.50 / 7.95, fp8 512x512x512 with the quantiser 10.5 / 11.2).  16-bit ones
+// where a launch is as long as the kernel (bf16 500x1000x40 3.34 / 3.8, f16 1200x1200x64, 361 tiles, 3.69 / 4.35;
+// bf16 1000x1000x256, 256 tiles of 4 K-steps, level at 4.5); past that the launch is hidden and unpacking stands in
+// front of the K loop (f16 1100x1003x200, 288 tiles of 4, 5.00 / 4.83, bf16 391x6864x288 6.50 / 6.43, 777x1001x1032
+// 8.11 / 8.07). Larger tiles have no such sizes: GemmArgs (bf16 1269x22136x312 49.3 / 48.8).
 template <int DT, int BM>
 constexpr bool kTileAlwaysPacks = BM == 64 && (DT == ASTERGEMM_FP8_E4M3 || DT == ASTERGEMM_MXFP4);
 inline bool packs_16_bit(int64_t grid, int ksteps) { return ksteps <= 4 && grid <= 512 && grid * ksteps <= 1024; }
@@ -32,7 +32,8 @@ int tile_ready() {
   static std::atomic<uint64_t> attr_devs{0}, packed_devs{0};
   constexpr int lds = tile_lds_bytes(DT, BM, BN, S);
   if constexpr (BM == 64)
-    if (int e = lds_attr_once(packed_devs, (const void*)gemm_tile_packed_kernel<DT, OUT, BM, BN, WM, WN, S>, lds)) return e;
+    if (int e = lds_attr_once(packed_devs, (const void*)gemm_tile_packed_kernel<DT, OUT, BM, BN, WM, WN, S>, lds))
+      return e;
   if constexpr (!kTileAlwaysPacks<DT, BM>)
     return lds_attr_once(attr_devs, (const void*)gemm_tile_kernel<DT, OUT, BM, BN, WM, WN, S>, lds);
   return 0;

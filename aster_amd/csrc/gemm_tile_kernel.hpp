@@ -99,14 +99,15 @@ __device__ __forceinline__ void map_tile(int bid, int tiles_m, int tiles_n,
   tn = r / rows;
 }
 
-// Workgroup b of `ranges` copies of a grid of `tiles` output tiles -> its K range and its number in the tile
-// grid (what map_tile takes).  A range is on as few XCDs as there are for it (8 / ranges of them, two ranges
-// on each for 16; where its tiles do not divide among them, or the ranges are no power of two, on all).  Its tiles lie side by side there and the XCD's L2 holds the range's rows once for all of them,
-// where with every range on every XCD each reads all of A.  Every range on every XCD / this, us, 128 x 128 tiles:
-// f16 1391x1024x8192 40.6 / 35.1, bf16 900x1024x8192 29.0 / 25.2, 634x1024x8192 25.7 / 23.9, 240x4096x11008 43.8 / 42.7,
-// fp8 558x1024x8192 29.5 / 27.9.  Not for MXFP4 (700x1024x8192 20.5 / 22.2, 162x4096x14336 22.7 / 23.3) and not on
-// 256 x 128 tiles, whose XCDs then stream weights a quarter of the row apart from memory: bf16 324x8192x28672 198 / 211,
-// 333x4096x14336 59.1 / 62.1 (weights in the last-level cache: 54.2 / 54.3).
+// Workgroup b of `ranges` copies of a grid of `tiles` output tiles -> its K range and its number in the tile grid
+// (what map_tile takes).  A range is on as few XCDs as there are for it (8 / ranges of them, two ranges on each for
+// 16; where its tiles do not divide among them, or the ranges are no power of two, on all).  Its tiles lie side by
+// side there and the XCD's L2 holds the range's rows once for all of them, where with every range on every XCD each
+// reads all of A.  Every range on every XCD / this, us, 128 x 128 tiles: f16 1391x1024x8192 40.6 / 35.1, bf16
+// 900x1024x8192 29.0 / 25.2, 634x1024x8192 25.7 / 23.9, 240x4096x11008 43.8 / 42.7, fp8 558x1024x8192 29.5 / 27.9.
+// Not for MXFP4 (700x1024x8192 20.5 / 22.2, 162x4096x14336 22.7 / 23.3) and not on 256 x 128 tiles, whose XCDs then
+// stream weights a quarter of the row apart from memory: bf16 324x8192x28672 198 / 211, 333x4096x14336 59.1 / 62.1
+// (weights in the last-level cache: 54.2 / 54.3).
 __device__ __forceinline__ void place_range(int b, int tiles, int ranges, int& range, int& bid) {
   const int xcds = ranges < 8 ? 8 / ranges : 1;  // XCDs of a range
   const int share = tiles / xcds;                // tiles of a range on one of them
