@@ -46,11 +46,12 @@ def queries(tmp_path_factory):
     (where / "queries.cpp").write_text(QUERIES)
     subprocess.run(["g++", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
                     str(where / "queries.cpp"), "-o", str(where / "queries.so")], check=True)
-    return str(where / "queries.so")
+    preload = [str(where / "queries.so")] + os.environ.get("LD_PRELOAD", "").split()   # before what is preloaded already
+    return dict(os.environ, LD_PRELOAD=" ".join(preload))
 
 
 def test_every_id_describes_sizes_that_no_kernel_takes(queries):
-    p = subprocess.run([sys.executable, "-c", WALK], cwd=ROOT, env=dict(os.environ, LD_PRELOAD=queries),
+    p = subprocess.run([sys.executable, "-c", WALK], cwd=ROOT, env=queries,
                        capture_output=True, text=True, timeout=300)
     assert p.returncode == 0 and "described" in p.stdout, (p.returncode, p.stdout[-200:], p.stderr[-2000:])
 
@@ -88,6 +89,6 @@ OWN, BF16, FP8 = (128, 256), 1, 2
      (640, 8192, 8192, FP8, (192, 128))],
 ], ids=["third", "second", "squares", "first"])
 def test_rounds_of_tiles_on_pre_shuffled_weights(queries, cases):
-    p = subprocess.run([sys.executable, "-c", TILES % cases], cwd=ROOT, env=dict(os.environ, LD_PRELOAD=queries),
+    p = subprocess.run([sys.executable, "-c", TILES % cases], cwd=ROOT, env=queries,
                        capture_output=True, text=True, timeout=300)
     assert p.returncode == 0 and "selected" in p.stdout, (p.returncode, p.stderr[-2000:])
