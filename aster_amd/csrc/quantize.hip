@@ -337,23 +337,29 @@ __global__ __launch_bounds__(1024) void quantize_fp8_kernel(const void* __restri
   if (threadIdx.x == 0) *scale = sc.s;
 }
 
-// Larger ones outside a capture (kFp8OneLaunchUncaptured): one launch, the source read once and kept in
-// registers from the maximum to the codes (the register files hold 128 MB; past 2^25 elements what is left over
-// is read twice).  What bounds it is the way of the maxima through memory, about 2 us, and from 4 M elements on
-// the bytes.  bf16, two launches -> this, back to back: 64 x 4096 7.3 -> 4.9 us, 333 x 4096 7.2 -> 6.3, 500 x
-// 8192 8.7 -> 7.5, 500 x 14336 12.1 -> 9.8, 4096 x 4096 19.0 -> 15.8, 8192 x 4096 31.6 -> 24.2, 8192 x 8192
+// Larger ones outside a capture, on a device of kFp8Slots CUs or more (kFp8OneLaunchUncaptured): one launch, the source
+// read once and kept in registers from the maximum to the codes (a tensor of up to 128 MB is held whole; of a larger one
+// 112 MB are, and the rest is read twice).  What bounds it is the way of the maxima through memory, about 2 us, and from
+// 4 M elements on the bytes.  bf16, two launches -> this, back to back: 64 x 4096 7.3 -> 4.9 us, 333 x 4096 7.2 -> 6.3,
+// 500 x 8192 8.7 -> 7.5, 500 x 14336 12.1 -> 9.8, 4096 x 4096 19.0 -> 15.8, 8192 x 4096 31.6 -> 24.2, 8192 x 8192
 // 73.9 -> 53.9, 8192 x 28672 240 -> 214.  Every workgroup leaves its maximum, with the tag of this launch
 // beside it in the same 8 bytes, in a slot of its own and reads everybody else's (agent scope: past the L2s,
 // which differ from XCD to XCD; a slot says all there is to know, so nothing has to be ordered with it).  No
 // wait depends on another workgroup being there: one that has not seen all slots after `patience` looks up the
-// missing shares in the source itself.
+// missing shares in the source itself, one after the other from a place that each workgroup draws for itself, and leaves
+// what it finds in the slot of the share (what the share's owner will store there).  So where other work holds CUs, the
+// workgroups that run read the shares of those that do not less than one and a half times between them, and those that
+// come later find every slot filled (beside a product of 2.8 ms on 224 CUs, two launches / this: 500 x 14336 60 / 73 us,
+// 4096 x 4096 92 / 143, 8192 x 8192 290 / 550; each workgroup for itself: until the product ends).
 //
 // The slots are kFp8SlotSets sets that launches take in turn.  Nothing is cleared: a tag is used once in 2^33
 // launches, and if two launches that run at the same time should ever share a set, what the one writes over of the
 // other's is looked up in the source as well.  A captured launch would repeat its tag at every replay, so
 // captures get the two launches above.
 constexpr int kFp8Slots = 256, kFp8SlotSets = 64;
-constexpr unsigned kFp8Patience = 5000;  // 50 us of the 100 MHz counter
+// Ticks of the 100 MHz counter before a workgroup gives up: 5 us, and half as long as a CU takes for its share at the
+// rate of a large copy (200 bytes a tick).  With the chip to itself the last maximum is 1 to 6 us behind the first.
+constexpr unsigned fp8_patience(int64_t src_bytes) { return 500 + (unsigned)(src_bytes / (kFp8Slots * 400)); }
 constexpr uint64_t kFp8Tags = ((uint64_t)1 << 33) - 1;
 __device__ uint64_t fp8_slots[kFp8SlotSets][kFp8Slots];
 
@@ -397,46 +403,65 @@ __global__ __launch_bounds__(T) void quantize_fp8_once_kernel(const void* __rest
   m = block_max<T / 64>(m);
   if (tid == 0)
     __hip_atomic_store(slots + blockIdx.x, tag << 31 | m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __shared__ int missing[kFp8Slots];
   bool seen = true;
+  auto look = [&]() {
+    const uint64_t s = __hip_atomic_load(slots + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (s >> 31 != tag) return;
+    const unsigned o = (unsigned)s & 0x7FFFFFFFu;
+    m = o > m ? o : m;
+    seen = true;
+  };
   if (tid < kFp8Slots) {
     const uint64_t began = wall_clock64();
-    seen = tid >= grid;
+    seen = tid >= grid || tid == (int)blockIdx.x;
     while (true) {
-      if (!seen) {
-        const uint64_t s = __hip_atomic_load(slots + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (s >> 31 == tag) {
-          const unsigned o = (unsigned)s & 0x7FFFFFFFu;
-          m = o > m ? o : m;
-          seen = true;
-        }
-      }
+      if (!seen) look();
       if (__all(seen) || wall_clock64() - began >= patience) break;
       __builtin_amdgcn_s_sleep(1);
     }
-    missing[tid] = !seen;
   }
-  if (__syncthreads_or(!seen)) {
-    __shared__ uint64_t late;
-    for (int w = 0; w < grid; ++w) {
-      if (!missing[w]) continue;
+  if (__builtin_amdgcn_readfirstlane(__syncthreads_or(!seen))) {
+    __shared__ int nearest;
+    unsigned mix = blockIdx.x * 0x9E3779B1u;
+    while (true) {
+      const int first = (int)__umulhi(mix, (unsigned)grid);  // another place for each workgroup and share
+      mix = (mix ^ mix >> 15) * 0x85EBCA6Bu + 0x9E3779B1u;
+      if (tid == 0) nearest = grid;
       __syncthreads();
-      if (tid == 0) late = __hip_atomic_load(slots + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (!seen) look();
+      if (!seen) atomicMin(&nearest, (tid - first + grid) % grid);
       __syncthreads();
-      if (late >> 31 == tag) {
-        const unsigned o = (unsigned)late & 0x7FFFFFFFu;
-        m = o > m ? o : m;
-        continue;
-      }
+      const int d = __builtin_amdgcn_readfirstlane(nearest);
+      if (d == grid) break;
+      const int w = (first + d) % grid;
+      constexpr int B = MORE ? 8 : U;  // in flight
       AbsMax<SRC> of_w;
-      for (index k = w * T + tid; k < ng; k += stride) of_w.fold(g[k]);
-      const unsigned b = of_w.bits();
-      m = b > m ? b : m;
-      if (w == 0)
-        for (int64_t k = (int64_t)ng * NE + tid; k < n; k += T) {
-          const unsigned e = __float_as_uint(load1<SRC>(src, k)) & 0x7FFFFFFFu;
-          m = e > m ? e : m;
-        }
+      for (index k = w * T + tid; k < ng; k += B * stride) {
+        i32x4 r[B];
+#pragma unroll
+        for (int b = 0; b < B; ++b) r[b] = g[k + b * stride < ng ? k + b * stride : ng - 1];
+#pragma unroll
+        for (int b = 0; b < B; ++b) of_w.fold(r[b]);
+      }
+      unsigned o = of_w.bits();
+      if (w == 0 && j < n) {
+        const unsigned e = __float_as_uint(load1<SRC>(src, j)) & 0x7FFFFFFFu;
+        o = e > o ? e : o;
+      }
+      o = block_max<T / 64>(o);
+      m = o > m ? o : m;
+      if (tid == 0) __hip_atomic_store(slots + w, tag << 31 | o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (tid == w) seen = true;
+    }
+    // The loads above have the registers of v, which is fetched again, from places that the compiler does not know: it
+    // would keep the first values or their addresses all the same.
+    const i32x4* again = g;
+    index at = i;
+    asm volatile("" : "+s"(again), "+v"(at));
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const index k = at + u * stride;
+      v[u] = again[k < ng ? k : ng - 1];
     }
   }
   const Fp8Scale sc(block_max<T / 64>(m));
@@ -732,7 +757,7 @@ extern "C" int astergemm_quantize_fp8_tensor(const void* dSrc, int src_dtype, in
       return;
     }
     if (once) {
-      launch_fp8_once<SRC>(dSrc, n, dDst, dScale, kFp8Patience, s);
+      launch_fp8_once<SRC>(dSrc, n, dDst, dScale, fp8_patience(n * Src<SRC>::kBytes), s);
       return;
     }
     // one partial maximum per workgroup, a multiple of 32 of them (128 bytes of dst), 1024 at most

@@ -464,6 +464,50 @@ def test_fp8_quantiser_sets_of_maxima_in_turn(dtype):
         assert torch.equal(qs[i], want)
 
 
+def test_fp8_quantiser_beside_a_kernel_that_holds_most_cus():
+    """A product keeps 224 CUs for longer than the quantiser runs: the workgroups that find a place look up the maxima of
+    the others between them, once, and not each for itself.  Against the two launches of a capture, which wait for nobody
+    (1.5 times as long as those; 30 times where every workgroup reads all missing shares); the bytes are the same."""
+    import torch
+    from time import perf_counter
+    n, (M, N, K) = 1 << 24, (3584, 4096, 65536)
+    a, b = (torch.zeros(r, K, device="cuda", dtype=torch.bfloat16) for r in (M, N))
+    c = torch.zeros(M, N, device="cuda", dtype=torch.bfloat16)
+    plan = AG.GemmPlan.create(M, N, K, "bf16", "bf16")
+    assert plan.info.grid_x == 224 and plan.info.lds_bytes == 160 * 1024
+    x = torch.randn(n, device="cuda").to(torch.bfloat16)
+    q = [torch.zeros(n, device="cuda", dtype=torch.uint8) for _ in range(2)]
+    s = torch.zeros(2, device="cuda")
+    busy, stream, graph = torch.cuda.Stream(), torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    call = lambda i: Q.quantize_fp8_tensor_device(x.data_ptr(), n, q[i].data_ptr(), s.data_ptr() + 4 * i, src_dtype="bf16",
+                                                  stream=stream.cuda_stream)
+    with torch.cuda.graph(graph, stream=stream):
+        call(1)
+
+    def replay():
+        with torch.cuda.stream(stream):
+            graph.replay()
+
+    def took(what):
+        torch.cuda.synchronize()
+        plan.run(a.data_ptr(), b.data_ptr(), c.data_ptr(), stream=busy.cuda_stream)
+        began = perf_counter()
+        while perf_counter() - began < 150e-6:      # the product's workgroups have their CUs
+            pass
+        e = [torch.cuda.Event(enable_timing=True) for _ in range(2)]
+        e[0].record(stream)
+        what()
+        e[1].record(stream)
+        torch.cuda.synchronize()
+        return e[0].elapsed_time(e[1])
+
+    print("quantize_fp8_tensor beside a product", flush=True)
+    eager, captured = (min(took(f) for _ in range(6)) for f in (lambda: call(0), replay))
+    assert torch.equal(q[0], q[1]) and s[0] == s[1]
+    assert eager <= 4 * captured, (eager, captured)
+
+
 @pytest.mark.parametrize("rows", [1, 15, 127, 128, 129, 300])
 @pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
 def test_mxfp4_quantiser_lane_order_edges(rows, dtype):
