@@ -777,10 +777,10 @@ extern "C" int astergemm_quantize_fp8_tensor(const void* dSrc, int src_dtype, in
 
 extern "C" int astergemm_diag_quantize_fp8(const void* dSrc, int src_dtype, int64_t n, uint8_t* dDst, float* dScale,
                                            unsigned patience, void* stream) {
-  if (!dSrc || !dDst || !dScale || n <= kFp8OneLaunch || (((uintptr_t)dSrc) & 15) || (((uintptr_t)dDst) & 3) ||
+  if (!dSrc || !dDst || !dScale || n <= kFp8OneLaunchUncaptured || (((uintptr_t)dSrc) & 15) || (((uintptr_t)dDst) & 3) ||
       !src_ok(src_dtype) || is_capturing((hipStream_t)stream)) {
     set_error("astergemm_diag_quantize_fp8: bad argument (more than %lld elements, no capture, otherwise as for "
-              "astergemm_quantize_fp8_tensor)", (long long)kFp8OneLaunch);
+              "astergemm_quantize_fp8_tensor)", (long long)kFp8OneLaunchUncaptured);
     return ASTERGEMM_EINVAL;
   }
   (void)hipGetLastError();

@@ -517,10 +517,11 @@ int astergemm_weight_config(const astergemm_weight_header* h, int64_t M, int dty
  * contrib/kittens/test/bench/bench_harness.py:31-41) and measures nothing.   */
 int astergemm_diag_mfma_rate(int dtype_ab, const void* dSample, int64_t sample_bytes,
                              int target_ms, double* tflops, void* stream);
-/* astergemm_quantize_fp8_tensor past 131072 elements, outside a capture, with
- * the time (ticks of 10 ns) after which a workgroup stops waiting for the
- * maxima of the others and looks them up in the source: the same bytes with
- * any value, 0 among them.                                                  */
+/* astergemm_quantize_fp8_tensor past 114688 elements, outside a capture and on
+ * 256 CUs or more (the form that reads its source once), with the time (ticks
+ * of 10 ns) after which a workgroup stops waiting for the maxima of the others
+ * and looks them up in the source: the same bytes with any value, 0 among
+ * them.                                                                     */
 int astergemm_diag_quantize_fp8(const void* dSrc, int src_dtype, int64_t n, uint8_t* dDst, float* dScale,
                                 unsigned patience, void* stream);
 

@@ -464,6 +464,57 @@ def test_fp8_quantiser_sets_of_maxima_in_turn(dtype):
         assert torch.equal(qs[i], want)
 
 
+@pytest.mark.parametrize("patience", [0, 5000])
+@pytest.mark.parametrize("dtype,n", [
+    ("bf16", 114689), ("f32", 114691), ("f16", 131072),           # from the first size on that the form takes
+    ("bf16", 1 << 20), ("f32", (1 << 21) + 3), ("bf16", (1 << 23) + 7), ("bf16", (1 << 24) + 5),    # 1 ... 16 groups
+    ("bf16", 3 * (1 << 23)), ("f32", 1 << 24), ("bf16", (1 << 26) + 70003), ("f32", (1 << 25) + 70001),  # 1024 threads
+])
+def test_fp8_quantiser_looks_up_the_maximum_anywhere(dtype, n, patience):
+    """A maximum, an infinity and a NaN in the first, a middle and the last element, in the last whole group and, of a
+    tensor that the registers do not hold, behind what they hold; without patience, so that workgroups look the shares
+    up, and with it: the bytes of the two launches (one up to 131072 elements) of a capture."""
+    import torch
+    src = {"f32": torch.float32, "bf16": torch.bfloat16, "f16": torch.float16}[dtype]
+    per = 4 if dtype == "f32" else 8
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    x = torch.randn(n, generator=g, device="cuda").clamp(-5, 5).to(src)
+    q = [torch.full((n + 16,), 0xAB, device="cuda", dtype=torch.uint8) for _ in range(2)]
+    s = [torch.zeros(1, device="cuda") for _ in range(2)]
+    torch.cuda.synchronize()
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        Q.quantize_fp8_tensor_device(x.data_ptr(), n, q[1].data_ptr(), s[1].data_ptr(), src_dtype=dtype,
+                                     stream=stream.cuda_stream)
+    held = 14 * 256 * 1024 * per
+    for at in [0, n // 2 + 5, n // per * per - 1, n - 1] + ([held + 9, (held + n) // 2] if n > 1 << 25 else []):
+        kept = x[at].clone()
+        for value, scale in ((-9.0, np.float32(9) / np.float32(448)), (float("-inf"), np.inf), (float("nan"), 1.0)):
+            x[at] = value
+            print(f"quantize_fp8_tensor {dtype} n={n} {value} at {at} patience {patience}", flush=True)
+            torch.cuda.synchronize()
+            graph.replay()
+            _capi.check(_capi.load().astergemm_diag_quantize_fp8(
+                x.data_ptr(), _capi.DTYPE_NAMES[dtype], n, q[0].data_ptr(), s[0].data_ptr(), patience, None))
+            torch.cuda.synchronize()
+            assert [v.item() for v in s] == [scale] * 2
+            assert torch.equal(q[0], q[1]) and bool((q[0][n:] == 0xAB).all())
+            q[0][:n].zero_()
+        x[at] = kept
+
+
+def test_the_diagnostic_entry_takes_what_the_form_takes():
+    import torch
+    x, s = torch.ones(114689, device="cuda"), torch.zeros(1, device="cuda")
+    q = torch.zeros(114692, device="cuda", dtype=torch.uint8)
+    run = lambda n: _capi.load().astergemm_diag_quantize_fp8(x.data_ptr(), _capi.DTYPE_NAMES["f32"], n, q.data_ptr(),
+                                                             s.data_ptr(), 100, None)
+    assert run(114688) == -22 and run(114689) == 0
+    torch.cuda.synchronize()
+    assert s.item() == np.float32(1) / np.float32(448) and bool((q[:114689] == 0x7E).all())
+
+
 def test_fp8_quantiser_beside_a_kernel_that_holds_most_cus():
     """A product keeps 224 CUs for longer than the quantiser runs: the workgroups that find a place look up the maxima of
     the others between them, once, and not each for itself.  Against the two launches of a capture, which wait for nobody
