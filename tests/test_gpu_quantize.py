@@ -504,6 +504,53 @@ def test_fp8_quantiser_looks_up_the_maximum_anywhere(dtype, n, patience):
         x[at] = kept
 
 
+@pytest.fixture
+def captured(monkeypatch):
+    """Q.quantize_fp8_tensor_device as a captured call, replayed: one launch up to 131072 elements, two past that,
+    which is what devices of fewer than 256 CUs run as well."""
+    import torch
+    eager = Q.quantize_fp8_tensor_device
+    graphs = []
+
+    def call(*args, **kw):
+        torch.cuda.synchronize()
+        stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            eager(*args, stream=stream.cuda_stream, **kw)
+        for _ in range(2):
+            graph.replay()
+            torch.cuda.synchronize()
+        graphs.append(graph)
+
+    monkeypatch.setattr(Q, "quantize_fp8_tensor_device", call)
+    return graphs
+
+
+@pytest.mark.parametrize("n", [114688, 114689, 131072, 131073, 131080, 262144, 262149, 300007, 524288, 524296, 2097159])
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+def test_fp8_quantiser_sizes_of_the_captured_forms(captured, n, dtype):
+    """Round the limit of the one launch in which every workgroup reads the whole tensor, of 64 workgroups of the second
+    launch (65 count on two levels: past 524288 16-bit elements, 262144 of fp32), whole and broken groups."""
+    test_fp8_quantiser_one_and_two_launch_forms(n, dtype)
+    assert len(captured) == 1
+
+
+@pytest.mark.parametrize("n", [2 ** 25 - 1, 2 ** 25, 2 ** 25 + 1029])
+def test_fp8_quantiser_captured_with_two_workgroups_per_cu(captured, n):
+    """2^25 elements and more: 512 workgroups in the second launch, 32 on each counter; one below, 256."""
+    test_fp8_quantiser_one_and_two_launch_forms(n, "bf16")
+    assert len(captured) == 1
+
+
+@pytest.mark.parametrize("case", ["zeros", "nan", "inf", "huge", "tiny", "subnormal", "2^60", "2^-60"])
+@pytest.mark.parametrize("dtype", ["f32", "bf16", "f16"])
+def test_fp8_quantiser_two_launch_edges_captured(captured, case, dtype):
+    """Scales that are no ordinary ones, the special element in the place of the partial maxima, in the middle and
+    behind the last whole group."""
+    test_fp8_quantiser_two_launch_edges(case, dtype)
+    assert captured
+
+
 def test_the_diagnostic_entry_takes_what_the_form_takes():
     import torch
     x, s = torch.ones(114689, device="cuda"), torch.zeros(1, device="cuda")
