@@ -201,6 +201,35 @@ KwaveForm fewest_rows(int64_t M, int64_t N, int cus, int* rows) {
   return f;
 }
 
+// Whether that is ahead of 128 x 128 tiles past 512 rows, by what either takes, us: one round of small tiles a wave's
+// share of the tile's loads and MFMAs over the row, and what all workgroups bring through the L2s; split K a range's
+// loads and the fp32 planes, to memory and back, one K loop the loads of a whole row, which few columns have in cache.
+// With few columns the planes weigh nothing, and tall tiles, of which 32 rows cover M, leave most CUs without one.
+// Fitted to 1342 sizes of 513 ... 4096 rows on 256 CUs, mean errors 5 % and 3 %.  Of the 1149 of them where K is split
+// 602 are taken, 16 of those by mistake (behind by 1 ... 5 %, one by 9), and 31 left where this was ahead by 3 ... 11 %;
+// by the bytes of the rows alone, 503 of those taken were behind, by up to 111 %.  Tiles of 128 rows are left: behind, or
+// ahead by no more than 15 %.
+bool ahead_past_512_rows(int dt, int64_t M, int64_t N, int64_t K, const KwaveForm& f) {
+  const bool mx = dt == ASTERGEMM_MXFP4;
+  const KwaveShape& t = shapes_of(dt, false)[f.shape];
+  if (t.bm >= 128) return false;
+  const int64_t rb = row_bytes(dt, K), g128 = (M + 127) / 128 * ((N + 127) / 128);
+  const int64_t tiles = (M + t.bm - 1) / t.bm * ((N + f.per - 1) / f.per);
+  // (the conditions of check_stream_splitk)
+  const bool splits = rb % kRowBytes == 0 && rb >= (mx ? 32 : 64) * kRowBytes && (!mx || K % 512 == 0) &&
+                      (M % 8 == 0 || g128 >= 8);
+  const int S = splits ? stream_split_of(g128, rb / kRowBytes, mx) : 0;
+  if (!mx && S == 0) return false;
+  const double rows = rb * 1e-6, tile = (double)t.bm * rows, all = (double)tiles * (t.bm + f.per) * rows;
+  const double own = mx ? 3.81 + 13.6 * tile + 0.206 * t.bn * tile + 0.0352 * all
+                        : 8.45 + 3.3 * tile + 0.118 * t.bn * tile + 0.0211 * all;
+  const double planes = (double)S * M * N * 4e-6;
+  const double other = S == 0 ? (N <= 128 ? 5100 : 6500) * rows
+                     : mx     ? 7.01 + 19.95 * 256 * rows / S + 0.389 * planes
+                              : 10.57 + 12.08 * 256 * rows / S + 0.298 * planes;
+  return own < 0.95 * other;
+}
+
 }  // namespace
 
 // Prompts of a few hundred tokens, 128 x 128 tiles (split K, or one K loop) / this, us:
@@ -215,11 +244,13 @@ KwaveForm fewest_rows(int64_t M, int64_t N, int cus, int* rows) {
 // The lines, measured on 256 CUs: operand rows per CU times their bytes, against tiles that read 256 rows or
 // split K further
 // (bf16 128x4096x14336, 2.8 MB here: 37.4 / 50.0; fp8 200x4096x14336 24.8 / 30.2; MXFP4 333x8192x8192 24.3 / 26.8).
-// More than 512 rows on few columns, operands of bytes, where small tiles are one round and no plane leaves the CUs:
+// More than 512 rows, operands of bytes (ahead_past_512_rows):
 //   fp8   560x1024x8192 19.6 / 17.1, 900x1024x8192 21.1 / 17.4, 1194x1024x8192 25.6 / 21.5, 1500x1024x8192 26.3 / 22.5,
-//         700x2048x8192 25.9 / 21.8; behind: 3000x512x8192 26.6 / 32.2, 1100x1024x16384 (2.6 MB) 32.2 / 37.7
+//         700x2048x8192 25.9 / 21.8; behind: 3000x512x8192 26.6 / 32.2 (nothing below 1024 columns is taken),
+//         1100x1024x16384 (2.6 MB) 32.2 / 37.7, 631x1904x9216 23.9 / 27.7, 762x1256x9216 21.9 / 25.0
 //   MXFP4 560x1024x8192 16.4 / 12.3, 1194x1024x8192 21.1 / 18.3, 2047x1024x8192 23.2 / 21.5, 600x2048x4096 14.2 / 10.6,
-//         1000x1024x4096 14.6 / 9.0, 3000x512x8192 21.9 / 20.3; behind: 800x4096x4096 (216 rows) 14.4 / 17.9
+//         1000x1024x4096 14.6 / 9.0, 3000x512x8192 21.9 / 20.3; behind: 800x4096x4096 (216 rows) 14.4 / 17.9,
+//         3000x64x14336 14.4 / 29.5, 4096x64x8192 13.7 / 23.6, 2047x256x14336 16.6 / 21.2, 4096x64x4096 11.0 / 14.6
 // 16-bit ones are behind from 700 rows on (1194x1024x8192 32.9 / 34.9).
 KwaveForm kwave_prompt_form(int dt, int64_t M, int64_t N, int64_t K, int cus) {
   const int64_t rb = row_bytes(dt, K);
@@ -234,7 +265,7 @@ KwaveForm kwave_prompt_form(int dt, int64_t M, int64_t N, int64_t K, int cus) {
   else if (dt == ASTERGEMM_FP8_E4M3)
     pays = M <= 128 ? own <= 1400000 : M <= 512 ? rows <= 128 && own <= 900000 : rows <= 160 && own <= 1350000;
   else pays = M <= 128 ? own <= 2200000 : rows <= 192 && own <= 1600000;
-  return pays ? f : KwaveForm{};
+  return pays && (M <= 512 || ahead_past_512_rows(dt, M, N, K, f)) ? f : KwaveForm{};
 }
 
 // Small products, general 64 x 64 tile kernel / this, us: bf16 300x300x2048 10.0 / 5.4 (32 x 32),

@@ -87,6 +87,16 @@ def test_k_over_waves_past_512_rows(gpu, M, N, K, dtype_ab, tile):
     test_k_over_waves(gpu, M, N, K, dtype_ab, "bf16", tile)
 
 
+@pytest.mark.parametrize("M,N,K,dtype_ab", [
+    (3000, 64, 14336, "mxfp4"), (4096, 64, 8192, "mxfp4"), (2047, 256, 14336, "mxfp4"), (2560, 16, 8192, "mxfp4"),
+    (4096, 64, 4096, "mxfp4"), (1400, 64, 14336, "mxfp4"), (631, 1904, 9216, "fp8_e4m3"), (762, 1256, 9216, "fp8_e4m3"),
+])
+def test_past_512_rows_where_splitting_k_over_waves_is_behind(gpu, M, N, K, dtype_ab):
+    """Few columns, whose planes weigh nothing, and rows too long for one round: 128 x 128 tiles."""
+    info = AG.GemmPlan.create(M, N, K, dtype_ab, "bf16").info
+    assert (info.wg_tile_m, info.wg_tile_n) == (128, 128), (info.name, info.wg_tile_m, info.wg_tile_n)
+
+
 @pytest.mark.parametrize("M,N,K", [(16, 4096, 14336), (50, 1000, 2304), (100, 200, 1032)])
 def test_non_finite_rows_stay_in_their_row(gpu, M, N, K):
     """The rows past M and N repeat the last one; a NaN there, and an infinity, reach their own row only."""
