@@ -564,7 +564,8 @@ __device__ __forceinline__ void mx4_store(uint8_t* packed, int64_t group, unsign
 // groups per lane lengthen that chain.  bf16, captured and replayed, U = 4 / 2 / 1: 16 x 4096 2.44 / 2.02 /
 // 1.92 us, 64 x 14336 2.5 / 2.2 / 2.0, 500 x 4096 2.8 / 2.4 / 2.2, 500 x 14336 4.7 / 4.1 / 4.1, 4096 x 4096 9.1
 // / 8.0 / 8.3, 8192 x 8192 33.2 / 29.1 / 29.3 (a large copy's rate): one while 2048 workgroups hold the source,
-// two past that.  CONTIG: ld == K, so block t sits at element 32 t and no (row, column) split is needed.
+// past that two, or four (mx4_four_groups).  CONTIG: ld == K, so block t sits at element 32 t and no (row, column)
+// split is needed.
 template <int SRC, bool CONTIG, int U>
 __global__ __launch_bounds__(256) void quantize_mxfp4_kernel(const void* __restrict__ src,
                                                              int64_t nblocks, unsigned bpr,
@@ -607,7 +608,9 @@ __global__ __launch_bounds__(256) void quantize_mxfp4_kernel(const void* __restr
 // written where they fall they are single bytes 256 apart (bf16 4096 x 4096 17.6 -> 10.9 us, 8192 x 8192 60.5
 // -> 32.0).  T threads, which for the same reason are many: 256 / 512 / 1024, captured and replayed, 333 x 4096
 // 5.5 / 4.0 / 3.6, 1024 x 4096 5.9 / 4.2 / 3.8, 1024 x 8192 7.5 / 5.7 / 5.6, 4096 x 4096 10.8 / 9.1 / 9.4, 4096
-// x 14336 27.4 / 27.4 / 27.1, 8192 x 8192 32.6 / 30.2 / 31.9.
+// x 14336 27.4 / 27.4 / 27.1, 8192 x 8192 32.6 / 30.2 / 31.9.  Up to 48 rows (fp32: 32) 256: rows past the end are
+// loaded and encoded too, those of the whole tile with more threads (fp32 1 x 4096 3.4 / - / 4.6, 32 x 4096 3.9 / - /
+// 4.8, 40 x 4096 5.3 / - / 4.8; bf16 1 x 4096 3.6 / - / 3.7, 64 x 4096 4.3 / - / 4.2).
 template <int SRC, int T>
 __global__ __launch_bounds__(T) void quantize_mxfp4_lanes_kernel(const void* __restrict__ src, int rows,
                                                                    unsigned bpr, int64_t ld,
@@ -654,6 +657,18 @@ __global__ __launch_bounds__(T) void quantize_mxfp4_lanes_kernel(const void* __r
         if ((b >> 1) * 16 + (int)(threadIdx.x & 15) < live) dst[b] = sc[threadIdx.x * 16 + b];
     }
   }
+}
+
+// Past one group per lane: four where a trip of all workgroups is more than three fifths full with them, rows with gaps
+// between them, which would otherwise take two trips with half of their loads in flight (bf16, two / four, replayed:
+// 3000 x 4096 of pitch 4104 8.3 / 7.25 us, 1000 x 14336 of 14344 8.7 / 8.3; fp32 4096 x 4096 of 4224 16.1 / 14.7; emptier:
+// bf16 2500 x 8192 of 8200 12.3 / 13.8, fp32 700 x 28672 of 28680 19.0 / 20.5), up to four trips (8192 x 8192 of 8200 and
+// 6000 x 14336 of 14344 level).  Rows without gaps only where two groups leave half of a second trip empty (bf16
+// 3000 x 4096 7.4 / 7.1; 1000 x 14336 7.8 / 8.05).
+bool mx4_four_groups(int64_t groups, bool contig) {
+  const int64_t trip = 4 * 256 * 2048, rest = groups % trip;
+  if (contig) return groups > trip * 59 / 100 && groups <= trip * 78 / 100;
+  return groups <= 4 * trip && (rest == 0 || rest > trip * 3 / 5);
 }
 
 // workgroups of 256 threads for `work_items` thread-items, at most 8 per compute unit
@@ -821,7 +836,8 @@ extern "C" int astergemm_quantize_mxfp4_ex(const void* dSrc, int src_dtype, int6
       auto go = [&](auto kern, int threads) {
         hipLaunchKernelGGL(kern, dim3(grid), dim3(threads), 0, st, dSrc, (int)rows, bpr, ld_src, dPacked, dScales);
       };
-      if (rows * K <= (int64_t)1 << 22) go(quantize_mxfp4_lanes_kernel<SRC, 1024>, 1024);
+      if (rows <= (SRC == ASTERGEMM_F32 ? 32 : 48)) go(quantize_mxfp4_lanes_kernel<SRC, 256>, 256);
+      else if (rows * K <= (int64_t)1 << 22) go(quantize_mxfp4_lanes_kernel<SRC, 1024>, 1024);
       else go(quantize_mxfp4_lanes_kernel<SRC, 512>, 512);
       return;
     }
@@ -834,6 +850,9 @@ extern "C" int astergemm_quantize_mxfp4_ex(const void* dSrc, int src_dtype, int6
     if (groups <= (int64_t)2048 * 256) {
       if (contig) go(quantize_mxfp4_kernel<SRC, true, 1>, 1);
       else go(quantize_mxfp4_kernel<SRC, false, 1>, 1);
+    } else if (mx4_four_groups(groups, contig)) {
+      if (contig) go(quantize_mxfp4_kernel<SRC, true, 4>, 4);
+      else go(quantize_mxfp4_kernel<SRC, false, 4>, 4);
     } else {
       if (contig) go(quantize_mxfp4_kernel<SRC, true, 2>, 2);
       else go(quantize_mxfp4_kernel<SRC, false, 2>, 2);

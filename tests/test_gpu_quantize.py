@@ -662,3 +662,16 @@ def test_mxfp4_quantiser_sizes_of_its_forms(rows, K, ld, dtype, layout):
     assert np.array_equal(scales, np.asarray(want_s).reshape(-1))
     for bf in (a, p, sc):
         bf.free()
+
+
+@pytest.mark.parametrize("rows,K,ld,dtype,layout", [
+    (1, 256, 0, "f32", "lanes128"), (32, 256, 0, "f32", "lanes128"), (33, 512, 520, "f32", "lanes128"),  # 256 threads, 1024
+    (48, 256, 264, "bf16", "lanes128"), (49, 512, 0, "f16", "lanes128"),
+    (2417, 4096, 0, "bf16", "rows"), (3000, 4096, 0, "f16", "rows"), (3195, 4096, 0, "bf16", "rows"),  # two, four, two
+    (1500, 4096, 0, "f32", "rows"),
+    (2457, 4096, 4104, "bf16", "rows"), (2458, 4096, 4104, "bf16", "rows"), (4096, 4096, 4104, "f16", "rows"),
+    (4097, 4096, 4104, "bf16", "rows"), (1300, 4096, 4224, "f32", "rows"), (2049, 4096, 4104, "f32", "rows"),
+])
+def test_mxfp4_quantiser_lines_between_its_forms(rows, K, ld, dtype, layout):
+    """Few rows in lane order, and two groups per lane or four."""
+    test_mxfp4_quantiser_sizes_of_its_forms(rows, K, ld, dtype, layout)
