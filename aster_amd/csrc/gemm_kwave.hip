@@ -205,10 +205,10 @@ KwaveForm fewest_rows(int64_t M, int64_t N, int cus, int* rows) {
 // share of the tile's loads and MFMAs over the row, and what all workgroups bring through the L2s; split K a range's
 // loads and the fp32 planes, to memory and back, one K loop the loads of a whole row, which few columns have in cache.
 // With few columns the planes weigh nothing, and tall tiles, of which 32 rows cover M, leave most CUs without one.
-// Fitted to 1342 sizes of 513 ... 4096 rows on 256 CUs, mean errors 5 % and 3 %.  Of the 1149 of them where K is split
-// 602 are taken, 16 of those by mistake (behind by 1 ... 5 %, one by 9), and 31 left where this was ahead by 3 ... 11 %;
-// by the bytes of the rows alone, 503 of those taken were behind, by up to 111 %.  Tiles of 128 rows are left: behind, or
-// ahead by no more than 15 %.
+// Fitted to 1342 sizes of 513 ... 4096 rows on 256 CUs, mean errors 5 % and 3 %.  Of the 1149 of them where K is
+// split 602 are taken, 16 of those by mistake (behind by 1 ... 5 %, one by 9), and 31 left where this was ahead by
+// 3 ... 11 %; by the bytes of the rows alone, 503 of those taken were behind, by up to 111 %.  Tiles of 128 rows are
+// left: behind, or ahead by no more than 15 %.
 bool ahead_past_512_rows(int dt, int64_t M, int64_t N, int64_t K, const KwaveForm& f) {
   const bool mx = dt == ASTERGEMM_MXFP4;
   const KwaveShape& t = shapes_of(dt, false)[f.shape];

@@ -41,7 +41,7 @@ inline int kwave_prompt(int dt, int out, const GemmArgs& a, int own_ready, hipSt
 // 1024 elements): bf16 2048x4096 57.9 / 52.8, 180 / 159, 18.4 / 18.0; 512x14336 73.1 / 57.5, 184 / 157, 16.9 / 15.8;
 // 1024x8192 57.3 / 52.1, 185 / 155, 18.0 / 17.4; with a K tail 2048x4096x4104 79.0 / 67.0.  fp32 outputs on rows
 // of 2 KiB are behind (f16 2048x4096x1024 21.2 / 21.9).  K loops from step 0 in both for these figures; as AUTO
-// runs them they start by XCD (step_order).
+// runs them they start by XCD, and odd tile rows swap the steps of a pair (step_order).
 inline bool pairs_tiles(int out, int64_t M, int64_t N, int64_t row_bytes, int cus) {
   const int64_t g128 = M / 128 * (N / 128);
   return M % 128 == 0 && N % 128 == 0 && row_bytes >= (out == ASTERGEMM_F32 ? 18 * 128 : 2048) &&

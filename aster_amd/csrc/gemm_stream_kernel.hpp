@@ -286,10 +286,13 @@ __device__ __forceinline__ void stream_mma(const i32x4& a, const i32x4& b, f32x4
 //   * Odd tile rows take the steps of a pair in the other order.  In the same order both tile rows of a panel wait
 //     for the same weights to come from memory, and what a CU reads from L2 queues behind them (a loop of these
 //     transfers alone, 192 x 128 tiles of 333x14336x4096: 47.7 us, activations only 13.4, weights only 25.7); so
-//     each fetches half of them and finds the other half in L2 (39.7).  bf16, three sets of weights in turn:
-//     333x14336x4096 48.2 -> 45.6, 333x11008x4096 43.8 -> 39.2, 200x11008x4096 36.1 -> 32.8, 333x8192x8192 65.3 ->
-//     62.5, 800x4096x11008 84.2 -> 81.9, 500x4096x14336 66.0 -> 64.0; fp8 and weights found in the last-level cache
-//     level.  By tile column as well, or in pairs of pairs: level with this.
+//     each fetches half of them and finds the other half in L2 (39.7).  By where the weights come from, not by their
+//     size: in turn with enough others that none is in the last-level cache, us: bf16 333x14336x4096 (117 MB)
+//     50.2 -> 46.3, 500x8192x4096 (67 MB) 43.6 -> 39.8, 640x4096x4096 (34 MB) 40.8 -> 36.0, 1024x4096x4096 42.6 ->
+//     40.1, 500x4096x14336 (split K) 133 -> 108, fp8 333x14336x4096 (59 MB) 28.0 -> 27.0, 640x4096x4096 (17 MB)
+//     21.9 -> 20.1; level past some 1800 rows.  Where the cache holds them it costs 0 to 6 %: 41.5 -> 42.1, 35.1 ->
+//     35.3, 31.0 -> 31.9, 35.8 -> 37.9, 80.5 -> 80.7, fp8 23.4 -> 24.3, 17.5 -> 17.7.  A line on the weights' bytes
+//     would part neither.  By tile column as well, or in pairs of pairs: level with this.
 // So which XCD and tile row a row of A is in decides the order of its fp32 sums, and equal rows may differ in the last
 // bits from one row of tiles to another; the bits of a config are the same on every run.
 struct StepOrder {

@@ -9,7 +9,8 @@
 // NaN and infinities to S|0x7F, signed zero), with the subnormal range rounded to nearest
 // even as the hardware converter does.  The MX block format is the one the scaled MFMA
 // expects (v_mfma_scale_f32_16x16x128_f8f6f4, e8m0 scale per 32 K-elements).
-// Both are HBM-bound byte work: one pass over the source (two for the per-tensor scale).
+// Both are HBM-bound byte work: one pass over the source, for the per-tensor scale where the register files hold it and
+// the launch is not captured, two elsewhere.
 #include <type_traits>
 
 #include "astergemm_internal.h"
@@ -262,9 +263,10 @@ __global__ __launch_bounds__(1024) void quantize_fp8_small_kernel(const void* __
     for (int j = ng * NE + threadIdx.x; j < n; j += 1024) dst[j] = (uint8_t)sc.code(load1<SRC>(src, j));
 }
 
-// Larger ones inside a capture in two launches (outside: quantize_fp8_once_kernel below).  The first leaves one maximum
-// per workgroup in the first 4 * gridDim.x bytes of dst (written over by the codes in the end) and clears the
-// counters of the second: *scale, and kFp8Counters of them behind the partial maxima.
+// Larger ones inside a capture, and on devices of fewer than kFp8Slots CUs, in two launches (elsewhere:
+// quantize_fp8_once_kernel below).  The first leaves one maximum per workgroup in the first 4 * gridDim.x bytes of dst
+// (written over by the codes in the end) and clears the counters of the second: *scale, and kFp8Counters of them behind
+// the partial maxima.
 constexpr int kFp8Counters = 16, kFp8CounterPitch = 32;  // a counter every 128 bytes of dst
 constexpr int kFp8CounterBytes = kFp8Counters * kFp8CounterPitch * 4;
 
@@ -337,20 +339,20 @@ __global__ __launch_bounds__(1024) void quantize_fp8_kernel(const void* __restri
   if (threadIdx.x == 0) *scale = sc.s;
 }
 
-// Larger ones outside a capture, on a device of kFp8Slots CUs or more (kFp8OneLaunchUncaptured): one launch, the source
-// read once and kept in registers from the maximum to the codes (a tensor of up to 128 MB is held whole; of a larger one
-// 112 MB are, and the rest is read twice).  What bounds it is the way of the maxima through memory, about 2 us, and from
-// 4 M elements on the bytes.  bf16, two launches -> this, back to back: 64 x 4096 7.3 -> 4.9 us, 333 x 4096 7.2 -> 6.3,
-// 500 x 8192 8.7 -> 7.5, 500 x 14336 12.1 -> 9.8, 4096 x 4096 19.0 -> 15.8, 8192 x 4096 31.6 -> 24.2, 8192 x 8192
-// 73.9 -> 53.9, 8192 x 28672 240 -> 214.  Every workgroup leaves its maximum, with the tag of this launch
-// beside it in the same 8 bytes, in a slot of its own and reads everybody else's (agent scope: past the L2s,
-// which differ from XCD to XCD; a slot says all there is to know, so nothing has to be ordered with it).  No
-// wait depends on another workgroup being there: one that has not seen all slots after `patience` looks up the
-// missing shares in the source itself, one after the other from a place that each workgroup draws for itself, and leaves
-// what it finds in the slot of the share (what the share's owner will store there).  So where other work holds CUs, the
-// workgroups that run read the shares of those that do not less than one and a half times between them, and those that
-// come later find every slot filled (beside a product of 2.8 ms on 224 CUs, two launches / this: 500 x 14336 60 / 73 us,
-// 4096 x 4096 92 / 143, 8192 x 8192 290 / 550; each workgroup for itself: until the product ends).
+// Larger ones outside a capture, on a device of kFp8Slots CUs or more (kFp8OneLaunchUncaptured): one launch, the
+// source read once and kept in registers from the maximum to the codes (a tensor of up to 128 MB is held whole; of a
+// larger one 112 MB are, and the rest is read twice).  What bounds it is the way of the maxima through memory, about
+// 2 us, and from 4 M elements on the bytes.  bf16, two launches -> this, back to back: 64 x 4096 7.3 -> 4.8 us,
+// 500 x 8192 8.7 -> 7.4, 500 x 14336 12.1 -> 9.6, 4096 x 4096 19.5 -> 16.1, 8192 x 4096 31.4 -> 24.5, 8192 x 8192
+// 70.6 -> 54.2, 8192 x 28672 240 -> 214.  Every workgroup leaves its maximum, with the tag of this launch beside it in
+// the same 8 bytes, in a slot of its own and reads everybody else's (agent scope: past the L2s, which differ from XCD
+// to XCD; a slot says all there is to know, so nothing has to be ordered with it).  No wait depends on another workgroup
+// being there: one that has not seen all slots after `patience` looks up the missing shares in the source itself, one
+// after the other from a place that each workgroup draws for itself, and leaves what it finds in the slot of the share
+// (what the share's owner will store there).  So where other work holds CUs, the workgroups that run read the shares of
+// those that do not less than one and a half times between them, and those that come later find every slot filled
+// (beside a product of 2.8 ms on 224 CUs, two launches / this: 500 x 14336 60 / 73 us, 4096 x 4096 92 / 143, 8192 x
+// 8192 290 / 550; each workgroup for itself: until the product ends).
 //
 // The slots are kFp8SlotSets sets that launches take in turn.  Nothing is cleared: a tag is used once in 2^33
 // launches, and if two launches that run at the same time should ever share a set, what the one writes over of the
@@ -659,12 +661,12 @@ __global__ __launch_bounds__(T) void quantize_mxfp4_lanes_kernel(const void* __r
   }
 }
 
-// Past one group per lane: four where a trip of all workgroups is more than three fifths full with them, rows with gaps
-// between them, which would otherwise take two trips with half of their loads in flight (bf16, two / four, replayed:
-// 3000 x 4096 of pitch 4104 8.3 / 7.25 us, 1000 x 14336 of 14344 8.7 / 8.3; fp32 4096 x 4096 of 4224 16.1 / 14.7; emptier:
-// bf16 2500 x 8192 of 8200 12.3 / 13.8, fp32 700 x 28672 of 28680 19.0 / 20.5), up to four trips (8192 x 8192 of 8200 and
-// 6000 x 14336 of 14344 level).  Rows without gaps only where two groups leave half of a second trip empty (bf16
-// 3000 x 4096 7.4 / 7.1; 1000 x 14336 7.8 / 8.05).
+// Past one group per lane: four where a trip of all workgroups is more than three fifths full with them, rows with
+// gaps between them, which would otherwise take two trips with half of their loads in flight (bf16, two / four,
+// replayed: 3000 x 4096 of pitch 4104 8.3 / 7.25 us, 1000 x 14336 of 14344 8.7 / 8.3; fp32 4096 x 4096 of 4224 16.1 /
+// 14.7; emptier: bf16 2500 x 8192 of 8200 12.3 / 13.8, fp32 700 x 28672 of 28680 19.0 / 20.5), up to four trips
+// (8192 x 8192 of 8200 and 6000 x 14336 of 14344 level).  Rows without gaps only where two groups leave half of a
+// second trip empty (bf16 3000 x 4096 7.4 / 7.1; 1000 x 14336 7.8 / 8.05).
 bool mx4_four_groups(int64_t groups, bool contig) {
   const int64_t trip = 4 * 256 * 2048, rest = groups % trip;
   if (contig) return groups > trip * 59 / 100 && groups <= trip * 78 / 100;
@@ -678,9 +680,10 @@ int blocks_for(int64_t work_items) {
 }
 
 // Up to this many elements every workgroup reads the whole source for the maximum: against two launches (bf16, back to
-// back: 65536 elements 4.1 / 6.8 us, 229376 7.5 / 6.8), and against quantize_fp8_once_kernel, which captures do not get
-// (with the product behind it: 16x14336x4096 14.5 / 15.0, 7x4096x14336 15.5 / 16.1, 12x8192x8192 17.4 / 16.5; past the
-// line 31x14336x4096 17.7 / 16.0, 9x4096x14336 17.4 / 15.7, 16x8192x8192 17.1 / 16.6).
+// back: 65536 elements 4.1 / 6.8 us, 229376 7.5 / 6.8), and against quantize_fp8_once_kernel, which captures do not
+// get (with the product behind it: 65536 elements, 16x14336x4096, 14.5 / 15.0).  Between 98304 and 114688 either is
+// ahead, by the product behind it (12x8192x8192, 98304, 17.4 / 16.5; 7x4096x14336, 100352, 15.5 / 16.1); past the line
+// that form was at each size measured (31x14336x4096 17.7 / 16.0, 9x4096x14336 17.4 / 15.7, 16x8192x8192 17.1 / 16.6).
 constexpr int64_t kFp8OneLaunch = 131072, kFp8OneLaunchUncaptured = 114688;
 
 }  // namespace

@@ -405,6 +405,12 @@ int astergemm_shuffle_scales_e8m0_lanes128(const uint8_t* src, uint8_t* dst, int
  * zero; the subnormal range rounds to nearest even.  *dScale is what
  * astergemm_operands.dScaleA / dScaleB take.  dDst 4-byte aligned.
  *
+ * Past 114688 elements, outside a capture and on 256 CUs or more, one launch
+ * reads the source once; its workgroups exchange their maxima, and what has
+ * not arrived after a few microseconds is looked up in the source: where other
+ * work holds CUs the call takes up to twice the time of the two launches that
+ * captures get, which wait for nobody.  The bytes are the same.
+ *
  * astergemm_quantize_mxfp4: rows x K elements (row stride ld_src elements,
  * 0 = K) -> dPacked[rows, K/2] (element 2j in the low nibble of byte j) and
  * dScales[rows, K/32] e8m0 bytes, the operand layout of the scaled MFMA
